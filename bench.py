@@ -50,8 +50,8 @@ METRIC = "force evals/s @512 H2O, mixed vs FP64 (same GPU, ΔF≤1e-5) + p99 ser
 FLOP_DIMER = 31600      # algorithmic FLOP per 2B dimer (value + gradient)
 FLOP_TRIMER = 113100    # algorithmic FLOP per 3B trimer (value + gradient)
 PEAK_FP64 = 78.6        # TFLOP/s, MI355X FP64 (vector and matrix peaks are equal)
-FLOP_SFAC = 12         # FLOP per (k vector, site) of the Ewald structure factors: the six multiply-adds of
-                       # mu_a cos(k.r) and mu_a sin(k.r) into S(k); the phase recurrence is not counted
+FLOP_SFAC = 8          # FLOP per (k vector, site) of the Ewald structure factors as matrix products: for the real
+                       # and the imaginary part one multiply-add with (l alpha + m beta) and one with gamma
 # HBM bytes per launch of k_el_sfac<false> at this workload, from rocprofv3 --pmc FETCH_SIZE /
 # WRITE_SIZE (KiB per dispatch) scaled by the same counters on a plain 512 MiB copy (FETCH x 2,
 # WRITE x 1); profiles/k_el_sfac_bench512_traffic.md
@@ -374,7 +374,7 @@ def main():
     kvec = int(ctx.elec_details()["k_vectors"])
     reps = max(5, min(args.steps, 20))
     _, ms_k3 = ctx.time_forces(reps)
-    ms_sf, flop_sf_lib = ctx.time_elec(reps)
+    ms_sf, _ = ctx.time_elec(reps)
     tf_k3 = nt * FLOP_TRIMER / (ms_k3 * 1e-3) / 1e12
     # algorithmic work of one launch: FLOP_SFAC per (k vector, polarizable site)
     flop_sf = FLOP_SFAC * kvec * box.nreal
@@ -549,17 +549,16 @@ def main():
                    "single_ms_heat_flux": 1e3 * parts["heat"] / args.steps,
                    "k_pip3b_ms": ms_k3, "k_pip3b_tflops": tf_k3, "k_pip3b_frac": tf_k3 / PEAK_FP64,
                    "sfac_launches_per_step": n_sfac},
-        "roofline": {"bound": "fp64-valu", "engine": "FP64 vector ALU (no dense contraction, so no MFMA; peak "
-                                                     "78.6 TFLOP/s)",
-                     "kernel": "k_el_sfac<false> (dipole structure factors, launched once per solver iteration)",
+        "roofline": {"bound": "fp64-mfma", "engine": "FP64 matrix cores (v_mfma_f64_16x16x4; FP64 vector and matrix "
+                                                     "peaks are equal, 78.6 TFLOP/s)",
+                     "kernel": "k_rs_sfac<2> (dipole structure factors, launched once per solver iteration)",
                      "achieved": achieved, "peak": PEAK_FP64, "unit": "TFLOP/s", "frac": achieved / PEAK_FP64,
                      "traffic": SFAC_TRAFFIC_BYTES,
                      "traffic_source": "copied from profiles/k_el_sfac_bench512_traffic.md (rocprofv3 --pmc FETCH_SIZE "
                                        "and WRITE_SIZE of this workload and build, scaled by a plain copy), bytes "
                                        "per launch; not measured in this run",
                      "kernel_ms": ms_sf, "flop_per_launch": flop_sf,
-                     "flop_per_unit": FLOP_SFAC, "units_per_launch": f"{kvec} k vectors x {box.nreal} sites",
-                     "frac_with_recurrence": flop_sf_lib / (ms_sf * 1e-3) / 1e12 / PEAK_FP64},
+                     "flop_per_unit": FLOP_SFAC, "units_per_launch": f"{kvec} k vectors x {box.nreal} sites"},
     }
     if not args.no_cpu:
         # in a child process that never touches the GPU (its all-core leg forks workers)

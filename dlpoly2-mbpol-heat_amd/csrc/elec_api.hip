@@ -15,32 +15,11 @@
 
 #define R4PIE0 138935.4835
 #define SQRPI 1.7724538509055159
-#ifndef EL_DCHUNK_MAX
-#define EL_DCHUNK_MAX 32      // site chunks of the dipole structure-factor pass (partials re-read by the sum)
-#endif
-#ifndef EL_SPLIT
-#define EL_SPLIT 2  // threads per k run in the structure-factor pass (elec_kernels.hip)
-#endif
 #ifndef EL_KCHUNK_WAVES
-#define EL_KCHUNK_WAVES 4096  // site-block x k-chunk product the reciprocal field passes aim at
+#define EL_KCHUNK_WAVES 4096  // site-block x k-chunk product the final reciprocal pass aims at
 #endif
 #ifndef EL_KCHUNK_RUNS
-#define EL_KCHUNK_RUNS 32     // at most this many k runs per chunk of the site-parallel passes
-#endif
-#ifndef EL_FCHUNK_WAVES
-#define EL_FCHUNK_WAVES 3072  // wavefronts the reciprocal field passes aim at
-#endif
-#ifndef EL_FCHUNK_RUNS
-#define EL_FCHUNK_RUNS 48     // at most this many k runs per chunk of the field passes
-#endif
-#ifndef EL_KG
-#define EL_KG 4               // run groups (wavefronts) per field block (elec_kernels.hip)
-#endif
-#ifndef EL_DCHUNK_WAVES
-#define EL_DCHUNK_WAVES 3072  // wavefronts the structure-factor passes aim at
-#endif
-#ifndef EL_SG
-#define EL_SG 4               // site groups (wavefronts) per structure-factor block (elec_kernels.hip)
+#define EL_KCHUNK_RUNS 32     // at most this many k runs per chunk of the final reciprocal pass
 #endif
 #define PI_D 3.141592653589793
 
@@ -106,10 +85,11 @@ void free_buffers(ElecBuffers& E)
     dfree(E.x); dfree(E.y); dfree(E.z); dfree(E.chge); dfree(E.polr); dfree(E.polr2); dfree(E.dg); dfree(E.tab);
     dfree(E.nbrA); dfree(E.cntA); dfree(E.nbrP); dfree(E.cntP); dfree(E.tens); dfree(E.tin);
     dfree(E.dip); dfree(E.dip0); dfree(E.efk); dfree(E.emu); dfree(E.efdc); dfree(E.efdd);
-    dfree(E.cg_p); dfree(E.cg_q); dfree(E.cg_r); dfree(E.cg_z); dfree(E.cg_minv); dfree(E.cg_tmu); dfree(E.cg_smu); dfree(E.cgblk);
-    dfree(E.cg_u); dfree(E.cg_w); dfree(E.cg_m); dfree(E.cg_s); dfree(E.cg_sp); dfree(E.cg_su); dfree(E.cg_sq); dfree(E.ksum); dfree(E.state); dfree(E.zero_state);
-    dfree(E.kv); dfree(E.klmn); dfree(E.runs); dfree(E.runk); dfree(E.phc); dfree(E.phs);
-    dfree(E.S); dfree(E.Spart); dfree(E.Sq); dfree(E.kc); dfree(E.kf); dfree(E.Fpart);
+    dfree(E.cg_p); dfree(E.cg_q); dfree(E.cg_r); dfree(E.cg_z); dfree(E.cg_minv); dfree(E.cg_tmu); dfree(E.cgblk);
+    dfree(E.cg_u); dfree(E.cg_w); dfree(E.cg_m); dfree(E.cg_s); dfree(E.ksum); dfree(E.state); dfree(E.zero_state);
+    dfree(E.kv); dfree(E.runs); dfree(E.runk); dfree(E.phc); dfree(E.phs); dfree(E.pht);
+    dfree(E.rs_pair); dfree(E.rs_ak); dfree(E.rs_kpos);
+    dfree(E.Spart); dfree(E.kf); dfree(E.Fpart);
     dfree(E.vk); dfree(E.vr); dfree(E.vs); dfree(E.vc); dfree(E.vdck); dfree(E.vdcr); dfree(E.vesp);
     dfree(E.fk); dfree(E.f2); dfree(E.f3); dfree(E.fsite); dfree(E.e1); dfree(E.e2); dfree(E.e3); dfree(E.ep);
     dfree(E.s1); dfree(E.w2); dfree(E.w3); dfree(E.fmsum); dfree(E.fmx); dfree(E.eout); dfree(E.wout);
@@ -203,6 +183,76 @@ int build_table(ElecState& S, double alpha, double rcut, std::string& err)
     return 0;
 }
 
+// The plan of the matrix passes (RsPlan) of the k list kv / klm: its (l, m) pairs by falling
+// largest |n| in groups of 16, the Ewald weights of (pair, +-n), where each k's sums lie, and
+// the site chunks.
+int build_rs(ElecState& S, const double* rc, const int* kmax, const std::vector<double>& kv,
+             const std::vector<int>& klm, std::string& err)
+{
+    ElecBuffers& E = S.E;
+    RsPlan& R = E.rs;
+    const int K = E.K;
+    struct Pair {
+        int l, m, nmax, first, last;   // k's [first, last)
+    };
+    std::vector<Pair> pr;
+    for (int k = 0; k < K; ++k) {
+        const int l = klm[3 * k], m = klm[3 * k + 1], n = std::abs(klm[3 * k + 2]);
+        if (pr.empty() || pr.back().l != l || pr.back().m != m) pr.push_back({l, m, 0, k, k});
+        pr.back().nmax = std::max(pr.back().nmax, n);
+        pr.back().last = k + 1;
+    }
+    std::stable_sort(pr.begin(), pr.end(), [](const Pair& a, const Pair& b) { return a.nmax > b.nmax; });
+    R.ng = std::max(1, ((int)pr.size() + 15) / 16);
+    R.ntiles = pr.empty() ? 1 : std::max(1, (pr[0].nmax + 7) / 8);
+    R.ky = kmax[0] + 1 + kmax[1];
+    R.kz = R.ky + kmax[1] + 1;
+    R.kt = R.kz + kmax[2] + 1;
+    for (int i = 0; i < 9; ++i) R.rc[i] = rc[i];
+    const int nn = 8 * R.ntiles + 1;
+    std::vector<int4> pair((size_t)16 * R.ng, make_int4(0, 0, 0, 0));
+    std::vector<double2> ak((size_t)16 * R.ng * nn, make_double2(0.0, 0.0));
+    std::vector<int> kpos(K);
+    for (size_t p = 0; p < pr.size(); ++p) {
+        // (the first pair of a group has its largest n)
+        pair[p] = make_int4(pr[p].l, pr[p].m, pr[p].nmax, (pr[p - p % 16].nmax + 7) / 8);
+        for (int k = pr[p].first; k < pr[p].last; ++k) {
+            const int n = klm[3 * k + 2], an = std::abs(n);
+            double2& a = ak[p * nn + an];
+            (n < 0 ? a.y : a.x) = kv[8 * (size_t)k + 3];
+            kpos[k] = (int)(p << 8) | (an << 1) | (n < 0);
+        }
+    }
+    // Site chunks: 8, one per XCD (blocks are dealt to the XCDs in turn, chunks fastest), or the
+    // next multiple of 8 that keeps a chunk's weights in LDS (RS_MAX_SPC); fewer where a chunk
+    // would be under 32 sites, a step of four for each of the 8 wavefronts.
+    auto chunks = [&](int n, int& nch, int& spc) {
+        const int want = 8 * ((n + 8 * RS_MAX_SPC - 1) / (8 * RS_MAX_SPC));
+        spc = std::min(RS_MAX_SPC, ((n + want - 1) / want + 31) / 32 * 32);
+        nch = (n + spc - 1) / spc;
+    };
+    chunks(3 * S.nw, R.nch, R.spc);
+    chunks(E.n, R.nchq, R.spcq);
+    dfree(E.rs_pair);
+    dfree(E.rs_ak);
+    dfree(E.rs_kpos);
+    dfree(E.pht);
+    dfree(E.Spart);
+    ECHK(dalloc(&E.rs_pair, pair.size()));
+    ECHK(dalloc(&E.rs_ak, ak.size()));
+    ECHK(dalloc(&E.rs_kpos, kpos.size()));
+    ECHK(dalloc(&E.pht, (size_t)(E.n + RS_PAD) * R.kt));
+    ECHK(dalloc(&E.Spart, (size_t)4 * std::max(R.nch, R.nchq) * R.ng * RS_SLOT(R.ntiles)));
+    ECHK(hipMemcpy(E.rs_pair, pair.data(), sizeof(int4) * pair.size(), hipMemcpyHostToDevice));
+    ECHK(hipMemcpy(E.rs_ak, ak.data(), sizeof(double2) * ak.size(), hipMemcpyHostToDevice));
+    ECHK(hipMemcpy(E.rs_kpos, kpos.data(), sizeof(int) * kpos.size(), hipMemcpyHostToDevice));
+    R.pair = E.rs_pair;
+    R.ak = E.rs_ak;
+    R.kpos = E.rs_kpos;
+    E.fchunks = R.ng;
+    return 0;
+}
+
 // k vectors of ewald1p.f:151-159, 248-345 in the reference's order (l = 0..kmax1, then
 // m, then n, half space), grouped into runs of consecutive n at fixed (l, m).
 int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha, std::string& err)
@@ -242,7 +292,7 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
     const double ralph = -0.25 / (alpha * alpha);
 
     std::vector<double> kv;
-    std::vector<int> runs, runk, klmn;
+    std::vector<int> runs, runk, klm;   // klm: l, m, n of every k
     if (kmax[0] + kmax[1] + kmax[2] + 3 > 80) {
         err = "kmax1 + kmax2 + kmax3 above 77 is not supported";
         return -1;
@@ -270,7 +320,8 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
                 const double akv2 = 2.0 * (rrksq - ralph);
                 const double rec[8] = {k0, k1, k2, akk, akv, akv2, 0.0, 0.0};
                 kv.insert(kv.end(), rec, rec + 8);
-                klmn.push_back((ll << 16) | ((mm + 128) << 8) | (nn + 128));
+                const int lmn[3] = {ll, mm, nn};
+                klm.insert(klm.end(), lmn, lmn + 3);
                 if (run_open < 0 || runs[4 * run_open + 3] == 8) {
                     run_open = (int)runk.size();
                     const int r4[4] = {ll, mm, nn, 0};
@@ -285,53 +336,23 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
         mmin = -kmax[1];
     }
     dfree(E.kv);
-    dfree(E.klmn);
     dfree(E.runs);
     dfree(E.runk);
-    dfree(E.S);
-    dfree(E.Sq);
-    dfree(E.kc);
     dfree(E.kf);
-    dfree(E.Spart);
     E.K = K;
     E.nrun = (int)runk.size();
     ECHK(dalloc(&E.kv, kv.size()));
     ECHK(dalloc(&E.runs, runs.size()));
     ECHK(dalloc(&E.runk, runk.size()));
     ECHK(hipMemcpy(E.kv, kv.data(), sizeof(double) * kv.size(), hipMemcpyHostToDevice));
-    ECHK(dalloc(&E.klmn, klmn.size()));
-    ECHK(hipMemcpy(E.klmn, klmn.data(), sizeof(int) * klmn.size(), hipMemcpyHostToDevice));
     ECHK(hipMemcpy(E.runs, runs.data(), sizeof(int) * runs.size(), hipMemcpyHostToDevice));
     ECHK(hipMemcpy(E.runk, runk.data(), sizeof(int) * runk.size(), hipMemcpyHostToDevice));
-    // site chunks of the structure-factor passes (their partials are re-read by the chunk
-    // sum): about EL_DCHUNK_WAVES wavefronts, EL_SG per block of 64 half-runs, and at least
-    // 64 sites per chunk
-    const int rblocks = (EL_SPLIT * E.nrun + 63) / 64;
-    const int nrow = 3 * S.nw;
-    E.schunks = std::max(1, std::min(16, std::min((E.n + 63) / 64, EL_DCHUNK_WAVES / (EL_SG * rblocks))));
-    E.dchunks = std::max(1, std::min(EL_DCHUNK_MAX, std::min((nrow + 63) / 64, EL_DCHUNK_WAVES / (EL_SG * rblocks))));
     // MBGPU_ELEC_WAVE_CHUNKS=1 (any nonzero integer) keeps the wavefront rule alone for the k
     // chunks of the final pass below (a test aid that compares chunkings); unset, empty or 0
     // leaves the bound on
     const char* wave_env = getenv("MBGPU_ELEC_WAVE_CHUNKS");
     const bool wave_rules_only = wave_env && atoi(wave_env) != 0;
-    E.spc = (E.n + E.schunks - 1) / E.schunks;
-    E.dspc = (nrow + E.dchunks - 1) / E.dchunks;
-    ECHK(dalloc(&E.S, (size_t)8 * K));
-    dfree(E.cg_smu);
-    dfree(E.cg_sp);
-    dfree(E.cg_su);
-    dfree(E.cg_sq);
-    ECHK(dalloc(&E.cg_smu, (size_t)6 * K));
-    ECHK(dalloc(&E.cg_sp, (size_t)6 * K));
-    ECHK(dalloc(&E.cg_su, (size_t)6 * K));
-    ECHK(dalloc(&E.cg_sq, (size_t)6 * K));
-    ECHK(dalloc(&E.Sq, (size_t)2 * K));
-    ECHK(dalloc(&E.kc, (size_t)16 * K));
     ECHK(dalloc(&E.kf, (size_t)16 * K));
-    ECHK(dalloc(&E.Spart, (size_t)std::max(8 * E.schunks, 6 * E.dchunks) * K));
-    ECHK(hipMemset(E.S, 0, sizeof(double) * 8 * K));
-    ECHK(hipMemset(E.kc, 0, sizeof(double) * 16 * K));
     // phase tables
     const int ks = std::max(std::max(kmax[0], kmax[1]), kmax[2]) + 1;
     if (ks != E.kstride) {
@@ -355,21 +376,7 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
         const int k0 = runk[r0], k1 = r1 < E.nrun ? runk[r1] : K;
         E.kmaxch = std::max(E.kmaxch, k1 - k0);
     }
-    // k chunks of the field passes: about EL_FCHUNK_WAVES wavefronts (EL_KG per block of
-    // 128 sites), at most EL_FCHUNK_RUNS runs per chunk (their constants are staged in LDS)
-    {
-        const int sblocks = (nrow + 127) / 128;
-        E.fchunks = std::max(1, std::min(E.nrun, EL_FCHUNK_WAVES / (EL_KG * sblocks)));
-        E.fchunks = std::max(E.fchunks, std::min(E.nrun, (E.nrun + EL_FCHUNK_RUNS - 1) / EL_FCHUNK_RUNS));
-        E.frpc = (E.nrun + E.fchunks - 1) / E.fchunks;
-        E.fchunks = (E.nrun + E.frpc - 1) / E.frpc;
-        E.fkmax = 0;
-        for (int c = 0; c < E.fchunks; ++c) {
-            const int r0 = c * E.frpc, r1 = std::min(E.nrun, r0 + E.frpc);
-            const int k0 = runk[r0], k1 = r1 < E.nrun ? runk[r1] : K;
-            E.fkmax = std::max(E.fkmax, k1 - k0);
-        }
-    }
+    if (build_rs(S, rc, kmax, kv, klm, err)) return -1;
     dfree(E.Fpart);
     ECHK(dalloc(&E.Fpart, std::max((size_t)E.kchunks * 16, (size_t)E.fchunks * 6) * E.n));
     // block partials of the final passes
@@ -405,7 +412,7 @@ int alloc_direct(ElecState& S, std::string& err)
     ECHK(dalloc(&E.blk, (size_t)E.nblk));
     E.K = E.nrun = 0;
     E.kchunks = E.fchunks = 1;
-    E.rpc = E.kmaxch = E.frpc = E.fkmax = 0;
+    E.rpc = E.kmaxch = 0;
     S.k_alpha = -1.0;   // a later periodic call builds its k list
     S.P.rvolm = 0.0;
     return 0;
@@ -531,8 +538,7 @@ int elec_configure(ElecState& S, int nw, const CellGeom& g, const double* cell, 
     P.rpc = S.E.rpc;
     P.kmaxch = S.E.kmaxch;
     P.fchunks = S.E.fchunks;
-    P.frpc = S.E.frpc;
-    P.fkmax = S.E.fkmax;
+    P.rs = S.E.rs;
     P.scale = 4.0 * P.rvolm * R4PIE0;
     P.scal1 = 2.0 * P.rvolm * R4PIE0;
     P.self_dd = 4.0 * R4PIE0 * P.alpha * P.alpha * P.alpha / SQRPI / 3.0;

@@ -22,6 +22,8 @@
 //     the remaining kernels of a batch of iterations into no-ops.
 #include <math.h>
 
+#include <algorithm>
+
 #include "mbgpu_internal.h"
 #include "gen/dms_table.inc"
 
@@ -29,7 +31,6 @@
 #define SQRPI 1.7724538509055159      // dl_params.inc
 #define TWOPI (2.0 * 3.141592653589793)
 #define EL_RUN 8                      // k vectors per run (consecutive n)
-#define EL_SCHUNK 64                  // sites per chunk of the structure-factor pass
 
 namespace {
 
@@ -521,15 +522,21 @@ __global__ void k_el_intra_prep(ElecDev P, const double* __restrict__ x, const d
 
 // Reciprocal-space phase tables of each site: cos / sin (l * 2 pi * s_a), s = rcell . r,
 // l = 0..kmax_a, by the reference's recurrence (ewald1p.f:196-241, 262-282), layout
-// phc/phs [a][l][n].
+// phc/phs [a][l][n] (for the final site pass) and pht[n][rs.kt] (for the matrix passes).
 __global__ void k_el_phase(ElecDev P, const double* __restrict__ x, const double* __restrict__ y,
                            const double* __restrict__ z, const double* __restrict__ rcell,
-                           double* __restrict__ phc, double* __restrict__ phs)
+                           double* __restrict__ phc, double* __restrict__ phs, double2* __restrict__ pht)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= P.n) return;
+    if (j >= P.n) {
+        // (the structure-factor pass reads up to RS_PAD sites past the last with weight 0)
+        if (j < P.n + RS_PAD)
+            for (int l = 0; l < P.rs.kt; ++l) pht[(long)j * P.rs.kt + l] = make_double2(0.0, 0.0);
+        return;
+    }
     const int ks = P.kstride;
     for (int a = 0; a < 3; ++a) {
+        double2* row = pht + (long)j * P.rs.kt + (a == 0 ? 0 : a == 1 ? P.rs.ky : P.rs.kz);
         const double ss = rcell[a] * x[j] + rcell[3 + a] * y[j] + rcell[6 + a] * z[j];
         const double c1 = cos(TWOPI * ss), s1 = sin(TWOPI * ss);
         double c = 1.0, s = 0.0;
@@ -544,6 +551,8 @@ __global__ void k_el_phase(ElecDev P, const double* __restrict__ x, const double
             }
             phc[((long)a * ks + l) * P.n + j] = c;
             phs[((long)a * ks + l) * P.n + j] = s;
+            row[l] = make_double2(c, s);
+            if (a == 1 && l > 0) row[-l] = make_double2(c, -s);
         }
     }
 }
@@ -568,411 +577,6 @@ __device__ __forceinline__ void run_phase(double el_c, double el_s, double em_c,
 }
 
 }  // namespace
-
-// Structure factors over a chunk of sites, k-parallel (ewald1p.f:342-438).  A block owns
-// 64 half-runs (lane = half-run: up to EL_HALF consecutive k at fixed l, m, stepping
-// exp(i k.r_j) along n by a complex recurrence) and EL_SG site groups (one wavefront
-// each): the block stages the phase tables of its site chunk in LDS, EL_TILE sites at a
-// time (rows l = lmin..lmax of a*, every |m| row of b*, every |n| row of c*, padded against
-// bank conflicts), wavefront w takes the tile's sites w, w + EL_SG, ..., and the EL_SG
-// partial sums of every k are added in LDS in group order before one partial per chunk is
-// written: Spart[chunk][k][NV], NV = 8 with charges (sum q ckr, sum q skr, sum mu ckr (3),
-// sum mu skr (3)), NV = 6 for the dipoles alone (the last six).  The dipole sums run over
-// polarizable sites only.
-#ifndef EL_TILE
-#define EL_TILE 16
-#endif
-#define EL_TROW (EL_TILE + 1)
-#ifndef EL_SPLIT
-#define EL_SPLIT 2                    // threads per k run in the structure-factor pass
-#endif
-#ifndef EL_SG
-#define EL_SG 4                       // site groups (wavefronts) per structure-factor block
-#endif
-#define EL_HALF (EL_RUN / EL_SPLIT)
-// With cgblk (the conjugate-gradient solver's partials, cgnb blocks), the pass first takes the
-// solver's stopping test for iteration `it` (cg_step; block (0, 0) records the scalars) and
-// does nothing once the dipoles have converged.
-template <bool CHG>
-__global__ __launch_bounds__(64 * EL_SG) void k_el_sfac(ElecDev P, int spc, const int* __restrict__ runs,
-                                                        const int* __restrict__ runk, const double* __restrict__ phc,
-                                                        const double* __restrict__ phs, const double* __restrict__ chge,
-                                                        const double* __restrict__ dip, double* __restrict__ Spart,
-                                                        double* __restrict__ state, const double* __restrict__ cgblk,
-                                                        int cgnb, int it)
-{
-    if (!CHG && state[2] != 0.0) return;
-    if (!CHG && cgblk &&
-        cg_step(P, it, cgnb, cgblk, state, blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64))
-        return;
-    extern __shared__ double lds[];
-    constexpr int NT = 64 * EL_SG;
-    constexpr int NV = CHG ? 8 : 6;
-    constexpr int Q0 = CHG ? 0 : 2;          // first accumulator component written
-    const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 6;
-    const int g = blockIdx.x * 64 + lane;
-    const int r = g / EL_SPLIT, half = g % EL_SPLIT;
-    const int chunk = blockIdx.y;
-    const int ns = CHG ? P.n : P.nrow;
-    const int j0 = chunk * spc, j1 = min(ns, j0 + spc);
-    const int rfirst = (blockIdx.x * 64) / EL_SPLIT;
-    const int rlast = min(P.nrun - 1, (blockIdx.x * 64 + 63) / EL_SPLIT);
-    const int lmin = runs[4 * rfirst], lmax = runs[4 * rlast];
-    const int nl = lmax - lmin + 1, nm = P.km[1] + 1, nn = P.km[2] + 1;
-    const int nrows = nl + nm + nn;
-    // (cos, sin) pairs of the tile's table rows, and (q, mu) of its sites, as double2 so
-    // that each entry is one 16-byte LDS read (dynamic LDS starts 16-byte aligned)
-    double2* tcs = reinterpret_cast<double2*>(lds);
-    double2* tw = tcs + nrows * EL_TROW;
-    const int ks = P.kstride;
-    int l = lmin, m = 0, nst = 1, cnt = 0;
-    if (r < P.nrun) {
-        l = runs[4 * r];
-        m = runs[4 * r + 1];
-        nst = runs[4 * r + 2] + EL_HALF * half;
-        cnt = min(EL_HALF, max(0, runs[4 * r + 3] - EL_HALF * half));
-        if (cnt == 0) nst = runs[4 * r + 2];
-    }
-    const int rowA = (l - lmin) * EL_TROW, rowB = (nl + abs(m)) * EL_TROW, rowC = (nl + nm + abs(nst)) * EL_TROW;
-    const int rowC1 = (nl + nm + 1) * EL_TROW;
-    double acc[EL_HALF][8];
-#pragma unroll
-    for (int t = 0; t < EL_HALF; ++t)
-#pragma unroll
-        for (int q = 0; q < 8; ++q) acc[t][q] = 0.0;
-    // tiles of EL_TILE sites, double-buffered: the next tile's table entries are loaded
-    // into registers while the current tile is consumed from LDS
-    constexpr int PF = (80 * EL_TILE + NT - 1) / NT;   // staged entries per thread (nrows <= 80)
-    double pc[PF], ps[PF], pw = 0.0;
-    auto fetch = [&](int t0) {
-        const int tn = min(EL_TILE, j1 - t0);
-#pragma unroll
-        for (int u = 0; u < PF; ++u) {
-            const int idx = tid + NT * u;
-            const int row = idx / EL_TILE, sidx = idx - row * EL_TILE;
-            pc[u] = 0.0;
-            ps[u] = 0.0;
-            if (row < nrows && sidx < tn) {
-                int a, ll;
-                if (row < nl) {
-                    a = 0;
-                    ll = lmin + row;
-                } else if (row < nl + nm) {
-                    a = 1;
-                    ll = row - nl;
-                } else {
-                    a = 2;
-                    ll = row - nl - nm;
-                }
-                const long o = ((long)a * ks + ll) * P.n + t0 + sidx;
-                pc[u] = phc[o];
-                ps[u] = phs[o];
-            }
-        }
-        if (tid < 4 * EL_TILE) {
-            // a site without an induced dipole carries mu = 0, so no test in the sums
-            const int sj = tid >> 2, w = tid & 3;
-            const int j = t0 + sj;
-            pw = 0.0;
-            if (sj < tn) {
-                if (w == 0) pw = chge[j];
-                else if (site_polr2(P, j) > 1.e-6) pw = dip[3 * j + w - 1];
-            }
-        }
-    };
-    if (j0 < j1) fetch(j0);
-    for (int t0 = j0; t0 < j1; t0 += EL_TILE) {
-        const int tn = min(EL_TILE, j1 - t0);
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < PF; ++u) {
-            const int idx = tid + NT * u;
-            const int row = idx / EL_TILE, sidx = idx - row * EL_TILE;
-            if (row < nrows) tcs[row * EL_TROW + sidx] = make_double2(pc[u], ps[u]);
-        }
-        if (tid < 4 * EL_TILE) reinterpret_cast<double*>(tw)[tid] = pw;
-        __syncthreads();
-        if (t0 + EL_TILE < j1) fetch(t0 + EL_TILE);
-        if (cnt > 0) {
-            // every thread steps EL_HALF k; terms past the end of its run are never stored
-#pragma unroll 2
-            for (int sj = grp; sj < tn; sj += EL_SG) {
-                const double2 A = tcs[rowA + sj], B = tcs[rowB + sj], C = tcs[rowC + sj], C1 = tcs[rowC1 + sj];
-                const double2 w01 = tw[2 * sj], w23 = tw[2 * sj + 1];
-                double ckr, skr;
-                run_phase(A.x, A.y, B.x, B.y, C.x, C.y, m, nst, ckr, skr);
-                const double q = w01.x, mx = w01.y, my = w23.x, mz = w23.y;
-#pragma unroll
-                for (int t = 0; t < EL_HALF; ++t) {
-                    if (CHG) {
-                        acc[t][0] += q * ckr;
-                        acc[t][1] += q * skr;
-                    }
-                    acc[t][2] += ckr * mx;
-                    acc[t][3] += ckr * my;
-                    acc[t][4] += ckr * mz;
-                    acc[t][5] += skr * mx;
-                    acc[t][6] += skr * my;
-                    acc[t][7] += skr * mz;
-                    const double cn = ckr * C1.x - skr * C1.y;
-                    skr = skr * C1.x + ckr * C1.y;
-                    ckr = cn;
-                }
-            }
-        }
-    }
-    // the site groups' sums, added in group order through LDS (the tiles are done with it);
-    // every thread reaches every barrier
-    double* red = lds;                                   // [EL_SG - 1][64][NV]
-#pragma unroll
-    for (int t = 0; t < EL_HALF; ++t) {
-        __syncthreads();
-        if (grp > 0)
-#pragma unroll
-            for (int q = 0; q < NV; ++q) red[((grp - 1) * 64 + lane) * NV + q] = acc[t][Q0 + q];
-        __syncthreads();
-        if (grp == 0)
-#pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                double v = acc[t][Q0 + q];
-                for (int w = 1; w < EL_SG; ++w) v += red[((w - 1) * 64 + lane) * NV + q];
-                acc[t][Q0 + q] = v;
-            }
-    }
-    if (grp != 0 || cnt == 0) return;
-    const int k0 = runk[r] + EL_HALF * half;
-#pragma unroll
-    for (int t = 0; t < EL_HALF; ++t)
-        if (t < cnt)
-#pragma unroll
-            for (int q = 0; q < NV; ++q) Spart[((long)chunk * P.K + k0 + t) * NV + q] = acc[t][Q0 + q];
-}
-
-// Sum the chunk partials and derive the per-k constants of the field passes: kc[k][0..5] =
-// (-k_a akk k.Ms, -k_a akk k.Mc) for the dipole field (ewald1p.f:759-767).  With CHG the
-// charge sums are stored in Sq[k][2] and kc[k][6..11] receives the charge-field constants
-// (k_a akk ckcs, -k_a akk ckss) (ewald1p.f:749-757).  A block sums 64 (k, component)
-// elements (8 k vectors); lanes 8k'..8k'+7 of the first wave hold the 8 sums of one k.
-template <bool CHG>
-__device__ void sreduce_block(const ElecDev& P, int blk, int schunks, const double* __restrict__ Spart,
-                              const double* __restrict__ kv, double* __restrict__ S, double* __restrict__ Sq,
-                              double* __restrict__ kc)
-{
-    // NV values per k in the partials (see k_el_sfac); a block sums EPB consecutive
-    // elements, a whole number of k
-    constexpr int NV = CHG ? 8 : 6, EPB = CHG ? 64 : 60, Q0 = CHG ? 0 : 2;
-    const int lane = threadIdx.x & 63;
-    const long e = (long)blk * EPB + lane;
-    const double v = chunk_sum64(Spart, (long)NV * P.K, schunks, e, lane < EPB && e < (long)NV * P.K);
-    if (threadIdx.x >= 64) return;
-    const int base = lane - lane % NV;
-    double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int q = 0; q < NV; ++q) s[Q0 + q] = __shfl(v, min(base + q, 63), 64);
-    const int k = (int)(e / NV);
-    if (lane % NV != 0 || lane >= EPB || k >= P.K) return;
-    if (CHG) {
-        Sq[2 * k] = s[0];
-        Sq[2 * k + 1] = s[1];
-    }
-#pragma unroll
-    for (int q = 2; q < 8; ++q) S[8 * k + q] = s[q];
-    const double kx = kv[8 * k], ky = kv[8 * k + 1], kz = kv[8 * k + 2], akk = kv[8 * k + 3];
-    const double skdmuckrs = kx * s[2] + ky * s[3] + kz * s[4];
-    const double skdmuskrs = kx * s[5] + ky * s[6] + kz * s[7];
-    double* c = kc + 16 * k;
-    c[0] = -kx * akk * skdmuskrs;
-    c[1] = -ky * akk * skdmuskrs;
-    c[2] = -kz * akk * skdmuskrs;
-    c[3] = -kx * akk * skdmuckrs;
-    c[4] = -ky * akk * skdmuckrs;
-    c[5] = -kz * akk * skdmuckrs;
-    if (CHG) {
-        c[6] = kx * akk * s[0];
-        c[7] = ky * akk * s[0];
-        c[8] = kz * akk * s[0];
-        c[9] = -kx * akk * s[1];
-        c[10] = -ky * akk * s[1];
-        c[11] = -kz * akk * s[1];
-    }
-}
-
-template <bool CHG>
-__global__ __launch_bounds__(256) void k_el_sreduce(ElecDev P, int schunks, const double* __restrict__ Spart,
-                                                    const double* __restrict__ kv, double* __restrict__ S,
-                                                    double* __restrict__ Sq, double* __restrict__ kc,
-                                                    const double* __restrict__ state)
-{
-    if (!CHG && state[2] != 0.0) return;
-    sreduce_block<CHG>(P, blockIdx.x, schunks, Spart, kv, S, Sq, kc);
-}
-
-// Reciprocal-space fields over a chunk of runs, site-parallel (ewald1p.f:749-769):
-// efdd_a += c_a skr + d_a ckr (dipole field), with CHG also efdc_a += e_a skr + f_a ckr
-// (charge field).  A block covers 128 sites (two per lane: j and j + 64) and EL_KG run
-// groups (one wavefront each, runs g, g + EL_KG, ... of the chunk); it stages the chunk's
-// runs and per-k constants in LDS, and the run groups' sums are added in LDS in group
-// order before one partial per chunk is written: Fpart[chunk][6][n] (components 0..2 the
-// dipole field, 3..5 the charge field).
-#ifndef EL_KG
-#define EL_KG 4                       // run groups (wavefronts) per field block
-#endif
-template <bool CHG>
-__global__ __launch_bounds__(64 * EL_KG) void k_el_kfield(ElecDev P, const int* __restrict__ runs,
-                                                          const int* __restrict__ runk, const double* __restrict__ phc,
-                                                          const double* __restrict__ phs, const double* __restrict__ kc,
-                                                          double* __restrict__ Fpart, const double* __restrict__ state)
-{
-    if (!CHG && state[2] != 0.0) return;
-    extern __shared__ double lds[];
-    constexpr int NC = CHG ? 12 : 6;
-    constexpr int NT = 64 * EL_KG;
-    const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 6;
-    const int chunk = blockIdx.y;
-    const int r0 = chunk * P.frpc, r1 = min(P.nrun, r0 + P.frpc);
-    const int nr = max(0, r1 - r0);
-    // two sites per lane share every constant read; lanes past the last site compute on a
-    // clamped site and store nothing (every thread reaches the barriers below).  The n = 1
-    // phase factors are loaded before the staging barrier, which completes them: loaded
-    // later, the wait for them inside the k loop would also wait for the run prefetches.
-    const int nrow = CHG ? P.n : P.nrow;
-    const int ja = blockIdx.x * 128 + lane, jb = ja + 64;
-    const bool ha = ja < nrow, hb = jb < nrow;
-    const int jA = ha ? ja : 0, jB = hb ? jb : jA;
-    const int ks = P.kstride;
-    const long o1 = ((long)2 * ks + 1) * P.n;
-    const double ca1 = phc[o1 + jA], sa1 = phs[o1 + jA], cb1 = phc[o1 + jB], sb1 = phs[o1 + jB];
-    double* sk = lds;                                          // [fkmax][NC]
-    int* sr = reinterpret_cast<int*>(lds + (long)P.fkmax * NC); // [frpc][4] runs
-    int* so = sr + 4 * P.frpc;                                  // [frpc] first k of each run - kbase
-    const int kbase = nr ? runk[r0] : 0;
-    const int nk = nr ? ((r1 < P.nrun ? runk[r1] : P.K) - kbase) : 0;
-    for (int idx = tid; idx < nk * NC; idx += NT) {
-        const int kk = idx / NC, q = idx - kk * NC;
-        sk[idx] = kc[16L * (kbase + kk) + q];
-    }
-    for (int idx = tid; idx < nr * 4; idx += NT) sr[idx] = runs[4 * r0 + idx];
-    for (int idx = tid; idx < nr; idx += NT) so[idx] = runk[r0 + idx] - kbase;
-    __syncthreads();
-    double fa[3] = {0, 0, 0}, fb[3] = {0, 0, 0}, ga[3] = {0, 0, 0}, gb[3] = {0, 0, 0};
-    // the phase-table entries of a run are loaded one run ahead (double-buffered in
-    // registers), so their latency overlaps the previous run's arithmetic
-    double qa[6], qb[6];
-    auto load_run = [&](int r) {
-        const int l = sr[4 * r], m = sr[4 * r + 1], n0 = sr[4 * r + 2];
-        const long oa = (long)l * P.n, ob = ((long)ks + abs(m)) * P.n, oc = ((long)2 * ks + abs(n0)) * P.n;
-        qa[0] = phc[oa + jA]; qa[1] = phs[oa + jA]; qa[2] = phc[ob + jA];
-        qa[3] = phs[ob + jA]; qa[4] = phc[oc + jA]; qa[5] = phs[oc + jA];
-        qb[0] = phc[oa + jB]; qb[1] = phs[oa + jB]; qb[2] = phc[ob + jB];
-        qb[3] = phs[ob + jB]; qb[4] = phc[oc + jB]; qb[5] = phs[oc + jB];
-    };
-    if (grp < nr) load_run(grp);
-    for (int r = grp; r < nr; r += EL_KG) {
-        const int m = sr[4 * r + 1], n0 = sr[4 * r + 2], cnt = sr[4 * r + 3], kk = so[r];
-        double cA, sA, cB, sB;
-        run_phase(qa[0], qa[1], qa[2], qa[3], qa[4], qa[5], m, n0, cA, sA);
-        run_phase(qb[0], qb[1], qb[2], qb[3], qb[4], qb[5], m, n0, cB, sB);
-        if (r + EL_KG < nr) load_run(r + EL_KG);
-#pragma unroll
-        for (int t = 0; t < EL_RUN; ++t) {
-            if (t < cnt) {
-                // one fused multiply-add per product into the accumulators
-                const double* c = sk + NC * (kk + t);
-                const double c0 = c[0], c1v = c[1], c2 = c[2], c3 = c[3], c4 = c[4], c5 = c[5];
-                fa[0] += c0 * sA;
-                fa[0] += c3 * cA;
-                fa[1] += c1v * sA;
-                fa[1] += c4 * cA;
-                fa[2] += c2 * sA;
-                fa[2] += c5 * cA;
-                fb[0] += c0 * sB;
-                fb[0] += c3 * cB;
-                fb[1] += c1v * sB;
-                fb[1] += c4 * cB;
-                fb[2] += c2 * sB;
-                fb[2] += c5 * cB;
-                if (CHG) {
-                    const double c6 = c[6], c7 = c[7], c8 = c[8], c9 = c[9], c10 = c[10], c11 = c[11];
-                    ga[0] += c6 * sA;
-                    ga[0] += c9 * cA;
-                    ga[1] += c7 * sA;
-                    ga[1] += c10 * cA;
-                    ga[2] += c8 * sA;
-                    ga[2] += c11 * cA;
-                    gb[0] += c6 * sB;
-                    gb[0] += c9 * cB;
-                    gb[1] += c7 * sB;
-                    gb[1] += c10 * cB;
-                    gb[2] += c8 * sB;
-                    gb[2] += c11 * cB;
-                }
-                const double na = cA * ca1 - sA * sa1;
-                sA = sA * ca1 + cA * sa1;
-                cA = na;
-                const double nb = cB * cb1 - sB * sb1;
-                sB = sB * cb1 + cB * sb1;
-                cB = nb;
-            }
-        }
-    }
-    // the run groups' sums, added in group order through LDS
-    constexpr int NQ = CHG ? 12 : 6;                           // values per lane
-    double v[12];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        v[q] = fa[q];
-        v[3 + q] = fb[q];
-        if (CHG) {
-            v[6 + q] = ga[q];
-            v[9 + q] = gb[q];
-        }
-    }
-    double* red = lds;                                         // [EL_KG - 1][64][NQ]
-    __syncthreads();
-    if (grp > 0)
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) red[((grp - 1) * 64 + lane) * NQ + q] = v[q];
-    __syncthreads();
-    if (grp != 0) return;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-        for (int w = 1; w < EL_KG; ++w) v[q] += red[((w - 1) * 64 + lane) * NQ + q];
-    double* out = Fpart + (long)chunk * 6 * P.n;
-    for (int q = 0; q < 3; ++q) {
-        if (ha) out[(long)q * P.n + ja] = v[q];
-        if (hb) out[(long)q * P.n + jb] = v[3 + q];
-        if (CHG) {
-            if (ha) out[(long)(3 + q) * P.n + ja] = v[6 + q];
-            if (hb) out[(long)(3 + q) * P.n + jb] = v[9 + q];
-        }
-    }
-}
-
-// Sum the field partials over the k chunks and scale (ewald1p.f:941-976): efdd =
-// scale * sum + self term; with CHG also efdc = scale * sum (iloop = 1).  Element
-// (component q, site j) = q * nrow + j, 64 per block.
-template <bool CHG>
-__global__ __launch_bounds__(256) void k_el_kfield_reduce(ElecDev P, const double* __restrict__ Fpart,
-                                                          const double* __restrict__ dip, double* __restrict__ efdd,
-                                                          double* __restrict__ efdc, const double* __restrict__ state)
-{
-    if (!CHG && state[2] != 0.0) return;
-    const int nrow = CHG ? P.n : P.nrow;
-    const int nq = CHG ? 6 : 3;
-    const int t = blockIdx.x * 64 + (threadIdx.x & 63);
-    const bool valid = t < nq * nrow;
-    const int q = valid ? t / nrow : 0, j = valid ? t - q * nrow : 0;
-    const double sum = chunk_sum64(Fpart, 6L * P.n, P.fchunks, (long)q * P.n + j, valid);
-    if (threadIdx.x >= 64 || !valid) return;
-    if (q < 3) {
-        const bool pol = site_polr2(P, j) > 1.e-6;
-        efdd[3 * j + q] = (pol ? P.scale * sum : 0.0) + P.self_dd * dip[3 * j + q];
-    } else {
-        efdc[3 * j + q - 3] = P.scale * sum;
-    }
-}
-
-// ============================================================ solver iteration ======
 
 // Real-space dipole field of one row (rfield.f:201-317 list pairs; 419-520 excluded
 // pairs): emu_i = sum_j T_ij mu_j.  One wavefront per site.
@@ -1016,6 +620,414 @@ __device__ void emu_row(const ElecDev& P, int i, int lane, const int* __restrict
         for (int q = 0; q < 3; ++q) emu[3 * i + q] = e[q];
 }
 
+// ------------------------------------------- Ewald sums as FP64 matrix products ------
+// S(k) = sum_j w_j(k) e^{i k.r_j} and the fields of a set of amplitudes U(k) at the sites,
+// over the k list of ewald1p.f:254-345 (k = (l, m, n)).  The list is taken by its (l, m) pairs,
+// 16 to a group.  With phi = l x + m y, C = cos phi, S = sin phi per (pair, site) and the
+// tables (cos n z, sin n z) per (n > 0, site),
+//   S(l, m, +-n) = sum_j w (C cz -+ S sz) + i sum_j w (S cz +- C sz):
+// the four sums of the two k are entries of the products [w C; w S] x [cz | sz] over the
+// sites, which the matrix cores form in 16 x 16 tiles (pairs x 8 n, cos and sin) four sites at
+// a time.  For dipoles w = k.mu = (l alpha + m beta) +- n gamma with alpha = 2 pi a*.mu, ...:
+// (l alpha + m beta) goes with the phases, n gamma with the table, in products of their own:
+// 8 FLOP per (k, site) where vector sums of the three components with a phase recurrence
+// took 20.  The field is the transposed product: with W = akk U the rows
+//   H_C = sum_n cz (W+c + W-c) + sz (W+s - W-s),  H_S = sum_n cz (W+s + W-s) + sz (W-c - W+c)
+// per (pair, site), and the same with n W for the c* component, are contracted over the pairs
+// with C, S, l and m on the spot.
+// FP64 matrix and vector instructions share the same units at the same peak here (a loop of
+// independent 16x16x4 products reaches 68-71 TFLOP/s, of vector multiply-adds 52), so what the
+// matrix form saves is instructions, phase recurrences and the idle time of few wavefronts:
+// one wavefront per SIMD already runs them at rate.
+// Measured against the vector form with phase recurrences (launches back to back, 2.4 us of each
+// the launch itself; structure factors with their chunk sum and the real-space field, then the
+// fields): 19.2 + 8.9 and 16.5 -> 10.3 and 11.6 us at 512 waters (9 966 k, 1 536 sites), 162 + 22
+// and 137 -> 62 and 58 us at 2 048 waters (33 530 k, 6 144 sites).  At 512 waters what is left is
+// latency (the products alone take 2.3 us a pass at rate), at 2 048 the matrix units are busy
+// half the time; the rest is phases and operand set-up on the same units.
+typedef double v4d __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ v4d mfma_f64(double a, double b, v4d c)
+{
+    // a: row lane % 16, column lane / 16; b: row lane / 16, column lane % 16;
+    // c[v]: row lane / 16 + 4 v, column lane % 16
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// One set of weights of a structure-factor launch: dipoles mu[3 j] (dip) or scalars v[j stride],
+// over the first ns sites.
+struct RsSrc {
+    const double* v;
+    int stride, dip, ns;
+};
+struct RsSrcs {
+    RsSrc s[4];
+};
+
+#define RS_NT 4                       // tiles of 8 n per block
+#define RS_WAVES 8                    // wavefronts per block
+
+// (cos phi, sin phi) of a pair from the table entries of l and m
+__device__ __forceinline__ void rs_phase(const double2 X, const double2 Y, double& c, double& s)
+{
+    c = X.x * Y.x - X.y * Y.y;
+    s = X.y * Y.x + X.x * Y.y;
+}
+
+// the value of the lane 8 further on within each row of 16 lanes
+__device__ __forceinline__ double row_ror8(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x128, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x128, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// A block's sums for one group of pairs, tiles [t0, t0 + NT) of n and one chunk of sites.  The
+// chunk's weights are staged in LDS (2 pi a*.mu, 2 pi b*.mu, 2 pi c*.mu and the scalar weight;
+// zero past the last site); wavefront w takes the steps of four sites w, w + 8, ..., with the
+// next step's table entries loaded while the current one is multiplied, and the eight
+// wavefronts' sums are added in order through LDS.
+template <int NT>
+__device__ void rs_sfac_block(const ElecDev& P, const RsSrc src, int spc, int g, int t0, int chunk,
+                              const double2* __restrict__ pht, double* __restrict__ out, double* lds)
+{
+    const RsPlan& R = P.rs;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int j0 = chunk * spc, nj = min(spc, src.ns - j0), nstep = (nj + 3) / 4;
+    for (int i = tid; i < 4 * nstep; i += 64 * RS_WAVES) {
+        double4 w = make_double4(0.0, 0.0, 0.0, 0.0);
+        if (i < nj) {
+            const double* v = src.v + (long)(j0 + i) * src.stride;
+            if (src.dip) {
+                const double mx = TWOPI * v[0], my = TWOPI * v[1], mz = TWOPI * v[2];
+                w.x = R.rc[0] * mx + R.rc[3] * my + R.rc[6] * mz;
+                w.y = R.rc[1] * mx + R.rc[4] * my + R.rc[7] * mz;
+                w.z = R.rc[2] * mx + R.rc[5] * my + R.rc[8] * mz;
+            } else {
+                w.w = v[0];
+            }
+        }
+        reinterpret_cast<double4*>(lds)[i] = w;
+    }
+    const int4 pr = R.pair[16 * g + (lane & 15)];
+    const int nt = max(0, min(NT, __builtin_amdgcn_readfirstlane(pr.w) - t0));
+    const int sl = lane >> 4;
+    const double dl = pr.x, dm = pr.y;
+    // byte offsets from the chunk's first site (a chunk is at most RS_MAX_SPC sites)
+    const char* base = reinterpret_cast<const char*>(pht + (long)j0 * R.kt);
+    const unsigned step = 64u * R.kt;                     // four sites
+    unsigned at = (4u * wv + sl) * 16u * R.kt;
+    const unsigned ox = 16u * pr.x, oy = 16u * (R.ky + pr.y);
+    unsigned oz[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        // past the largest n of the list any entry of the table will do: no k takes the sum
+        const int n = 8 * (t0 + t) + 1 + (lane & 7);
+        oz[t] = 16u * (R.kz + min(n, P.km[2])) + (lane & 8);
+    }
+    v4d ac[NT], as[NT], gc[NT], gs[NT];      // sums with l alpha + m beta (or the scalar), with gamma
+#pragma unroll
+    for (int t = 0; t < NT; ++t) ac[t] = as[t] = gc[t] = gs[t] = (v4d){0.0, 0.0, 0.0, 0.0};
+    double c0 = 0.0, s0 = 0.0;
+    double2 X, Y;
+    double z[NT];
+    auto load = [&](unsigned o) {
+        X = *reinterpret_cast<const double2*>(base + (o + ox));
+        Y = *reinterpret_cast<const double2*>(base + (o + oy));
+#pragma unroll
+        for (int t = 0; t < NT; ++t) z[t] = *reinterpret_cast<const double*>(base + (o + oz[t]));
+    };
+    if (wv < nstep) load(at);
+    __syncthreads();
+    for (int st = wv; st < nstep; st += RS_WAVES) {
+        const double4 w = reinterpret_cast<const double4*>(lds)[4 * st + sl];
+        double c, s, zc[NT];
+        rs_phase(X, Y, c, s);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) zc[t] = z[t];
+        at += RS_WAVES * step;
+        if (st + RS_WAVES < nstep) load(at);
+        const double wp = w.w + dl * w.x + dm * w.y;
+        const double wc = wp * c, ws = wp * s;
+        c0 += wc;
+        s0 += ws;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            if (t < nt) {
+                ac[t] = mfma_f64(wc, zc[t], ac[t]);
+                as[t] = mfma_f64(ws, zc[t], as[t]);
+                if (src.dip) {
+                    const double zg = w.z * zc[t];
+                    gc[t] = mfma_f64(c, zg, gc[t]);
+                    gs[t] = mfma_f64(s, zg, gs[t]);
+                }
+            }
+    }
+    // S(+n), S(-n) of each wavefront (lanes of cos columns: real parts, of sin columns: imaginary
+    // parts), then the wavefronts' sums in order; every thread reaches every barrier
+    const bool sinc = lane & 8;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        if (t >= nt) break;
+        const double n = 8 * (t0 + t) + 1 + (lane & 7);
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const double g0 = n * gc[t][v], g1 = n * gs[t][v];
+            const double a0 = ac[t][v] + g0, b0 = ac[t][v] - g0;
+            const double a1 = row_ror8(as[t][v] + g1), b1 = row_ror8(as[t][v] - g1);
+            lds[512 * wv + 64 * v + lane] = sinc ? a0 + a1 : a0 - a1;
+            lds[512 * wv + 256 + 64 * v + lane] = sinc ? b1 - b0 : b0 + b1;
+        }
+        __syncthreads();
+        double r = 0.0;
+#pragma unroll
+        for (int q = 0; q < RS_WAVES; ++q) r += lds[512 * q + tid];
+        out[512 * (t0 + t) + tid] = r;
+    }
+    if (t0 == 0) {
+        c0 += __shfl_xor(c0, 16, 64);
+        s0 += __shfl_xor(s0, 16, 64);
+        c0 += __shfl_xor(c0, 32, 64);
+        s0 += __shfl_xor(s0, 32, 64);
+        __syncthreads();
+        if (lane < 16) {
+            lds[32 * wv + lane] = c0;
+            lds[32 * wv + 16 + lane] = s0;
+        }
+        __syncthreads();
+        if (tid < 32) {
+            double s = 0.0;
+#pragma unroll
+            for (int q = 0; q < RS_WAVES; ++q) s += lds[32 * q + tid];
+            out[512L * R.ntiles + tid] = s;
+        }
+    }
+}
+
+// Blocks [0, nsb) form the structure factors: block = (set, group of pairs, tile group, chunk),
+// chunks fastest, into Spart[set][chunk][group][slot].  The others form the real-space field emu
+// of the first set's dipoles, a row per wavefront (both parts need the dipoles alone, so one
+// launch holds the two).  With cgblk (the conjugate-gradient solver's partials, cgnb blocks) the
+// pass first takes the solver's stopping test for iteration `it` (cg_step; block 0 records the
+// scalars) and does nothing once the dipoles have converged.
+template <int NT>
+__global__ __launch_bounds__(64 * RS_WAVES) void k_rs_sfac(ElecDev P, RsSrcs src, int nsb, int nch, int spc,
+                                                           const double2* __restrict__ pht,
+                                                           double* __restrict__ Spart, const int* __restrict__ nbrP,
+                                                           const int* __restrict__ cntP,
+                                                           const double* __restrict__ tens,
+                                                           const double* __restrict__ tin, double* __restrict__ emu,
+                                                           double* __restrict__ state,
+                                                           const double* __restrict__ cgblk, int cgnb, int it)
+{
+    if (state[2] != 0.0) return;
+    if (cgblk && cg_step(P, it, cgnb, cgblk, state, blockIdx.x == 0 && threadIdx.x < 64)) return;
+    extern __shared__ double lds[];
+    const RsPlan& R = P.rs;
+    int b = blockIdx.x;
+    if (b >= nsb) {
+        emu_row(P, (b - nsb) * RS_WAVES + (threadIdx.x >> 6), threadIdx.x & 63, nbrP, cntP, tens, tin, src.s[0].v, emu);
+        return;
+    }
+    // chunks fastest: with 8 chunks (one per XCD, see build_rs) the blocks of an XCD read the
+    // same sites, and the groups with the most n, which take longest, start first
+    const int ntg = (R.ntiles + NT - 1) / NT;
+    const int chunk = b % nch;
+    b /= nch;
+    const int tg = b % ntg;
+    b /= ntg;
+    const int g = b % R.ng, set = b / R.ng;
+    const long slot = RS_SLOT(R.ntiles);
+    rs_sfac_block<NT>(P, src.s[set], spc, g, NT * tg, chunk, pht,
+                      Spart + (((long)set * nch + chunk) * R.ng + g) * slot, lds);
+}
+
+// S(l, m, +n) = v[0] + i v[1] and S(l, m, -n) = v[2] + i v[3] of pair p of a group, n > 0, added
+// over the chunks in order: base = the slot of chunk 0, cs = stride from chunk to chunk.
+__device__ __forceinline__ void rs_sums(const double* __restrict__ base, long cs, int nch, int p, int n, double (&v)[4])
+{
+    const double* s = base + 512 * ((n - 1) >> 3) + 64 * (p >> 2) + 16 * (p & 3) + ((n - 1) & 7);
+    v[0] = v[1] = v[2] = v[3] = 0.0;
+#pragma unroll 4
+    for (int ch = 0; ch < nch; ++ch, s += cs) {
+        v[0] += s[0];
+        v[1] += s[8];
+        v[2] += s[256];
+        v[3] += s[264];
+    }
+}
+
+// Reciprocal fields (ewald1p.f:749-769, without the prefactor): a block takes one group of pairs
+// and 16 RS_WAVES tpw sites (wavefront w the 16-site tiles w, w + 8, ...).  It first adds the
+// group's structure factors over the chunks and lays the weighted amplitudes out in LDS as the
+// matrix operands (W of the comment above: H_C, H_S, and both with n W), then each wavefront
+// multiplies them with its sites' tables, 4 n at a time, and contracts the 16 pairs' rows.  Set 0
+// gives the dipole field, -sum_k k akk (cos Uc + sin Us) with U = S of the dipoles, into
+// components 0..2 of Fpart[group][6][n]; set 1 the charge field, U = (Qs, -Qc), into components
+// 3..5.  MORE: lists with more than RS_NT tiles of n, whose amplitudes take LDS in turns.
+template <bool MORE>
+__global__ __launch_bounds__(64 * RS_WAVES, 4) void k_rs_field(ElecDev P, int nch, int tpw, int nsb,
+                                                               const double2* __restrict__ pht,
+                                                               const double* __restrict__ Spart,
+                                                               double* __restrict__ Fpart,
+                                                               const double* __restrict__ state)
+{
+    if (state[2] != 0.0) return;
+    __shared__ double W[4][2][8 * RS_NT][16];          // [H_C, H_S, n H_C, n H_S][cos, sin][n][pair]
+    __shared__ double W0[2][16];                       // n = 0: [C, S]
+    const RsPlan& R = P.rs;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    // site blocks fastest: see k_rs_sfac
+    const int sb = blockIdx.x % nsb, g = (blockIdx.x / nsb) % R.ng, set = blockIdx.x / (nsb * R.ng);
+    const int row = lane & 15, quad = lane >> 4;
+    const int nt = __builtin_amdgcn_readfirstlane(R.pair[16 * g].w);
+    const int nn = 8 * R.ntiles + 1;
+    const long slot = RS_SLOT(R.ntiles), cs = slot * R.ng;
+    const double* base = Spart + ((long)set * nch * R.ng + g) * slot;
+    // the amplitudes of tiles [t0, t0 + ntt); every thread of the block takes part
+    auto amplitudes = [&](int t0, int ntt) {
+        for (int i = tid; i < 128 * ntt; i += 64 * RS_WAVES) {
+            // consecutive threads: n of the tile, then pairs, as the sums lie
+            const int p = ((i >> 3) & 3) + 4 * ((i >> 5) & 3), nl = 8 * (i >> 7) + (i & 7), n = 8 * t0 + nl + 1;
+            double v[4];
+            rs_sums(base, cs, nch, p, n, v);
+            const double2 a = R.ak[(long)(16 * g + p) * nn + n];
+            double uc = v[0], us = v[1], dc = v[2], ds = v[3];
+            if (set) {
+                uc = v[1];
+                us = -v[0];
+                dc = v[3];
+                ds = -v[2];
+            }
+            uc *= a.x;
+            us *= a.x;
+            dc *= a.y;
+            ds *= a.y;
+            const double fn = n;
+            W[0][0][nl][p] = uc + dc;
+            W[0][1][nl][p] = us - ds;
+            W[1][0][nl][p] = us + ds;
+            W[1][1][nl][p] = dc - uc;
+            W[2][0][nl][p] = fn * (uc - dc);
+            W[2][1][nl][p] = fn * (us + ds);
+            W[3][0][nl][p] = fn * (us - ds);
+            W[3][1][nl][p] = -fn * (uc + dc);
+        }
+    };
+    if (wv == RS_WAVES - 1 && lane < 16) {
+        double c = 0.0, s = 0.0;
+        const double* q = base + 512L * R.ntiles + lane;
+        for (int ch = 0; ch < nch; ++ch, q += cs) {
+            c += q[0];
+            s += q[16];
+        }
+        const double a = R.ak[(long)(16 * g + lane) * nn].x;
+        W0[0][lane] = a * (set ? s : c);
+        W0[1][lane] = a * (set ? -c : s);
+    }
+    if (!MORE) amplitudes(0, nt);
+    double dl[4], dm[4];
+    int ox[4], oy[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int4 pr = R.pair[16 * g + quad + 4 * v];
+        dl[v] = pr.x;
+        dm[v] = pr.y;
+        ox[v] = pr.x;
+        oy[v] = R.ky + pr.y;
+    }
+    __syncthreads();
+    for (int tl = 0; tl < tpw; ++tl) {
+        const int jr = 16 * ((sb * tpw + tl) * RS_WAVES + wv) + row;
+        if (!MORE && jr - row >= P.nrow) break;        // (a wavefront's tile is all past the end)
+        const bool ok = jr < P.nrow;
+        const int j = ok ? jr : P.nrow - 1;
+        const double2* p = pht + (long)j * R.kt;
+        v4d hc, hs, gc, gs;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            hc[v] = W0[0][quad + 4 * v];
+            hs[v] = W0[1][quad + 4 * v];
+            gc[v] = gs[v] = 0.0;
+        }
+        double2 X[4], Y[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            X[v] = p[ox[v]];
+            Y[v] = p[oy[v]];
+        }
+        for (int t0 = 0; t0 < nt; t0 += RS_NT) {
+            const int ntt = min(RS_NT, nt - t0);
+            if (MORE) {
+                __syncthreads();
+                amplitudes(t0, ntt);
+                __syncthreads();
+            }
+#pragma unroll 2
+            for (int q = 0; q < 2 * ntt; ++q) {
+                const int nl = 4 * q + quad, n = min(8 * t0 + nl + 1, P.km[2]);
+                const double2 z = p[R.kz + n];
+                hc = mfma_f64(W[0][0][nl][row], z.x, hc);
+                hs = mfma_f64(W[1][0][nl][row], z.x, hs);
+                gc = mfma_f64(W[2][0][nl][row], z.x, gc);
+                gs = mfma_f64(W[3][0][nl][row], z.x, gs);
+                hc = mfma_f64(W[0][1][nl][row], z.y, hc);
+                hs = mfma_f64(W[1][1][nl][row], z.y, hs);
+                gc = mfma_f64(W[2][1][nl][row], z.y, gc);
+                gs = mfma_f64(W[3][1][nl][row], z.y, gs);
+            }
+        }
+        // contract the pairs: components along a*, b*, c*, then Cartesian
+        double fa = 0.0, fb = 0.0, fc = 0.0;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            double c, s;
+            rs_phase(X[v], Y[v], c, s);
+            const double t = c * hc[v] + s * hs[v];
+            fa += dl[v] * t;
+            fb += dm[v] * t;
+            fc += c * gc[v] + s * gs[v];
+        }
+        fa += __shfl_xor(fa, 16, 64);
+        fb += __shfl_xor(fb, 16, 64);
+        fc += __shfl_xor(fc, 16, 64);
+        fa += __shfl_xor(fa, 32, 64);
+        fb += __shfl_xor(fb, 32, 64);
+        fc += __shfl_xor(fc, 32, 64);
+        if (ok && quad < 3) {
+            const double e = R.rc[3 * quad] * fa + R.rc[3 * quad + 1] * fb + R.rc[3 * quad + 2] * fc;
+            Fpart[((long)g * 6 + 3 * set + quad) * P.n + j] = -TWOPI * e;
+        }
+    }
+}
+
+// Sum the field partials over the k chunks and scale (ewald1p.f:941-976): efdd =
+// scale * sum + self term; with CHG also efdc = scale * sum (iloop = 1), at the sites that
+// can carry a dipole.  Element (component q, site j) = q * nrow + j, 64 per block.
+template <bool CHG>
+__global__ __launch_bounds__(256) void k_el_kfield_reduce(ElecDev P, const double* __restrict__ Fpart,
+                                                          const double* __restrict__ dip, double* __restrict__ efdd,
+                                                          double* __restrict__ efdc, const double* __restrict__ state)
+{
+    if (!CHG && state[2] != 0.0) return;
+    const int nrow = P.nrow;
+    const int nq = CHG ? 6 : 3;
+    const int t = blockIdx.x * 64 + (threadIdx.x & 63);
+    const bool valid = t < nq * nrow;
+    const int q = valid ? t / nrow : 0, j = valid ? t - q * nrow : 0;
+    const double sum = chunk_sum64(Fpart, 6L * P.n, P.fchunks, (long)q * P.n + j, valid);
+    if (threadIdx.x >= 64 || !valid) return;
+    if (q < 3) {
+        const bool pol = site_polr2(P, j) > 1.e-6;
+        efdd[3 * j + q] = (pol ? P.scale * sum : 0.0) + P.self_dd * dip[3 * j + q];
+    } else {
+        efdc[3 * j + q - 3] = P.scale * sum;
+    }
+}
+
+// ============================================================ solver iteration ======
+
 // emu for four rows per block.  With cgblk (the conjugate-gradient solver's partials, cgnb
 // blocks), the solver's stopping test for iteration `it` comes first (cg_step; block 0
 // records the scalars) and the kernel does nothing once the dipoles have converged.
@@ -1028,26 +1040,6 @@ __global__ __launch_bounds__(256) void k_el_emu(ElecDev P, const int* __restrict
     if (state[2] != 0.0) return;
     if (cgblk && cg_step(P, it, cgnb, cgblk, state, blockIdx.x == 0 && threadIdx.x < 64)) return;
     emu_row(P, blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & 63, nbrP, cntP, tens, tin, dip, emu);
-}
-
-// One launch for two independent parts of an application of the dipole-field operator:
-// blocks [0, nsr) sum the dipole structure factors (k_el_sreduce<false>), the others form
-// the real-space field emu, four rows per block.
-__global__ __launch_bounds__(256) void k_el_sreduce_emu(ElecDev P, int nsr, int schunks, const double* __restrict__ Spart,
-                                                        const double* __restrict__ kv, double* __restrict__ S,
-                                                        double* __restrict__ Sq, double* __restrict__ kc,
-                                                        const int* __restrict__ nbrP, const int* __restrict__ cntP,
-                                                        const double* __restrict__ tens, const double* __restrict__ tin,
-                                                        const double* __restrict__ dip, double* __restrict__ emu,
-                                                        const double* __restrict__ state)
-{
-    if (state[2] != 0.0) return;
-    const int b = blockIdx.x;
-    if (b < nsr) {
-        sreduce_block<false>(P, b, schunks, Spart, kv, S, Sq, kc);
-        return;
-    }
-    emu_row(P, (b - nsr) * 4 + (threadIdx.x >> 6), threadIdx.x & 63, nbrP, cntP, tens, tin, dip, emu);
 }
 
 // SOR update (iter.f:58-89) and per-block sums of |dmu|^2 and of the dipole count.
@@ -1123,32 +1115,20 @@ __global__ __launch_bounds__(64) void k_el_converge(ElecDev P, int nb, const dou
 //   partials of g = r.u and d = w.u, from which cg_step forms the next alpha and beta
 // (u = M^-1 r, w = A u, s = A p, q = M^-1 s, z = A q throughout).  It starts from
 // r = E0 - A mu0, u = M^-1 r and one extra application of A for w = A u.  T mu, which the
-// final passes need, follows mu as T mu += alpha (D p - s); with the Ewald sum over k the
-// dipole structure factors follow it too: S(q) = S(m) + beta S(q), S(p) = S(u) + beta S(p),
-// S(mu) += alpha S(p), S(u) -= alpha S(q).  The scalars need no grid-wide synchronization:
+// final passes need, follows mu as T mu += alpha (D p - s).  The scalars need no grid-wide synchronization:
 // the first kernel of each iteration sums the update's block partials in every wavefront
 // (cg_step) and its first block records them for the update.
 
-// S(mu) of the start dipoles (the dipole part of the preparation's structure factors)
-__global__ __launch_bounds__(256) void k_cg_smu_init(ElecDev P, const double* __restrict__ S, double* __restrict__ Smu)
-{
-    const long e = (long)blockIdx.x * 256 + threadIdx.x;
-    if (e < 6L * P.K) Smu[e] = S[8 * (e / 6) + 2 + e % 6];
-}
-
-// Fields and structure factors of the converged dipoles for the final passes, from the
-// quantities the solver carried along with mu: emu = T mu (real and reciprocal parts
-// together), efdd = 0, S = S(mu)
+// Fields of the converged dipoles for the final passes, from T mu, which the solver carried
+// along with mu: emu = T mu (real and reciprocal parts together), efdd = 0
 __global__ __launch_bounds__(256) void k_cg_final_fields(ElecDev P, const double* __restrict__ tmu,
-                                                         const double* __restrict__ Smu, double* __restrict__ emu,
-                                                         double* __restrict__ efdd, double* __restrict__ S)
+                                                         double* __restrict__ emu, double* __restrict__ efdd)
 {
-    const long e = (long)blockIdx.x * 256 + threadIdx.x;
-    if (e < 3L * P.nrow) {
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e < 3 * P.nrow) {
         emu[e] = tmu[e];
         efdd[e] = 0.0;
     }
-    if (e < 6L * P.K) S[8 * (e / 6) + 2 + e % 6] = Smu[e];
 }
 
 // packed index of (i, j) in a symmetric 9 x 9 matrix stored as its lower triangle
@@ -1310,43 +1290,22 @@ __global__ __launch_bounds__(256) void k_cg_init(ElecDev P, const double* __rest
 // and the first wavefront adds the quarters in order and updates the rows; the new w of
 // each water is shared through LDS for m = M^-1 w.  Block partials (r.u, w.u,
 // |polr2 r / r4pie0|^2, dipole count, max |m_i|) per water block.  INIT sets w = A u and
-// leaves mu, r, u as they are.  The blocks after the waters' (Ewald sum over k) carry the
-// dipole structure factors (INIT: S(u) = S(m), S(q) = S(p) = 0).
+// leaves mu, r, u as they are.
 #define CG_WPB 7
 template <bool INIT>
-__global__ __launch_bounds__(256) void k_cg_update(ElecDev P, int nbw, const double* __restrict__ Fpart,
+__global__ __launch_bounds__(256) void k_cg_update(ElecDev P, const double* __restrict__ Fpart,
                                                    const double* __restrict__ emu, const double* __restrict__ minv,
                                                    double* __restrict__ m, double* __restrict__ dip,
                                                    double* __restrict__ r, double* __restrict__ u,
                                                    double* __restrict__ wv, double* __restrict__ z,
                                                    double* __restrict__ qv, double* __restrict__ sv,
                                                    double* __restrict__ pv, double* __restrict__ tmu,
-                                                   const double* __restrict__ S, double* __restrict__ Sx,
-                                                   double* __restrict__ Sp, double* __restrict__ Su,
-                                                   double* __restrict__ Sqr, double* __restrict__ blk,
+                                                   double* __restrict__ blk,
                                                    const double* __restrict__ state)
 {
     if (state[2] != 0.0) return;
     const double alpha = INIT ? 0.0 : state[4], beta = INIT ? 0.0 : state[5];
     const int tid = threadIdx.x;
-    if ((int)blockIdx.x >= nbw) {
-        const long e = (long)(blockIdx.x - nbw) * 256 + tid;
-        if (e >= 6L * P.K) return;
-        const double sm = S[8 * (e / 6) + 2 + e % 6];
-        if (INIT) {
-            Su[e] = sm;
-            Sqr[e] = 0.0;
-            Sp[e] = 0.0;
-        } else {
-            const double sq = sm + beta * Sqr[e];
-            const double sp = Su[e] + beta * Sp[e];
-            Sqr[e] = sq;
-            Sp[e] = sp;
-            Sx[e] += alpha * sp;
-            Su[e] -= alpha * sq;
-        }
-        return;
-    }
     __shared__ double part[4][64];
     __shared__ double ws[64];
     __shared__ double wmax[4];
@@ -1459,19 +1418,41 @@ __global__ __launch_bounds__(256) void k_el_polar(ElecDev P, const double* __res
 
 // Per-k scalars of the final reciprocal pass (ewald1p.f:696-730): akk (Qc^2 + Qs^2),
 // akk |summu|^2 and the six omg components; block partials [nb][8].  Also stores, per k,
-// the constants the site pass needs in kf[k][16].
+// the constants the site pass needs in kf[k][16].  The structure factors of mu_x, mu_y, mu_z
+// and of the charges (sets 0..3 of Spart) are added over the chunks here.
 __global__ __launch_bounds__(256) void k_el_kscal(ElecDev P, const double* __restrict__ kv,
-                                                  const double* __restrict__ S, const double* __restrict__ Sq,
-                                                  double* __restrict__ kf, double* __restrict__ blk)
+                                                  const double* __restrict__ Spart, double* __restrict__ kf,
+                                                  double* __restrict__ blk)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (k < P.K) {
         const double kx = kv[8 * k], ky = kv[8 * k + 1], kz = kv[8 * k + 2], akk = kv[8 * k + 3];
         const double akv = kv[8 * k + 4];
-        const double Qc = Sq[2 * k], Qs = Sq[2 * k + 1];
-        const double Mc[3] = {S[8 * k + 2], S[8 * k + 3], S[8 * k + 4]};
-        const double Ms[3] = {S[8 * k + 5], S[8 * k + 6], S[8 * k + 7]};
+        const RsPlan& R = P.rs;
+        const int pos = R.kpos[k], pg = pos >> 8, n = (pos >> 1) & 127;
+        const long slot = RS_SLOT(R.ntiles), cs = slot * R.ng;
+        double Fc[4], Fs[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const double* base = Spart + ((long)w * R.nchq * R.ng + (pg >> 4)) * slot;
+            if (n == 0) {
+                const double* q = base + 512L * R.ntiles + (pg & 15);
+                Fc[w] = Fs[w] = 0.0;
+                for (int ch = 0; ch < R.nchq; ++ch, q += cs) {
+                    Fc[w] += q[0];
+                    Fs[w] += q[16];
+                }
+            } else {
+                double u[4];
+                rs_sums(base, cs, R.nchq, pg & 15, n, u);
+                Fc[w] = (pos & 1) ? u[2] : u[0];
+                Fs[w] = (pos & 1) ? u[3] : u[1];
+            }
+        }
+        const double Qc = Fc[3], Qs = Fs[3];
+        const double Mc[3] = {Fc[0], Fc[1], Fc[2]};
+        const double Ms[3] = {Fs[0], Fs[1], Fs[2]};
         const double kk[3] = {kx, ky, kz};
         const double skdmuckrs = kx * Mc[0] + ky * Mc[1] + kz * Mc[2];
         const double skdmuskrs = kx * Ms[0] + ky * Ms[1] + kz * Ms[2];
@@ -2172,21 +2153,41 @@ __global__ void k_el_zero(double* __restrict__ p, long n)
 namespace {
 inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 // dynamic LDS of the reciprocal-space passes (bytes)
-inline size_t sfac_lds(const ElecDev& P)
-{
-    // the tile of table rows and site weights, reused afterwards for the site-group sums
-    const size_t tile = 2 * EL_TROW * (size_t)(P.km[0] + P.km[1] + P.km[2] + 3) + 4 * EL_TILE;
-    const size_t red = (size_t)(EL_SG - 1) * 64 * 8;
-    return sizeof(double) * (tile > red ? tile : red);
-}
-inline size_t kfield_lds(const ElecDev& P)
-{
-    // per-k constants (12), runs (4 ints) and run offsets (1 int), then the run-group sums
-    const size_t stage = (size_t)P.fkmax * 12 + (5 * (size_t)P.frpc + 1) / 2 + 1;
-    const size_t red = (size_t)(EL_KG - 1) * 64 * 12;
-    return sizeof(double) * (stage > red ? stage : red);
-}
+inline size_t rs_lds(int spc) { return sizeof(double) * std::max(512L * RS_WAVES, 4L * spc); }
 inline size_t kfinal_lds(const ElecDev& P) { return sizeof(double) * ((size_t)P.kmaxch * EL_KF + 2 * (size_t)P.rpc + 2); }
+
+// Structure factors of nset sets of weights over nch chunks of spc sites; with emu also the
+// real-space field of set 0 (dipoles).  Tiles of n per block: as many as the list needs, up to 4
+// (more are spread over blocks; each costs 16 accumulator registers).
+template <int NT>
+void rs_launch_sfac_t(const ElecBuffers& E, const ElecDev& P, const RsSrcs& src, int nset, int nch, int spc, bool emu,
+                      double* state, const double* cgblk, int cgnb, int it, hipStream_t s)
+{
+    const int nsb = P.rs.ng * ceil_div(P.rs.ntiles, NT) * nch * nset;
+    hipLaunchKernelGGL(k_rs_sfac<NT>, dim3(nsb + (emu ? ceil_div(P.nrow, RS_WAVES) : 0)), dim3(64 * RS_WAVES), rs_lds(spc),
+                       s, P, src, nsb, nch, spc, E.pht, E.Spart, E.nbrP, E.cntP, E.tens, E.tin, E.emu, state, cgblk,
+                       cgnb, it);
+}
+void rs_launch_sfac(const ElecBuffers& E, const ElecDev& P, const RsSrcs& src, int nset, int nch, int spc, bool emu,
+                    double* state, const double* cgblk, int cgnb, int it, hipStream_t s)
+{
+    auto f = P.rs.ntiles == 1   ? rs_launch_sfac_t<1>
+             : P.rs.ntiles == 2 ? rs_launch_sfac_t<2>
+             : P.rs.ntiles == 3 ? rs_launch_sfac_t<3>
+                                : rs_launch_sfac_t<4>;
+    f(E, P, src, nset, nch, spc, emu, state, cgblk, cgnb, it, s);
+}
+// The fields of nset sets of structure factors summed over nch chunks: 16-site tiles per
+// wavefront so that there are about two blocks per CU (each block first adds its group's chunks).
+void rs_launch_field(const ElecBuffers& E, const ElecDev& P, int nset, int nch, hipStream_t s)
+{
+    const int tiles = ceil_div(P.nrow, 16 * RS_WAVES);
+    const int tpw = std::max(1L, std::min((long)tiles, (long)tiles * P.rs.ng / 448));
+    const int nsb = ceil_div(tiles, tpw);
+    auto k = P.rs.ntiles > RS_NT ? k_rs_field<true> : k_rs_field<false>;
+    hipLaunchKernelGGL(k, dim3(nsb * P.rs.ng * nset), dim3(64 * RS_WAVES), 0, s, P, nch, tpw, nsb, E.pht, E.Spart,
+                       E.Fpart, E.state);
+}
 }
 
 int el_launch_setup(ElecBuffers& E, const ElecDev& P, CellList& cells, hipStream_t s)
@@ -2238,7 +2239,7 @@ int el_launch_prep(ElecBuffers& E, const ElecDev& P, const double* rcell_dev, co
         // field partials (one chunk), so that the reductions form efdd (the self term is 0
         // without an Ewald split) and efdc
         el_launch_zero(E.Fpart, 6L * P.n, s);
-        hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.n, 64)), dim3(256), 0, s, one_chunk(P),
+        hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.nrow, 64)), dim3(256), 0, s, one_chunk(P),
                            E.Fpart, E.dip, E.efdd, E.efdc, E.state);
         return (int)hipGetLastError();
     }
@@ -2256,21 +2257,18 @@ int el_launch_prep(ElecBuffers& E, const ElecDev& P, const double* rcell_dev, co
         sp_launch_spread(*sp->B, *sp->G, P.n, E.chge, E.dip, spec, g, true, nullptr, s);
         sp_launch_convolve(*sp->B, *sp->G, g, 2, true, nullptr, s);
         sp_launch_field(*sp->B, *sp->G, P.n, g, 2, sp->kap, E.Fpart, P.n, nullptr, s);
-        hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.n, 64)), dim3(256), 0, s, one_chunk(P),
+        hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.nrow, 64)), dim3(256), 0, s, one_chunk(P),
                            E.Fpart, E.dip, E.efdd, E.efdc, E.state);
         return (int)hipGetLastError();
     }
-    hipLaunchKernelGGL(k_el_phase, dim3(ceil_div(P.n, 64)), dim3(64), 0, s, P, E.x, E.y, E.z, rcell_dev, E.phc,
-                       E.phs);
-    // charge structure factors and the iloop = 1 reciprocal fields
-    hipLaunchKernelGGL(k_el_sfac<true>, dim3(ceil_div((long)EL_SPLIT * P.nrun, 64), E.schunks), dim3(64 * EL_SG), sfac_lds(P), s, P, E.spc,
-                       E.runs, E.runk, E.phc, E.phs, E.chge, E.dip, E.Spart, E.state, nullptr, 0, 0);
-    hipLaunchKernelGGL(k_el_sreduce<true>, dim3(ceil_div(8L * P.K, 64)), dim3(256), 0, s, P, E.schunks, E.Spart, E.kv, E.S,
-                       E.Sq, E.kc, E.state);
-    hipLaunchKernelGGL(k_el_kfield<true>, dim3(ceil_div(P.n, 128), P.fchunks), dim3(64 * EL_KG), kfield_lds(P), s, P, E.runs,
-                       E.runk, E.phc, E.phs, E.kc, E.Fpart, E.state);
-    hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.n, 64)), dim3(256), 0, s, P, E.Fpart, E.dip, E.efdd,
-                       E.efdc, E.state);
+    hipLaunchKernelGGL(k_el_phase, dim3(ceil_div(P.n + RS_PAD, 64)), dim3(64), 0, s, P, E.x, E.y, E.z, rcell_dev, E.phc,
+                       E.phs, E.pht);
+    // structure factors of the start dipoles and of the charges, and the iloop = 1 fields
+    rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.n}, {E.chge, 1, 0, P.n}}}, 2, P.rs.nchq, P.rs.spcq, false, E.state, nullptr, 0,
+                   0, s);
+    rs_launch_field(E, P, 2, P.rs.nchq, s);
+    hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.nrow, 64)), dim3(256), 0, s, P, E.Fpart, E.dip,
+                       E.efdd, E.efdc, E.state);
     return (int)hipGetLastError();
 }
 
@@ -2285,17 +2283,14 @@ int el_launch_iteration(ElecBuffers& E, const ElecDev& P, int first, const ElecS
     } else if (!first) {
         // reciprocal dipole field from the current dipoles (the first iteration's came
         // with the charge field)
-        hipLaunchKernelGGL(k_el_sfac<false>, dim3(ceil_div((long)EL_SPLIT * P.nrun, 64), E.dchunks), dim3(64 * EL_SG), sfac_lds(P), s, P,
-                           E.dspc, E.runs, E.runk, E.phc, E.phs, E.chge, E.dip, E.Spart, E.state, nullptr, 0, 0);
-        hipLaunchKernelGGL(k_el_sreduce<false>, dim3(ceil_div(6L * P.K, 60)), dim3(256), 0, s, P, E.dchunks, E.Spart, E.kv,
-                           E.S, E.Sq, E.kc, E.state);
-        hipLaunchKernelGGL(k_el_kfield<false>, dim3(ceil_div(P.nrow, 128), P.fchunks), dim3(64 * EL_KG), kfield_lds(P), s, P,
-                           E.runs, E.runk, E.phc, E.phs, E.kc, E.Fpart, E.state);
+        rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.nrow}}}, 1, P.rs.nch, P.rs.spc, true, E.state, nullptr, 0, 0, s);
+        rs_launch_field(E, P, 1, P.rs.nch, s);
         hipLaunchKernelGGL(k_el_kfield_reduce<false>, dim3(ceil_div(3L * P.nrow, 64)), dim3(256), 0, s, P, E.Fpart, E.dip,
                            E.efdd, E.efdc, E.state);
     }
-    hipLaunchKernelGGL(k_el_emu, dim3(ceil_div(P.nrow, 4)), dim3(256), 0, s, P, E.nbrP, E.cntP, E.tens, E.tin, E.dip,
-                       E.emu, E.state, nullptr, 0, 0);
+    if (first || sp)
+        hipLaunchKernelGGL(k_el_emu, dim3(ceil_div(P.nrow, 4)), dim3(256), 0, s, P, E.nbrP, E.cntP, E.tens, E.tin, E.dip,
+                           E.emu, E.state, nullptr, 0, 0);
     const int nb = ceil_div(P.nrow, 256);
     hipLaunchKernelGGL(k_el_sor, dim3(nb), dim3(256), 0, s, P, E.efk, E.emu, E.efdd, E.efdc, E.dip, E.blk, E.state);
     hipLaunchKernelGGL(k_el_converge, dim3(1), dim3(64), 0, s, P, nb, E.blk, E.state);
@@ -2304,17 +2299,12 @@ int el_launch_iteration(ElecBuffers& E, const ElecDev& P, int first, const ElecS
 
 // The dipole-field operator applied to the solver's m (emu: real-space rows; Fpart: the
 // reciprocal field's partials), for the k-sum: structure factors (taking the stopping test
-// of iteration `it` first when `check`), their sum and emu in one launch, the field.
+// of iteration `it` first when `check`) and emu in one launch, then the field.
 static void el_cg_apply_ksum(ElecBuffers& E, const ElecDev& P, bool check, int it, hipStream_t s)
 {
-    const int nbw = ceil_div(P.nw, CG_WPB), nsr = ceil_div(6 * P.K, 60);
-    hipLaunchKernelGGL(k_el_sfac<false>, dim3(ceil_div((long)EL_SPLIT * P.nrun, 64), E.dchunks), dim3(64 * EL_SG),
-                       sfac_lds(P), s, P, E.dspc, E.runs, E.runk, E.phc, E.phs, E.chge, E.cg_m, E.Spart, E.state,
-                       check ? E.cgblk : nullptr, nbw, it);
-    hipLaunchKernelGGL(k_el_sreduce_emu, dim3(nsr + ceil_div(P.nrow, 4)), dim3(256), 0, s, P, nsr, E.dchunks, E.Spart,
-                       E.kv, E.S, E.Sq, E.kc, E.nbrP, E.cntP, E.tens, E.tin, E.cg_m, E.emu, E.state);
-    hipLaunchKernelGGL(k_el_kfield<false>, dim3(ceil_div(P.nrow, 128), P.fchunks), dim3(64 * EL_KG), kfield_lds(P), s, P,
-                       E.runs, E.runk, E.phc, E.phs, E.kc, E.Fpart, E.state);
+    rs_launch_sfac(E, P, {{{E.cg_m, 3, 1, P.nrow}}}, 1, P.rs.nch, P.rs.spc, true, E.state, check ? E.cgblk : nullptr,
+                   ceil_div(P.nw, CG_WPB), it, s);
+    rs_launch_field(E, P, 1, P.rs.nch, s);
 }
 
 // The same for the particle mesh (emu first, with the stopping test when `check`) and for no
@@ -2331,15 +2321,12 @@ static void el_cg_update(ElecBuffers& E, const ElecDev& P, const ElecSpme* sp, b
 {
     const int nbw = ceil_div(P.nw, CG_WPB);
     const ElecDev Q = sp ? one_chunk(P) : P;
-    const int nsb = sp ? 0 : ceil_div(6 * P.K, 256);
     if (init)
-        hipLaunchKernelGGL(k_cg_update<true>, dim3(nbw + nsb), dim3(256), 0, s, Q, nbw, E.Fpart, E.emu, E.cg_minv,
-                           E.cg_m, E.dip, E.cg_r, E.cg_u, E.cg_w, E.cg_z, E.cg_q, E.cg_s, E.cg_p, E.cg_tmu, E.S,
-                           E.cg_smu, E.cg_sp, E.cg_su, E.cg_sq, E.cgblk, E.state);
+        hipLaunchKernelGGL(k_cg_update<true>, dim3(nbw), dim3(256), 0, s, Q, E.Fpart, E.emu, E.cg_minv, E.cg_m, E.dip,
+                           E.cg_r, E.cg_u, E.cg_w, E.cg_z, E.cg_q, E.cg_s, E.cg_p, E.cg_tmu, E.cgblk, E.state);
     else
-        hipLaunchKernelGGL(k_cg_update<false>, dim3(nbw + nsb), dim3(256), 0, s, Q, nbw, E.Fpart, E.emu, E.cg_minv,
-                           E.cg_m, E.dip, E.cg_r, E.cg_u, E.cg_w, E.cg_z, E.cg_q, E.cg_s, E.cg_p, E.cg_tmu, E.S,
-                           E.cg_smu, E.cg_sp, E.cg_su, E.cg_sq, E.cgblk, E.state);
+        hipLaunchKernelGGL(k_cg_update<false>, dim3(nbw), dim3(256), 0, s, Q, E.Fpart, E.emu, E.cg_minv, E.cg_m, E.dip,
+                           E.cg_r, E.cg_u, E.cg_w, E.cg_z, E.cg_q, E.cg_s, E.cg_p, E.cg_tmu, E.cgblk, E.state);
 }
 
 // conjugate-gradient start: residual of the start dipoles (their fields came with the
@@ -2353,19 +2340,14 @@ int el_launch_cg_init(ElecBuffers& E, const ElecDev& P, const ElecSpme* sp, hipS
                        E.emu, E.state, nullptr, 0, 0);
     hipLaunchKernelGGL(k_cg_init, dim3(nbw), dim3(256), 0, s, P, E.efk, E.efdc, E.emu, E.efdd, E.dip, E.cg_minv, E.cg_r,
                        E.cg_u, E.cg_m, E.cg_z, E.cg_q, E.cg_s, E.cg_p, E.cg_tmu);
-    if (!sp) {
-        hipLaunchKernelGGL(k_cg_smu_init, dim3(ceil_div(6L * P.K, 256)), dim3(256), 0, s, P, E.S, E.cg_smu);
-        el_cg_apply_ksum(E, P, false, 0, s);
-    } else {
-        el_cg_apply_other(E, P, *sp, false, 0, s);
-    }
+    if (!sp) el_cg_apply_ksum(E, P, false, 0, s);
+    else el_cg_apply_other(E, P, *sp, false, 0, s);
     el_cg_update(E, P, sp, true, s);
     return (int)hipGetLastError();
 }
 
 // Iteration `it` (0-based): the stopping test and scalars from the last update's partials,
 // n = A m (real-space rows, structure factors, reciprocal field), then the vector update.
-// With the particle mesh or no reciprocal space the structure factors are not carried.
 int el_launch_cg_iteration(ElecBuffers& E, const ElecDev& P, int it, const ElecSpme* sp, hipStream_t s)
 {
     if (sp) el_cg_apply_other(E, P, *sp, true, it, s);
@@ -2381,8 +2363,7 @@ int el_time_sfac(ElecBuffers& E, const ElecDev& P, int reps, hipEvent_t a, hipEv
 {
     (void)hipEventRecord(a, s);
     for (int r = 0; r < reps; ++r)
-        hipLaunchKernelGGL(k_el_sfac<false>, dim3(ceil_div((long)EL_SPLIT * P.nrun, 64), E.dchunks), dim3(64 * EL_SG), sfac_lds(P), s, P,
-                           E.dspc, E.runs, E.runk, E.phc, E.phs, E.chge, E.dip, E.Spart, E.zero_state, nullptr, 0, 0);
+        rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.nrow}}}, 1, P.rs.nch, P.rs.spc, false, E.zero_state, nullptr, 0, 0, s);
     (void)hipEventRecord(b, s);
     return (int)hipGetLastError();
 }
@@ -2390,14 +2371,11 @@ int el_time_sfac(ElecBuffers& E, const ElecDev& P, int reps, hipEvent_t a, hipEv
 int el_launch_final(ElecBuffers& E, const ElecDev& P, int distribute, double g34, double gln34, int refresh,
                     const ElecSpme* sp, hipStream_t s)
 {
-    // fields and structure factors of the final dipoles: carried along by the conjugate-
-    // gradient solver; the SOR path keeps those of its last iteration, as the reference does
-    // (the particle mesh carries no structure factors)
-    if (refresh) {
-        const ElecDev Q = sp ? one_chunk(P) : P;
-        hipLaunchKernelGGL(k_cg_final_fields, dim3(ceil_div(std::max(3L * Q.nrow, 6L * Q.K), 256)), dim3(256), 0, s, Q,
-                           E.cg_tmu, E.cg_smu, E.emu, E.efdd, E.S);
-    }
+    // fields of the final dipoles: carried along by the conjugate-gradient solver; the SOR path
+    // keeps those of its last iteration, as the reference does
+    if (refresh)
+        hipLaunchKernelGGL(k_cg_final_fields, dim3(ceil_div(3L * P.nrow, 256)), dim3(256), 0, s, P, E.cg_tmu, E.emu,
+                           E.efdd);
     // k-sum: one partial per 256 k; particle mesh: one per 4 sites (k_sp_elec_final's blocks)
     const int nsb = ceil_div(P.n, 256), nwb = ceil_div(P.nw, 64), nkb = sp ? ceil_div(P.n, 4) : ceil_div(P.K, 256);
     double* b_pol = E.blk;                       // [nsb]
@@ -2434,15 +2412,12 @@ int el_launch_final(ElecBuffers& E, const ElecDev& P, int distribute, double g34
         sp_launch_influence(B, G, g + B.ng_cap, 4, false, nullptr, s);
         sp_launch_fft(B, G, g, 11, true, nullptr, s, false);
         sp_launch_elec_final(B, G, P.n, E.chge, E.dip, g, sp->kap, E.ksum, b_ks, s);
-    } else if (!refresh) {
-        // structure factors of the converged dipoles (already computed with the refreshed fields)
-        hipLaunchKernelGGL(k_el_sfac<false>, dim3(ceil_div((long)EL_SPLIT * P.nrun, 64), E.dchunks), dim3(64 * EL_SG), sfac_lds(P), s, P,
-                           E.dspc, E.runs, E.runk, E.phc, E.phs, E.chge, E.dip, E.Spart, E.zero_state, nullptr, 0, 0);
-        hipLaunchKernelGGL(k_el_sreduce<false>, dim3(ceil_div(6L * P.K, 60)), dim3(256), 0, s, P, E.dchunks, E.Spart, E.kv, E.S, E.Sq, E.kc,
-                           (const double*)E.zero_state);
     }
     if (!sp) {
-        hipLaunchKernelGGL(k_el_kscal, dim3(nkb), dim3(256), 0, s, P, E.kv, E.S, E.Sq, E.kf, b_ks);
+        // structure factors of mu_x, mu_y, mu_z of the converged dipoles and of the charges
+        rs_launch_sfac(E, P, {{{E.dip, 3, 0, P.nrow}, {E.dip + 1, 3, 0, P.nrow}, {E.dip + 2, 3, 0, P.nrow}, {E.chge, 1, 0, P.n}}},
+                       4, P.rs.nchq, P.rs.spcq, false, E.zero_state, nullptr, 0, 0, s);
+        hipLaunchKernelGGL(k_el_kscal, dim3(nkb), dim3(256), 0, s, P, E.kv, E.Spart, E.kf, b_ks);
         hipLaunchKernelGGL(k_el_kfinal, dim3(ceil_div(P.n, 256), P.kchunks), dim3(256), kfinal_lds(P), s, P, E.runs,
                            E.runk, E.phc, E.phs, E.kv, E.kf, E.chge, E.dip, E.Fpart);
         hipLaunchKernelGGL(k_el_ksum, dim3(ceil_div(15L * P.n, 64)), dim3(256), 0, s, P, E.Fpart, E.ksum);

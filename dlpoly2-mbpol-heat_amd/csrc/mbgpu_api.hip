@@ -1784,7 +1784,7 @@ int mbgpu_time_elec(mbgpu_ctx* c, int reps, double* ms_sfac, double* flop_sfac)
     const int npol = 2 * S.nw * (S.P.polr2[1] > 1.e-6) + S.nw * (S.P.polr2[0] > 1.e-6) +
                      S.nw * (S.P.polr2[2] > 1.e-6);
     if (ms_sfac) *ms_sfac = ms / reps;
-    if (flop_sfac) *flop_sfac = 18.0 * S.P.K * npol;
+    if (flop_sfac) *flop_sfac = 8.0 * S.P.K * npol;
     return 0;
 }
 

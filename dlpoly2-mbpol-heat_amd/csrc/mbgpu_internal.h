@@ -122,6 +122,24 @@ struct MbBuffers {
 
 // ------------------------------------------------------------------ electrostatics ----
 
+// The k list as the matrix passes take it (k_rs_sfac, k_rs_field): its (l, m) pairs in
+// groups of 16, pairs with many n first, and n in tiles of 8.  A slot of structure factors
+// holds, per tile, [+n, -n][16 pairs][re, im][8 n], then the n = 0 ones
+// [re, im][16 pairs].
+struct RsPlan {
+    int ng, ntiles;                // groups of 16 pairs, most tiles of 8 n in a group
+    int kt, ky, kz;                // entries per site of the phase table pht; its m = 0 and n = 0 (m from -km to km)
+    int nch, spc;                  // site chunks of the dipole passes, sites per chunk
+    int nchq, spcq;                // the same over all sites (charges, final pass)
+    double rc[9];                  // inverse cell
+    const int4* pair;              // [ng * 16] l, m, largest |n|, tiles of the group
+    const double2* ak;             // [ng * 16][8 ntiles + 1] akk of (l, m, +n) and (l, m, -n), 0 where not in the list
+    const int* kpos;               // [K] (group * 16 + pair) << 8 | |n| << 1 | (n < 0)
+};
+#define RS_SLOT(ntiles) (512L * (ntiles) + 32)
+#define RS_PAD 4                      // sites past the last that the passes may read
+#define RS_MAX_SPC 1024               // most sites of a chunk (their weights are staged in LDS)
+
 // Kernel-argument block of the polarizable electrostatics (passed by value).
 struct ElecDev {
     int nw, n, nreal, nrow;        // waters, sites (4nw), real atoms (3nw), rows carrying dipoles
@@ -134,18 +152,24 @@ struct ElecDev {
     double drewd;                  // B-function table spacing
     int compat_qd;                 // qdforce M column as the reference (n_water + imol)
     int capA, capP;                // neighbour-row capacities (all partners / polarizable partners)
-    int K, nrun, kchunks;          // k vectors, runs of consecutive n, k chunks of the site-parallel passes
+    int K, nrun, kchunks;          // k vectors, runs of consecutive n, k chunks of the final pass
     int rpc, kmaxch;               // runs per k chunk, most k vectors in one chunk (final pass)
-    int fchunks, frpc, fkmax;      // the same for the field passes
+    int fchunks;                   // partials of a field pass (k-sum: the groups of rs)
     int km[3], kstride;            // kmax per axis, phase-table stride (max kmax + 1)
+    RsPlan rs;                     // k-sum: the (l, m) pairs and chunks of the matrix passes
     double scale, scal1, rvolm, self_dd;   // 4 rvolm r4pie0, 2 rvolm r4pie0, 2 pi/V, 4 r4pie0 a^3/(3 sqrt(pi))
 };
 
 // Device buffers of the electrostatics (owned by the context).
 struct ElecBuffers {
-    int n = 0, capA = 0, capP = 0, K = 0, nrun = 0, kchunks = 0, schunks = 0, ntab = 0, kstride = 0;
-    int spc = 0, dchunks = 0, dspc = 0, rpc = 0, kmaxch = 0;   // site chunks of the structure-factor passes
-    int fchunks = 0, frpc = 0, fkmax = 0;                      // k chunks of the field passes
+    int n = 0, capA = 0, capP = 0, K = 0, nrun = 0, kchunks = 0, ntab = 0, kstride = 0;
+    int rpc = 0, kmaxch = 0;                                   // k chunks of the final pass
+    int fchunks = 0;                                           // partials of a field pass
+    RsPlan rs{};                                               // k-sum: plan of the matrix passes
+    int4* rs_pair = nullptr;                                   // its arrays (see RsPlan)
+    double2* rs_ak = nullptr;
+    int* rs_kpos = nullptr;
+    double2* pht = nullptr;                                    // [n][kt] (cos, sin) of l, m, n per site
     double *x = nullptr, *y = nullptr, *z = nullptr;          // [n] site positions
     double *chge = nullptr, *polr = nullptr, *polr2 = nullptr; // [n]
     double* dg = nullptr;                                      // [nw][6] DMS derivatives
@@ -159,21 +183,18 @@ struct ElecBuffers {
     double *cg_p = nullptr, *cg_q = nullptr, *cg_r = nullptr, *cg_z = nullptr;                // [3n] solver vectors
     double *cg_u = nullptr, *cg_w = nullptr, *cg_m = nullptr, *cg_s = nullptr;                // [3n]
     double* cg_minv = nullptr;                                 // [nw][45] inverse preconditioner blocks
-    double *cg_tmu = nullptr, *cg_smu = nullptr;               // [3n] T mu, [K][6] S(mu) carried by the solver
-    double *cg_sp = nullptr, *cg_su = nullptr, *cg_sq = nullptr;   // [K][6] S(p), S(u), S(q) carried by the solver
+    double* cg_tmu = nullptr;                                  // [3n] T mu carried by the solver
     double* cgblk = nullptr;                                   // block partials of the solver kernels
     double* ksum = nullptr;                                    // [16][n] chunk sums of the final pass
     double* state = nullptr;                                   // [16] solver scalars
     double* kv = nullptr;                                      // [K][8] kx ky kz akk akv akv2 . .
     int* runs = nullptr;                                       // [nrun][4] l, m, n0, count; k0 in runk
     int* runk = nullptr;                                       // [nrun] index of the run's first k
-    int* klmn = nullptr;                                       // [K] l << 16 | (m+128) << 8 | (n+128)
     double *phc = nullptr, *phs = nullptr;                     // [3][kstride][n] cos / sin of l*2pi*s_a
-    double *S = nullptr, *Spart = nullptr;                     // [K][8], [schunks][K][8]
-    double* Sq = nullptr;                                      // [K][2] charge structure factors
-    double *kc = nullptr, *kf = nullptr;                       // [K][16] per-k constants of the passes
+    double* Spart = nullptr;                                   // [4][chunks][groups][slot] structure-factor sums
+    double* kf = nullptr;                                      // [K][16] per-k constants of the final pass
     double* zero_state = nullptr;                              // [8] zeros (solver state of final passes)
-    double* Fpart = nullptr;                                   // [kchunks][16][n] site partials
+    double* Fpart = nullptr;                                   // [kchunks][16][n], [fchunks][6][n] site partials
     double *vk = nullptr, *vr = nullptr, *vs = nullptr, *vc = nullptr, *vdck = nullptr, *vdcr = nullptr,
            *vesp = nullptr;                                    // [n]
     double *fk = nullptr, *f2 = nullptr, *f3 = nullptr, *fsite = nullptr;  // [3n]

@@ -446,8 +446,9 @@ int mbgpu_time_forces(mbgpu_ctx* ctx, int reps, double* ms_per_eval, double* ms_
 /* Timing helper: `reps` launches of the reciprocal-space dipole structure-factor kernel on
  * the dipoles of the last mbgpu_polar_electrostatics(_dev) call, timed with HIP events on
  * the library's stream.  Returns the mean milliseconds per launch and the algorithmic
- * FLOP of one launch: 18 per (k vector, polarizable site) -- six multiply-adds of the
- * dipole components into Re/Im S(k) and the complex phase recurrence along n. */
+ * FLOP of one launch: 8 per (k vector, polarizable site) -- the real and the imaginary part
+ * of S(k) each take one multiply-add with the dipole's a* and b* components and one with
+ * its c* component. */
 int mbgpu_time_elec(mbgpu_ctx* ctx, int reps, double* ms_sfac, double* flop_sfac);
 
 #ifdef __cplusplus
