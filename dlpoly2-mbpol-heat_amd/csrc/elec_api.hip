@@ -21,6 +21,10 @@
 #ifndef EL_KCHUNK_RUNS
 #define EL_KCHUNK_RUNS 32     // at most this many k runs per chunk of the final reciprocal pass
 #endif
+// Most solver iterations enqueued (or captured in a graph) at once.  SOR from zero dipoles takes
+// 70 to 80: with a bound of 64 a captured evaluation always ended unconverged and the one-call
+// evaluation was repeated launch by launch (216 waters: 6.05 -> 3.03 ms with the bound at 256).
+#define EL_MAX_BATCH 256
 #define PI_D 3.141592653589793
 
 namespace {
@@ -632,7 +636,7 @@ int elec_batch(const ElecState& S)
 {
     int gb = 0;
     if (S.last_iters > 0) {
-        gb = std::min(S.last_iters + 2, 64);
+        gb = std::min(S.last_iters + 2, EL_MAX_BATCH);
         if (S.gbatch >= S.last_iters && S.gbatch <= S.last_iters + 8) gb = S.gbatch;
     }
     if (const char* ev = getenv("MBGPU_GRAPH_BATCH")) gb = gb ? std::min(gb, std::max(1, atoi(ev))) : 0;
@@ -801,7 +805,7 @@ int elec_evaluate(ElecState& S, int max_iter, int distribute, int solver, hipStr
     // with clamped counts, so an overflowed attempt runs in bounds and is simply repeated
     // with larger rows, from the same start dipoles (kept in dip0).
     for (int attempt = from_graph ? -1 : (S.gexec && herr ? 1 : 0); attempt >= 0 || from_graph;) {
-        int launched = 0, batch = S.last_iters > 0 ? std::min(S.last_iters + 2, 64) : (solver == 1 ? 8 : 12);
+        int launched = 0, batch = S.last_iters > 0 ? std::min(S.last_iters + 2, EL_MAX_BATCH) : (solver == 1 ? 8 : 12);
         int rc = 0;
         if (from_graph) {
             // continue after the graph's iterations
