@@ -152,7 +152,7 @@ int alloc_rows(ElecState& S, int capA, int capP, std::string& err)
     E.capP = capP;
     ECHK(dalloc(&E.nbrA, (size_t)E.n * capA));
     ECHK(dalloc(&E.nbrP, (size_t)E.n * capP));
-    ECHK(dalloc(&E.tens, (size_t)6 * E.n * capP));
+    ECHK(dalloc(&E.tens, (size_t)E.n * capP));
     return 0;
 }
 
@@ -493,6 +493,8 @@ int elec_configure(ElecState& S, int nw, const CellGeom& g, const double* cell, 
         P.polr2[i] = p->polr2[i];
         P.km[i] = p->kmax[i];
     }
+    for (int i = 0; i < 3; ++i)
+        for (int j = 0; j < 3; ++j) P.bbi[i][j] = 1.0 / pow(p->polr[i] * p->polr[j], 1.0 / 6.0);
     P.athole = p->athole;
     P.athole12 = p->athole12;
     P.athole13 = p->athole13;

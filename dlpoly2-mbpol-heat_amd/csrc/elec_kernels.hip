@@ -144,6 +144,12 @@ __device__ __forceinline__ double site_polr2(const ElecDev& P, int i)
     return i >= P.nreal ? P.polr2[2] : ((i % 3) == 0 ? P.polr2[0] : P.polr2[1]);
 }
 
+// 0 O, 1 H, 2 M
+__device__ __forceinline__ int site_type(const ElecDev& P, int i)
+{
+    return i >= P.nreal ? 2 : ((i % 3) == 0 ? 0 : 1);
+}
+
 // erfcc.f: Numerical Recipes erfc with single-precision literals promoted to double.
 __device__ double erfcc_nr(double x)
 {
@@ -212,11 +218,17 @@ __device__ double gammq_nr(double a, double x, double gln)
     return exp(lf) * h;
 }
 
-// 3-point interpolation of the B-function table (rfield.f:102-120, ewald2p.f:160-178)
-__device__ __forceinline__ void table_interp(const double* __restrict__ t, double drewd, double rr, double* bbb)
+// 3-point interpolation of the B-function table (rfield.f:102-120, ewald2p.f:160-178); without
+// an Ewald split the functions vanish (an isolated cluster)
+__device__ __forceinline__ void table_interp(const ElecDev& P, const double* __restrict__ t, double rr, double* bbb)
 {
-    const int ll = (int)(rr / drewd);
-    const double ppp = rr / drewd - (double)ll;
+    if (P.alpha < 1.0e-6) {
+        bbb[0] = bbb[1] = bbb[2] = bbb[3] = 0.0;
+        return;
+    }
+    const double q = rr / P.drewd;
+    const int ll = (int)q;
+    const double ppp = q - (double)ll;
     const double* r0 = t + 4 * ll;
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
@@ -404,72 +416,65 @@ __global__ __launch_bounds__(64) void k_el_nbr(ElecDev P, const double* __restri
 
 // Per-row set-up of the real-space fields (rfield.f:62-323): the charge field of the row's
 // partners (iloop = 1 part, with the lads smearing) and the Thole-damped dipole tensors of
-// its polarizable partners (stored SoA [6][n][capP]).  One wavefront per site.
+// its polarizable partners, T = t2 d d^T - t1 1 with d the imaged separation, stored as their
+// radial factors (t1, t2) [n][capP]: the solver reads them every iteration, and 16 bytes and a
+// separation formed again cost less there than the six components did (emu_row).  One
+// wavefront per site, one pass over its partners: row P holds the polarizable ones in row A's
+// order, so a partner's place in it is the count of those before.
 __global__ __launch_bounds__(64) void k_el_prep(ElecDev P, const double* __restrict__ x,
                                                 const double* __restrict__ y, const double* __restrict__ z,
                                                 const double* __restrict__ chge, const double* __restrict__ tab,
                                                 const int* __restrict__ nbrA, const int* __restrict__ cntA,
-                                                const int* __restrict__ nbrP, const int* __restrict__ cntP,
-                                                double* __restrict__ tens, double* __restrict__ efk)
+                                                double2* __restrict__ tens, double* __restrict__ efk)
 {
     const int i = blockIdx.x;
     const int lane = threadIdx.x;
     if (i >= P.n) return;
-    const double pi_ = site_polr(P, i);
+    const bool poli = site_polr2(P, i) > 1.e-6;
+    const int ti = site_type(P, i);
+    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     double e[3] = {0.0, 0.0, 0.0};
     const int na = cntA[i];
-    for (int s = lane; s < na; s += 64) {
-        const int j = nbrA[(long)i * P.capA + s];
+    int np = 0;
+    for (int base = 0; base < na; base += 64) {
+        const int s = base + lane;
+        const bool in = s < na;
+        const int j = in ? nbrA[(long)i * P.capA + s] : i;
+        const bool inP = in && poli && site_polr2(P, j) > 1.e-6;
+        const unsigned long long bP = __ballot(inP);
+        const int sp = np + __popcll(bP & below);
+        np += __popcll(bP);
+        if (!in) continue;
         double d[3];
         const double r2 = sep(P, x, y, z, i, j, d);
         const double rr = sqrt(r2);
-        if (!(P.rcut > rr)) continue;
-        double bbb[4];
-        table_interp(tab, P.drewd, rr, bbb);
-        const double r3i = 1.0 / (rr * rr * rr);
-        const double bb = pow(pi_ * site_polr(P, j), 1.0 / 6.0);
-        const double u = rr / bb;
-        const double arob4 = P.ascd * (u * u) * (u * u);
-        const double dum1 = exp(-arob4);
-        double eki = R4PIE0 * chge[j] * (bbb[1] + r3i);
-        eki = eki - R4PIE0 * chge[j] * dum1 * r3i;
-        e[0] += eki * d[0];
-        e[1] += eki * d[1];
-        e[2] += eki * d[2];
+        double t1 = 0.0, t2 = 0.0;
+        if (P.rcut > rr) {
+            double bbb[4];
+            table_interp(P, tab, rr, bbb);
+            const double rri = 1.0 / rr, rsqi = rri * rri;
+            const double r3i = rri * rsqi;
+            const double u = rr * P.bbi[ti][site_type(P, j)];
+            const double u4 = (u * u) * (u * u);
+            const double dumq = exp(-P.ascd * u4);
+            const double eki = R4PIE0 * chge[j] * (bbb[1] + r3i * (1.0 - dumq));
+            e[0] += eki * d[0];
+            e[1] += eki * d[1];
+            e[2] += eki * d[2];
+            if (inP) {
+                const double arob4 = P.athole * u4;
+                const double dum1 = exp(-arob4);
+                const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
+                t1 = R4PIE0 * (bbb[1] + r3i * (1.0 - dum1));
+                t2 = R4PIE0 * (bbb[2] + 3.0 * r3i * rsqi * (1.0 - dum2));
+            }
+        }
+        // (a partner of the row's margin past rcut has no tensor)
+        if (inP && sp < P.capP) tens[(long)i * P.capP + sp] = make_double2(t1, t2);
     }
     for (int q = 0; q < 3; ++q) e[q] = wsum(e[q]);
     if (lane == 0)
         for (int q = 0; q < 3; ++q) efk[3 * i + q] = e[q];
-    const int np = cntP[i];
-    const long nc = (long)P.n * P.capP;
-    for (int s = lane; s < np; s += 64) {
-        const int j = nbrP[(long)i * P.capP + s];
-        double d[3];
-        const double r2 = sep(P, x, y, z, i, j, d);
-        const double rr = sqrt(r2);
-        double dt[6] = {0, 0, 0, 0, 0, 0};
-        if (P.rcut > rr) {
-            double bbb[4];
-            table_interp(tab, P.drewd, rr, bbb);
-            const double rsqi = 1.0 / r2;
-            const double r3i = 1.0 / (rr * rr * rr);
-            const double r5i = r3i * rsqi;
-            const double bb = pow(pi_ * site_polr(P, j), 1.0 / 6.0);
-            const double u = rr / bb;
-            const double arob4 = P.athole * (u * u) * (u * u);
-            const double dum1 = exp(-arob4);
-            const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
-            const double rij[6] = {d[0] * d[0], d[0] * d[1], d[0] * d[2], d[1] * d[1], d[1] * d[2], d[2] * d[2]};
-#pragma unroll
-            for (int q = 0; q < 6; ++q) {
-                const bool dg_ = (q == 0 || q == 3 || q == 5);
-                dt[q] = R4PIE0 * ((3.0 * rij[q] * r5i - (dg_ ? r3i : 0.0)) + rij[q] * bbb[2] - (dg_ ? bbb[1] : 0.0));
-                dt[q] = dt[q] - (3.0 * rij[q] * r5i * dum2 - (dg_ ? dum1 * r3i : 0.0)) * R4PIE0;
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < 6; ++q) tens[q * nc + (long)i * P.capP + s] = dt[q];
-    }
 }
 
 // Excluded (intramolecular) pairs of each water (rfield.f:327-525): charge field with the
@@ -579,31 +584,38 @@ __device__ __forceinline__ void run_phase(double el_c, double el_s, double em_c,
 }  // namespace
 
 // Real-space dipole field of one row (rfield.f:201-317 list pairs; 419-520 excluded
-// pairs): emu_i = sum_j T_ij mu_j.  One wavefront per site.
-__device__ void emu_row(const ElecDev& P, int i, int lane, const int* __restrict__ nbrP, const int* __restrict__ cntP,
-                        const double* __restrict__ tens, const double* __restrict__ tin,
+// pairs): emu_i = sum_j T_ij mu_j with T_ij = t2 d d^T - t1 1, by one wavefront, or by the WPR
+// of a block of 64 WPR threads (which all call it).  Bound by the factors' bytes (88 MB a pass
+// for a 701-water cluster, 230 MB when the six tensor components were stored: 38.5 -> 28.7 us) and,
+// with one wavefront to a long row, by the chain of its gathers.
+template <int WPR>
+__device__ void emu_row(const ElecDev& P, int i, int t, const double* __restrict__ x, const double* __restrict__ y,
+                        const double* __restrict__ z, const int* __restrict__ nbrP, const int* __restrict__ cntP,
+                        const double2* __restrict__ tens, const double* __restrict__ tin,
                         const double* __restrict__ dip, double* __restrict__ emu)
 {
     if (i >= P.nrow) return;
-    const long nc = (long)P.n * P.capP;
     double e[3] = {0, 0, 0};
     const int np = cntP[i];
-    for (int s = lane; s < np; s += 64) {
+#pragma unroll 2
+    for (int s = t; s < np; s += 64 * WPR) {
         const long o = (long)i * P.capP + s;
         const int j = nbrP[o];
+        const double2 tt = tens[o];
         const double mx = dip[3 * j], my = dip[3 * j + 1], mz = dip[3 * j + 2];
-        const double t0 = tens[o], t1 = tens[nc + o], t2 = tens[2 * nc + o];
-        const double t3 = tens[3 * nc + o], t4 = tens[4 * nc + o], t5 = tens[5 * nc + o];
-        e[0] += t0 * mx + t1 * my + t2 * mz;
-        e[1] += t1 * mx + t3 * my + t4 * mz;
-        e[2] += t2 * mx + t4 * my + t5 * mz;
+        double d[3];
+        (void)sep(P, x, y, z, i, j, d);
+        const double f = tt.y * (d[0] * mx + d[1] * my + d[2] * mz);
+        e[0] += f * d[0] - tt.x * mx;
+        e[1] += f * d[1] - tt.x * my;
+        e[2] += f * d[2] - tt.x * mz;
     }
     // excluded partners of the same water on lanes 0 and 1: the other two real sites (the M
     // site carries no induced dipole and its entries are not part of the solve); pair order
     // of tin: (O,H1) (O,H2) (O,M) (H1,H2) (H1,M) (H2,M)
-    if (lane < 2) {
+    if (t < 2) {
         const int w = i / 3, si = i - 3 * w;
-        const int pt = lane < si ? lane : lane + 1;
+        const int pt = t < si ? t : t + 1;
         const int a = min(si, pt), b = max(si, pt);
         const int pr = a == 0 ? b - 1 : 3;
         const int j = 3 * w + pt;
@@ -615,9 +627,13 @@ __device__ void emu_row(const ElecDev& P, int i, int lane, const int* __restrict
             e[2] += dt[2] * mx + dt[4] * my + dt[5] * mz;
         }
     }
-    for (int q = 0; q < 3; ++q) e[q] = wsum(e[q]);
-    if (lane == 0)
-        for (int q = 0; q < 3; ++q) emu[3 * i + q] = e[q];
+    if constexpr (WPR == 1) {
+        for (int q = 0; q < 3; ++q) e[q] = wsum(e[q]);
+        if (t == 0)
+            for (int q = 0; q < 3; ++q) emu[3 * i + q] = e[q];
+    } else {
+        block_sum_store(e, emu + 3 * i);
+    }
 }
 
 // ------------------------------------------- Ewald sums as FP64 matrix products ------
@@ -814,9 +830,10 @@ __device__ void rs_sfac_block(const ElecDev& P, const RsSrc src, int spc, int g,
 template <int NT>
 __global__ __launch_bounds__(64 * RS_WAVES) void k_rs_sfac(ElecDev P, RsSrcs src, int nsb, int nch, int spc,
                                                            const double2* __restrict__ pht,
-                                                           double* __restrict__ Spart, const int* __restrict__ nbrP,
-                                                           const int* __restrict__ cntP,
-                                                           const double* __restrict__ tens,
+                                                           double* __restrict__ Spart, const double* __restrict__ x,
+                                                           const double* __restrict__ y, const double* __restrict__ z,
+                                                           const int* __restrict__ nbrP, const int* __restrict__ cntP,
+                                                           const double2* __restrict__ tens,
                                                            const double* __restrict__ tin, double* __restrict__ emu,
                                                            double* __restrict__ state,
                                                            const double* __restrict__ cgblk, int cgnb, int it)
@@ -827,7 +844,8 @@ __global__ __launch_bounds__(64 * RS_WAVES) void k_rs_sfac(ElecDev P, RsSrcs src
     const RsPlan& R = P.rs;
     int b = blockIdx.x;
     if (b >= nsb) {
-        emu_row(P, (b - nsb) * RS_WAVES + (threadIdx.x >> 6), threadIdx.x & 63, nbrP, cntP, tens, tin, src.s[0].v, emu);
+        emu_row<1>(P, (b - nsb) * RS_WAVES + (threadIdx.x >> 6), threadIdx.x & 63, x, y, z, nbrP, cntP, tens, tin,
+                src.s[0].v, emu);
         return;
     }
     // chunks fastest: with 8 chunks (one per XCD, see build_rs) the blocks of an XCD read the
@@ -1028,18 +1046,23 @@ __global__ __launch_bounds__(256) void k_el_kfield_reduce(ElecDev P, const doubl
 
 // ============================================================ solver iteration ======
 
-// emu for four rows per block.  With cgblk (the conjugate-gradient solver's partials, cgnb
-// blocks), the solver's stopping test for iteration `it` comes first (cg_step; block 0
-// records the scalars) and the kernel does nothing once the dipoles have converged.
-__global__ __launch_bounds__(256) void k_el_emu(ElecDev P, const int* __restrict__ nbrP, const int* __restrict__ cntP,
-                                                const double* __restrict__ tens, const double* __restrict__ tin,
+// emu for a row per WPR wavefronts, blocks of four.  With cgblk (the conjugate-gradient
+// solver's partials, cgnb blocks), the solver's stopping test for iteration `it` comes first
+// (cg_step; block 0 records the scalars) and the kernel does nothing once the dipoles have
+// converged.
+template <int WPR>
+__global__ __launch_bounds__(256) void k_el_emu(ElecDev P, const double* __restrict__ x, const double* __restrict__ y,
+                                                const double* __restrict__ z, const int* __restrict__ nbrP,
+                                                const int* __restrict__ cntP, const double2* __restrict__ tens,
+                                                const double* __restrict__ tin,
                                                 const double* __restrict__ dip, double* __restrict__ emu,
                                                 double* __restrict__ state, const double* __restrict__ cgblk, int cgnb,
                                                 int it)
 {
     if (state[2] != 0.0) return;
     if (cgblk && cg_step(P, it, cgnb, cgblk, state, blockIdx.x == 0 && threadIdx.x < 64)) return;
-    emu_row(P, blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & 63, nbrP, cntP, tens, tin, dip, emu);
+    constexpr int T = 64 * WPR;
+    emu_row<WPR>(P, blockIdx.x * (4 / WPR) + threadIdx.x / T, threadIdx.x % T, x, y, z, nbrP, cntP, tens, tin, dip, emu);
 }
 
 // SOR update (iter.f:58-89) and per-block sums of |dmu|^2 and of the dipole count.
@@ -1679,7 +1702,7 @@ __global__ __launch_bounds__(64) void k_el_pairs(ElecDev P, const double* __rest
         if (!(P.rcut * P.rcut > rsq)) continue;
         const double rrr = sqrt(rsq);
         double bbb[4];
-        table_interp(tab, P.drewd, rrr, bbb);
+        table_interp(P, tab, rrr, bbb);
         const double rri = 1.0 / rrr, rsqi = 1.0 / rsq;
         const double r3i = 1.0 / (rrr * rrr * rrr);
         const double r5i = r3i * rsqi;
@@ -2156,6 +2179,20 @@ inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 inline size_t rs_lds(int spc) { return sizeof(double) * std::max(512L * RS_WAVES, 4L * spc); }
 inline size_t kfinal_lds(const ElecDev& P) { return sizeof(double) * ((size_t)P.kmaxch * EL_KF + 2 * (size_t)P.rpc + 2); }
 
+// The real-space field of dip: four wavefronts to a row where rows are long (a cluster's hold
+// every other polarizable site; 300 waters 8.7 -> 7.3 us, 701 waters 28.7 -> 23.4), one where a
+// block per row costs more than it shortens (2048-water box, 305 partners: 15.2 against 22.6).
+void launch_emu(const ElecBuffers& E, const ElecDev& P, const double* dip, double* state, const double* cgblk, int cgnb,
+                int it, hipStream_t s)
+{
+    if (P.capP >= 512 && P.g.imcon == 0)
+        hipLaunchKernelGGL(k_el_emu<4>, dim3(P.nrow), dim3(256), 0, s, P, E.x, E.y, E.z, E.nbrP, E.cntP, E.tens, E.tin,
+                           dip, E.emu, state, cgblk, cgnb, it);
+    else
+        hipLaunchKernelGGL(k_el_emu<1>, dim3(ceil_div(P.nrow, 4)), dim3(256), 0, s, P, E.x, E.y, E.z, E.nbrP, E.cntP,
+                           E.tens, E.tin, dip, E.emu, state, cgblk, cgnb, it);
+}
+
 // Structure factors of nset sets of weights over nch chunks of spc sites; with emu also the
 // real-space field of set 0 (dipoles).  Tiles of n per block: as many as the list needs, up to 4
 // (more are spread over blocks; each costs 16 accumulator registers).
@@ -2165,7 +2202,7 @@ void rs_launch_sfac_t(const ElecBuffers& E, const ElecDev& P, const RsSrcs& src,
 {
     const int nsb = P.rs.ng * ceil_div(P.rs.ntiles, NT) * nch * nset;
     hipLaunchKernelGGL(k_rs_sfac<NT>, dim3(nsb + (emu ? ceil_div(P.nrow, RS_WAVES) : 0)), dim3(64 * RS_WAVES), rs_lds(spc),
-                       s, P, src, nsb, nch, spc, E.pht, E.Spart, E.nbrP, E.cntP, E.tens, E.tin, E.emu, state, cgblk,
+                       s, P, src, nsb, nch, spc, E.pht, E.Spart, E.x, E.y, E.z, E.nbrP, E.cntP, E.tens, E.tin, E.emu, state, cgblk,
                        cgnb, it);
 }
 void rs_launch_sfac(const ElecBuffers& E, const ElecDev& P, const RsSrcs& src, int nset, int nch, int spc, bool emu,
@@ -2231,8 +2268,8 @@ static inline ElecDev one_chunk(const ElecDev& P)
 int el_launch_prep(ElecBuffers& E, const ElecDev& P, const double* rcell_dev, const ElecSpme* sp, hipStream_t s)
 {
     const int nwb = ceil_div(P.nw, 64);
-    hipLaunchKernelGGL(k_el_prep, dim3(P.n), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.tab, E.nbrA, E.cntA, E.nbrP,
-                       E.cntP, E.tens, E.efk);
+    hipLaunchKernelGGL(k_el_prep, dim3(P.n), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.tab, E.nbrA, E.cntA,
+                       E.tens, E.efk);
     hipLaunchKernelGGL(k_el_intra_prep, dim3(nwb), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.tin, E.efk);
     if (sp && !sp->B) {
         // no reciprocal space (an isolated cluster): zero fields, in the layout of the k-sum
@@ -2289,8 +2326,7 @@ int el_launch_iteration(ElecBuffers& E, const ElecDev& P, int first, const ElecS
                            E.efdd, E.efdc, E.state);
     }
     if (first || sp)
-        hipLaunchKernelGGL(k_el_emu, dim3(ceil_div(P.nrow, 4)), dim3(256), 0, s, P, E.nbrP, E.cntP, E.tens, E.tin, E.dip,
-                           E.emu, E.state, nullptr, 0, 0);
+        launch_emu(E, P, E.dip, E.state, nullptr, 0, 0, s);
     const int nb = ceil_div(P.nrow, 256);
     hipLaunchKernelGGL(k_el_sor, dim3(nb), dim3(256), 0, s, P, E.efk, E.emu, E.efdd, E.efdc, E.dip, E.blk, E.state);
     hipLaunchKernelGGL(k_el_converge, dim3(1), dim3(64), 0, s, P, nb, E.blk, E.state);
@@ -2312,8 +2348,7 @@ static void el_cg_apply_ksum(ElecBuffers& E, const ElecDev& P, bool check, int i
 static void el_cg_apply_other(ElecBuffers& E, const ElecDev& P, const ElecSpme& sp, bool check, int it, hipStream_t s)
 {
     const int nbw = ceil_div(P.nw, CG_WPB);
-    hipLaunchKernelGGL(k_el_emu, dim3(ceil_div(P.nrow, 4)), dim3(256), 0, s, P, E.nbrP, E.cntP, E.tens, E.tin, E.cg_m,
-                       E.emu, E.state, check ? E.cgblk : nullptr, nbw, it);
+    launch_emu(E, P, E.cg_m, E.state, check ? E.cgblk : nullptr, nbw, it, s);
     if (sp.B) el_spme_dipole_field(E, sp, P.nrow, E.cg_m, E.state, s, 9);
 }
 
@@ -2336,8 +2371,7 @@ int el_launch_cg_init(ElecBuffers& E, const ElecDev& P, const ElecSpme* sp, hipS
 {
     const int nbw = ceil_div(P.nw, 256);
     hipLaunchKernelGGL(k_cg_block, dim3(nbw), dim3(256), 0, s, P, E.x, E.y, E.z, E.cg_minv);
-    hipLaunchKernelGGL(k_el_emu, dim3(ceil_div(P.nrow, 4)), dim3(256), 0, s, P, E.nbrP, E.cntP, E.tens, E.tin, E.dip,
-                       E.emu, E.state, nullptr, 0, 0);
+    launch_emu(E, P, E.dip, E.state, nullptr, 0, 0, s);
     hipLaunchKernelGGL(k_cg_init, dim3(nbw), dim3(256), 0, s, P, E.efk, E.efdc, E.emu, E.efdd, E.dip, E.cg_minv, E.cg_r,
                        E.cg_u, E.cg_m, E.cg_z, E.cg_q, E.cg_s, E.cg_p, E.cg_tmu);
     if (!sp) el_cg_apply_ksum(E, P, false, 0, s);

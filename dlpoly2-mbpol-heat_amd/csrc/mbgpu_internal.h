@@ -148,6 +148,7 @@ struct ElecDev {
     double rcut, alpha, gamma, q_o;
     double polr[3], polr2[3];      // O, H, M
     double athole, athole12, athole13, ascc, ascd;
+    double bbi[3][3];              // (polr_i polr_j)^(-1/6) by site types
     double toler, omega;
     double drewd;                  // B-function table spacing
     int compat_qd;                 // qdforce M column as the reference (n_water + imol)
@@ -176,7 +177,7 @@ struct ElecBuffers {
     double* tab = nullptr;                                     // [(ntab+1)*4] B-function table
     int *nbrA = nullptr, *cntA = nullptr;                      // [n][capA] partners within rcut
     int *nbrP = nullptr, *cntP = nullptr;                      // [n][capP] polarizable partners
-    double* tens = nullptr;                                    // [6][n*capP] dipole tensors
+    double2* tens = nullptr;                                   // [n][capP] radial factors of the dipole tensors
     double* tin = nullptr;                                     // [nw][6 pairs][6] intramolecular tensors
     double *dip = nullptr, *efk = nullptr, *emu = nullptr, *efdc = nullptr, *efdd = nullptr;  // [3n]
     double* dip0 = nullptr;                                    // [3n] start dipoles of the evaluation
