@@ -1664,12 +1664,49 @@ __global__ __launch_bounds__(256) void k_el_kfinal_reduce(ElecDev P, const doubl
     block_sum_store(v, blk + 2 * blockIdx.x);
 }
 
+namespace {
+
+// Sums over the wavefront of 24 values per lane: each step halves the values a lane carries
+// (25 exchanges instead of 144 for 24 butterflies).  Returns the sum of value `k` (on every lane
+// whose k is below 24), always added in the same order.
+__device__ __forceinline__ double wave_sum24(const double (&v)[24], int lane, int& k)
+{
+    double a[12], b[6], c[4], d[2];
+    const bool h5 = lane & 32, h4 = lane & 16, h3 = lane & 8, h2 = lane & 4, h1 = lane & 2;
+#pragma unroll
+    for (int q = 0; q < 12; ++q) a[q] = (h5 ? v[q + 12] : v[q]) + __shfl_xor(h5 ? v[q] : v[q + 12], 32, 64);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) b[q] = (h4 ? a[q + 6] : a[q]) + __shfl_xor(h4 ? a[q] : a[q + 6], 16, 64);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) c[q] = (h3 ? b[q + 3] : b[q]) + __shfl_xor(h3 ? b[q] : b[q + 3], 8, 64);
+    c[3] = 0.0;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) d[q] = (h2 ? c[q + 2] : c[q]) + __shfl_xor(h2 ? c[q] : c[q + 2], 4, 64);
+    double e = (h1 ? d[1] : d[0]) + __shfl_xor(h1 ? d[0] : d[1], 2, 64);
+    e += __shfl_xor(e, 1, 64);
+    const int r = 2 * h2 + h1;
+    k = r < 3 ? 12 * h5 + 6 * h4 + 3 * h3 + r : 24;
+    return e;
+}
+
+}  // namespace
+
 // Real-space pair terms of one row (ewald2p.f:118-600; nthole = 4, lacs, lads): forces,
 // per-atom energy, ESP parts, and the row's force-matrix contraction W_i (real partners
 // only; for an M-site row the partner sums sum_j F and sum_j F (x) x_j, from which the
 // M-row redistribution builds W of O, H1, H2).  Each pair is seen from both of its rows,
 // so block partials carry half of each pair's energy, virial and stress.  One wavefront
 // per site; partials [n][8]: energy, virial, stress (xx xy xz yy yz zz).
+//
+// Bound by FP64 arithmetic.  The smeared charge-charge energy (exp(-x) - x^1/4 Gamma(3/4)
+// Q(3/4, x)) / r, x = ascc u^4, is the dear part (the reference's continued fraction: tens of
+// divisions) and below 1e-26 of 1 / r from x = PAIR_XNEAR on, under a hundred-thousandth of the
+// last place of erfc(alpha r) / r at any real cut-off, so it is left out there: that leaves the
+// partners within 2.3 (H-H) to 3.9 A (O-O), a few per row, which are gathered in LDS and taken
+// 64 at a time instead of one or two lanes of each step.  With one exp less, the powers from
+// the host's table and the sums in 25 exchanges: 365 -> 107 us for a 701-water cluster, 46 -> 30
+// at 512 waters, 161 -> 94 at 2 048.
+#define PAIR_XNEAR 60.0
 __global__ __launch_bounds__(64) void k_el_pairs(ElecDev P, const double* __restrict__ x,
                                                  const double* __restrict__ y, const double* __restrict__ z,
                                                  const double* __restrict__ chge, const double* __restrict__ dip,
@@ -1680,140 +1717,136 @@ __global__ __launch_bounds__(64) void k_el_pairs(ElecDev P, const double* __rest
                                                  double* __restrict__ w2, double* __restrict__ fmsum,
                                                  double* __restrict__ fmx, double* __restrict__ blk)
 {
+    __shared__ double2 near[128];                      // (x, qj / r) of near partners waiting
+    __shared__ double sums[24];
     const int i = blockIdx.x;
     const int lane = threadIdx.x;
     if (i >= P.n) return;
+    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const double qi = chge[i];
-    const double pi_ = site_polr(P, i);
+    const int ti = site_type(P, i);
     const bool poli = site_polr2(P, i) > 1.e-6;
     const double mi[3] = {dip[3 * i], dip[3 * i + 1], dip[3 * i + 2]};
+    const double xi[3] = {x[i], y[i], z[i]};
     const bool mrow = i >= P.nreal;
-    double fsum[3] = {0, 0, 0}, esum = 0.0, vrs = 0.0, vdcs = 0.0, W[9], red[8];
+    // [0..2] force, [3] energy / 2, [4] vr, [5] vdcr, [6..14] W, [15..20] stress, [21..23] fm; without
+    // R4PIE0 until the end
+    double v[24];
 #pragma unroll
-    for (int t = 0; t < 9; ++t) W[t] = 0.0;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) red[t] = 0.0;
-    double fm[3] = {0, 0, 0};
+    for (int t = 0; t < 24; ++t) v[t] = 0.0;
+    double smq = 0.0;                                  // sum of q_j sm
+    int nnear = 0;
+    auto smear = [&](int cnt) {
+        if (lane < cnt) {
+            const double2 p = near[lane];
+            smq += (exp(-p.x) - sqrt(sqrt(p.x)) * g34 * gammq_nr(0.75, p.x, gln34)) * p.y;
+        }
+    };
     const int na = cntA[i];
-    for (int s = lane; s < na; s += 64) {
-        const int j = nbrA[(long)i * P.capA + s];
-        double d[3];
-        const double rsq = sep(P, x, y, z, i, j, d);
-        if (!(P.rcut * P.rcut > rsq)) continue;
-        const double rrr = sqrt(rsq);
-        double bbb[4];
-        table_interp(P, tab, rrr, bbb);
-        const double rri = 1.0 / rrr, rsqi = 1.0 / rsq;
-        const double r3i = 1.0 / (rrr * rrr * rrr);
-        const double r5i = r3i * rsqi;
-        const double qj = chge[j];
-        const double cicj = qi * qj;
-        const double edum = cicj * (bbb[0] + 1.0 / rrr) * R4PIE0;
-        double espdum = (bbb[0] + 1.0 / rrr) * R4PIE0;
-        double ffac = cicj * (r3i + bbb[1]) * R4PIE0;
-        const double bb = pow(pi_ * site_polr(P, j), 1.0 / 6.0);
-        const double u = rrr / bb, u4 = (u * u) * (u * u);
-        double eng;
-        {
-            const double arob4 = P.ascc * u4;
-            const double dum1 = exp(-arob4);
-            const double sm = (dum1 - pow(arob4, 0.25) * g34 * gammq_nr(0.75, arob4, gln34)) / rrr * R4PIE0;
-            eng = edum - cicj * sm;
-            esum += 0.5 * edum;
-            esum += -cicj * 0.5 * sm;
-            espdum -= sm;
-            ffac -= cicj * r3i * dum1 * R4PIE0;
-        }
-        const double mj[3] = {dip[3 * j], dip[3 * j + 1], dip[3 * j + 2]};
-        const double rdmui = mi[0] * d[0] + mi[1] * d[1] + mi[2] * d[2];
-        const double rdmuj = mj[0] * d[0] + mj[1] * d[1] + mj[2] * d[2];
-        const double facmu0 = (qj * rdmui - qi * rdmuj) * (-3.0) * r5i * R4PIE0;
-        const double facmui0 = r3i * qj * R4PIE0;
-        const double facmuj0 = -r3i * qi * R4PIE0;
-        double facmu = facmu0 - (qj * rdmui - qi * rdmuj) * bbb[2] * R4PIE0;
-        double dfacmui = facmui0 + bbb[1] * qj * R4PIE0;
-        double dfacmuj = facmuj0 - bbb[1] * qi * R4PIE0;
-        double espdcdum = (bbb[1] + r3i) * R4PIE0;
-        {
-            const double arob4 = P.ascd * u4;
-            const double dum1 = exp(-arob4);
-            const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
-            facmu -= facmu0 * dum2;
-            dfacmui -= facmui0 * dum1;
-            dfacmuj -= facmuj0 * dum1;
-            espdcdum -= r3i * dum1 * R4PIE0;
-        }
-        if (poli && site_polr2(P, j) > 1.e-6) {
-            const double dpidpj = mi[0] * mj[0] + mi[1] * mj[1] + mi[2] * mj[2];
-            facmu += ((dpidpj * 3.0 + rdmui * rdmuj * rsqi * (-15.0)) * r5i + bbb[2] * dpidpj - bbb[3] * rdmui * rdmuj) *
-                     R4PIE0;
-            dfacmui += (3.0 * r5i + bbb[2]) * rdmuj * R4PIE0;
-            dfacmuj += (3.0 * r5i + bbb[2]) * rdmui * R4PIE0;
-            const double facmu1 = -15.0 * rdmui * rdmuj * rsqi * r5i * R4PIE0;
-            const double facmu2 = 3.0 * dpidpj * r5i * R4PIE0;
-            const double dfacmui1 = 3.0 * rdmuj * r5i * R4PIE0;
-            const double dfacmuj1 = 3.0 * rdmui * r5i * R4PIE0;
-            const double arob4 = P.athole * u4;
-            const double dum1 = exp(-arob4);
-            const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
-            const double bb4 = (bb * bb) * (bb * bb);
-            const double dum3 = 4.0 * P.athole * (4.0 * arob4 - 1.0) * dum1 * rsqi / bb4;
-            const double dum4 = 4.0 * P.athole * dum1 * rrr / bb4;
-            facmu = facmu - facmu1 * dum2 - facmu2 * dum1 + rdmui * rdmuj * dum3 * rri * R4PIE0 -
-                    dpidpj * rsqi * dum4 * R4PIE0;
-            dfacmui -= dfacmui1 * dum2;
-            dfacmuj -= dfacmuj1 * dum2;
-        }
-        const double dfac[3] = {dfacmui * mi[0] + dfacmuj * mj[0], dfacmui * mi[1] + dfacmuj * mj[1],
-                                dfacmui * mi[2] + dfacmuj * mj[2]};
-        ffac += facmu;
-        const double virdum = dfac[0] * d[0] + dfac[1] * d[1] + dfac[2] * d[2];
-        const double fv[3] = {ffac * d[0] + dfac[0], ffac * d[1] + dfac[1], ffac * d[2] + dfac[2]};
-        for (int q = 0; q < 3; ++q) fsum[q] += fv[q];
-        vrs += qj * espdum;
-        vdcs += rdmuj * espdcdum;
-        red[0] += 0.5 * eng;
-        red[1] += 0.5 * (-ffac * rsq - virdum);
-        red[2] += 0.5 * d[0] * fv[0];
-        red[3] += 0.5 * d[0] * fv[1];
-        red[4] += 0.5 * d[0] * fv[2];
-        red[5] += 0.5 * d[1] * fv[1];
-        red[6] += 0.5 * d[1] * fv[2];
-        red[7] += 0.5 * d[2] * fv[2];
-        if (j < P.nreal) {
-            if (!mrow) {
-                const double dr[3] = {x[i] - x[j], y[i] - y[j], z[i] - z[j]};
-                for (int a = 0; a < 3; ++a)
-                    for (int b = 0; b < 3; ++b) W[3 * a + b] += fv[a] * dr[b];
-            } else {
-                const double xj[3] = {x[j], y[j], z[j]};
+    for (int base = 0; base < na; base += 64) {
+        const int s = base + lane;
+        const int j = s < na ? nbrA[(long)i * P.capA + s] : i;
+        double d[3] = {0.0, 0.0, 0.0};
+        double rsq = P.rcut * P.rcut;
+        if (s < na) rsq = sep(P, x, y, z, i, j, d);
+        const bool in = s < na && P.rcut * P.rcut > rsq;
+        double xc = PAIR_XNEAR, qr = 0.0;
+        if (in) {
+            const double rrr = sqrt(rsq);
+            double bbb[4];
+            table_interp(P, tab, rrr, bbb);
+            const double rri = 1.0 / rrr, rsqi = rri * rri;
+            const double r3i = rri * rsqi, r5i = r3i * rsqi;
+            const double qj = chge[j];
+            const double u = rrr * P.bbi[ti][site_type(P, j)];
+            const double u4 = (u * u) * (u * u);
+            const double espdum = bbb[0] + rri;
+            xc = P.ascc * u4;
+            qr = qj * rri;
+            const double dumd = exp(-P.ascd * u4);
+            const double dumc = P.ascc == P.ascd ? dumd : exp(-xc);
+            const double cicj = qi * qj;
+            double ffac = cicj * (r3i * (1.0 - dumc) + bbb[1]);
+            const double mj[3] = {dip[3 * j], dip[3 * j + 1], dip[3 * j + 2]};
+            const double rdmui = mi[0] * d[0] + mi[1] * d[1] + mi[2] * d[2];
+            const double rdmuj = mj[0] * d[0] + mj[1] * d[1] + mj[2] * d[2];
+            const double dumd2 = (1.0 + (4.0 / 3.0) * (P.ascd * u4)) * dumd;
+            const double b1 = bbb[1] + r3i * (1.0 - dumd);
+            ffac -= (qj * rdmui - qi * rdmuj) * (3.0 * r5i * (1.0 - dumd2) + bbb[2]);
+            double dfi = b1 * qj, dfj = -b1 * qi;
+            if (poli && site_polr2(P, j) > 1.e-6) {
+                const double dpidpj = mi[0] * mj[0] + mi[1] * mj[1] + mi[2] * mj[2];
+                const double rr2 = rdmui * rdmuj;
+                const double arob4 = P.athole * u4;
+                const double dum1 = exp(-arob4);
+                const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
+                const double c3 = 3.0 * r5i * (1.0 - dum2) + bbb[2];
+                // 4 a dum1 / b^4 = 4 arob4 dum1 / r^4
+                const double dum34 = 4.0 * arob4 * dum1 * (rsqi * rsqi);
+                ffac += dpidpj * (3.0 * r5i * (1.0 - dum1) + bbb[2] - rri * dum34) -
+                        rr2 * (15.0 * (rsqi * r5i) * (1.0 - dum2) + bbb[3] - dum34 * (4.0 * arob4 - 1.0) * r3i);
+                dfi += c3 * rdmuj;
+                dfj += c3 * rdmui;
+            }
+            double fv[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                fv[q] = ffac * d[q] + dfi * mi[q] + dfj * mj[q];
+                v[q] += fv[q];
+            }
+            v[3] += cicj * espdum;
+            v[4] += qj * espdum;
+            v[5] += rdmuj * b1;
+            v[15] += d[0] * fv[0];
+            v[16] += d[0] * fv[1];
+            v[17] += d[0] * fv[2];
+            v[18] += d[1] * fv[1];
+            v[19] += d[1] * fv[2];
+            v[20] += d[2] * fv[2];
+            if (j < P.nreal) {
+                // raw separations, or the partner's position for an M-site row
+                const double xr[3] = {mrow ? x[j] : xi[0] - x[j], mrow ? y[j] : xi[1] - y[j], mrow ? z[j] : xi[2] - z[j]};
+#pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    fm[a] += fv[a];
-                    for (int b = 0; b < 3; ++b) W[3 * a + b] += fv[a] * xj[b];
+#pragma unroll
+                    for (int b = 0; b < 3; ++b) v[6 + 3 * a + b] += fv[a] * xr[b];
+                    v[21 + a] += fv[a];
                 }
             }
         }
-    }
-    for (int q = 0; q < 3; ++q) fsum[q] = wsum(fsum[q]);
-    for (int q = 0; q < 3; ++q) fm[q] = wsum(fm[q]);
-    for (int t = 0; t < 9; ++t) W[t] = wsum(W[t]);
-    esum = wsum(esum);
-    vrs = wsum(vrs);
-    vdcs = wsum(vdcs);
-    for (int t = 0; t < 8; ++t) red[t] = wsum(red[t]);
-    if (lane == 0) {
-        for (int q = 0; q < 3; ++q) f2[3 * i + q] = fsum[q];
-        e2[i] = esum;
-        vr[i] = vrs;
-        vdcr[i] = vdcs;
-        if (!mrow) {
-            for (int t = 0; t < 9; ++t) w2[9 * i + t] = W[t];
-        } else {
-            for (int q = 0; q < 3; ++q) fmsum[3 * i + q] = fm[q];
-            for (int t = 0; t < 9; ++t) fmx[9 * i + t] = W[t];
+        const bool isnear = xc < PAIR_XNEAR;
+        const unsigned long long bn = __ballot(isnear);
+        if (isnear) near[nnear + __popcll(bn & below)] = make_double2(xc, qr);
+        nnear += __popcll(bn);
+        __syncthreads();
+        if (nnear >= 64) {
+            smear(64);
+            const double2 rest = near[64 + lane];
+            __syncthreads();
+            near[lane] = rest;
+            nnear -= 64;
+            __syncthreads();
         }
-        for (int t = 0; t < 8; ++t) blk[8 * i + t] = red[t];
     }
+    smear(nnear);
+    v[4] -= smq;
+    v[3] = 0.5 * (v[3] - qi * smq);
+#pragma unroll
+    for (int t = 15; t < 21; ++t) v[t] *= 0.5;
+    int k;
+    const double t = R4PIE0 * wave_sum24(v, lane, k);
+    if (k < 24) sums[k] = t;
+    __syncthreads();
+    if (lane < 3) f2[3 * i + lane] = sums[lane];
+    if (lane == 3) e2[i] = sums[3];
+    if (lane == 4) vr[i] = sums[4];
+    if (lane == 5) vdcr[i] = sums[5];
+    if (lane >= 6 && lane < 15) (mrow ? fmx : w2)[9 * i + lane - 6] = sums[lane];
+    if (lane >= 15 && lane < 21) blk[8 * i + 2 + lane - 15] = sums[lane];
+    if (lane >= 21 && lane < 24 && mrow) fmsum[3 * i + lane - 21] = sums[lane];
+    // the virial is minus the trace of the stress (both halved)
+    if (lane == 24) blk[8 * i] = sums[3];
+    if (lane == 25) blk[8 * i + 1] = -(sums[15] + sums[18] + sums[20]);
 }
 
 namespace {
