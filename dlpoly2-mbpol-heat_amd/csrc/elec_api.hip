@@ -131,7 +131,7 @@ int alloc_sites(ElecState& S, int nw, std::string& err)
     ECHK(dalloc(&E.s1, (size_t)9 * n)); ECHK(dalloc(&E.w2, (size_t)9 * n)); ECHK(dalloc(&E.w3, (size_t)9 * n));
     ECHK(dalloc(&E.fmsum, (size_t)3 * n)); ECHK(dalloc(&E.fmx, (size_t)9 * n));
     ECHK(dalloc(&E.eout, nreal)); ECHK(dalloc(&E.wout, (size_t)9 * nreal)); ECHK(dalloc(&E.sout, (size_t)9 * nreal));
-    ECHK(dalloc(&E.scal, 64)); ECHK(dalloc(&E.err, 4)); ECHK(dalloc(&S.rcell, 9));
+    ECHK(dalloc(&E.scal, 64)); ECHK(dalloc(&E.err, 4));
     ECHK(dalloc(&E.pk, 64));
     if (!S.hpk) ECHK(hipHostMalloc((void**)&S.hpk, sizeof(double) * 64, hipHostMallocDefault));
     ECHK(hipMemset(E.zero_state, 0, 8 * sizeof(double)));
@@ -390,7 +390,6 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
     dfree(E.blk);
     E.nblk = nsb + 8 * nkb + 2 * nsb + 8 * E.n + 24 * nwb + 2 * nsb + 64;
     ECHK(dalloc(&E.blk, (size_t)E.nblk));
-    ECHK(hipMemcpy(S.rcell, rc, sizeof(double) * 9, hipMemcpyHostToDevice));
     S.P.rvolm = twopi / volm;
     for (int i = 0; i < 9; ++i) S.k_cell[i] = cell[i];
     for (int i = 0; i < 3; ++i) S.k_kmax[i] = kmax[i];
@@ -428,7 +427,6 @@ void elec_release(ElecState& S)
 {
     elec_drop_graph(S);
     free_buffers(S.E);
-    dfree(S.rcell);
     if (S.hpk) (void)hipHostFree(S.hpk);
     S.hpk = nullptr;
     if (S.sp) {
@@ -561,23 +559,15 @@ int enqueue_attempt(ElecState& S, const ElecSpme* sp, int solver, bool first, in
     ElecBuffers& E = S.E;
     const ElecDev& P = S.P;
     {
-        // the start dipoles kept (or restored), and the four int flags cleared
-        double* d[2] = {first ? E.dip0 : E.dip, reinterpret_cast<double*>(E.err)};
-        const double* sr[2] = {first ? E.dip : E.dip0, nullptr};
-        const long len[2] = {3L * P.n, 2};
-        el_launch_copy_segs(2, d, sr, len, s);
+        // the start dipoles kept (or restored); the four int flags, the solver state and T mu
+        // cleared
+        double* d[4] = {first ? E.dip0 : E.dip, reinterpret_cast<double*>(E.err), E.state, E.emu};
+        const double* sr[4] = {first ? E.dip : E.dip0, nullptr, nullptr, nullptr};
+        const long len[4] = {3L * P.n, 2, 16, 3L * P.n};
+        el_launch_copy_segs(4, d, sr, len, s);
     }
-    int rc = el_launch_setup(E, P, S.cells, s);
-    if (rc) return rc;
-    {
-        // solver state and T mu cleared; M sites carry no induced dipole (polr2 = 0): any
-        // start value cleared
-        double* d[3] = {E.state, E.emu, E.dip + 3 * P.nreal};
-        const double* sr[3] = {nullptr, nullptr, nullptr};
-        const long len[3] = {16, 3L * P.n, 3L * (P.n - P.nreal)};
-        el_launch_copy_segs(3, d, sr, len, s);
-    }
-    rc = el_launch_prep(E, P, S.rcell, sp, s);
+    int rc = el_launch_setup(E, P, S.cells, solver == 1, sp == nullptr, s);
+    if (!rc) rc = el_launch_prep(E, P, solver == 1, sp, s);
     if (!rc && solver == 1) rc = el_launch_cg_init(E, P, sp, s);
     for (int b = 0; !rc && b < nbatch; ++b)
         rc = solver == 1 ? el_launch_cg_iteration(E, P, b, sp, s) : el_launch_iteration(E, P, b == 0, sp, s);
@@ -597,7 +587,6 @@ std::vector<unsigned char> graph_key(const ElecState& S, int distribute, int sol
     add(&S.P, sizeof S.P);
     add(&S.E, sizeof S.E);
     add(&S.cells, sizeof S.cells);
-    add(&S.rcell, sizeof S.rcell);
     const int v[5] = {distribute, solver, nbatch, S.recip, S.P.g.imcon};
     add(v, sizeof v);
     if (S.recip && S.sp && S.spg) {

@@ -277,11 +277,12 @@ __device__ __forceinline__ double sep(const ElecDev& P, const double* __restrict
 
 // M sites (dlpoly_cmd.f:2041-2057) and DMS charges with their derivatives
 // (qdetermine.f90:118-259; new charge assignment).  One thread per water.
-__global__ void k_el_sites(ElecDev P, double* __restrict__ x, double* __restrict__ y, double* __restrict__ z,
-                           double* __restrict__ chge, double* __restrict__ dg)
+__device__ __forceinline__ void water_sites(const ElecDev& P, int w, double* __restrict__ x, double* __restrict__ y,
+                                            double* __restrict__ z, double* __restrict__ chge, double* __restrict__ dg,
+                                            double* __restrict__ dip)
 {
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= P.nw) return;
+    // an M site carries no induced dipole (polr2 = 0): any start value cleared
+    for (int q = 0; q < 3; ++q) dip[3 * (P.nreal + w) + q] = 0.0;
     const int io = 3 * w, m = P.nreal + w;
     double r1v[3], r2v[3];
     {
@@ -316,19 +317,33 @@ __global__ void k_el_sites(ElecDev P, double* __restrict__ x, double* __restrict
         f3[j] = f3[j - 1] * x3;
     }
     double p1 = 0.0, p2 = 0.0, g11 = 0.0, g12 = 0.0, g21 = 0.0, g22 = 0.0, g1c = 0.0, g2c = 0.0;
+    // (the derivatives' common 1 / reoh once per sum: a division in each of the 84 terms' four
+    // made this 17 us of one thread's latency, with the preconditioner's 15 after it: now 8.4 for both)
 #pragma unroll
     for (int j = 1; j < DMS_NTERMS; ++j) {
         const int a = dms_idx[j][0], b = dms_idx[j][1], c = dms_idx[j][2];
-        const double cf = dms_coef[j];
-        p1 = p1 + cf * f1[a] * f2[b] * f3[c];
-        p2 = p2 + cf * f1[b] * f2[a] * f3[c];
-        g11 = g11 + cf * (a - 1) * f1[a - 1] * f2[b] * f3[c] / reoh;
-        g12 = g12 + cf * (b - 1) * f1[a] * f2[b - 1] * f3[c] / reoh;
-        g21 = g21 + cf * (b - 1) * f1[b - 1] * f2[a] * f3[c] / reoh;
-        g22 = g22 + cf * (a - 1) * f1[b] * f2[a - 1] * f3[c] / reoh;
-        g1c = g1c + cf * (c - 1) * f1[a] * f2[b] * f3[c - 1];
-        g2c = g2c + cf * (c - 1) * f1[b] * f2[a] * f3[c - 1];
+        const double cf3 = dms_coef[j] * f3[c];
+        const double ab = f1[a] * f2[b], ba = f1[b] * f2[a];
+        p1 += cf3 * ab;
+        p2 += cf3 * ba;
+        if (a > 1) {
+            g11 += ((a - 1) * cf3) * (f1[a - 1] * f2[b]);
+            g22 += ((a - 1) * cf3) * (f1[b] * f2[a - 1]);
+        }
+        if (b > 1) {
+            g12 += ((b - 1) * cf3) * (f1[a] * f2[b - 1]);
+            g21 += ((b - 1) * cf3) * (f1[b - 1] * f2[a]);
+        }
+        if (c > 1) {
+            const double d3 = (c - 1) * dms_coef[j] * f3[c - 1];
+            g1c += d3 * ab;
+            g2c += d3 * ba;
+        }
     }
+    g11 /= reoh;
+    g12 /= reoh;
+    g21 /= reoh;
+    g22 /= reoh;
     // DMS parameters (module.f90:818-826)
     const double b1dms = 1.0, adms = 0.2999 * 0.529177249, bdms = -0.6932;
     const double c0 = 1.0099, c1 = -0.1801, c2 = 0.0892;
@@ -339,8 +354,8 @@ __global__ void k_el_sites(ElecDev P, double* __restrict__ x, double* __restrict
     const double leg = c0 + pl1 * c1 + pl2 * c2;
     const double pr1 = pow(r1, bdms), pr2 = pow(r2, bdms);
     const double pc0 = adms * (pr1 + pr2) * leg;
-    const double dpc0dr1 = adms * (bdms * pow(r1, bdms - 1)) * leg;
-    const double dpc0dr2 = adms * (bdms * pow(r2, bdms - 1)) * leg;
+    const double dpc0dr1 = adms * (bdms * (pr1 / r1)) * leg;
+    const double dpc0dr2 = adms * (bdms * (pr2 / r2)) * leg;
     const double dpc0dcos = adms * (pr1 + pr2) * (c1 + 3.0 * c2 * pl1);
     double* G = dg + 6 * w;
     G[0] = g11 * damp + p1 * ddampdr1 + dpc0dr1;
@@ -359,19 +374,173 @@ __global__ void k_el_sites(ElecDev P, double* __restrict__ x, double* __restrict
     chge[m] = -(q1 + q2);
 }
 
+// packed index of (i, j) in a symmetric 9 x 9 matrix stored as its lower triangle
+__device__ __forceinline__ constexpr int tri9(int i, int j) { return i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i; }
+
+// Per water: the preconditioner block M = diag(r4pie0 / polr2) - r4pie0 T_damped over the
+// intramolecular pairs (the Thole-damped dipole tensor of rfield.f:419-520 without its Ewald
+// split: M only has to be close to A's block, it does not move the fixed point), inverted
+// by Cholesky and stored packed (45 values per water).  Rows of sites without a dipole are
+// decoupled unit rows.  A block that is not positive definite falls back to the diagonal.
+__device__ __forceinline__ void water_block(const ElecDev& P, int w, const double* __restrict__ x,
+                                            const double* __restrict__ y, const double* __restrict__ z,
+                                            double* __restrict__ minv)
+{
+    double a[45];
+    bool on[3];
+#pragma unroll
+    for (int q = 0; q < 45; ++q) a[q] = 0.0;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+        const double p2 = site_polr2(P, 3 * w + s);
+        on[s] = p2 > P.toler;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) a[tri9(3 * s + c, 3 * s + c)] = on[s] ? R4PIE0 / p2 : 1.0;
+    }
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int t = s + 1; t < 3; ++t) {
+            const int i = 3 * w + s, j = 3 * w + t;
+            if (!(on[s] && on[t] && site_polr2(P, i) > 1.e-6 && site_polr2(P, j) > 1.e-6)) continue;
+            double d[3];
+            const double r2 = sep(P, x, y, z, i, j, d);
+            const double rr = sqrt(r2);
+            const double r3i = 1.0 / (rr * r2), r5i = r3i / r2;
+            const double u = rr * P.bbi[site_type(P, i)][site_type(P, j)];
+            const double arob4 = (s == 0 ? P.athole12 : P.athole13) * (u * u) * (u * u);
+            const double dum1 = exp(-arob4);
+            const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    a[tri9(3 * t + e, 3 * s + c)] =
+                        -R4PIE0 * (3.0 * d[c] * d[e] * r5i * (1.0 - dum2) - (c == e ? r3i * (1.0 - dum1) : 0.0));
+        }
+    // Cholesky M = L L^T in place; the diagonal of L is kept as its inverse
+    bool ok = true;
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+        for (int j = 0; j <= i; ++j) {
+            double v = a[tri9(i, j)];
+#pragma unroll
+            for (int k = 0; k < j; ++k) v -= a[tri9(i, k)] * a[tri9(j, k)];
+            if (i == j) {
+                ok = ok && v > 0.0;
+                a[tri9(i, i)] = 1.0 / sqrt(fmax(v, 1.e-300));
+            } else {
+                a[tri9(i, j)] = v * a[tri9(j, j)];
+            }
+        }
+    // X = L^-1 (lower), then M^-1 = X^T X
+    double X[45];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        X[tri9(i, i)] = a[tri9(i, i)];
+#pragma unroll
+        for (int j = 0; j < i; ++j) {
+            double v = 0.0;
+#pragma unroll
+            for (int k = j; k < i; ++k) v += a[tri9(i, k)] * X[tri9(k, j)];
+            X[tri9(i, j)] = -v * a[tri9(i, i)];
+        }
+    }
+    double* m = minv + 45L * w;
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+        for (int j = 0; j <= i; ++j) {
+            double v = 0.0;
+#pragma unroll
+            for (int k = i; k < 9; ++k) v += X[tri9(k, i)] * X[tri9(k, j)];
+            ok = ok && isfinite(v);
+            a[tri9(i, j)] = v;
+        }
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+        for (int j = 0; j <= i; ++j) {
+            const int s = i / 3;
+            const double jac = (i == j && on[s]) ? site_polr2(P, 3 * w + s) / R4PIE0 : 0.0;
+            m[tri9(i, j)] = ok ? a[tri9(i, j)] : jac;
+        }
+}
+
+// Blocks [0, nb): the M sites and charges; blocks [nb, 2 nb) (conjugate gradients): the
+// preconditioner's inverse blocks, which need the real atoms alone.  One thread per water, both
+// a chain of one thread's latency, side by side.
+__global__ __launch_bounds__(64) void k_el_waters(ElecDev P, int nb, double* __restrict__ x, double* __restrict__ y,
+                                                  double* __restrict__ z, double* __restrict__ chge,
+                                                  double* __restrict__ dg, double* __restrict__ dip,
+                                                  double* __restrict__ minv)
+{
+    const bool second = (int)blockIdx.x >= nb;
+    const int w = (blockIdx.x - (second ? nb : 0)) * 64 + threadIdx.x;
+    if (w >= P.nw) return;
+    if (second) water_block(P, w, x, y, z, minv);
+    else water_sites(P, w, x, y, z, chge, dg, dip);
+}
+
+// Reciprocal-space phase tables of each site: cos / sin (l * 2 pi * s_a), s = rcell . r,
+// l = 0..kmax_a, by the reference's recurrence (ewald1p.f:196-241, 262-282), layout
+// phc/phs [a][l][n] (for the final site pass) and pht[n][rs.kt] (for the matrix passes).
+__device__ __forceinline__ void site_phases(const ElecDev& P, int j, const double* __restrict__ x,
+                                            const double* __restrict__ y, const double* __restrict__ z,
+                                            double* __restrict__ phc, double* __restrict__ phs,
+                                            double2* __restrict__ pht)
+{
+    const double* rcell = P.rs.rc;
+    if (j >= P.n) {
+        // (the structure-factor pass reads up to RS_PAD sites past the last with weight 0)
+        if (j < P.n + RS_PAD)
+            for (int l = 0; l < P.rs.kt; ++l) pht[(long)j * P.rs.kt + l] = make_double2(0.0, 0.0);
+        return;
+    }
+    const int ks = P.kstride;
+    for (int a = 0; a < 3; ++a) {
+        double2* row = pht + (long)j * P.rs.kt + (a == 0 ? 0 : a == 1 ? P.rs.ky : P.rs.kz);
+        const double ss = rcell[a] * x[j] + rcell[3 + a] * y[j] + rcell[6 + a] * z[j];
+        const double c1 = cos(TWOPI * ss), s1 = sin(TWOPI * ss);
+        double c = 1.0, s = 0.0;
+        for (int l = 0; l <= P.km[a]; ++l) {
+            if (l == 1) {
+                c = c1;
+                s = s1;
+            } else if (l > 1) {
+                const double cs = c;
+                c = cs * c1 - s * s1;
+                s = s * c1 + cs * s1;
+            }
+            phc[((long)a * ks + l) * P.n + j] = c;
+            phs[((long)a * ks + l) * P.n + j] = s;
+            row[l] = make_double2(c, s);
+            if (a == 1 && l > 0) row[-l] = make_double2(c, -s);
+        }
+    }
+}
+
 // Neighbour rows: every site of another water within rcut (superset by a relative 1e-9 of
 // rcut^2; each kernel applies the reference's own test), found in the 27 link cells around
 // the site when the box holds three cells per axis (the Verlet list over link cells of
 // parlink.f), else by a scan of every site; either way in an order fixed by the positions.
 // Row P holds the partners of a polarizable site that are polarizable.  One wavefront per
-// site.
-__global__ __launch_bounds__(64) void k_el_nbr(ElecDev P, const double* __restrict__ x,
+// site.  The first nph blocks (k-sum) form the phase tables instead, 64 sites each: both parts
+// need the sites alone.
+__global__ __launch_bounds__(64) void k_el_nbr(ElecDev P, int nph, const double* __restrict__ x,
                                                const double* __restrict__ y, const double* __restrict__ z,
                                                int* __restrict__ nbrA, int* __restrict__ cntA,
-                                               int* __restrict__ nbrP, int* __restrict__ cntP, int* __restrict__ err)
+                                               int* __restrict__ nbrP, int* __restrict__ cntP, int* __restrict__ err,
+                                               double* __restrict__ phc, double* __restrict__ phs,
+                                               double2* __restrict__ pht)
 {
-    const int i = blockIdx.x;
+    const int i = (int)blockIdx.x - nph;
     const int lane = threadIdx.x;
+    if (i < 0) {
+        site_phases(P, blockIdx.x * 64 + lane, x, y, z, phc, phs, pht);
+        return;
+    }
     if (i >= P.n) return;
     const int wi = water_of(P, i);
     const bool poli = site_polr2(P, i) > 1.e-6;
@@ -421,11 +590,16 @@ __global__ __launch_bounds__(64) void k_el_nbr(ElecDev P, const double* __restri
 // separation formed again cost less there than the six components did (emu_row).  One
 // wavefront per site, one pass over its partners: row P holds the polarizable ones in row A's
 // order, so a partner's place in it is the count of those before.
+// Lanes 0..2 add the excluded (intramolecular) pairs of the site (rfield.f:327-525): the charge
+// field with the -erf kernel, and from the lower site of each real pair the dipole tensor (Ewald +
+// Applequist - Thole with athole12/athole13), stored tin[nw][pair][6] for pairs (O,H1) (O,H2)
+// (O,M) (H1,H2) (H1,M) (H2,M); those of the M site, which carries no dipole, are not used.
 __global__ __launch_bounds__(64) void k_el_prep(ElecDev P, const double* __restrict__ x,
                                                 const double* __restrict__ y, const double* __restrict__ z,
                                                 const double* __restrict__ chge, const double* __restrict__ tab,
                                                 const int* __restrict__ nbrA, const int* __restrict__ cntA,
-                                                double2* __restrict__ tens, double* __restrict__ efk)
+                                                double2* __restrict__ tens, double* __restrict__ tin,
+                                                double* __restrict__ efk)
 {
     const int i = blockIdx.x;
     const int lane = threadIdx.x;
@@ -434,6 +608,39 @@ __global__ __launch_bounds__(64) void k_el_prep(ElecDev P, const double* __restr
     const int ti = site_type(P, i);
     const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     double e[3] = {0.0, 0.0, 0.0};
+    if (lane < 3) {
+        const int w = water_of(P, i), a = i < P.nreal ? i - 3 * w : 3, b = lane < a ? lane : lane + 1;
+        const int j = b < 3 ? 3 * w + b : P.nreal + w;
+        double d[3];
+        const double r2 = sep(P, x, y, z, i, j, d);
+        const double rr = sqrt(r2);
+        const double rri = 1.0 / rr, rsqi = rri * rri;
+        const double r3i = rri * rsqi;
+        double bbb[4];
+        bfun_direct(P.alpha, rr, rsqi, bbb);
+        const double ek = R4PIE0 * chge[j] * bbb[1];
+        e[0] = ek * d[0];
+        e[1] = ek * d[1];
+        e[2] = ek * d[2];
+        if (a < b && b < 3) {
+            double t1 = 0.0, t2 = 0.0;
+            if (poli && site_polr2(P, j) > 1.e-6) {
+                const double u = rr * P.bbi[ti][site_type(P, j)];
+                const double arob4 = (a == 0 ? P.athole12 : P.athole13) * (u * u) * (u * u);
+                const double dum1 = exp(-arob4);
+                const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
+                t1 = bbb[1] + r3i * (1.0 - dum1);
+                t2 = bbb[2] + 3.0 * r3i * rsqi * (1.0 - dum2);
+            }
+            double* o = tin + 36 * w + 6 * (a == 0 ? b - 1 : 3);
+            o[0] = t2 * d[0] * d[0] - t1;
+            o[1] = t2 * d[0] * d[1];
+            o[2] = t2 * d[0] * d[2];
+            o[3] = t2 * d[1] * d[1] - t1;
+            o[4] = t2 * d[1] * d[2];
+            o[5] = t2 * d[2] * d[2] - t1;
+        }
+    }
     const int na = cntA[i];
     int np = 0;
     for (int base = 0; base < na; base += 64) {
@@ -475,91 +682,6 @@ __global__ __launch_bounds__(64) void k_el_prep(ElecDev P, const double* __restr
     for (int q = 0; q < 3; ++q) e[q] = wsum(e[q]);
     if (lane == 0)
         for (int q = 0; q < 3; ++q) efk[3 * i + q] = e[q];
-}
-
-// Excluded (intramolecular) pairs of each water (rfield.f:327-525): charge field with the
-// -erf kernel and the dipole tensors (Ewald + Applequist - Thole with athole12/athole13),
-// stored [nw][pair][6] for pairs (O,H1) (O,H2) (O,M) (H1,H2) (H1,M) (H2,M).
-__global__ void k_el_intra_prep(ElecDev P, const double* __restrict__ x, const double* __restrict__ y,
-                                const double* __restrict__ z, const double* __restrict__ chge,
-                                double* __restrict__ tin, double* __restrict__ efk)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= P.nw) return;
-    const int s[4] = {3 * w, 3 * w + 1, 3 * w + 2, P.nreal + w};
-    int pr = 0;
-    for (int a = 0; a < 4; ++a)
-        for (int b = a + 1; b < 4; ++b, ++pr) {
-            const int i = s[a], j = s[b];
-            double d[3];
-            const double r2 = sep(P, x, y, z, i, j, d);
-            const double rr = sqrt(r2);
-            const double rsqi = 1.0 / r2;
-            const double r3i = 1.0 / (rr * r2);
-            const double r5i = r3i * rsqi;
-            double bbb[4];
-            bfun_direct(P.alpha, rr, rsqi, bbb);
-            const double eki = R4PIE0 * chge[j] * bbb[1];
-            const double ekj = R4PIE0 * chge[i] * bbb[1];
-            for (int q = 0; q < 3; ++q) {
-                efk[3 * i + q] += eki * d[q];
-                efk[3 * j + q] -= ekj * d[q];
-            }
-            double dt[6] = {0, 0, 0, 0, 0, 0};
-            if (site_polr2(P, i) > 1.e-6 && site_polr2(P, j) > 1.e-6) {
-                const double bb = pow(site_polr(P, i) * site_polr(P, j), 1.0 / 6.0);
-                const double u = rr / bb;
-                const double ath = (i % 3 == 0 || j % 3 == 0) ? P.athole12 : P.athole13;
-                const double arob4 = ath * (u * u) * (u * u);
-                const double dum1 = exp(-arob4);
-                const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
-                const double rij[6] = {d[0] * d[0], d[0] * d[1], d[0] * d[2], d[1] * d[1], d[1] * d[2], d[2] * d[2]};
-                for (int q = 0; q < 6; ++q) {
-                    const bool dg_ = (q == 0 || q == 3 || q == 5);
-                    dt[q] = rij[q] * bbb[2] - (dg_ ? bbb[1] : 0.0);
-                    dt[q] = dt[q] + 3.0 * rij[q] * r5i - (dg_ ? r3i : 0.0);
-                    dt[q] = dt[q] - 3.0 * rij[q] * r5i * dum2 + (dg_ ? dum1 * r3i : 0.0);
-                }
-            }
-            for (int q = 0; q < 6; ++q) tin[36 * w + 6 * pr + q] = dt[q];
-        }
-}
-
-// Reciprocal-space phase tables of each site: cos / sin (l * 2 pi * s_a), s = rcell . r,
-// l = 0..kmax_a, by the reference's recurrence (ewald1p.f:196-241, 262-282), layout
-// phc/phs [a][l][n] (for the final site pass) and pht[n][rs.kt] (for the matrix passes).
-__global__ void k_el_phase(ElecDev P, const double* __restrict__ x, const double* __restrict__ y,
-                           const double* __restrict__ z, const double* __restrict__ rcell,
-                           double* __restrict__ phc, double* __restrict__ phs, double2* __restrict__ pht)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= P.n) {
-        // (the structure-factor pass reads up to RS_PAD sites past the last with weight 0)
-        if (j < P.n + RS_PAD)
-            for (int l = 0; l < P.rs.kt; ++l) pht[(long)j * P.rs.kt + l] = make_double2(0.0, 0.0);
-        return;
-    }
-    const int ks = P.kstride;
-    for (int a = 0; a < 3; ++a) {
-        double2* row = pht + (long)j * P.rs.kt + (a == 0 ? 0 : a == 1 ? P.rs.ky : P.rs.kz);
-        const double ss = rcell[a] * x[j] + rcell[3 + a] * y[j] + rcell[6 + a] * z[j];
-        const double c1 = cos(TWOPI * ss), s1 = sin(TWOPI * ss);
-        double c = 1.0, s = 0.0;
-        for (int l = 0; l <= P.km[a]; ++l) {
-            if (l == 1) {
-                c = c1;
-                s = s1;
-            } else if (l > 1) {
-                const double cs = c;
-                c = cs * c1 - s * s1;
-                s = s * c1 + cs * s1;
-            }
-            phc[((long)a * ks + l) * P.n + j] = c;
-            phs[((long)a * ks + l) * P.n + j] = s;
-            row[l] = make_double2(c, s);
-            if (a == 1 && l > 0) row[-l] = make_double2(c, -s);
-        }
-    }
 }
 
 // ======================================================= reciprocal-space passes ======
@@ -1154,155 +1276,72 @@ __global__ __launch_bounds__(256) void k_cg_final_fields(ElecDev P, const double
     }
 }
 
-// packed index of (i, j) in a symmetric 9 x 9 matrix stored as its lower triangle
-__device__ __forceinline__ constexpr int tri9(int i, int j) { return i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i; }
-
-// Per water: the preconditioner block M = diag(r4pie0 / polr2) - r4pie0 T_damped over the
-// intramolecular pairs (the Thole-damped dipole tensor of rfield.f:419-520 without its Ewald
-// split: M only has to be close to A's block, it does not move the fixed point), inverted
-// by Cholesky and stored packed (45 values per water).  Rows of sites without a dipole are
-// decoupled unit rows.  A block that is not positive definite falls back to the diagonal.
-__global__ __launch_bounds__(256) void k_cg_block(ElecDev P, const double* __restrict__ x,
-                                                  const double* __restrict__ y, const double* __restrict__ z,
-                                                  double* __restrict__ minv)
+// The reciprocal fields of the start dipoles (efdd, with the self term) and of the charges (efdc)
+// from their chunk partials, as k_el_kfield_reduce<true>; r = E0 + T mu0 - D mu0 (T mu0 = emu +
+// efdd), u = M^-1 r, T mu = T mu0; the first application of A goes to m = u; z, q, s, p start at
+// zero.  A block takes CG_WPB waters, a row per lane, as k_cg_update: a quarter of the chunks per
+// wavefront, then the first wavefront has the rows.
+#define CG_WPB 7
+__global__ __launch_bounds__(256) void k_cg_init(ElecDev P, const double* __restrict__ Fpart,
+                                                 const double* __restrict__ efk, double* __restrict__ efdc,
+                                                 const double* __restrict__ emu, double* __restrict__ efdd,
+                                                 const double* __restrict__ dip, const double* __restrict__ minv,
+                                                 double* __restrict__ r, double* __restrict__ u, double* __restrict__ m,
+                                                 double* __restrict__ z, double* __restrict__ qv,
+                                                 double* __restrict__ sv, double* __restrict__ pv,
+                                                 double* __restrict__ tmu)
 {
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= P.nw) return;
-    double a[45];
-    bool on[3];
-#pragma unroll
-    for (int q = 0; q < 45; ++q) a[q] = 0.0;
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-        const double p2 = site_polr2(P, 3 * w + s);
-        on[s] = p2 > P.toler;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) a[tri9(3 * s + c, 3 * s + c)] = on[s] ? R4PIE0 / p2 : 1.0;
-    }
-#pragma unroll
-    for (int s = 0; s < 3; ++s)
-#pragma unroll
-        for (int t = s + 1; t < 3; ++t) {
-            const int i = 3 * w + s, j = 3 * w + t;
-            if (!(on[s] && on[t] && site_polr2(P, i) > 1.e-6 && site_polr2(P, j) > 1.e-6)) continue;
-            double d[3];
-            const double r2 = sep(P, x, y, z, i, j, d);
-            const double rr = sqrt(r2);
-            const double r3i = 1.0 / (rr * r2), r5i = r3i / r2;
-            const double bb = pow(site_polr(P, i) * site_polr(P, j), 1.0 / 6.0);
-            const double u = rr / bb;
-            const double arob4 = (s == 0 ? P.athole12 : P.athole13) * (u * u) * (u * u);
-            const double dum1 = exp(-arob4);
-            const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-#pragma unroll
-                for (int e = 0; e < 3; ++e)
-                    a[tri9(3 * t + e, 3 * s + c)] =
-                        -R4PIE0 * (3.0 * d[c] * d[e] * r5i * (1.0 - dum2) - (c == e ? r3i * (1.0 - dum1) : 0.0));
-        }
-    // Cholesky M = L L^T in place
-    bool ok = true;
-#pragma unroll
-    for (int i = 0; i < 9; ++i)
-#pragma unroll
-        for (int j = 0; j <= i; ++j) {
-            double v = a[tri9(i, j)];
-#pragma unroll
-            for (int k = 0; k < j; ++k) v -= a[tri9(i, k)] * a[tri9(j, k)];
-            if (i == j) {
-                ok = ok && v > 0.0;
-                a[tri9(i, i)] = sqrt(fmax(v, 1.e-300));
-            } else {
-                a[tri9(i, j)] = v / a[tri9(j, j)];
-            }
-        }
-    // X = L^-1 (lower), then M^-1 = X^T X
-    double X[45];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        X[tri9(i, i)] = 1.0 / a[tri9(i, i)];
-#pragma unroll
-        for (int j = 0; j < i; ++j) {
-            double v = 0.0;
-#pragma unroll
-            for (int k = j; k < i; ++k) v += a[tri9(i, k)] * X[tri9(k, j)];
-            X[tri9(i, j)] = -v / a[tri9(i, i)];
+    __shared__ double part[4][2][64];
+    __shared__ double rs[64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wl = lane / 9, i = lane - 9 * wl;
+    const int w = blockIdx.x * CG_WPB + wl;
+    const bool act = lane < 9 * CG_WPB && w < P.nw;
+    const int o = 9 * w + i, j = 3 * w + i / 3, c = i % 3;
+    const double p2 = act ? site_polr2(P, j) : 0.0;
+    const bool on = act && p2 > P.toler;
+    double sd = 0.0, sc = 0.0;
+    if (act) {
+        const int c0 = (P.fchunks * wave) / 4, c1 = (P.fchunks * (wave + 1)) / 4;
+        const double* f = Fpart + (long)c * P.n + j;
+        const long cs = 6L * P.n;
+#pragma unroll 4
+        for (int ch = c0; ch < c1; ++ch) {
+            sd += f[ch * cs];
+            sc += f[ch * cs + 3L * P.n];
         }
     }
-    double* m = minv + 45L * w;
-#pragma unroll
-    for (int i = 0; i < 9; ++i)
-#pragma unroll
-        for (int j = 0; j <= i; ++j) {
-            double v = 0.0;
-#pragma unroll
-            for (int k = i; k < 9; ++k) v += X[tri9(k, i)] * X[tri9(k, j)];
-            ok = ok && isfinite(v);
-            a[tri9(i, j)] = v;
-        }
-#pragma unroll
-    for (int i = 0; i < 9; ++i)
-#pragma unroll
-        for (int j = 0; j <= i; ++j) {
-            const int s = i / 3;
-            const double jac = (i == j && on[s]) ? site_polr2(P, 3 * w + s) / R4PIE0 : 0.0;
-            m[tri9(i, j)] = ok ? a[tri9(i, j)] : jac;
-        }
-}
-
-// z = M^-1 r for one water (rows of sites without a dipole stay zero)
-__device__ __forceinline__ void cg_precondition(const double* __restrict__ m, const double (&r)[9],
-                                                const bool (&on)[3], double (&z)[9])
-{
-    double mm[45];
-#pragma unroll
-    for (int q = 0; q < 45; ++q) mm[q] = m[q];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        double v = 0.0;
-#pragma unroll
-        for (int j = 0; j < 9; ++j) v += mm[tri9(i, j)] * r[j];
-        z[i] = on[i / 3] ? v : 0.0;
-    }
-}
-
-// r = E0 + T mu0 - D mu0 (T mu0 = emu + efdd of the start dipoles), u = M^-1 r, T mu = T mu0;
-// the first application of A goes to m = u; z, q, s, p start at zero.  One thread per water.
-__global__ __launch_bounds__(256) void k_cg_init(ElecDev P, const double* __restrict__ efk,
-                                                 const double* __restrict__ efdc, const double* __restrict__ emu,
-                                                 const double* __restrict__ efdd, const double* __restrict__ dip,
-                                                 const double* __restrict__ minv, double* __restrict__ r,
-                                                 double* __restrict__ u, double* __restrict__ m, double* __restrict__ z,
-                                                 double* __restrict__ qv, double* __restrict__ sv,
-                                                 double* __restrict__ pv, double* __restrict__ tmu)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= P.nw) return;
-    double rr[9], uu[9];
-    bool on[3];
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-        const double p2 = site_polr2(P, 3 * w + s);
-        on[s] = p2 > P.toler;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const int o = 9 * w + 3 * s + c;
-            tmu[o] = emu[o] + efdd[o];
-            rr[3 * s + c] = on[s] ? (efk[o] + efdc[o] + emu[o] + efdd[o]) - R4PIE0 * dip[o] / p2 : 0.0;
-        }
-    }
-    cg_precondition(minv + 45L * w, rr, on, uu);
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-        const int o = 9 * w + q;
-        r[o] = rr[q];
-        u[o] = uu[q];
-        m[o] = uu[q];
+    part[wave][0][lane] = sd;
+    part[wave][1][lane] = sc;
+    __syncthreads();
+    double rr = 0.0;
+    if (wave == 0 && act) {
+        sd = ((part[0][0][lane] + part[1][0][lane]) + part[2][0][lane]) + part[3][0][lane];
+        sc = ((part[0][1][lane] + part[1][1][lane]) + part[2][1][lane]) + part[3][1][lane];
+        const double mu = dip[o];
+        const double ed = (p2 > 1.e-6 ? P.scale * sd : 0.0) + P.self_dd * mu, ec = P.scale * sc;
+        const double t = emu[o] + ed;
+        efdd[o] = ed;
+        efdc[o] = ec;
+        tmu[o] = t;
+        rr = on ? (efk[o] + ec + t) - R4PIE0 * mu / p2 : 0.0;
+        r[o] = rr;
         z[o] = 0.0;
         qv[o] = 0.0;
         sv[o] = 0.0;
         pv[o] = 0.0;
+    }
+    if (wave == 0) rs[lane] = rr;
+    __syncthreads();
+    if (wave == 0 && act) {
+        double uu = 0.0;
+        if (on) {
+            const double* mi = minv + 45L * w;
+#pragma unroll
+            for (int k = 0; k < 9; ++k) uu += mi[tri9(i, k)] * rs[9 * wl + k];
+        }
+        u[o] = uu;
+        m[o] = uu;
     }
 }
 
@@ -1314,7 +1353,6 @@ __global__ __launch_bounds__(256) void k_cg_init(ElecDev P, const double* __rest
 // each water is shared through LDS for m = M^-1 w.  Block partials (r.u, w.u,
 // |polr2 r / r4pie0|^2, dipole count, max |m_i|) per water block.  INIT sets w = A u and
 // leaves mu, r, u as they are.
-#define CG_WPB 7
 template <bool INIT>
 __global__ __launch_bounds__(256) void k_cg_update(ElecDev P, const double* __restrict__ Fpart,
                                                    const double* __restrict__ emu, const double* __restrict__ minv,
@@ -2260,15 +2298,19 @@ void rs_launch_field(const ElecBuffers& E, const ElecDev& P, int nset, int nch, 
 }
 }
 
-int el_launch_setup(ElecBuffers& E, const ElecDev& P, CellList& cells, hipStream_t s)
+// The sites and charges (and with cg the preconditioner), the neighbour rows (and with ksum the
+// phase tables).
+int el_launch_setup(ElecBuffers& E, const ElecDev& P, CellList& cells, bool cg, bool ksum, hipStream_t s)
 {
-    const int nwb = ceil_div(P.nw, 64);
-    hipLaunchKernelGGL(k_el_sites, dim3(nwb), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.dg);
+    const int nwb = ceil_div(P.nw, 64), nph = ksum ? ceil_div(P.n + RS_PAD, 64) : 0;
+    hipLaunchKernelGGL(k_el_waters, dim3(cg ? 2 * nwb : nwb), dim3(64), 0, s, P, nwb, E.x, E.y, E.z, E.chge, E.dg,
+                       E.dip, E.cg_minv);
     if (P.cells.on) {
         const int rc = cells_build(cells, P.n, E.x, E.y, E.z, 1, s);
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(k_el_nbr, dim3(P.n), dim3(64), 0, s, P, E.x, E.y, E.z, E.nbrA, E.cntA, E.nbrP, E.cntP, E.err);
+    hipLaunchKernelGGL(k_el_nbr, dim3(nph + P.n), dim3(64), 0, s, P, nph, E.x, E.y, E.z, E.nbrA, E.cntA, E.nbrP, E.cntP,
+                       E.err, E.phc, E.phs, E.pht);
     return (int)hipGetLastError();
 }
 
@@ -2298,22 +2340,19 @@ static inline ElecDev one_chunk(const ElecDev& P)
     return Q;
 }
 
-int el_launch_prep(ElecBuffers& E, const ElecDev& P, const double* rcell_dev, const ElecSpme* sp, hipStream_t s)
+// The charge fields and dipole tensors of every row, then the reciprocal fields of the start
+// dipoles and of the charges as partials (Fpart); the real-space field of the start dipoles; for
+// SOR also the sums of the partials (the conjugate-gradient start forms its own).
+int el_launch_prep(ElecBuffers& E, const ElecDev& P, bool cg, const ElecSpme* sp, hipStream_t s)
 {
-    const int nwb = ceil_div(P.nw, 64);
-    hipLaunchKernelGGL(k_el_prep, dim3(P.n), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.tab, E.nbrA, E.cntA,
-                       E.tens, E.efk);
-    hipLaunchKernelGGL(k_el_intra_prep, dim3(nwb), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.tin, E.efk);
+    hipLaunchKernelGGL(k_el_prep, dim3(P.n), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.tab, E.nbrA, E.cntA, E.tens,
+                       E.tin, E.efk);
     if (sp && !sp->B) {
         // no reciprocal space (an isolated cluster): zero fields, in the layout of the k-sum
         // field partials (one chunk), so that the reductions form efdd (the self term is 0
         // without an Ewald split) and efdc
         el_launch_zero(E.Fpart, 6L * P.n, s);
-        hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.nrow, 64)), dim3(256), 0, s, one_chunk(P),
-                           E.Fpart, E.dip, E.efdd, E.efdc, E.state);
-        return (int)hipGetLastError();
-    }
-    if (sp) {
+    } else if (sp) {
         // particle mesh: splines of every site, then the fields of the start dipoles (grid 0)
         // and of the charges (grid 1) at every site, in the layout of the k-sum field partials
         sp_launch_prep(*sp->B, *sp->G, P.n, E.x, E.y, E.z, s);
@@ -2327,18 +2366,16 @@ int el_launch_prep(ElecBuffers& E, const ElecDev& P, const double* rcell_dev, co
         sp_launch_spread(*sp->B, *sp->G, P.n, E.chge, E.dip, spec, g, true, nullptr, s);
         sp_launch_convolve(*sp->B, *sp->G, g, 2, true, nullptr, s);
         sp_launch_field(*sp->B, *sp->G, P.n, g, 2, sp->kap, E.Fpart, P.n, nullptr, s);
-        hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.nrow, 64)), dim3(256), 0, s, one_chunk(P),
-                           E.Fpart, E.dip, E.efdd, E.efdc, E.state);
-        return (int)hipGetLastError();
+    } else {
+        // structure factors of the start dipoles and of the charges, and the iloop = 1 fields
+        rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.n}, {E.chge, 1, 0, P.n}}}, 2, P.rs.nchq, P.rs.spcq, true, E.state, nullptr,
+                       0, 0, s);
+        rs_launch_field(E, P, 2, P.rs.nchq, s);
     }
-    hipLaunchKernelGGL(k_el_phase, dim3(ceil_div(P.n + RS_PAD, 64)), dim3(64), 0, s, P, E.x, E.y, E.z, rcell_dev, E.phc,
-                       E.phs, E.pht);
-    // structure factors of the start dipoles and of the charges, and the iloop = 1 fields
-    rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.n}, {E.chge, 1, 0, P.n}}}, 2, P.rs.nchq, P.rs.spcq, false, E.state, nullptr, 0,
-                   0, s);
-    rs_launch_field(E, P, 2, P.rs.nchq, s);
-    hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.nrow, 64)), dim3(256), 0, s, P, E.Fpart, E.dip,
-                       E.efdd, E.efdc, E.state);
+    if (sp) launch_emu(E, P, E.dip, E.state, nullptr, 0, 0, s);
+    if (!cg)
+        hipLaunchKernelGGL(k_el_kfield_reduce<true>, dim3(ceil_div(6L * P.nrow, 64)), dim3(256), 0, s,
+                           sp ? one_chunk(P) : P, E.Fpart, E.dip, E.efdd, E.efdc, E.state);
     return (int)hipGetLastError();
 }
 
@@ -2358,8 +2395,8 @@ int el_launch_iteration(ElecBuffers& E, const ElecDev& P, int first, const ElecS
         hipLaunchKernelGGL(k_el_kfield_reduce<false>, dim3(ceil_div(3L * P.nrow, 64)), dim3(256), 0, s, P, E.Fpart, E.dip,
                            E.efdd, E.efdc, E.state);
     }
-    if (first || sp)
-        launch_emu(E, P, E.dip, E.state, nullptr, 0, 0, s);
+    // (the first iteration's came with the preparation)
+    if (!first && sp) launch_emu(E, P, E.dip, E.state, nullptr, 0, 0, s);
     const int nb = ceil_div(P.nrow, 256);
     hipLaunchKernelGGL(k_el_sor, dim3(nb), dim3(256), 0, s, P, E.efk, E.emu, E.efdd, E.efdc, E.dip, E.blk, E.state);
     hipLaunchKernelGGL(k_el_converge, dim3(1), dim3(64), 0, s, P, nb, E.blk, E.state);
@@ -2398,15 +2435,13 @@ static void el_cg_update(ElecBuffers& E, const ElecDev& P, const ElecSpme* sp, b
 }
 
 // conjugate-gradient start: residual of the start dipoles (their fields came with the
-// charge fields of the preparation, plus the real-space dipole field here), u = M^-1 r, and
+// charge fields of the preparation), u = M^-1 r, and
 // the first application of A, to u, for w = A u
 int el_launch_cg_init(ElecBuffers& E, const ElecDev& P, const ElecSpme* sp, hipStream_t s)
 {
-    const int nbw = ceil_div(P.nw, 256);
-    hipLaunchKernelGGL(k_cg_block, dim3(nbw), dim3(256), 0, s, P, E.x, E.y, E.z, E.cg_minv);
-    launch_emu(E, P, E.dip, E.state, nullptr, 0, 0, s);
-    hipLaunchKernelGGL(k_cg_init, dim3(nbw), dim3(256), 0, s, P, E.efk, E.efdc, E.emu, E.efdd, E.dip, E.cg_minv, E.cg_r,
-                       E.cg_u, E.cg_m, E.cg_z, E.cg_q, E.cg_s, E.cg_p, E.cg_tmu);
+    hipLaunchKernelGGL(k_cg_init, dim3(ceil_div(P.nw, CG_WPB)), dim3(256), 0, s, sp ? one_chunk(P) : P, E.Fpart, E.efk,
+                       E.efdc, E.emu, E.efdd, E.dip, E.cg_minv, E.cg_r, E.cg_u, E.cg_m, E.cg_z, E.cg_q, E.cg_s, E.cg_p,
+                       E.cg_tmu);
     if (!sp) el_cg_apply_ksum(E, P, false, 0, s);
     else el_cg_apply_other(E, P, *sp, false, 0, s);
     el_cg_update(E, P, sp, true, s);

@@ -218,8 +218,8 @@ struct ElecSpme {
     const SpmeGeom* G;
     double kap;          // V / (8 pi): from the full-space mesh sums to the half-space k sums
 };
-int el_launch_setup(ElecBuffers& E, const ElecDev& P, CellList& cells, hipStream_t s);
-int el_launch_prep(ElecBuffers& E, const ElecDev& P, const double* rcell_dev, const ElecSpme* sp, hipStream_t s);
+int el_launch_setup(ElecBuffers& E, const ElecDev& P, CellList& cells, bool cg, bool ksum, hipStream_t s);
+int el_launch_prep(ElecBuffers& E, const ElecDev& P, bool cg, const ElecSpme* sp, hipStream_t s);
 int el_launch_iteration(ElecBuffers& E, const ElecDev& P, int first, const ElecSpme* sp, hipStream_t s);
 int el_launch_final(ElecBuffers& E, const ElecDev& P, int distribute, double g34, double gln34, int refresh,
                     const ElecSpme* sp, hipStream_t s);
@@ -257,7 +257,6 @@ struct ElecState {
     double k_cell[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};     // key of the k-vector list
     int k_kmax[3] = {0, 0, 0};
     double k_alpha = -1.0, k_rcut = -1.0;
-    double* rcell = nullptr;            // [9] device copy of the inverse cell
     double scal[48];                    // host copy of the reduced scalars
     double* hpk = nullptr;              // pinned host copy of E.pk (EL_PK_N doubles)
     double out[20];                     // eng_ew1p, eng_ew2p, eng_ew3p, eng_polar, eng_cpe, vir_cpe,
