@@ -94,12 +94,15 @@ void free_buffers(ElecBuffers& E)
     dfree(E.kv); dfree(E.runs); dfree(E.runk); dfree(E.phc); dfree(E.phs); dfree(E.pht);
     dfree(E.rs_pair); dfree(E.rs_ak); dfree(E.rs_kpos);
     dfree(E.Spart); dfree(E.kf); dfree(E.Fpart);
-    dfree(E.vk); dfree(E.vr); dfree(E.vs); dfree(E.vc); dfree(E.vdck); dfree(E.vdcr); dfree(E.vesp);
-    dfree(E.fk); dfree(E.f2); dfree(E.f3); dfree(E.fsite); dfree(E.e1); dfree(E.e2); dfree(E.e3); dfree(E.ep);
-    dfree(E.s1); dfree(E.w2); dfree(E.w3); dfree(E.fmsum); dfree(E.fmx); dfree(E.eout); dfree(E.wout);
+    dfree(E.vr); dfree(E.vdcr); dfree(E.vesp); dfree(E.f2); dfree(E.fsite); dfree(E.e1); dfree(E.e2);
+    dfree(E.w2); dfree(E.fmsum); dfree(E.fmx); dfree(E.eout); dfree(E.wout);
     dfree(E.sout); dfree(E.blk); dfree(E.scal); dfree(E.err); dfree(E.pk);
     E.n = E.capA = E.capP = E.K = E.nrun = 0;
 }
+
+// doubles of block partials in E.blk: the final passes' (nkb blocks of 8 per-k sums, 8 per site, 24
+// per 16 waters), or SOR's 2 per 256 rows
+int final_partials(int n, int nw, int nkb) { return 8 * nkb + 8 * n + 24 * ((nw + 15) / 16) + 2 * (n / 256 + 1); }
 
 // site-sized buffers (allocated once per context size)
 int alloc_sites(ElecState& S, int nw, std::string& err)
@@ -123,12 +126,9 @@ int alloc_sites(ElecState& S, int nw, std::string& err)
     ECHK(dalloc(&E.cgblk, (size_t)5 * ((nw + 6) / 7) + 64));
     ECHK(dalloc(&E.ksum, (size_t)16 * n));
     ECHK(dalloc(&E.state, 16)); ECHK(dalloc(&E.zero_state, 8));
-    ECHK(dalloc(&E.vk, n)); ECHK(dalloc(&E.vr, n)); ECHK(dalloc(&E.vs, n)); ECHK(dalloc(&E.vc, n));
-    ECHK(dalloc(&E.vdck, n)); ECHK(dalloc(&E.vdcr, n)); ECHK(dalloc(&E.vesp, n));
-    ECHK(dalloc(&E.fk, (size_t)3 * n)); ECHK(dalloc(&E.f2, (size_t)3 * n)); ECHK(dalloc(&E.f3, (size_t)3 * n));
-    ECHK(dalloc(&E.fsite, (size_t)3 * n));
-    ECHK(dalloc(&E.e1, n)); ECHK(dalloc(&E.e2, n)); ECHK(dalloc(&E.e3, n)); ECHK(dalloc(&E.ep, n));
-    ECHK(dalloc(&E.s1, (size_t)9 * n)); ECHK(dalloc(&E.w2, (size_t)9 * n)); ECHK(dalloc(&E.w3, (size_t)9 * n));
+    ECHK(dalloc(&E.vr, n)); ECHK(dalloc(&E.vdcr, n)); ECHK(dalloc(&E.vesp, n));
+    ECHK(dalloc(&E.f2, (size_t)3 * n)); ECHK(dalloc(&E.fsite, (size_t)3 * n));
+    ECHK(dalloc(&E.e1, n)); ECHK(dalloc(&E.e2, n)); ECHK(dalloc(&E.w2, (size_t)9 * n));
     ECHK(dalloc(&E.fmsum, (size_t)3 * n)); ECHK(dalloc(&E.fmx, (size_t)9 * n));
     ECHK(dalloc(&E.eout, nreal)); ECHK(dalloc(&E.wout, (size_t)9 * nreal)); ECHK(dalloc(&E.sout, (size_t)9 * nreal));
     ECHK(dalloc(&E.scal, 64)); ECHK(dalloc(&E.err, 4));
@@ -385,10 +385,9 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
     ECHK(dalloc(&E.Fpart, std::max((size_t)E.kchunks * 16, (size_t)E.fchunks * 6) * E.n));
     // block partials of the final passes
     // (the particle-mesh final pass writes a partial per 4 sites where the k sum writes one
-    // per 256 k)
-    const int nsb = (E.n + 255) / 256, nkb = std::max((K + 255) / 256, (E.n + 3) / 4), nwb = (S.nw + 63) / 64;
+    // per 64 k)
     dfree(E.blk);
-    E.nblk = nsb + 8 * nkb + 2 * nsb + 8 * E.n + 24 * nwb + 2 * nsb + 64;
+    E.nblk = final_partials(E.n, S.nw, std::max((K + 63) / 64, (E.n + 3) / 4));
     ECHK(dalloc(&E.blk, (size_t)E.nblk));
     S.P.rvolm = twopi / volm;
     for (int i = 0; i < 9; ++i) S.k_cell[i] = cell[i];
@@ -409,9 +408,8 @@ int alloc_direct(ElecState& S, std::string& err)
     ElecBuffers& E = S.E;
     dfree(E.Fpart);
     ECHK(dalloc(&E.Fpart, (size_t)6 * E.n));
-    const int nsb = (E.n + 255) / 256, nkb = (E.n + 3) / 4, nwb = (S.nw + 63) / 64;
     dfree(E.blk);
-    E.nblk = nsb + 8 * nkb + 2 * nsb + 8 * E.n + 24 * nwb + 2 * nsb + 64;
+    E.nblk = final_partials(E.n, S.nw, (E.n + 3) / 4);
     ECHK(dalloc(&E.blk, (size_t)E.nblk));
     E.K = E.nrun = 0;
     E.kchunks = E.fchunks = 1;

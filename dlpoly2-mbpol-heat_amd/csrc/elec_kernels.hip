@@ -1264,18 +1264,6 @@ __global__ __launch_bounds__(64) void k_el_converge(ElecDev P, int nb, const dou
 // the first kernel of each iteration sums the update's block partials in every wavefront
 // (cg_step) and its first block records them for the update.
 
-// Fields of the converged dipoles for the final passes, from T mu, which the solver carried
-// along with mu: emu = T mu (real and reciprocal parts together), efdd = 0
-__global__ __launch_bounds__(256) void k_cg_final_fields(ElecDev P, const double* __restrict__ tmu,
-                                                         double* __restrict__ emu, double* __restrict__ efdd)
-{
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e < 3 * P.nrow) {
-        emu[e] = tmu[e];
-        efdd[e] = 0.0;
-    }
-}
-
 // The reciprocal fields of the start dipoles (efdd, with the self term) and of the charges (efdc)
 // from their chunk partials, as k_el_kfield_reduce<true>; r = E0 + T mu0 - D mu0 (T mu0 = emu +
 // efdd), u = M^-1 r, T mu = T mu0; the first application of A goes to m = u; z, q, s, p start at
@@ -1452,31 +1440,6 @@ __global__ __launch_bounds__(64) void k_cg_check(ElecDev P, int it, int nb, cons
 
 // ================================================================ final passes ======
 
-// Polarization energy per site (coulomb_polar.f:58-103).
-__global__ __launch_bounds__(256) void k_el_polar(ElecDev P, const double* __restrict__ efk,
-                                                  const double* __restrict__ emu, const double* __restrict__ efdd,
-                                                  const double* __restrict__ efdc, const double* __restrict__ dip,
-                                                  double* __restrict__ ep, double* __restrict__ blk)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double v[1] = {0.0};
-    if (i < P.n) {
-        double e = 0.0;
-        const double p2 = site_polr2(P, i);
-        if (p2 > 1.e-6) {
-            double s = 0.0;
-            for (int q = 0; q < 3; ++q)
-                s += dip[3 * i + q] * (efk[3 * i + q] + efdc[3 * i + q] + 0.5 * (emu[3 * i + q] + efdd[3 * i + q]) + 0.0);
-            const double edum = dip[3 * i] * dip[3 * i] + dip[3 * i + 1] * dip[3 * i + 1] + dip[3 * i + 2] * dip[3 * i + 2];
-            e = -s;
-            e = e + R4PIE0 * edum / p2 / 2.0;
-        }
-        ep[i] = e;
-        v[0] = e;
-    }
-    block_sum_store(v, blk + blockIdx.x);
-}
-
 // Per-k scalars of the final reciprocal pass (ewald1p.f:696-730): akk (Qc^2 + Qs^2),
 // akk |summu|^2 and the six omg components; block partials [nb][8].  Also stores, per k,
 // the constants the site pass needs in kf[k][16].  The structure factors of mu_x, mu_y, mu_z
@@ -1485,35 +1448,33 @@ __global__ __launch_bounds__(256) void k_el_kscal(ElecDev P, const double* __res
                                                   const double* __restrict__ Spart, double* __restrict__ kf,
                                                   double* __restrict__ blk)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    // four lanes per k, a set of structure factors each
+    const int k = blockIdx.x * 64 + threadIdx.x / 4, w = threadIdx.x & 3;
     double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    double mc = 0.0, ms = 0.0;
     if (k < P.K) {
-        const double kx = kv[8 * k], ky = kv[8 * k + 1], kz = kv[8 * k + 2], akk = kv[8 * k + 3];
-        const double akv = kv[8 * k + 4];
         const RsPlan& R = P.rs;
         const int pos = R.kpos[k], pg = pos >> 8, n = (pos >> 1) & 127;
         const long slot = RS_SLOT(R.ntiles), cs = slot * R.ng;
-        double Fc[4], Fs[4];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const double* base = Spart + ((long)w * R.nchq * R.ng + (pg >> 4)) * slot;
-            if (n == 0) {
-                const double* q = base + 512L * R.ntiles + (pg & 15);
-                Fc[w] = Fs[w] = 0.0;
-                for (int ch = 0; ch < R.nchq; ++ch, q += cs) {
-                    Fc[w] += q[0];
-                    Fs[w] += q[16];
-                }
-            } else {
-                double u[4];
-                rs_sums(base, cs, R.nchq, pg & 15, n, u);
-                Fc[w] = (pos & 1) ? u[2] : u[0];
-                Fs[w] = (pos & 1) ? u[3] : u[1];
+        const double* base = Spart + ((long)w * R.nchq * R.ng + (pg >> 4)) * slot;
+        if (n == 0) {
+            const double* q = base + 512L * R.ntiles + (pg & 15);
+            for (int ch = 0; ch < R.nchq; ++ch, q += cs) {
+                mc += q[0];
+                ms += q[16];
             }
+        } else {
+            double u[4];
+            rs_sums(base, cs, R.nchq, pg & 15, n, u);
+            mc = (pos & 1) ? u[2] : u[0];
+            ms = (pos & 1) ? u[3] : u[1];
         }
-        const double Qc = Fc[3], Qs = Fs[3];
-        const double Mc[3] = {Fc[0], Fc[1], Fc[2]};
-        const double Ms[3] = {Fs[0], Fs[1], Fs[2]};
+    }
+    const double Mc[3] = {__shfl(mc, 0, 4), __shfl(mc, 1, 4), __shfl(mc, 2, 4)}, Qc = __shfl(mc, 3, 4);
+    const double Ms[3] = {__shfl(ms, 0, 4), __shfl(ms, 1, 4), __shfl(ms, 2, 4)}, Qs = __shfl(ms, 3, 4);
+    if (k < P.K && w == 0) {
+        const double kx = kv[8 * k], ky = kv[8 * k + 1], kz = kv[8 * k + 2], akk = kv[8 * k + 3];
+        const double akv = kv[8 * k + 4];
         const double kk[3] = {kx, ky, kz};
         const double skdmuckrs = kx * Mc[0] + ky * Mc[1] + kz * Mc[2];
         const double skdmuskrs = kx * Ms[0] + ky * Ms[1] + kz * Ms[2];
@@ -1674,32 +1635,6 @@ __global__ __launch_bounds__(256) void k_el_ksum(ElecDev P, const double* __rest
     const bool valid = e < 15L * P.n;
     const double v = chunk_sum64(Fpart, 16L * P.n, P.kchunks, e, valid);
     if (threadIdx.x < 64 && valid) ksum[e] = v;
-}
-
-// Per-site results of the final reciprocal pass from the chunk sums, with the prefactors
-// (ewald1p.f:941-1001): fk = scale * f, vesp_k, vesp_dc_k = scale * ..., e_ew1p = scal1 * e +
-// self energy, s_ew1p = -scal1 * s, vesp_s.  Block partials [nb][2]: sum of q^2.
-__global__ __launch_bounds__(256) void k_el_kfinal_reduce(ElecDev P, const double* __restrict__ ksum,
-                                                          const double* __restrict__ chge, double* __restrict__ fk,
-                                                          double* __restrict__ vk, double* __restrict__ vdck,
-                                                          double* __restrict__ vs, double* __restrict__ e1,
-                                                          double* __restrict__ s1, double* __restrict__ blk)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    double v[2] = {0.0, 0.0};
-    if (j < P.n) {
-        double a[15];
-        for (int t = 0; t < 15; ++t) a[t] = ksum[(long)t * P.n + j];
-        const double q = chge[j];
-        for (int t = 0; t < 3; ++t) fk[3 * j + t] = P.scale * a[t];
-        vk[j] = a[3] * P.scale;
-        vdck[j] = a[4] * P.scale;
-        vs[j] = -2.0 * R4PIE0 * q * P.alpha / SQRPI;
-        e1[j] = -R4PIE0 * P.alpha * q * q / SQRPI + P.scal1 * a[5];
-        for (int t = 0; t < 9; ++t) s1[9 * j + t] = -(P.scal1 * a[6 + t]);
-        v[0] = q * q;
-    }
-    block_sum_store(v, blk + 2 * blockIdx.x);
 }
 
 namespace {
@@ -1887,330 +1822,260 @@ __global__ __launch_bounds__(64) void k_el_pairs(ElecDev P, const double* __rest
     if (lane == 25) blk[8 * i + 1] = -(sums[15] + sums[18] + sums[20]);
 }
 
-namespace {
-
-// force-matrix entry F at (row a, column b) of water-local work: contraction into the
-// per-atom tensors of the water's real atoms (M rows moved to O, H1, H2), columns of
-// real atoms only, diagonal entries skipped (heatcurrent.f90:541-555, 711-719).
-__device__ void fm_local(const ElecDev& P, const double* x, const double* y, const double* z, int a, int b,
-                         const double* F, double* w3)
+// The end of an evaluation, four lanes per water (lane a: site O, H1, H2, M), 16 waters per
+// wavefront.  In turn: the site's reciprocal results from the final pass's sums ksum, with the
+// prefactors (ewald1p.f:941-1001; null: no reciprocal space); its polarization energy
+// (coulomb_polar.f:58-103); the excluded pairs with the other three sites (ewald3p.f:80-391, every
+// pair seen from both of its sites); the ESP (forces.f:876-880); the charge-derivative forces on
+// O, H1, H2 (qdforce.f90:70-566; the charges do not depend on M); and the site forces and the
+// per-real-atom outputs of the heat-current decomposition, with the M site's share moved onto
+// O, H1, H2 (dlpoly_cmd.f:2583-2606, heatcurrent.f90:302-555): fout (3 per site; M forces moved
+// when distribute != 0), eout (energy ew1p + ew2p + ew3p + polar), sout (ew1p stress), wout
+// (force-matrix contraction; columns of real atoms only, diagonal entries skipped,
+// heatcurrent.f90:541-555, 711-719).  emu + efdd is the dipoles' own field (efdd null: emu holds
+// both).  Block partials [24]: polar, q^2, excluded pairs (energy, virial, stress 6), qd (virial,
+// stress 6), the angular terms of the per-atom qd stresses (qdforce.f90:504-531, the ones recorded
+// without HEAT_STRESS; 6).
+// Bound by one lane's latency: six launches of one thread per water or site before (polar 4, sums 5,
+// excluded pairs 18, ESP 5, qd 26, outputs 9 us at 512 waters), 16.7 us as one.
+__global__ __launch_bounds__(64) void k_el_water_final(
+    ElecDev P, int distribute, const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z,
+    const double* __restrict__ chge, const double* __restrict__ dip, const double* __restrict__ dg,
+    const double* __restrict__ ksum, const double* __restrict__ efk, const double* __restrict__ efdc,
+    const double* __restrict__ emu, const double* __restrict__ efdd, const double* __restrict__ f2,
+    const double* __restrict__ e2, const double* __restrict__ vr, const double* __restrict__ vdcr,
+    const double* __restrict__ w2, const double* __restrict__ fmsum, const double* __restrict__ fmx,
+    double* __restrict__ e1, double* __restrict__ vesp, double* __restrict__ fout, double* __restrict__ eout,
+    double* __restrict__ sout, double* __restrict__ wout, double* __restrict__ blk)
 {
-    if (b >= P.nreal) return;
-    if (a < P.nreal) {
-        if (a == b) return;
-        const double dr[3] = {x[a] - x[b], y[a] - y[b], z[a] - z[b]};
+    const int lane = threadIdx.x, a = lane & 3;
+    const int wr = blockIdx.x * 16 + (lane >> 2);
+    const bool live = wr < P.nw;
+    const int w = live ? wr : P.nw - 1;                // (lanes past the last water repeat it, unused)
+    const int i = a < 3 ? 3 * w + a : P.nreal + w;
+    const double wt = a == 0 ? 1.0 - P.gamma : 0.5 * P.gamma;
+    double red[24];
+#pragma unroll
+    for (int t = 0; t < 24; ++t) red[t] = 0.0;
+    // the water's sites
+    double xs[4][3], qs[4], mus[4][3];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const int j = b < 3 ? 3 * w + b : P.nreal + w;
+        xs[b][0] = x[j];
+        xs[b][1] = y[j];
+        xs[b][2] = z[j];
+        qs[b] = chge[j];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) mus[b][q] = dip[3 * j + q];
+    }
+    const double xi[3] = {x[i], y[i], z[i]}, qi = chge[i];
+    const double mi[3] = {dip[3 * i], dip[3 * i + 1], dip[3 * i + 2]};
+    const double p2 = site_polr2(P, i);
+    // reciprocal space
+    double f[3], vk = 0.0, vd = 0.0, e = 0.0, st[9];
+    double kz[15];
+#pragma unroll
+    for (int t = 0; t < 15; ++t) kz[t] = ksum ? ksum[(long)t * P.n + i] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) f[q] = P.scale * kz[q] + f2[3 * i + q];
+    vk = kz[3] * P.scale;
+    vd = kz[4] * P.scale;
+    const double er = -R4PIE0 * P.alpha * qi * qi / SQRPI + P.scal1 * kz[5];
+#pragma unroll
+    for (int t = 0; t < 9; ++t) st[t] = -(P.scal1 * kz[6 + t]);
+    red[1] = qi * qi;
+    // polarization
+    if (p2 > 1.e-6) {
+        double t = 0.0, m2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const double own = efdd ? emu[3 * i + q] + efdd[3 * i + q] : emu[3 * i + q];
+            t += mi[q] * (efk[3 * i + q] + efdc[3 * i + q] + 0.5 * own);
+            m2 += mi[q] * mi[q];
+        }
+        red[0] = R4PIE0 * m2 / p2 / 2.0 - t;
+    }
+    e = er + e2[i] + red[0];
+    // excluded pairs: F = force on this site from site b
+    double vc = 0.0, W[9], FM[3] = {0.0, 0.0, 0.0};    // FM: force on M from this real site
+#pragma unroll
+    for (int t = 0; t < 9; ++t) W[t] = 0.0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        if (b == a) continue;
+        const int j = b < 3 ? 3 * w + b : P.nreal + w;
+        double d[3] = {xi[0] - xs[b][0], xi[1] - xs[b][1], xi[2] - xs[b][2]};
+        image_vec(P.g, d[0], d[1], d[2]);
+        const double rsq = norm2_nc(d[0], d[1], d[2]);
+        const double rrr = sqrt(rsq);
+        const double rri = 1.0 / rrr, rsqi = rri * rri;
+        const double r3i = rri * rsqi, r5i = r3i * rsqi;
+        double bbb[4];
+        bfun_direct(P.alpha, rrr, rsqi, bbb);
+        const double qj = qs[b], cicj = qi * qj;
+        const double rdmui = mi[0] * d[0] + mi[1] * d[1] + mi[2] * d[2];
+        const double rdmuj = mus[b][0] * d[0] + mus[b][1] * d[1] + mus[b][2] * d[2];
+        double ffac = cicj * bbb[1] - (qj * rdmui - qi * rdmuj) * bbb[2];
+        double dfi = bbb[1] * qj, dfj = -bbb[1] * qi;
+        if (p2 > 1.e-6 && site_polr2(P, j) > 1.e-6) {
+            const double dpidpj = mi[0] * mus[b][0] + mi[1] * mus[b][1] + mi[2] * mus[b][2];
+            const double rr2 = rdmui * rdmuj;
+            const double ath = (a == 0 || b == 0) ? P.athole12 : P.athole13;
+            const double u = rrr * P.bbi[site_type(P, i)][site_type(P, j)];
+            const double arob4 = ath * (u * u) * (u * u);
+            const double dum1 = exp(-arob4);
+            const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
+            const double c3 = 3.0 * r5i * (1.0 - dum2) + bbb[2];
+            const double dum34 = 4.0 * arob4 * dum1 * (rsqi * rsqi);
+            ffac += dpidpj * (3.0 * r5i * (1.0 - dum1) + bbb[2] - rri * dum34) -
+                    rr2 * (15.0 * (rsqi * r5i) * (1.0 - dum2) + bbb[3] - dum34 * (4.0 * arob4 - 1.0) * r3i);
+            dfi += c3 * rdmuj;
+            dfj += c3 * rdmui;
+        }
+        double F[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            F[q] = R4PIE0 * (ffac * d[q] + dfi * mi[q] + dfj * mus[b][q]);
+            f[q] += F[q];
+        }
+        const double eh = 0.5 * cicj * bbb[0] * R4PIE0;
+        e += eh;
+        vc += R4PIE0 * (qj * bbb[0] + rdmuj * bbb[1]);
+        red[2] += eh;
+        red[4] += 0.5 * d[0] * F[0];
+        red[5] += 0.5 * d[0] * F[1];
+        red[6] += 0.5 * d[0] * F[2];
+        red[7] += 0.5 * d[1] * F[1];
+        red[8] += 0.5 * d[1] * F[2];
+        red[9] += 0.5 * d[2] * F[2];
+        if (b < 3) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) W[3 * p + q] += F[p] * (xi[q] - xs[b][q]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) FM[q] = -F[q];
+        }
+    }
+    red[3] = -(red[4] + red[7] + red[9]);
+    // the M row's entries moved to O, H1, H2 (the M lane's own W is not used)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        const double G[3] = {__shfl(FM[0], b, 4), __shfl(FM[1], b, 4), __shfl(FM[2], b, 4)};
+        if (b == a) continue;
+#pragma unroll
         for (int p = 0; p < 3; ++p)
-            for (int q = 0; q < 3; ++q) w3[9 * a + 3 * p + q] += F[p] * dr[q];
-        return;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) W[3 * p + q] += wt * G[p] * (xi[q] - xs[b][q]);
     }
-    const int w = a - P.nreal;
-    const double wt[3] = {1.0 - P.gamma, 0.5 * P.gamma, 0.5 * P.gamma};
-    for (int t = 0; t < 3; ++t) {
-        const int r = 3 * w + t;
-        if (r == b) continue;
-        const double dr[3] = {x[r] - x[b], y[r] - y[b], z[r] - z[b]};
-        for (int p = 0; p < 3; ++p)
-            for (int q = 0; q < 3; ++q) w3[9 * r + 3 * p + q] += wt[t] * F[p] * dr[q];
-    }
-}
-
-}  // namespace
-
-// Excluded-pair corrections of each water (ewald3p.f:80-391).  Writes the water's rows of
-// f3, e3, vc, w3 (all zero-initialised by this kernel) and block partials [nb][8]:
-// energy, virial, stress.
-__global__ __launch_bounds__(64) void k_el_intra_final(ElecDev P, const double* __restrict__ x,
-                                                       const double* __restrict__ y, const double* __restrict__ z,
-                                                       const double* __restrict__ chge, const double* __restrict__ dip,
-                                                       double* __restrict__ f3, double* __restrict__ e3,
-                                                       double* __restrict__ vc, double* __restrict__ w3,
-                                                       double* __restrict__ blk)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    double red[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (w < P.nw) {
-        // the water's four sites (O, H1, H2, M); every sum of the water's rows is kept in
-        // registers (slots 0..3, fully unrolled) and stored once
-        const int s[4] = {3 * w, 3 * w + 1, 3 * w + 2, P.nreal + w};
-        double xs[4][3];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            xs[a][0] = x[s[a]];
-            xs[a][1] = y[s[a]];
-            xs[a][2] = z[s[a]];
-        }
-        double fl[4][3], el[4], vl[4], wl[3][9];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            fl[a][0] = fl[a][1] = fl[a][2] = 0.0;
-            el[a] = vl[a] = 0.0;
-        }
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int t = 0; t < 9; ++t) wl[a][t] = 0.0;
-        const double wt[3] = {1.0 - P.gamma, 0.5 * P.gamma, 0.5 * P.gamma};
-        // force-matrix contraction of the pair force F on slot ai from slot bi (fm_local)
-        auto fml = [&](int ai, int bi, const double (&F)[3]) {
-            if (bi == 3) return;
-            if (ai < 3) {
-                if (ai == bi) return;
-#pragma unroll
-                for (int p = 0; p < 3; ++p)
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) wl[ai][3 * p + q] += F[p] * (xs[ai][q] - xs[bi][q]);
-                return;
-            }
-#pragma unroll
-            for (int t = 0; t < 3; ++t) {
-                if (t == bi) continue;
-#pragma unroll
-                for (int p = 0; p < 3; ++p)
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) wl[t][3 * p + q] += wt[t] * F[p] * (xs[t][q] - xs[bi][q]);
-            }
-        };
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = a + 1; b < 4; ++b) {
-                const int i = s[a], j = s[b];
-                double d[3];
-                const double rsq = sep(P, x, y, z, i, j, d);
-                const double rrr = sqrt(rsq);
-                const double rri = 1.0 / rrr, rsqi = 1.0 / rsq;
-                const double r3i = 1.0 / (rrr * rrr * rrr);
-                const double r5i = r3i * rsqi;
-                double bbb[4];
-                bfun_direct(P.alpha, rrr, rsqi, bbb);
-                const double qi = chge[i], qj = chge[j];
-                const double cicj = qi * qj;
-                red[0] += cicj * bbb[0] * R4PIE0;
-                el[a] += 0.5 * cicj * bbb[0] * R4PIE0;
-                el[b] += 0.5 * cicj * bbb[0] * R4PIE0;
-                const double espdum = bbb[0] * R4PIE0;
-                const double espdcdum = bbb[1] * R4PIE0;
-                double ffac = cicj * bbb[1] * R4PIE0;
-                const double mi[3] = {dip[3 * i], dip[3 * i + 1], dip[3 * i + 2]};
-                const double mj[3] = {dip[3 * j], dip[3 * j + 1], dip[3 * j + 2]};
-                const double rdmui = mi[0] * d[0] + mi[1] * d[1] + mi[2] * d[2];
-                const double rdmuj = mj[0] * d[0] + mj[1] * d[1] + mj[2] * d[2];
-                double facmu = (qj * rdmui - qi * rdmuj) * (-bbb[2]) * R4PIE0;
-                double dfacmui = bbb[1] * qj * R4PIE0;
-                double dfacmuj = -bbb[1] * qi * R4PIE0;
-                if (site_polr2(P, i) > 1.e-6 && site_polr2(P, j) > 1.e-6) {
-                    const double dpidpj = mi[0] * mj[0] + mi[1] * mj[1] + mi[2] * mj[2];
-                    facmu += (bbb[2] * dpidpj - bbb[3] * rdmui * rdmuj) * R4PIE0;
-                    dfacmui += bbb[2] * rdmuj * R4PIE0;
-                    dfacmuj += bbb[2] * rdmui * R4PIE0;
-                    const double facmu1 = -15.0 * rdmui * rdmuj * rsqi * r5i * R4PIE0;
-                    const double facmu2 = 3.0 * dpidpj * r5i * R4PIE0;
-                    facmu = facmu + facmu1 + facmu2;
-                    const double dfacmuidd = 3.0 * rdmuj * r5i * R4PIE0;
-                    const double dfacmujdd = 3.0 * rdmui * r5i * R4PIE0;
-                    dfacmui += dfacmuidd;
-                    dfacmuj += dfacmujdd;
-                    const double bb = pow(site_polr(P, i) * site_polr(P, j), 1.0 / 6.0);
-                    const double ath = (i % 3 == 0 || j % 3 == 0) ? P.athole12 : P.athole13;
-                    const double u = rrr / bb;
-                    const double arob4 = ath * (u * u) * (u * u);
-                    const double dum1 = exp(-arob4);
-                    const double dum2 = (1.0 + (4.0 / 3.0) * arob4) * dum1;
-                    const double bb4 = (bb * bb) * (bb * bb);
-                    const double dum3 = 4.0 * ath * (4.0 * arob4 - 1.0) * dum1 * rsqi / bb4;
-                    const double dum4 = 4.0 * ath * dum1 * rrr / bb4;
-                    facmu = facmu - facmu1 * dum2 - facmu2 * dum1 + rdmui * rdmuj * dum3 * rri * R4PIE0 -
-                            dpidpj * rsqi * dum4 * R4PIE0;
-                    dfacmui -= dfacmuidd * dum2;
-                    dfacmuj -= dfacmujdd * dum2;
-                }
-                const double dfac[3] = {dfacmui * mi[0] + dfacmuj * mj[0], dfacmui * mi[1] + dfacmuj * mj[1],
-                                        dfacmui * mi[2] + dfacmuj * mj[2]};
-                ffac += facmu;
-                const double fv[3] = {ffac * d[0] + dfac[0], ffac * d[1] + dfac[1], ffac * d[2] + dfac[2]};
-                const double virdum = dfac[0] * d[0] + dfac[1] * d[1] + dfac[2] * d[2];
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    fl[a][q] += fv[q];
-                    fl[b][q] -= fv[q];
-                }
-                const double mf[3] = {-fv[0], -fv[1], -fv[2]};
-                fml(a, b, fv);
-                fml(b, a, mf);
-                red[1] += -ffac * rsq - virdum;
-                red[2] += d[0] * fv[0];
-                red[3] += d[0] * fv[1];
-                red[4] += d[0] * fv[2];
-                red[5] += d[1] * fv[1];
-                red[6] += d[1] * fv[2];
-                red[7] += d[2] * fv[2];
-                vl[a] += qj * espdum;
-                vl[b] += qi * espdum;
-                vl[a] += rdmuj * espdcdum;
-                vl[b] -= rdmui * espdcdum;
-            }
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const int i = s[a];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) f3[3 * i + q] = fl[a][q];
-            e3[i] = el[a];
-            vc[i] = vl[a];
-        }
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int t = 0; t < 9; ++t) w3[9L * s[a] + t] = wl[a][t];
-    }
-    block_sum_store(red, blk + 8 * blockIdx.x);
-}
-
-// ESP at every site (forces.f:876-880).
-__global__ void k_el_vesp(int n, const double* __restrict__ vk, const double* __restrict__ vr,
-                          const double* __restrict__ vs, const double* __restrict__ vc, const double* __restrict__ vdck,
-                          const double* __restrict__ vdcr, double* __restrict__ vesp)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) vesp[i] = vk[i] + vr[i] + vs[i] + vc[i] + vdck[i] + vdcr[i] + 0.0;
-}
-
-// Charge-derivative forces of each water (qdforce.f90:70-566): adds to the water's rows
-// of f3 and w3; block partials [nb][8]: 0, virial, stress.
-__global__ __launch_bounds__(64) void k_el_qd(ElecDev P, const double* __restrict__ x, const double* __restrict__ y,
-                                              const double* __restrict__ z, const double* __restrict__ dg,
-                                              const double* __restrict__ vesp, double* __restrict__ f3,
-                                              double* __restrict__ w3, double* __restrict__ blk)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    // [0..7] energy (unused), virial, stress6; [8..13] the angular terms of the per-atom qd
-    // stresses (qdforce.f90:504-531, the ones recorded without HEAT_STRESS), summed
-    double red[16] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    if (w < P.nw) {
-        const int io = 3 * w, ih1 = io + 1, ih2 = io + 2, im = P.nreal + w;
-        const int site[4] = {io, ih1, ih2, im};
+    // ESP
+    const double ve = vk + vr[i] + -2.0 * R4PIE0 * qi * P.alpha / SQRPI + vc + vd + vdcr[i];
+    const double vt1 = __shfl(ve, 1, 4), vt2 = __shfl(ve, 2, 4), vt3 = __shfl(ve, 3, 4);
+    // charge derivatives
+    {
         const double* G = dg + 6 * w;   // dp1dr1, dp1dr2, dp2dr1, dp2dr2, dp1dcos, dp2dcos
-        double r1v[3], r2v[3];
-        sep(P, x, y, z, ih1, io, r1v);
-        sep(P, x, y, z, ih2, io, r2v);
+        double r1v[3] = {xs[1][0] - xs[0][0], xs[1][1] - xs[0][1], xs[1][2] - xs[0][2]};
+        double r2v[3] = {xs[2][0] - xs[0][0], xs[2][1] - xs[0][1], xs[2][2] - xs[0][2]};
+        double r3v[3] = {xs[1][0] - xs[2][0], xs[1][1] - xs[2][1], xs[1][2] - xs[2][2]};
+        image_vec(P.g, r1v[0], r1v[1], r1v[2]);
+        image_vec(P.g, r2v[0], r2v[1], r2v[2]);
+        image_vec(P.g, r3v[0], r3v[1], r3v[2]);
         const double r1 = sqrt(r1v[0] * r1v[0] + r1v[1] * r1v[1] + r1v[2] * r1v[2]);
         const double r2 = sqrt(r2v[0] * r2v[0] + r2v[1] * r2v[1] + r2v[2] * r2v[2]);
         const double rdot = r1v[0] * r2v[0] + r1v[1] * r2v[1] + r1v[2] * r2v[2];
-        const double cost = rdot / (r1 * r2);
+        const double r1i = 1.0 / r1, r2i = 1.0 / r2;
+        const double cost = rdot * (r1i * r2i);
         const double r3 = sqrt(r1 * r1 + r2 * r2 - 2.0 * r1 * r2 * cost);
         const double sint = sqrt(1.0 - cost * cost);
-        const double cott = cost / sint;
-        const double r1sqr = r1 * r1, r2sqr = r2 * r2;
-        double dr[3][4][3];
-        for (int k = 0; k < 3; ++k)
-            for (int s = 0; s < 4; ++s)
-                for (int q = 0; q < 3; ++q) dr[k][s][q] = 0.0;
-        for (int q = 0; q < 3; ++q) {
-            dr[0][1][q] = r1v[q] / r1;
-            dr[0][0][q] = -dr[0][1][q];
-            dr[1][2][q] = r2v[q] / r2;
-            dr[1][0][q] = -dr[1][2][q];
-            dr[2][1][q] = cott * (r1v[q] / r1sqr - r2v[q] / rdot);
-            dr[2][2][q] = cott * (r2v[q] / r2sqr - r1v[q] / rdot);
-            dr[2][0][q] = -dr[2][1][q] - dr[2][2][q];
-        }
+        const double cott = cost / sint, rdi = 1.0 / rdot;
         const double tmp = P.gamma / 2.0 / (1.0 - P.gamma);
-        double dq[4][4][3];
-        for (int s = 0; s < 4; ++s)
+        if (a < 3) {
+            const int col = P.compat_qd ? P.nw + w : P.nreal + w;
+            double xc[3] = {0.0, 0.0, 0.0};
+            if (col < P.nreal) {
+                xc[0] = x[col];
+                xc[1] = y[col];
+                xc[2] = z[col];
+            }
+#pragma unroll
             for (int q = 0; q < 3; ++q) {
-                const double dp1 = G[0] * dr[0][s][q] + G[1] * dr[1][s][q] - sint * G[4] * dr[2][s][q];
-                const double dp2 = G[2] * dr[0][s][q] + G[3] * dr[1][s][q] - sint * G[5] * dr[2][s][q];
-                dq[0][s][q] = 0.0;
-                dq[1][s][q] = dp1 * (tmp + 1.0) + dp2 * tmp;
-                dq[2][s][q] = dp2 * (tmp + 1.0) + dp1 * tmp;
-                dq[3][s][q] = -(dq[1][s][q] + dq[2][s][q]);
-            }
-        for (int j = 0; j < 4; ++j) {
-            const double vt = vesp[site[j]];
-            const int col = (j < 3) ? site[j] : (P.compat_qd ? P.nw + w : im);
-            for (int s = 0; s < 4; ++s) {
-                const double F[3] = {-dq[j][s][0] * vt, -dq[j][s][1] * vt, -dq[j][s][2] * vt};
-                for (int q = 0; q < 3; ++q) f3[3 * site[s] + q] += F[q];
-                fm_local(P, x, y, z, site[s], col, F, w3);
+                // derivatives of r1, r2 and theta by this site
+                const double a1 = r1v[q] * r1i, a2 = r2v[q] * r2i;
+                const double t1 = cott * (a1 * r1i - r2v[q] * rdi), t2 = cott * (a2 * r2i - r1v[q] * rdi);
+                const double d1 = a == 0 ? -a1 : a == 1 ? a1 : 0.0;
+                const double d2 = a == 0 ? -a2 : a == 2 ? a2 : 0.0;
+                const double dt = a == 0 ? -t1 - t2 : a == 1 ? t1 : t2;
+                const double dp1 = G[0] * d1 + G[1] * d2 - sint * G[4] * dt;
+                const double dp2 = G[2] * d1 + G[3] * d2 - sint * G[5] * dt;
+                const double dq1 = dp1 * (tmp + 1.0) + dp2 * tmp;
+                const double dq2 = dp2 * (tmp + 1.0) + dp1 * tmp;
+                const double F1 = -dq1 * vt1, F2 = -dq2 * vt2, F3 = (dq1 + dq2) * vt3;
+                f[q] += F1 + F2 + F3;
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    if (a != 1) W[3 * q + r] += F1 * (xi[r] - xs[1][r]);
+                    if (a != 2) W[3 * q + r] += F2 * (xi[r] - xs[2][r]);
+                    if (col < P.nreal && col != i) W[3 * q + r] += F3 * (xi[r] - xc[r]);
+                }
             }
         }
-        double dqdr12[4] = {0, 0, 0, 0}, dqdr13[4] = {0, 0, 0, 0}, dqdcos[4] = {0, 0, 0, 0};
-        dqdr12[1] = G[0] + (G[0] + G[2]) * tmp;
-        dqdr13[1] = G[1] + (G[1] + G[3]) * tmp;
-        dqdcos[1] = G[4] + (G[4] + G[5]) * tmp;
-        dqdr12[2] = G[2] + (G[0] + G[2]) * tmp;
-        dqdr13[2] = G[3] + (G[1] + G[3]) * tmp;
-        dqdcos[2] = G[5] + (G[4] + G[5]) * tmp;
-        dqdr12[3] = -(G[0] + G[2]) / (1.0 - P.gamma);
-        dqdr13[3] = -(G[1] + G[3]) / (1.0 - P.gamma);
-        dqdcos[3] = -(G[4] + G[5]) / (1.0 - P.gamma);
-        double rv[2][3], r3v[3];
-        sep(P, x, y, z, io, ih1, rv[0]);
-        sep(P, x, y, z, io, ih2, rv[1]);
-        sep(P, x, y, z, ih1, ih2, r3v);
-        const double rr1 = sqrt(rv[0][0] * rv[0][0] + rv[0][1] * rv[0][1] + rv[0][2] * rv[0][2]);
-        const double rr2 = sqrt(rv[1][0] * rv[1][0] + rv[1][1] * rv[1][1] + rv[1][2] * rv[1][2]);
-        const double rr3 = sqrt(r3v[0] * r3v[0] + r3v[1] * r3v[1] + r3v[2] * r3v[2]);
-        const double dcosdr12 = (r1 - r2 * cost) / r1 / r2;
-        const double dcosdr13 = (r2 - r1 * cost) / r1 / r2;
-        const double dcosdr23 = -r3 / r1 / r2;
+        // this site's charge in the virial and stress
+        const double g0 = a == 1 ? G[0] + (G[0] + G[2]) * tmp : a == 2 ? G[2] + (G[0] + G[2]) * tmp
+                        : a == 3 ? -(G[0] + G[2]) / (1.0 - P.gamma) : 0.0;
+        const double g1 = a == 1 ? G[1] + (G[1] + G[3]) * tmp : a == 2 ? G[3] + (G[1] + G[3]) * tmp
+                        : a == 3 ? -(G[1] + G[3]) / (1.0 - P.gamma) : 0.0;
+        const double gc = a == 1 ? G[4] + (G[4] + G[5]) * tmp : a == 2 ? G[5] + (G[4] + G[5]) * tmp
+                        : a == 3 ? -(G[4] + G[5]) / (1.0 - P.gamma) : 0.0;
+        const double rr3i = 1.0 / sqrt(r3v[0] * r3v[0] + r3v[1] * r3v[1] + r3v[2] * r3v[2]);
+        const double c12 = (r1 - r2 * cost) * r1i * r2i * r1i, c13 = (r2 - r1 * cost) * r1i * r2i * r2i;
+        const double c23 = -r3 * r1i * r2i * rr3i;
         const int sa[6] = {0, 0, 0, 1, 1, 2}, sb[6] = {0, 1, 2, 1, 2, 2};
-        for (int i = 0; i < 4; ++i) {
-            const double vt = vesp[site[i]];
-            for (int pr = 0; pr < 2; ++pr) {
-                const double dqdr = pr == 0 ? dqdr12[i] : dqdr13[i];
-                const double* r = rv[pr];
-                const double rjk = pr == 0 ? rr1 : rr2;
-                for (int t = 0; t < 6; ++t) red[2 + t] -= vt * dqdr * r[sa[t]] * r[sb[t]] / rjk;
-                red[1] += vt * rjk * dqdr;
-            }
-            double dc[6];
-            for (int t = 0; t < 6; ++t)
-                dc[t] = dcosdr12 * rv[0][sa[t]] * rv[0][sb[t]] / rr1 + dcosdr13 * rv[1][sa[t]] * rv[1][sb[t]] / rr2 +
-                        dcosdr23 * r3v[sa[t]] * r3v[sb[t]] / rr3;
-            for (int t = 0; t < 6; ++t) red[2 + t] -= vt * dqdcos[i] * dc[t];
-            for (int t = 0; t < 6; ++t) red[8 + t] += vt * dqdcos[i] * dc[t];
-            red[1] += vt * (dc[0] + dc[3] + dc[5]) * dqdcos[i];
+        double dc[6];
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+            const double p1 = r1v[sa[t]] * r1v[sb[t]], p2r = r2v[sa[t]] * r2v[sb[t]], p3 = r3v[sa[t]] * r3v[sb[t]];
+            dc[t] = c12 * p1 + c13 * p2r + c23 * p3;
+            red[11 + t] = -ve * (g0 * r1i * p1 + g1 * r2i * p2r + gc * dc[t]);
+            red[17 + t] = ve * gc * dc[t];
         }
+        red[10] = ve * (r1 * g0 + r2 * g1 + gc * (dc[0] + dc[3] + dc[5]));
     }
-    block_sum_store(red, blk + 16 * blockIdx.x);
-}
-
-// Site forces and the per-real-atom outputs of the heat-current decomposition, with the
-// M-site redistribution (dlpoly_cmd.f:2583-2606, heatcurrent.f90:302-555).  One thread
-// per water: fout (3 per site; M forces moved to O, H1, H2 when distribute != 0),
-// eout (energy ew1p + ew2p + ew3p + polar), sout (ew1p stress), wout (force-matrix
-// contraction) for O, H1, H2.
-__global__ void k_el_combine(ElecDev P, int distribute, const double* __restrict__ x, const double* __restrict__ y,
-                             const double* __restrict__ z, const double* __restrict__ fk, const double* __restrict__ f2,
-                             const double* __restrict__ f3, const double* __restrict__ e1, const double* __restrict__ e2,
-                             const double* __restrict__ e3, const double* __restrict__ ep,
-                             const double* __restrict__ s1, const double* __restrict__ w2,
-                             const double* __restrict__ w3, const double* __restrict__ fmsum,
-                             const double* __restrict__ fmx, double* __restrict__ fout, double* __restrict__ eout,
-                             double* __restrict__ sout, double* __restrict__ wout)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= P.nw) return;
-    const int m = P.nreal + w;
-    const double wt[3] = {1.0 - P.gamma, P.gamma / 2.0, P.gamma / 2.0};
-    double fm[3];
-    for (int q = 0; q < 3; ++q) fm[q] = fk[3 * m + q] + f2[3 * m + q] + f3[3 * m + q];
-    const double em = e1[m] + e2[m] + e3[m] + ep[m];
-    for (int t = 0; t < 3; ++t) {
-        const int r = 3 * w + t;
-        for (int q = 0; q < 3; ++q) {
-            const double f = fk[3 * r + q] + f2[3 * r + q] + f3[3 * r + q];
-            fout[3 * r + q] = distribute ? f + wt[t] * fm[q] : f;
+    // outputs, the M site's share moved onto the real atoms
+    double fm[3], sm[9];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) fm[q] = __shfl(f[q], 3, 4);
+#pragma unroll
+    for (int t = 0; t < 9; ++t) sm[t] = __shfl(st[t], 3, 4);
+    const double em = __shfl(e, 3, 4);
+    if (live) {
+        e1[i] = er;
+        vesp[i] = ve;
+        if (a < 3) {
+            const int m = P.nreal + w;
+            eout[i] = e + wt * em;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) fout[3 * i + q] = distribute ? f[q] + wt * fm[q] : f[q];
+#pragma unroll
+            for (int t = 0; t < 9; ++t) sout[9 * i + t] = st[t] + wt * sm[t];
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    wout[9 * i + 3 * p + q] = w2[9 * i + 3 * p + q] + W[3 * p + q] +
+                                              wt * (fmsum[3 * m + p] * xi[q] - fmx[9 * m + 3 * p + q]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) fout[3 * i + q] = distribute ? 0.0 : f[q];
         }
-        eout[r] = (e1[r] + e2[r] + e3[r] + ep[r]) + wt[t] * em;
-        for (int q = 0; q < 9; ++q) sout[9 * r + q] = s1[9 * r + q] + wt[t] * s1[9 * m + q];
-        const double xr[3] = {x[r], y[r], z[r]};
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b)
-                wout[9 * r + 3 * a + b] =
-                    w2[9 * r + 3 * a + b] + w3[9 * r + 3 * a + b] + wt[t] * (fmsum[3 * m + a] * xr[b] - fmx[9 * m + 3 * a + b]);
+    } else {
+#pragma unroll
+        for (int t = 0; t < 24; ++t) red[t] = 0.0;
     }
-    for (int q = 0; q < 3; ++q) fout[3 * m + q] = distribute ? 0.0 : fm[q];
+    int k;
+    const double t = wave_sum24(red, lane, k);
+    if (k < 24 && (lane & 1) == 0) blk[24L * blockIdx.x + k] = t;
 }
 
 // Fixed-order sums of block partials: set b has nb[b] blocks of stride[b] values, of which
@@ -2473,28 +2338,12 @@ int el_time_sfac(ElecBuffers& E, const ElecDev& P, int reps, hipEvent_t a, hipEv
 int el_launch_final(ElecBuffers& E, const ElecDev& P, int distribute, double g34, double gln34, int refresh,
                     const ElecSpme* sp, hipStream_t s)
 {
-    // fields of the final dipoles: carried along by the conjugate-gradient solver; the SOR path
-    // keeps those of its last iteration, as the reference does
-    if (refresh)
-        hipLaunchKernelGGL(k_cg_final_fields, dim3(ceil_div(3L * P.nrow, 256)), dim3(256), 0, s, P, E.cg_tmu, E.emu,
-                           E.efdd);
-    // k-sum: one partial per 256 k; particle mesh: one per 4 sites (k_sp_elec_final's blocks)
-    const int nsb = ceil_div(P.n, 256), nwb = ceil_div(P.nw, 64), nkb = sp ? ceil_div(P.n, 4) : ceil_div(P.K, 256);
-    double* b_pol = E.blk;                       // [nsb]
-    double* b_ks = b_pol + nsb;                  // [nkb][8]
-    double* b_q2 = b_ks + 8L * nkb;              // [nsb][2]
-    double* b_p2 = b_q2 + 2L * nsb;              // [n][8]
-    double* b_p3 = b_p2 + 8L * P.n;              // [nwb][8]
-    double* b_qd = b_p3 + 8L * nwb;              // [nwb][16]
-    hipLaunchKernelGGL(k_el_polar, dim3(nsb), dim3(256), 0, s, P, E.efk, E.emu, E.efdd, E.efdc, E.dip, E.ep, b_pol);
-    if (sp && !sp->B) {
-        // no reciprocal space: zero site sums and per-block partials for the k-sum's final
-        // kernel (forces, ESP, per-atom energy and stress of the reciprocal part all 0)
-        double* d[2] = {E.ksum, b_ks};
-        const double* sr[2] = {nullptr, nullptr};
-        const long len[2] = {15L * P.n, 8L * nkb};
-        el_launch_copy_segs(2, d, sr, len, s);
-    } else if (sp) {
+    // k-sum: one partial per 64 k; particle mesh: one per 4 sites (k_sp_elec_final's blocks)
+    const int nwb = ceil_div(P.nw, 16), nkb = !sp ? ceil_div(P.K, 64) : sp->B ? ceil_div(P.n, 4) : 0;
+    double* b_ks = E.blk;                        // [nkb][8]
+    double* b_p2 = b_ks + 8L * nkb;              // [n][8]
+    double* b_w = b_p2 + 8L * P.n;               // [nwb][24]
+    if (sp && sp->B) {
         // particle mesh: grids 0..4 hold q + mu, q, and mu_x, mu_y, mu_z as charges; the
         // stress kernels of grid 0 go to grids 5..10; every per-site quantity of the k-sum
         // site pass then comes from one gather (k_sp_elec_final), in the k-sum pass's units
@@ -2524,23 +2373,21 @@ int el_launch_final(ElecBuffers& E, const ElecDev& P, int distribute, double g34
                            E.runk, E.phc, E.phs, E.kv, E.kf, E.chge, E.dip, E.Fpart);
         hipLaunchKernelGGL(k_el_ksum, dim3(ceil_div(15L * P.n, 64)), dim3(256), 0, s, P, E.Fpart, E.ksum);
     }
-    hipLaunchKernelGGL(k_el_kfinal_reduce, dim3(nsb), dim3(256), 0, s, P, E.ksum, E.chge, E.fk, E.vk, E.vdck, E.vs,
-                       E.e1, E.s1, b_q2);
     hipLaunchKernelGGL(k_el_pairs, dim3(P.n), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.dip, E.tab, E.nbrA, E.cntA,
                        g34, gln34, E.f2, E.e2, E.vr, E.vdcr, E.w2, E.fmsum, E.fmx, b_p2);
-    hipLaunchKernelGGL(k_el_intra_final, dim3(nwb), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.dip, E.f3, E.e3, E.vc,
-                       E.w3, b_p3);
-    hipLaunchKernelGGL(k_el_vesp, dim3(nsb), dim3(256), 0, s, P.n, E.vk, E.vr, E.vs, E.vc, E.vdck, E.vdcr, E.vesp);
-    hipLaunchKernelGGL(k_el_qd, dim3(nwb), dim3(64), 0, s, P, E.x, E.y, E.z, E.dg, E.vesp, E.f3, E.w3, b_qd);
-    hipLaunchKernelGGL(k_el_combine, dim3(nwb), dim3(64), 0, s, P, distribute, E.x, E.y, E.z, E.fk, E.f2, E.f3, E.e1,
-                       E.e2, E.e3, E.ep, E.s1, E.w2, E.w3, E.fmsum, E.fmx, E.fsite, E.eout, E.sout, E.wout);
-    // scalars: [0] eng_polar, [1..8] k sums (engc, engdum, omg6), [9..10] sum q^2,
-    // [11..18] pairs (energy, virial, stress6), [19..26] excluded pairs, [27..34] qd,
+    // the dipoles' own field: carried along by the conjugate-gradient solver as T mu; the SOR path
+    // keeps that of its last iteration, as the reference does
+    hipLaunchKernelGGL(k_el_water_final, dim3(nwb), dim3(64), 0, s, P, distribute, E.x, E.y, E.z, E.chge, E.dip, E.dg,
+                       sp && !sp->B ? nullptr : E.ksum, E.efk, E.efdc, refresh ? E.cg_tmu : E.emu,
+                       refresh ? nullptr : E.efdd, E.f2, E.e2, E.vr, E.vdcr, E.w2, E.fmsum, E.fmx, E.e1, E.vesp, E.fsite,
+                       E.eout, E.sout, E.wout, b_w);
+    // scalars: [0] eng_polar, [1..8] k sums (engc, engdum, omg6), [9] sum q^2, [11..18] pairs
+    // (energy, virial, stress6), [19..26] excluded pairs, [28..34] qd (virial, stress6),
     // [35..40] angular per-atom qd stresses
     SumSets ss{};
-    const double* sb[7] = {b_pol, b_ks, b_q2, b_p2, b_p3, b_qd, b_qd + 8};
-    const int snb[7] = {nsb, nkb, nsb, P.n, nwb, nwb, nwb}, sst[7] = {1, 8, 2, 8, 8, 16, 16};
-    const int snv[7] = {1, 8, 2, 8, 8, 8, 6}, soff[7] = {0, 1, 9, 11, 19, 27, 35};
+    const double* sb[7] = {b_ks, b_p2, b_w, b_w + 1, b_w + 2, b_w + 10, b_w + 17};
+    const int snb[7] = {nkb, P.n, nwb, nwb, nwb, nwb, nwb}, sst[7] = {8, 8, 24, 24, 24, 24, 24};
+    const int snv[7] = {8, 8, 1, 1, 8, 7, 6}, soff[7] = {1, 11, 0, 9, 19, 28, 35};
     ss.nsv = 0;
     for (int q = 0; q < 7; ++q) {
         ss.blk[q] = sb[q];

@@ -196,11 +196,10 @@ struct ElecBuffers {
     double* kf = nullptr;                                      // [K][16] per-k constants of the final pass
     double* zero_state = nullptr;                              // [8] zeros (solver state of final passes)
     double* Fpart = nullptr;                                   // [kchunks][16][n], [fchunks][6][n] site partials
-    double *vk = nullptr, *vr = nullptr, *vs = nullptr, *vc = nullptr, *vdck = nullptr, *vdcr = nullptr,
-           *vesp = nullptr;                                    // [n]
-    double *fk = nullptr, *f2 = nullptr, *f3 = nullptr, *fsite = nullptr;  // [3n]
-    double *e1 = nullptr, *e2 = nullptr, *e3 = nullptr, *ep = nullptr;     // [n]
-    double *s1 = nullptr, *w2 = nullptr, *w3 = nullptr;        // [9n]
+    double *vr = nullptr, *vdcr = nullptr, *vesp = nullptr;    // [n]
+    double *f2 = nullptr, *fsite = nullptr;                    // [3n]
+    double *e1 = nullptr, *e2 = nullptr;                       // [n]
+    double* w2 = nullptr;                                      // [9n]
     double *fmsum = nullptr, *fmx = nullptr;                   // [3n], [9n] M-row sums of ewald2p
     double *eout = nullptr, *wout = nullptr, *sout = nullptr;  // [nreal], [9 nreal] x2: per real atom
     double* blk = nullptr;                                     // [nblk][16] block partials
