@@ -18,10 +18,8 @@
 #include "mbgpu_internal.h"
 
 int mb_launch_lists(MbBuffers& B, const CellGeom& g, hipStream_t s);
-int mb_launch_dimers(MbBuffers& B, const int* ncnt, int ncap, const CellGeom& g, bool gather, hipStream_t s);
-int mb_launch_trimers(MbBuffers& B, const int* ncnt, int ncap, int blk_off, const CellGeom& g, bool gather,
-                      hipStream_t s);
-int mb_launch_accumulate(MbBuffers& B, double* fx, double* fy, double* fz, hipStream_t s);
+int mb_launch_clusters(MbBuffers& B, int cap2, int cap3, const CellGeom& g, bool gather, hipStream_t s);
+int mb_launch_accumulate(MbBuffers& B, double* fx, double* fy, double* fz, bool clear_f, hipStream_t s);
 int md_launch_stage(int stage, int nr, double dt, const double* mass, double* x, double* y, double* z, double* vx,
                     double* vy, double* vz, double* fx, double* fy, double* fz, double* fsite, double* ekin,
                     double* blk, double* out, hipStream_t s);
@@ -285,7 +283,6 @@ int alloc_fixed(mbgpu_ctx* c)
     HIPCHK(dalloc(&B.tcnt, nw));
     HIPCHK(dalloc(&B.toff, nw));
     HIPCHK(dalloc(&B.counts, 4));
-    HIPCHK(dalloc(&B.is_water, (size_t)4 * ((na + 3) / 4)));
     HIPCHK(dalloc(&B.scal, 16));
     HIPCHK(dalloc(&B.atomic_energy, na));
     HIPCHK(dalloc(&B.heat_w, (size_t)9 * na));
@@ -404,9 +401,8 @@ int build_lists(mbgpu_ctx* c)
 int run_clusters(mbgpu_ctx* c, double* fx, double* fy, double* fz)
 {
     MbBuffers& B = c->B;
-    int rc = mb_launch_dimers(B, B.counts, (int)B.dcap, c->geom, true, c->stream);
-    if (!rc) rc = mb_launch_trimers(B, B.counts + 1, (int)B.tcap, (int)((B.dcap + 127) / 128), c->geom, true, c->stream);
-    if (!rc) rc = mb_launch_accumulate(B, fx, fy, fz, c->stream);
+    int rc = mb_launch_clusters(B, (int)B.dcap, (int)B.tcap, c->geom, true, c->stream);
+    if (!rc) rc = mb_launch_accumulate(B, fx, fy, fz, false, c->stream);
     if (rc) return fail(rc, "cluster kernels failed (%d)", rc);
     return 0;
 }
@@ -470,8 +466,7 @@ int leaf_eval(int nmon, const double* const* w, double* E, double* gout)
     // one cluster (the count 1 in counts[0] and counts[1]), stride 1
     const int one[2] = {1, 1};
     HIPCHK(hipMemcpyAsync(B.counts, one, sizeof one, hipMemcpyHostToDevice, c->stream));
-    int rc = nmon == 2 ? mb_launch_dimers(B, B.counts, 1, c->geom, false, c->stream)
-                       : mb_launch_trimers(B, B.counts + 1, 1, 0, c->geom, false, c->stream);
+    int rc = mb_launch_clusters(B, nmon == 2 ? 1 : 0, nmon == 2 ? 0 : 1, c->geom, false, c->stream);
     if (rc) return fail(rc, "leaf kernels failed");
     HIPCHK(hipMemcpyAsync(E, nmon == 2 ? B.e2 : B.e3, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipMemcpyAsync(gout, nmon == 2 ? B.g2 : B.g3, sizeof(double) * 9 * nmon, hipMemcpyDeviceToHost,
@@ -613,15 +608,9 @@ int full_enqueue_mbpol_water(mbgpu_ctx* c, double* x, double* y, double* z, doub
                              hipStream_t a)
 {
     MbBuffers& B = c->B;
-    if (fx) {
-        el_launch_zero(fx, B.natms, a);
-        el_launch_zero(fy, B.natms, a);
-        el_launch_zero(fz, B.natms, a);
-    }
     int rc = mb_launch_lists(B, c->geom, a);
-    if (!rc) rc = mb_launch_dimers(B, B.counts, (int)B.dcap, c->geom, true, a);
-    if (!rc) rc = mb_launch_trimers(B, B.counts + 1, (int)B.tcap, (int)((B.dcap + 127) / 128), c->geom, true, a);
-    if (!rc) rc = mb_launch_accumulate(B, fx, fy, fz, a);
+    if (!rc) rc = mb_launch_clusters(B, (int)B.dcap, (int)B.tcap, c->geom, true, a);
+    if (!rc) rc = mb_launch_accumulate(B, fx, fy, fz, true, a);
     if (!rc) rc = water_enqueue(c->wt, x, y, z, fx, fy, fz, a);
     if (rc) return fail(rc, "MB-pol or water-term kernels failed: %s", hipGetErrorString((hipError_t)rc));
     return 0;
@@ -788,7 +777,7 @@ void mbgpu_destroy(mbgpu_ctx* c)
     dfree(B.tcnt); dfree(B.toff); dfree(B.counts); dfree(B.dimers); dfree(B.trimers);
     dfree(B.clus2); dfree(B.xv2); dfree(B.part2); dfree(B.e2); dfree(B.g2); dfree(B.s2);
     dfree(B.clus3); dfree(B.xv3); dfree(B.part3); dfree(B.e3); dfree(B.g3); dfree(B.s3);
-    dfree(B.is_water); dfree(B.nbr2l); dfree(B.cnt2l); dfree(B.kmask); dfree(B.rowoff); dfree(B.blk); dfree(B.scal); dfree(B.atomic_energy); dfree(B.heat_w); dfree(B.fout);
+    dfree(B.nbr2l); dfree(B.cnt2l); dfree(B.kmask); dfree(B.rowoff); dfree(B.blk); dfree(B.scal); dfree(B.atomic_energy); dfree(B.heat_w); dfree(B.fout);
     dfree(B.cs2); dfree(B.cs3);
     cells_free(B.cells);
     dfree(B.xv2f); dfree(B.part2f); dfree(B.cs2f); dfree(B.xv3f); dfree(B.part3f); dfree(B.cs3f);
@@ -1745,11 +1734,8 @@ int mbgpu_time_forces(mbgpu_ctx* c, int reps, double* ms_per_eval, double* ms_pi
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     for (int r = 0; r < reps; ++r) {
         if (build_lists(c)) return -1;
-        int rc = mb_launch_dimers(B, B.counts, (int)B.dcap, c->geom, true, c->stream);
-        if (!rc)
-            rc = mb_launch_trimers(B, B.counts + 1, (int)B.tcap, (int)((B.dcap + 127) / 128), c->geom, true,
-                                   c->stream);
-        if (!rc) rc = mb_launch_accumulate(B, nullptr, nullptr, nullptr, c->stream);
+        int rc = mb_launch_clusters(B, (int)B.dcap, (int)B.tcap, c->geom, true, c->stream);
+        if (!rc) rc = mb_launch_accumulate(B, nullptr, nullptr, nullptr, false, c->stream);
         if (rc) return fail(rc, "timing run failed");
         double s[16];
         HIPCHK(hipMemcpyAsync(s, B.scal, sizeof s, hipMemcpyDeviceToHost, c->stream));
@@ -1759,7 +1745,7 @@ int mbgpu_time_forces(mbgpu_ctx* c, int reps, double* ms_per_eval, double* ms_pi
     HIPCHK(hipEventElapsedTime(&total, c->ev0, c->ev1));
     // the 3-body polynomial kernel alone, same stream
     HIPCHK(hipEventRecord(c->ev2, c->stream));
-    for (int r = 0; r < reps; ++r) launch_pip3b_f64(B.xv3, B.part3, B.counts + 1, (int)B.tcap, B.cs3, c->stream);
+    for (int r = 0; r < reps; ++r) launch_pip_f64(B.counts, nullptr, nullptr, 0, nullptr, B.xv3, B.part3, (int)B.tcap, B.cs3, c->stream);
     HIPCHK(hipEventRecord(c->ev3, c->stream));
     HIPCHK(hipEventSynchronize(c->ev3));
     HIPCHK(hipEventElapsedTime(&k3, c->ev2, c->ev3));

@@ -35,14 +35,15 @@ inline hipError_t mbgpu_alloc(T** p, size_t n)
     return e;
 }
 
-// Launch wrappers for the generated polynomial kernels (pip2b.hip / pip3b.hip): the first
-// *ncnt clusters (a device count) of buffers laid out with stride ncap, ncap lanes launched.
-// xv: variables SoA [nvars][ncap]; part: SoA [nslices][nvars+1][ncap]; cs: coefficient stream.
-void launch_pip2b_f64(const double* xv, double* part, const int* ncnt, int ncap, const double* cs, hipStream_t s);
-void launch_pip3b_f64(const double* xv, double* part, const int* ncnt, int ncap, const double* cs, hipStream_t s);
-// FP32 instantiations of the same code (mixed-precision mode)
-void launch_pip2b_f32(const float* xv, float* part, const int* ncnt, int ncap, const float* cs, hipStream_t s);
-void launch_pip3b_f32(const float* xv, float* part, const int* ncnt, int ncap, const float* cs, hipStream_t s);
+// Launch wrappers for the generated polynomial kernels (pip_f64.hip, pip_f32.hip): the first
+// counts[0] dimers and counts[1] trimers (device counts) of buffers laid out with strides cap2 and
+// cap3, as many lanes launched (0: none).  xv: variables SoA [nvars][cap]; part: SoA
+// [nslices][nvars+1][cap]; cs: coefficient streams.
+void launch_pip_f64(const int* counts, const double* xv2, double* part2, int cap2, const double* cs2, const double* xv3,
+                    double* part3, int cap3, const double* cs3, hipStream_t s);
+// the same in FP32 (mixed-precision mode)
+void launch_pip_f32(const int* counts, const float* xv2, float* part2, int cap2, const float* cs2, const float* xv3,
+                    float* part3, int cap3, const float* cs3, hipStream_t s);
 int pip2b_nslices();
 int pip3b_nslices();
 int pip2b_stream_len();
@@ -102,7 +103,6 @@ struct MbBuffers {
     // accumulators
     long long* acc = nullptr;      // fixed-point sums: [2][13*natms] (high halves, low halves) of
                                    // forces (3n), energies (n), heat-flux tensors (9n)
-    unsigned char* is_water = nullptr;  // natms (rounded up to 4)
     double* blk = nullptr;         // per-block partial scalars
     int nblk_cap = 0;
     double* scal = nullptr;        // [16] reduced scalars

@@ -6,10 +6,10 @@
 //   image_monomers   mbpol.f90:1275-1301     k_image_monomers
 //   pair predicate   mbpol.f90:496-503       k_neighbours (|img(O_i-O_j)|^2 <= r2f^2)
 //   triple predicate mbpol.f90:843-869       k_trimers (some monomer within r3f of both)
-//   re-imaging       mbpol.f90:505-509,875-882  k_gather2 / k_gather3
-//   2B leaf          mbpol-2b-poly.cpp:358-682  k_setup2 + pip2b + k_finish2
-//   3B leaf          mbpol-3b-poly.cpp:148-312  k_setup3 + pip3b + k_finish3
-//   accumulation     mbpol.f90:519-653, 896-1067  k_accum2 / k_accum3
+//   re-imaging       mbpol.f90:505-509,875-882  k_clusters (gather2, gather3)
+//   2B leaf          mbpol-2b-poly.cpp:358-682  k_clusters (setup2) + k_pip + k_finish (finish2)
+//   3B leaf          mbpol-3b-poly.cpp:148-312  k_clusters (setup3) + k_pip + k_finish (finish3)
+//   accumulation     mbpol.f90:519-653, 896-1067  k_gather_water
 //   heat-current bookkeeping  heatcurrent.f90 update_energy_mbpol / update_forces, contracted
 //                    per atom as W_i = sum_j F_ij (x) (x_i - x_j) (heatcurrent.f90:716-719)
 #include <stdio.h>
@@ -156,11 +156,6 @@ __device__ __forceinline__ void block_reduce_store(const double* vals, int n, do
 
 // ===================================================================== kernels ======
 
-__global__ void k_zero_ll(long long* __restrict__ p, long n)
-{
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = 0;
-}
-
 __global__ void k_zero_i(int* __restrict__ p, int n)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -302,17 +297,29 @@ __global__ __launch_bounds__(64) void k_neighbours(int nw, const double* __restr
 // The count pass records, per row, the bit mask of kept partners and the number of kept
 // pairs before the row, so that the position of any kept pair in c's output range is
 // toff[c] + rowoff[c][p] + popcount(mask[c][p] below bit q); k_gather_water uses this to
-// find the trimers of a water without atomics.
+// find the trimers of a water without atomics.  The fill pass also writes the dimers (c, j > c).
 template <bool FILL>
 __global__ __launch_bounds__(64) void k_trimers(int nw, const double* __restrict__ mon, CellGeom g,
                                                 const int* __restrict__ nbr3, const int* __restrict__ cnt3,
                                                 int* __restrict__ tcnt, const int* __restrict__ toff,
                                                 unsigned long long* __restrict__ kmask, int* __restrict__ rowoff,
-                                                int* __restrict__ trimers, long tcap)
+                                                int* __restrict__ trimers, long tcap, int cap2,
+                                                const int* __restrict__ nbr2, const int* __restrict__ cnt2,
+                                                const int* __restrict__ off2, int* __restrict__ dimers, long dcap)
 {
     const int c = blockIdx.x;
     const int lane = threadIdx.x;
     if (c >= nw) return;
+    if (FILL) {
+        const int n2 = min(cnt2[c], cap2);
+        for (int q = lane; q < n2; q += 64) {
+            const long d = (long)off2[c] + q;
+            if (d < dcap) {
+                dimers[2 * d] = c;
+                dimers[2 * d + 1] = nbr2[(long)c * cap2 + q];
+            }
+        }
+    }
     const int n = min(cnt3[c], 64);
     const int* S = nbr3 + (long)c * 64;
     const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -361,10 +368,13 @@ __global__ __launch_bounds__(64) void k_trimers(int nw, const double* __restrict
     }
 }
 
-// Exclusive prefix sum of n counts (one block of 1024 threads); total to *total.
-__global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ cnt, int n, int* __restrict__ off,
-                                               int* __restrict__ total)
+// Exclusive prefix sums of n counts, one block of 1024 threads per set: dimers per water, then
+// trimers per centre; totals to total[0], total[1].
+__global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ cnt2, const int* __restrict__ cnt3, int n,
+                                               int* __restrict__ off2, int* __restrict__ off3, int* __restrict__ total)
 {
+    const int* __restrict__ cnt = blockIdx.x ? cnt3 : cnt2;
+    int* __restrict__ off = blockIdx.x ? off3 : off2;
     __shared__ long wsum[16];
     const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
     const int per = (n + 1023) / 1024;
@@ -386,7 +396,7 @@ __global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ cnt, int 
             wsum[w] = acc;
             acc += v;
         }
-        *total = (int)acc;
+        total[blockIdx.x] = (int)acc;
     }
     __syncthreads();
     long acc = wsum[wid] + inc - s;
@@ -396,28 +406,10 @@ __global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ cnt, int 
     }
 }
 
-__global__ void k_fill_dimers(int nw, int cap2, const int* __restrict__ nbr2, const int* __restrict__ cnt2,
-                              const int* __restrict__ off2, int* __restrict__ dimers, long dcap)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nw) return;
-    const int n = min(cnt2[i], cap2);
-    for (int q = 0; q < n; ++q) {
-        const long d = (long)off2[i] + q;
-        if (d < dcap) {
-            dimers[2 * d] = i;
-            dimers[2 * d + 1] = nbr2[(long)i * cap2 + q];
-        }
-    }
-}
-
 // Re-image a dimer around its second water (mbpol.f90:496-509); SoA [18][nd].
-__global__ void k_gather2(const int* __restrict__ ncnt, int ncap, const int* __restrict__ dimers, const double* __restrict__ mon, CellGeom g,
-                          double* __restrict__ clus)
+__device__ __forceinline__ void gather2(int d, int ncap, const int* __restrict__ dimers, const double* __restrict__ mon,
+                                        const CellGeom& g, double* __restrict__ clus)
 {
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nd = min(*ncnt, ncap);
-    if (d >= nd) return;
     double w1[9], w2[9];
     load_mon(mon, dimers[2 * d], w1);
     load_mon(mon, dimers[2 * d + 1], w2);
@@ -437,12 +429,9 @@ __global__ void k_gather2(const int* __restrict__ ncnt, int ncap, const int* __r
 }
 
 // Re-image a trimer around its middle water (mbpol.f90:843-882); SoA [27][nt].
-__global__ void k_gather3(const int* __restrict__ ncnt, int ncap, const int* __restrict__ trimers, const double* __restrict__ mon, CellGeom g,
-                          double* __restrict__ clus)
+__device__ __forceinline__ void gather3(int t, int ncap, const int* __restrict__ trimers, const double* __restrict__ mon,
+                                        const CellGeom& g, double* __restrict__ clus)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nt = min(*ncnt, ncap);
-    if (t >= nt) return;
     double w1[9], w2[9], w3[9];
     load_mon(mon, trimers[3 * t], w1);
     load_mon(mon, trimers[3 * t + 1], w2);
@@ -470,11 +459,9 @@ __global__ void k_gather3(const int* __restrict__ ncnt, int ncap, const int* __r
 
 // 2B variables (mbpol-2b-poly.cpp:358-445): SoA [31][nd]; xvf (may be NULL) receives the
 // same values rounded to FP32 for the mixed-precision polynomial
-__global__ void k_setup2(const int* __restrict__ ncnt, int ncap, const double* __restrict__ clus, double* __restrict__ xv, float* __restrict__ xvf)
+__device__ __forceinline__ void setup2(int d, int ncap, const double* __restrict__ clus, double* __restrict__ xv,
+                                       float* __restrict__ xvf)
 {
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nd = min(*ncnt, ncap);
-    if (d >= nd) return;
     double w[18], s[30], a1[3], a2[3], b1[3], b2[3];
 #pragma unroll
     for (int k = 0; k < 18; ++k) w[k] = clus[(long)k * ncap + d];
@@ -484,9 +471,9 @@ __global__ void k_setup2(const int* __restrict__ ncnt, int ncap, const double* _
         const V2Def v = c2_vars[n];
         const double dx = s[3 * v.s1] - s[3 * v.s2], dy = s[3 * v.s1 + 1] - s[3 * v.s2 + 1],
                      dz = s[3 * v.s1 + 2] - s[3 * v.s2 + 2];
-        const double r = sqrt(dx * dx + dy * dy + dz * dz);
-        const double e = exp(c2_k[v.k] * ((double)v.d0 - r));
-        const double val = v.kind ? e * (1.0 / r) : e;
+        const double r2 = dx * dx + dy * dy + dz * dz, rinv = rsqrt(r2);
+        const double e = exp(c2_k[v.k] * ((double)v.d0 - r2 * rinv));
+        const double val = v.kind ? e * rinv : e;
         xv[(long)n * ncap + d] = val;
         if (xvf) xvf[(long)n * ncap + d] = (float)val;
     }
@@ -511,7 +498,7 @@ __device__ __forceinline__ void cluster_virial(const double* w, const double* g,
     }
 }
 
-// Sum the slice partials, apply the chain rule through the variables and extra points and
+// From the polynomial and its gradients (slice sums), apply the chain rule through the variables and extra points and
 // the switch (mbpol-2b-poly.cpp:447-682).  Record: E (kcal/mol) and dE/dx of the 6 atoms;
 // block partials of energy, virial and stress.
 // sum of the raw (un-imaged) positions of the atoms of the NMON waters ids[0..NMON)
@@ -533,16 +520,14 @@ __device__ __forceinline__ void cluster_raw_sum(const int* ids, const int* __res
     }
 }
 
-__global__ __launch_bounds__(128) void k_finish2(const int* __restrict__ ncnt, int ncap, int nsl, const double* __restrict__ clus,
-                                                 const double* __restrict__ xv, const double* __restrict__ part,
-                                                 double* __restrict__ erec, double* __restrict__ grec,
-                                                 double* __restrict__ blk, const int* __restrict__ dimers,
-                                                 const int* __restrict__ wbase, const double* __restrict__ x,
-                                                 const double* __restrict__ y, const double* __restrict__ z,
-                                                 double* __restrict__ srec)
+__device__ __forceinline__ void finish2(int d, int ncnt, int ncap, const double* __restrict__ clus,
+                                        const double* __restrict__ xv, const double* __restrict__ part,
+                                        double* __restrict__ erec, double* __restrict__ grec, double* __restrict__ blk,
+                                        const int* __restrict__ dimers, const int* __restrict__ wbase,
+                                        const double* __restrict__ x, const double* __restrict__ y,
+                                        const double* __restrict__ z, double* __restrict__ srec)
 {
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nd = min(*ncnt, ncap);
+    const int nd = min(ncnt, ncap);
     double red[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (d < nd && dimers) {
         double S[3];
@@ -564,28 +549,20 @@ __global__ __launch_bounds__(128) void k_finish2(const int* __restrict__ ncnt, i
             for (int k = 0; k < 18; ++k) gout[k] = 0.0;
         } else {
             dimer_sites(w, s, a1, a2, b1, b2);
-            double E = 0.0;
-            for (int q = 0; q < nsl; ++q) E += part[((long)q * 32) * ncap + d];
+            const double E = part[d];
             double xg[30];
 #pragma unroll
             for (int k = 0; k < 30; ++k) xg[k] = 0.0;
 #pragma unroll
             for (int n = 0; n < 31; ++n) {
-                double gn = 0.0;
-                for (int q = 0; q < nsl; ++q) gn += part[((long)q * 32 + 1 + n) * ncap + d];
+                const double gn = part[(long)(1 + n) * ncap + d];
                 const V2Def v = c2_vars[n];
                 const double dd[3] = {s[3 * v.s1] - s[3 * v.s2], s[3 * v.s1 + 1] - s[3 * v.s2 + 1],
                                       s[3 * v.s1 + 2] - s[3 * v.s2 + 2]};
-                const double r = sqrt(dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2]);
+                const double rinv = rsqrt(dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2]);
                 const double val = xv[(long)n * ncap + d];
                 const double k = c2_k[v.k];
-                double gg;
-                if (v.kind) {
-                    const double rinv = 1.0 / r;
-                    gg = -(k + rinv) * val * rinv;
-                } else {
-                    gg = -k * val / r;
-                }
+                const double gg = v.kind ? -(k + rinv) * val * rinv : -k * val * rinv;
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
                     const double t = gn * (dd[i] * gg);
@@ -617,12 +594,10 @@ __global__ __launch_bounds__(128) void k_finish2(const int* __restrict__ ncnt, i
     block_reduce_store(red, 8, blk + 8 * blockIdx.x);
 }
 
-// 3B variables (mbpol-3b-poly.cpp:170-206): SoA [36][nt]; xvf as in k_setup2
-__global__ void k_setup3(const int* __restrict__ ncnt, int ncap, const double* __restrict__ clus, double* __restrict__ xv, float* __restrict__ xvf)
+// 3B variables (mbpol-3b-poly.cpp:170-206): SoA [36][nt]; xvf as in setup2
+__device__ __forceinline__ void setup3(int t, int ncap, const double* __restrict__ clus, double* __restrict__ xv,
+                                       float* __restrict__ xvf)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nt = min(*ncnt, ncap);
-    if (t >= nt) return;
     double w[27];
 #pragma unroll
     for (int k = 0; k < 27; ++k) w[k] = clus[(long)k * ncap + t];
@@ -639,17 +614,15 @@ __global__ void k_setup3(const int* __restrict__ ncnt, int ncap, const double* _
 }
 
 // mbpol-3b-poly.cpp:208-312: switch s = sab*sac + sab*sbc + sac*sbc, chain rule, switch
-// gradients.  Record: E (kcal/mol) and dE/dx of the 9 atoms; block partials as k_finish2.
-__global__ __launch_bounds__(128) void k_finish3(const int* __restrict__ ncnt, int ncap, int nsl, const double* __restrict__ clus,
-                                                 const double* __restrict__ xv, const double* __restrict__ part,
-                                                 double* __restrict__ erec, double* __restrict__ grec,
-                                                 double* __restrict__ blk, const int* __restrict__ trimers,
-                                                 const int* __restrict__ wbase, const double* __restrict__ x,
-                                                 const double* __restrict__ y, const double* __restrict__ z,
-                                                 double* __restrict__ srec)
+// gradients.  Record: E (kcal/mol) and dE/dx of the 9 atoms; block partials as finish2.
+__device__ __forceinline__ void finish3(int t, int ncnt, int ncap, const double* __restrict__ clus,
+                                        const double* __restrict__ xv, const double* __restrict__ part,
+                                        double* __restrict__ erec, double* __restrict__ grec, double* __restrict__ blk,
+                                        const int* __restrict__ trimers, const int* __restrict__ wbase,
+                                        const double* __restrict__ x, const double* __restrict__ y,
+                                        const double* __restrict__ z, double* __restrict__ srec)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nt = min(*ncnt, ncap);
+    const int nt = min(ncnt, ncap);
     double red[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (t < nt && trimers) {
         double S[3];
@@ -662,8 +635,7 @@ __global__ __launch_bounds__(128) void k_finish3(const int* __restrict__ ncnt, i
         double w[27];
 #pragma unroll
         for (int k = 0; k < 27; ++k) w[k] = clus[(long)k * ncap + t];
-        double E = 0.0;
-        for (int q = 0; q < nsl; ++q) E += part[((long)q * 37) * ncap + t];
+        const double E = part[t];
         double rab[3], rac[3], rbc[3];
 #pragma unroll
         for (int n = 0; n < 3; ++n) {
@@ -684,15 +656,13 @@ __global__ __launch_bounds__(128) void k_finish3(const int* __restrict__ ncnt, i
         for (int k = 0; k < 27; ++k) gc[k] = 0.0;
 #pragma unroll
         for (int n = 0; n < 36; ++n) {
-            double gn = 0.0;
-            for (int q = 0; q < nsl; ++q) gn += part[((long)q * 37 + 1 + n) * ncap + t];
-            gn *= sw;
+            const double gn = sw * part[(long)(1 + n) * ncap + t];
             const V3Def v = c3_vars[n];
             const double dx[3] = {w[3 * v.a1] - w[3 * v.a2], w[3 * v.a1 + 1] - w[3 * v.a2 + 1],
                                   w[3 * v.a1 + 2] - w[3 * v.a2 + 2]};
-            const double dd = sqrt(dx[0] * dx[0] + dx[1] * dx[1] + dx[2] * dx[2]);
+            const double rinv = rsqrt(dx[0] * dx[0] + dx[1] * dx[1] + dx[2] * dx[2]);
             const double k = c3_k[v.cls];
-            const double gg = -k * gn * xv[(long)n * ncap + t] / dd;
+            const double gg = -k * gn * xv[(long)n * ncap + t] * rinv;
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
                 gc[3 * v.a1 + i] += gg * dx[i];
@@ -716,6 +686,70 @@ __global__ __launch_bounds__(128) void k_finish3(const int* __restrict__ ncnt, i
         cluster_virial<27>(w, gc, red);
     }
     block_reduce_store(red, 8, blk + 8 * blockIdx.x);
+}
+
+// Both cluster pipelines in one launch per step: blocks [0, nb2) take dimers, the others trimers
+// (neither needs the other, and apart each step was two launches of a few microseconds' work).
+// A cluster's sites, re-imaged from the lists (`gather`), and its polynomial variables.
+__global__ __launch_bounds__(128) void k_clusters(int nb2, const int* __restrict__ counts, int cap2, int cap3, int gather,
+                                                  const int* __restrict__ dimers, const int* __restrict__ trimers,
+                                                  const double* __restrict__ mon, CellGeom g, double* __restrict__ clus2,
+                                                  double* __restrict__ xv2, float* __restrict__ xv2f,
+                                                  double* __restrict__ clus3, double* __restrict__ xv3,
+                                                  float* __restrict__ xv3f)
+{
+    if ((int)blockIdx.x < nb2) {
+        const int d = blockIdx.x * 128 + threadIdx.x;
+        if (d >= min(counts[0], cap2)) return;
+        if (gather) gather2(d, cap2, dimers, mon, g, clus2);
+        setup2(d, cap2, clus2, xv2, xv2f);
+    } else {
+        const int t = (blockIdx.x - nb2) * 128 + threadIdx.x;
+        if (t >= min(counts[1], cap3)) return;
+        if (gather) gather3(t, cap3, trimers, mon, g, clus3);
+        setup3(t, cap3, clus3, xv3, xv3f);
+    }
+}
+
+// The polynomials' slice partials of every (variable, cluster) added in FP64 and slice order into
+// slice 0 of part (from the FP32 ones pf where the polynomial ran in FP32); clusters at or past the
+// count skipped.  n2 = 32 cap2 and n3 = 37 cap3 elements.
+__device__ __forceinline__ void slice_sum(long i, long n, int nsl, const float* __restrict__ pf, double* __restrict__ part)
+{
+    double s = pf ? (double)pf[i] : part[i];
+    if (pf)
+        for (int q = 1; q < nsl; ++q) s += (double)pf[q * n + i];
+    else
+        for (int q = 1; q < nsl; ++q) s += part[q * n + i];
+    part[i] = s;
+}
+__global__ __launch_bounds__(256) void k_slice_sums(int nb2, const int* __restrict__ counts, int cap2, int cap3, int nsl2,
+                                                    int nsl3, const float* __restrict__ pf2, double* __restrict__ part2,
+                                                    const float* __restrict__ pf3, double* __restrict__ part3)
+{
+    if ((int)blockIdx.x < nb2) {
+        const long n = 32L * cap2, i = blockIdx.x * 256L + threadIdx.x;
+        if (i < n && i % cap2 < counts[0]) slice_sum(i, n, nsl2, pf2, part2);
+    } else {
+        const long n = 37L * cap3, i = (blockIdx.x - nb2) * 256L + threadIdx.x;
+        if (i < n && i % cap3 < counts[1]) slice_sum(i, n, nsl3, pf3, part3);
+    }
+}
+
+struct FinishArgs {
+    const double *clus2, *xv2, *part2, *clus3, *xv3, *part3, *x, *y, *z;
+    double *e2, *g2, *s2, *e3, *g3, *s3, *blk;
+    const int *dimers, *trimers, *wbase, *counts;
+    int cap2, cap3;
+};
+__global__ __launch_bounds__(128) void k_finish(int nb2, FinishArgs A)
+{
+    if ((int)blockIdx.x < nb2)
+        finish2(blockIdx.x * 128 + threadIdx.x, A.counts[0], A.cap2, A.clus2, A.xv2, A.part2, A.e2, A.g2, A.blk, A.dimers,
+                A.wbase, A.x, A.y, A.z, A.s2);
+    else
+        finish3((blockIdx.x - nb2) * 128 + threadIdx.x, A.counts[1], A.cap3, A.clus3, A.xv3, A.part3, A.e3, A.g3, A.blk,
+                A.trimers, A.wbase, A.x, A.y, A.z, A.s3);
 }
 
 // position of value v in the ascending list L[0..n) (v is known to be present)
@@ -755,6 +789,30 @@ struct GatherArgs {
     const double *e2, *g2, *s2, *e3, *g3, *s3, *x, *y, *z;
     double *fx, *fy, *fz, *fout, *ae, *hw;
 };
+
+// Sums over the wavefront of N values per lane into out[0..N): at each step a lane keeps half of its
+// values and passes the others on (first, cnt: the place and number of those it holds).
+template <int N, int O>
+__device__ __forceinline__ void fold_sums(const long long (&v)[N], int lane, int first, int cnt, long long* out)
+{
+    constexpr int H = (N + 1) / 2;
+    const bool up = lane & O;
+    long long r[H];
+#pragma unroll
+    for (int q = 0; q < H; ++q) {
+        const long long hi = q + H < N ? v[q + H < N ? q + H : 0] : 0;
+        r[q] = (up ? hi : v[q]) + __shfl_xor(up ? v[q] : hi, O, 64);
+    }
+    first += up ? H : 0;
+    cnt = up ? max(cnt - H, 0) : min(cnt, H);
+    if constexpr (O > 1) {
+        fold_sums<H, O / 2>(r, lane, first, cnt, out);
+    } else {
+#pragma unroll
+        for (int q = 0; q < H; ++q)
+            if (q < cnt) out[first + q] = r[q];
+    }
+}
 
 #define GATHER_THREADS 256
 #define GATHER_MAXLEAF 4096   // >= 64 centres x 63 pairs: cannot overflow with 64-entry short lists
@@ -853,19 +911,16 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_water(GatherArgs A)
                 for (int q = 0; q < 3; ++q) acc(10 + 9 * a + 3 * pp + q, fa[pp] * rr[q]);
         }
     }
-    // exact combination: wavefront shuffles, then the wavefronts through LDS
+    // exact combination: exchanges that halve the sums a lane carries (76 instead of 444 for 74
+    // butterflies), then the wavefronts through LDS
     const int lane = tid & 63, wid = tid >> 6;
+    long long v[74];
 #pragma unroll
     for (int k = 0; k < 37; ++k) {
-        for (int off = 32; off > 0; off >>= 1) {
-            hi[k] += __shfl_down(hi[k], off, 64);
-            lo[k] += __shfl_down(lo[k], off, 64);
-        }
-        if (lane == 0) {
-            red[wid][k] = hi[k];
-            red[wid][37 + k] = lo[k];
-        }
+        v[k] = hi[k];
+        v[37 + k] = lo[k];
     }
+    fold_sums<74, 32>(v, lane, 0, 74, red[wid]);
     __syncthreads();
     if (tid < 37) {
         long long h = 0, l = 0;
@@ -887,55 +942,17 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_water(GatherArgs A)
     }
 }
 
-// Sum the nsl slice partials of every (variable, cluster) into slice 0, in slice order:
-// n = rows x ncap elements, clusters at or past the count skipped.
-__global__ void k_slice_sum(long n, int nsl, const int* __restrict__ ncnt, int ncap, double* __restrict__ part)
-{
-    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i >= n || i % ncap >= *ncnt) return;
-    double s = part[i];
-    for (int q = 1; q < nsl; ++q) s += part[q * n + i];
-    part[i] = s;
-}
-
-// FP64 sum of the nsl FP32 slice partials of every (variable, cluster), in slice order.
-__global__ void k_slice_sum_f(long n, int nsl, const int* __restrict__ ncnt, int ncap, const float* __restrict__ pf,
-                              double* __restrict__ part)
-{
-    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i >= n || i % ncap >= *ncnt) return;
-    double s = (double)pf[i];
-    for (int q = 1; q < nsl; ++q) s += (double)pf[q * n + i];
-    part[i] = s;
-}
-
-// Zero the per-atom outputs of the sites that are not water atoms (M sites).
-__global__ void k_zero_other_sites(int natms, const unsigned char* __restrict__ is_water, double* __restrict__ fout,
-                                   double* __restrict__ ae, double* __restrict__ hw)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= natms || is_water[i]) return;
-    fout[3 * i] = fout[3 * i + 1] = fout[3 * i + 2] = 0.0;
-    ae[i] = 0.0;
-    for (int k = 0; k < 9; ++k) hw[9L * i + k] = 0.0;
-}
-
-__global__ void k_mark_water(int nw, const int* __restrict__ wbase, unsigned char* __restrict__ is_water)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= nw) return;
-    const int o = wbase[w];
-    is_water[o] = is_water[o + 1] = is_water[o + 2] = 1;
-}
-
-// Fixed-order sum of nb block partials (8 values each): one wavefront per value.
-__global__ __launch_bounds__(512) void k_reduce_blocks(const double* __restrict__ blk, int nb, double* __restrict__ out)
+// Fixed-order sums of block partials (8 values each), one wavefront per value: block 0 the first nb0
+// into out[0..7], block 1 the next nb1 into out[8..15].
+__global__ __launch_bounds__(512) void k_reduce_blocks(const double* __restrict__ blk, int nb0, int nb1,
+                                                       double* __restrict__ out)
 {
     const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int first = blockIdx.x ? nb0 : 0, nb = blockIdx.x ? nb1 : nb0;
     double s = 0.0;
-    for (int b = lane; b < nb; b += 64) s += blk[8L * b + q];
+    for (int b = lane; b < nb; b += 64) s += blk[8L * (first + b) + q];
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-    if (lane == 0) out[q] = s;
+    if (lane == 0) out[8 * blockIdx.x + q] = s;
 }
 
 // Heat flux (compute_heat_flux2, heatcurrent.f90:703-728) from per-atom quantities:
@@ -988,80 +1005,59 @@ int mb_launch_lists(MbBuffers& B, const CellGeom& g, hipStream_t s)
     }
     hipLaunchKernelGGL(k_neighbours, dim3(nw), dim3(64), 0, s, nw, B.mon, g, B.cells.V, B.cap2, B.nbr2, B.cnt2,
                        B.nbr2l, B.cnt2l, B.cap3, B.nbr3, B.cnt3, B.counts + 2);
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, B.cnt2, nw, B.off2, B.counts + 0);
-    hipLaunchKernelGGL(k_fill_dimers, dim3((nw + 127) / 128), dim3(128), 0, s, nw, B.cap2, B.nbr2, B.cnt2, B.off2,
-                       B.dimers, B.dcap);
     hipLaunchKernelGGL(k_trimers<false>, dim3(nw), dim3(64), 0, s, nw, B.mon, g, B.nbr3, B.cnt3, B.tcnt, B.toff,
-                       B.kmask, B.rowoff, B.trimers, B.tcap);
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, B.tcnt, nw, B.toff, B.counts + 1);
+                       B.kmask, B.rowoff, B.trimers, B.tcap, B.cap2, B.nbr2, B.cnt2, B.off2, B.dimers, B.dcap);
+    hipLaunchKernelGGL(k_scan, dim3(2), dim3(1024), 0, s, B.cnt2, B.tcnt, nw, B.off2, B.toff, B.counts);
     hipLaunchKernelGGL(k_trimers<true>, dim3(nw), dim3(64), 0, s, nw, B.mon, g, B.nbr3, B.cnt3, B.tcnt, B.toff,
-                       B.kmask, B.rowoff, B.trimers, B.tcap);
+                       B.kmask, B.rowoff, B.trimers, B.tcap, B.cap2, B.nbr2, B.cnt2, B.off2, B.dimers, B.dcap);
     return (int)hipGetLastError();
 }
 
-// Cluster pipeline of the dimers: ncnt (device) dimers of a buffer laid out with stride and
-// grid ncap, so that the launches do not depend on the count (a graph may hold them); block
-// partials of (energy, virial, stress) go to B.blk[0 .. 8*ceil(ncap/128)), zero for the
-// blocks past the count.
-int mb_launch_dimers(MbBuffers& B, const int* ncnt, int ncap, const CellGeom& g, bool gather, hipStream_t s)
+// Cluster pipelines of the dimers and trimers: B.counts (device) clusters of buffers laid out with
+// strides and grids cap2 and cap3 (0: none), so that the launches do not depend on the counts (a
+// graph may hold them); block partials of (energy, virial, stress) go to B.blk, ceil(cap2/128)
+// blocks of the dimers' and then the trimers', zero for the blocks past a count.
+int mb_launch_clusters(MbBuffers& B, int cap2, int cap3, const CellGeom& g, bool gather, hipStream_t s)
 {
-    if (ncap <= 0) return 0;
-    const int nb = (ncap + 127) / 128;
-    if (gather) hipLaunchKernelGGL(k_gather2, dim3(nb), dim3(128), 0, s, ncnt, ncap, B.dimers, B.mon, g, B.clus2);
-    const long n = 32L * ncap;
-    if (B.mixed & 1) {
-        hipLaunchKernelGGL(k_setup2, dim3(nb), dim3(128), 0, s, ncnt, ncap, B.clus2, B.xv2, B.xv2f);
-        launch_pip2b_f32(B.xv2f, B.part2f, ncnt, ncap, B.cs2f, s);
-        hipLaunchKernelGGL(k_slice_sum_f, dim3((n + 255) / 256), dim3(256), 0, s, n, pip2b_nslices(), ncnt, ncap,
-                           B.part2f, B.part2);
-    } else {
-        hipLaunchKernelGGL(k_setup2, dim3(nb), dim3(128), 0, s, ncnt, ncap, B.clus2, B.xv2, nullptr);
-        launch_pip2b_f64(B.xv2, B.part2, ncnt, ncap, B.cs2, s);
-        hipLaunchKernelGGL(k_slice_sum, dim3((n + 255) / 256), dim3(256), 0, s, n, pip2b_nslices(), ncnt, ncap,
-                           B.part2);
-    }
-    hipLaunchKernelGGL(k_finish2, dim3(nb), dim3(128), 0, s, ncnt, ncap, 1, B.clus2, B.xv2, B.part2, B.e2, B.g2,
-                       B.blk, gather ? B.dimers : nullptr, B.wbase, B.x, B.y, B.z, B.s2);
-    return (int)hipGetLastError();
-}
-
-// Same for trimers; block partials after blk_off blocks of the dimers'.
-int mb_launch_trimers(MbBuffers& B, const int* ncnt, int ncap, int blk_off, const CellGeom& g, bool gather,
-                      hipStream_t s)
-{
-    if (ncap <= 0) return 0;
-    const int nb = (ncap + 127) / 128;
-    if (gather) hipLaunchKernelGGL(k_gather3, dim3(nb), dim3(128), 0, s, ncnt, ncap, B.trimers, B.mon, g, B.clus3);
-    const long n = 37L * ncap;
-    if (B.mixed & 2) {
-        hipLaunchKernelGGL(k_setup3, dim3(nb), dim3(128), 0, s, ncnt, ncap, B.clus3, B.xv3, B.xv3f);
-        launch_pip3b_f32(B.xv3f, B.part3f, ncnt, ncap, B.cs3f, s);
-        hipLaunchKernelGGL(k_slice_sum_f, dim3((n + 255) / 256), dim3(256), 0, s, n, pip3b_nslices(), ncnt, ncap,
-                           B.part3f, B.part3);
-    } else {
-        hipLaunchKernelGGL(k_setup3, dim3(nb), dim3(128), 0, s, ncnt, ncap, B.clus3, B.xv3, nullptr);
-        launch_pip3b_f64(B.xv3, B.part3, ncnt, ncap, B.cs3, s);
-        hipLaunchKernelGGL(k_slice_sum, dim3((n + 255) / 256), dim3(256), 0, s, n, pip3b_nslices(), ncnt, ncap,
-                           B.part3);
-    }
-    hipLaunchKernelGGL(k_finish3, dim3(nb), dim3(128), 0, s, ncnt, ncap, 1, B.clus3, B.xv3, B.part3, B.e3, B.g3,
-                       B.blk + 8L * blk_off, gather ? B.trimers : nullptr, B.wbase, B.x, B.y, B.z, B.s3);
+    if (cap2 <= 0 && cap3 <= 0) return 0;
+    const int nb2 = (cap2 + 127) / 128, nb3 = (cap3 + 127) / 128;
+    const bool f2 = B.mixed & 1, f3 = B.mixed & 2;
+    hipLaunchKernelGGL(k_clusters, dim3(nb2 + nb3), dim3(128), 0, s, nb2, B.counts, cap2, cap3, gather ? 1 : 0, B.dimers,
+                       B.trimers, B.mon, g, B.clus2, B.xv2, f2 ? B.xv2f : nullptr, B.clus3, B.xv3, f3 ? B.xv3f : nullptr);
+    if (!f2 || !f3)
+        launch_pip_f64(B.counts, B.xv2, B.part2, f2 ? 0 : cap2, B.cs2, B.xv3, B.part3, f3 ? 0 : cap3, B.cs3, s);
+    if (f2 || f3)
+        launch_pip_f32(B.counts, B.xv2f, B.part2f, f2 ? cap2 : 0, B.cs2f, B.xv3f, B.part3f, f3 ? cap3 : 0, B.cs3f, s);
+    const int ns2 = (int)((32L * cap2 + 255) / 256), ns3 = (int)((37L * cap3 + 255) / 256);
+    hipLaunchKernelGGL(k_slice_sums, dim3(ns2 + ns3), dim3(256), 0, s, ns2, B.counts, cap2, cap3, pip2b_nslices(),
+                       pip3b_nslices(), f2 ? B.part2f : nullptr, B.part2, f3 ? B.part3f : nullptr, B.part3);
+    FinishArgs A;
+    A.clus2 = B.clus2; A.xv2 = B.xv2; A.part2 = B.part2; A.clus3 = B.clus3; A.xv3 = B.xv3; A.part3 = B.part3;
+    A.x = B.x; A.y = B.y; A.z = B.z;
+    A.e2 = B.e2; A.g2 = B.g2; A.s2 = B.s2; A.e3 = B.e3; A.g3 = B.g3; A.s3 = B.s3; A.blk = B.blk;
+    A.dimers = gather ? B.dimers : nullptr;
+    A.trimers = gather ? B.trimers : nullptr;
+    A.wbase = B.wbase; A.counts = B.counts; A.cap2 = cap2; A.cap3 = cap3;
+    hipLaunchKernelGGL(k_finish, dim3(nb2 + nb3), dim3(128), 0, s, nb2, A);
     return (int)hipGetLastError();
 }
 
 // Per-water gather of the cluster records (the lists' dimers and trimers, strides dcap and
 // tcap) into per-atom forces, energies and heat-flux tensors; scal[0..7] = 2B (energy,
 // virial, stress 6), scal[8..15] = 3B.
-int mb_launch_accumulate(MbBuffers& B, double* fx, double* fy, double* fz, hipStream_t s)
+int mb_launch_accumulate(MbBuffers& B, double* fx, double* fy, double* fz, bool clear_f, hipStream_t s)
 {
     const int na = B.natms, nw = B.nw;
     const int nb2 = (int)((B.dcap + 127) / 128), nb3 = (int)((B.tcap + 127) / 128);
     if (nb2 + nb3 > B.nblk_cap) return -1;
-    hipLaunchKernelGGL(k_zero_i, dim3((na + 1023) / 1024), dim3(256), 0, s, reinterpret_cast<int*>(B.is_water),
-                       (na + 3) / 4);
-    hipLaunchKernelGGL(k_mark_water, dim3((nw + 255) / 256), dim3(256), 0, s, nw, B.wbase, B.is_water);
-    hipLaunchKernelGGL(k_zero_other_sites, dim3((na + 255) / 256), dim3(256), 0, s, na, B.is_water, B.fout,
-                       B.atomic_energy, B.heat_w);
+    {
+        // the per-atom outputs (the gather writes the water atoms', M sites keep 0); with clear_f
+        // also the caller's forces
+        double* d[6] = {B.fout, B.atomic_energy, B.heat_w, fx, fy, fz};
+        const double* sr[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+        const long len[6] = {3L * na, na, 9L * na, na, na, na};
+        el_launch_copy_segs(fx && clear_f ? 6 : 3, d, sr, len, s);
+    }
     GatherArgs A;
     A.nw = nw; A.nd = (int)B.dcap; A.nt = (int)B.tcap; A.cap2 = B.cap2;
     A.wbase = B.wbase; A.dimers = B.dimers; A.trimers = B.trimers;
@@ -1071,9 +1067,7 @@ int mb_launch_accumulate(MbBuffers& B, double* fx, double* fy, double* fz, hipSt
     A.x = B.x; A.y = B.y; A.z = B.z;
     A.fx = fx; A.fy = fy; A.fz = fz; A.fout = B.fout; A.ae = B.atomic_energy; A.hw = B.heat_w;
     hipLaunchKernelGGL(k_gather_water, dim3(nw), dim3(GATHER_THREADS), 0, s, A);
-    hipLaunchKernelGGL(k_zero_i, dim3(1), dim3(64), 0, s, reinterpret_cast<int*>(B.scal), 32);
-    if (nb2) hipLaunchKernelGGL(k_reduce_blocks, dim3(1), dim3(512), 0, s, B.blk, nb2, B.scal);
-    if (nb3) hipLaunchKernelGGL(k_reduce_blocks, dim3(1), dim3(512), 0, s, B.blk + 8L * nb2, nb3, B.scal + 8);
+    hipLaunchKernelGGL(k_reduce_blocks, dim3(2), dim3(512), 0, s, B.blk, nb2, nb3, B.scal);
     return (int)hipGetLastError();
 }
 
@@ -1085,6 +1079,6 @@ int mb_launch_heat_flux(int nreal, const double* vx, const double* vy, const dou
     if (nb > nblk_cap) return -1;
     hipLaunchKernelGGL(k_heat_flux, dim3(nb), dim3(256), 0, s, nreal, vx, vy, vz, ekin, epot, epot2, w, w2, sew,
                        blk);
-    hipLaunchKernelGGL(k_reduce_blocks, dim3(1), dim3(512), 0, s, blk, nb, out);
+    hipLaunchKernelGGL(k_reduce_blocks, dim3(1), dim3(512), 0, s, blk, nb, 0, out);
     return (int)hipGetLastError();
 }
