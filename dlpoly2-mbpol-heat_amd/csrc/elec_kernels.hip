@@ -97,12 +97,24 @@ __device__ double chunk_sum64(const double* __restrict__ in, long cs, int nc, lo
 // g = r.u and d = w.u (the Chronopoulos-Gear recurrence), and a power of two of about
 // 1 / max |m_i| for the particle mesh's spreading of m.  state = [iterations, rms step, done, g,
 // alpha, beta, -, d, -, m scale].  Returns true when the dipoles have converged.
-__device__ bool cg_step(const ElecDev& P, int it, int nb, const double* __restrict__ blk, double* __restrict__ state,
-                        bool record)
+// In two parts, so that a kernel can issue its other loads between: cg_load starts the loads of the
+// first 64 blocks' partials, cg_finish adds the others and decides.
+struct CgSums {
+    double a, b, c, d, e;
+};
+__device__ __forceinline__ CgSums cg_load(int nb, const double* __restrict__ blk)
 {
     const int lane = threadIdx.x & 63;
-    double a = 0.0, b = 0.0, c = 0.0, d = 0.0, e = 0.0;
-    for (int k = lane; k < nb; k += 64) {
+    CgSums s = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if (lane < nb) s = {blk[5 * lane], blk[5 * lane + 1], blk[5 * lane + 2], blk[5 * lane + 3], blk[5 * lane + 4]};
+    return s;
+}
+__device__ __forceinline__ bool cg_finish(const ElecDev& P, const CgSums& s0, int it, int nb,
+                                          const double* __restrict__ blk, double* __restrict__ state, bool record)
+{
+    const int lane = threadIdx.x & 63;
+    double a = s0.a, b = s0.b, c = s0.c, d = s0.d, e = s0.e;
+    for (int k = lane + 64; k < nb; k += 64) {
         a += blk[5 * k];
         b += blk[5 * k + 1];
         c += blk[5 * k + 2];
@@ -131,6 +143,12 @@ __device__ bool cg_step(const ElecDev& P, int it, int nb, const double* __restri
         }
     }
     return done;
+}
+
+__device__ __forceinline__ bool cg_step(const ElecDev& P, int it, int nb, const double* __restrict__ blk,
+                                        double* __restrict__ state, bool record)
+{
+    return cg_finish(P, cg_load(nb, blk), it, nb, blk, state, record);
 }
 
 __device__ __forceinline__ int water_of(const ElecDev& P, int i) { return i < P.nreal ? i / 3 : i - P.nreal; }
@@ -825,27 +843,31 @@ __device__ __forceinline__ double row_ror8(double v)
 // zero past the last site); wavefront w takes the steps of four sites w, w + 8, ..., with the
 // next step's table entries loaded while the current one is multiplied, and the eight
 // wavefronts' sums are added in order through LDS.
-template <int NT>
-__device__ void rs_sfac_block(const ElecDev& P, const RsSrc src, int spc, int g, int t0, int chunk,
-                              const double2* __restrict__ pht, double* __restrict__ out, double* lds)
+// `go` (the solver's stopping test) is called by every thread once the first loads are under way;
+// nothing is written if it returns false.
+template <int NT, class Go>
+__device__ __forceinline__ void rs_sfac_block(const ElecDev& P, const RsSrc src, int spc, int g, int t0, int chunk,
+                                              const double2* __restrict__ pht, double* __restrict__ out, double* lds,
+                                              Go&& go)
 {
     const RsPlan& R = P.rs;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int j0 = chunk * spc, nj = min(spc, src.ns - j0), nstep = (nj + 3) / 4;
-    for (int i = tid; i < 4 * nstep; i += 64 * RS_WAVES) {
-        double4 w = make_double4(0.0, 0.0, 0.0, 0.0);
+    // (a chunk has at most two sites per thread)
+    static_assert(RS_MAX_SPC <= 2 * 64 * RS_WAVES, "");
+    double mv[2][3];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int i = tid + 64 * RS_WAVES * h;
+        const double* v = src.v + (long)(j0 + i) * src.stride;
+        mv[h][0] = mv[h][1] = mv[h][2] = 0.0;
         if (i < nj) {
-            const double* v = src.v + (long)(j0 + i) * src.stride;
+            mv[h][0] = v[0];
             if (src.dip) {
-                const double mx = TWOPI * v[0], my = TWOPI * v[1], mz = TWOPI * v[2];
-                w.x = R.rc[0] * mx + R.rc[3] * my + R.rc[6] * mz;
-                w.y = R.rc[1] * mx + R.rc[4] * my + R.rc[7] * mz;
-                w.z = R.rc[2] * mx + R.rc[5] * my + R.rc[8] * mz;
-            } else {
-                w.w = v[0];
+                mv[h][1] = v[1];
+                mv[h][2] = v[2];
             }
         }
-        reinterpret_cast<double4*>(lds)[i] = w;
     }
     const int4 pr = R.pair[16 * g + (lane & 15)];
     const int nt = max(0, min(NT, __builtin_amdgcn_readfirstlane(pr.w) - t0));
@@ -876,6 +898,22 @@ __device__ void rs_sfac_block(const ElecDev& P, const RsSrc src, int spc, int g,
         for (int t = 0; t < NT; ++t) z[t] = *reinterpret_cast<const double*>(base + (o + oz[t]));
     };
     if (wv < nstep) load(at);
+    if (!go()) return;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int i = tid + 64 * RS_WAVES * h;
+        if (i < 4 * nstep) {
+            double4 w = make_double4(0.0, 0.0, 0.0, mv[h][0]);
+            if (src.dip) {
+                const double mx = TWOPI * mv[h][0], my = TWOPI * mv[h][1], mz = TWOPI * mv[h][2];
+                w.x = R.rc[0] * mx + R.rc[3] * my + R.rc[6] * mz;
+                w.y = R.rc[1] * mx + R.rc[4] * my + R.rc[7] * mz;
+                w.z = R.rc[2] * mx + R.rc[5] * my + R.rc[8] * mz;
+                w.w = 0.0;
+            }
+            reinterpret_cast<double4*>(lds)[i] = w;
+        }
+    }
     __syncthreads();
     for (int st = wv; st < nstep; st += RS_WAVES) {
         const double4 w = reinterpret_cast<const double4*>(lds)[4 * st + sl];
@@ -960,14 +998,20 @@ __global__ __launch_bounds__(64 * RS_WAVES) void k_rs_sfac(ElecDev P, RsSrcs src
                                                            double* __restrict__ state,
                                                            const double* __restrict__ cgblk, int cgnb, int it)
 {
-    if (state[2] != 0.0) return;
-    if (cgblk && cg_step(P, it, cgnb, cgblk, state, blockIdx.x == 0 && threadIdx.x < 64)) return;
     extern __shared__ double lds[];
     const RsPlan& R = P.rs;
+    const double done = state[2];
+    CgSums cg = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if (cgblk) cg = cg_load(cgnb, cgblk);
+    auto go = [&]() {
+        if (done != 0.0) return false;
+        return !(cgblk && cg_finish(P, cg, it, cgnb, cgblk, state, blockIdx.x == 0 && threadIdx.x < 64));
+    };
     int b = blockIdx.x;
     if (b >= nsb) {
+        if (!go()) return;
         emu_row<1>(P, (b - nsb) * RS_WAVES + (threadIdx.x >> 6), threadIdx.x & 63, x, y, z, nbrP, cntP, tens, tin,
-                src.s[0].v, emu);
+                   src.s[0].v, emu);
         return;
     }
     // chunks fastest: with 8 chunks (one per XCD, see build_rs) the blocks of an XCD read the
@@ -980,7 +1024,7 @@ __global__ __launch_bounds__(64 * RS_WAVES) void k_rs_sfac(ElecDev P, RsSrcs src
     const int g = b % R.ng, set = b / R.ng;
     const long slot = RS_SLOT(R.ntiles);
     rs_sfac_block<NT>(P, src.s[set], spc, g, NT * tg, chunk, pht,
-                      Spart + (((long)set * nch + chunk) * R.ng + g) * slot, lds);
+                      Spart + (((long)set * nch + chunk) * R.ng + g) * slot, lds, go);
 }
 
 // S(l, m, +n) = v[0] + i v[1] and S(l, m, -n) = v[2] + i v[3] of pair p of a group, n > 0, added
@@ -1013,7 +1057,7 @@ __global__ __launch_bounds__(64 * RS_WAVES, 4) void k_rs_field(ElecDev P, int nc
                                                                double* __restrict__ Fpart,
                                                                const double* __restrict__ state)
 {
-    if (state[2] != 0.0) return;
+    const double done = state[2];
     __shared__ double W[4][2][8 * RS_NT][16];          // [H_C, H_S, n H_C, n H_S][cos, sin][n][pair]
     __shared__ double W0[2][16];                       // n = 0: [C, S]
     const RsPlan& R = P.rs;
@@ -1025,14 +1069,21 @@ __global__ __launch_bounds__(64 * RS_WAVES, 4) void k_rs_field(ElecDev P, int nc
     const int nn = 8 * R.ntiles + 1;
     const long slot = RS_SLOT(R.ntiles), cs = slot * R.ng;
     const double* base = Spart + ((long)set * nch * R.ng + g) * slot;
-    // the amplitudes of tiles [t0, t0 + ntt); every thread of the block takes part
+    // the amplitudes of tiles [t0, t0 + ntt); every thread of the block takes part (ntt <= RS_NT: one
+    // (pair, n) each)
+    static_assert(128 * RS_NT <= 64 * RS_WAVES, "");
+    // consecutive threads: n of the tile, then pairs, as the sums lie
+    const int ap = ((tid >> 3) & 3) + 4 * ((tid >> 5) & 3), an = 8 * (tid >> 7) + (tid & 7);
+    double v[4];
+    double2 ak;
+    auto sums = [&](int t0, int ntt) {
+        if (tid < 128 * ntt) {
+            rs_sums(base, cs, nch, ap, 8 * t0 + an + 1, v);
+            ak = R.ak[(long)(16 * g + ap) * nn + 8 * t0 + an + 1];
+        }
+    };
     auto amplitudes = [&](int t0, int ntt) {
-        for (int i = tid; i < 128 * ntt; i += 64 * RS_WAVES) {
-            // consecutive threads: n of the tile, then pairs, as the sums lie
-            const int p = ((i >> 3) & 3) + 4 * ((i >> 5) & 3), nl = 8 * (i >> 7) + (i & 7), n = 8 * t0 + nl + 1;
-            double v[4];
-            rs_sums(base, cs, nch, p, n, v);
-            const double2 a = R.ak[(long)(16 * g + p) * nn + n];
+        if (tid < 128 * ntt) {
             double uc = v[0], us = v[1], dc = v[2], ds = v[3];
             if (set) {
                 uc = v[1];
@@ -1040,21 +1091,22 @@ __global__ __launch_bounds__(64 * RS_WAVES, 4) void k_rs_field(ElecDev P, int nc
                 dc = v[3];
                 ds = -v[2];
             }
-            uc *= a.x;
-            us *= a.x;
-            dc *= a.y;
-            ds *= a.y;
-            const double fn = n;
-            W[0][0][nl][p] = uc + dc;
-            W[0][1][nl][p] = us - ds;
-            W[1][0][nl][p] = us + ds;
-            W[1][1][nl][p] = dc - uc;
-            W[2][0][nl][p] = fn * (uc - dc);
-            W[2][1][nl][p] = fn * (us + ds);
-            W[3][0][nl][p] = fn * (us - ds);
-            W[3][1][nl][p] = -fn * (uc + dc);
+            uc *= ak.x;
+            us *= ak.x;
+            dc *= ak.y;
+            ds *= ak.y;
+            const double fn = 8 * t0 + an + 1;
+            W[0][0][an][ap] = uc + dc;
+            W[0][1][an][ap] = us - ds;
+            W[1][0][an][ap] = us + ds;
+            W[1][1][an][ap] = dc - uc;
+            W[2][0][an][ap] = fn * (uc - dc);
+            W[2][1][an][ap] = fn * (us + ds);
+            W[3][0][an][ap] = fn * (us - ds);
+            W[3][1][an][ap] = -fn * (uc + dc);
         }
     };
+    if (!MORE) sums(0, nt);
     if (wv == RS_WAVES - 1 && lane < 16) {
         double c = 0.0, s = 0.0;
         const double* q = base + 512L * R.ntiles + lane;
@@ -1066,17 +1118,18 @@ __global__ __launch_bounds__(64 * RS_WAVES, 4) void k_rs_field(ElecDev P, int nc
         W0[0][lane] = a * (set ? s : c);
         W0[1][lane] = a * (set ? -c : s);
     }
-    if (!MORE) amplitudes(0, nt);
     double dl[4], dm[4];
     int ox[4], oy[4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int4 pr = R.pair[16 * g + quad + 4 * v];
-        dl[v] = pr.x;
-        dm[v] = pr.y;
-        ox[v] = pr.x;
-        oy[v] = R.ky + pr.y;
+    for (int q = 0; q < 4; ++q) {
+        const int4 pr = R.pair[16 * g + quad + 4 * q];
+        dl[q] = pr.x;
+        dm[q] = pr.y;
+        ox[q] = pr.x;
+        oy[q] = R.ky + pr.y;
     }
+    if (done != 0.0) return;
+    if (!MORE) amplitudes(0, nt);
     __syncthreads();
     for (int tl = 0; tl < tpw; ++tl) {
         const int jr = 16 * ((sb * tpw + tl) * RS_WAVES + wv) + row;
@@ -1100,6 +1153,7 @@ __global__ __launch_bounds__(64 * RS_WAVES, 4) void k_rs_field(ElecDev P, int nc
         for (int t0 = 0; t0 < nt; t0 += RS_NT) {
             const int ntt = min(RS_NT, nt - t0);
             if (MORE) {
+                sums(t0, ntt);
                 __syncthreads();
                 amplitudes(t0, ntt);
                 __syncthreads();
@@ -1352,7 +1406,7 @@ __global__ __launch_bounds__(256) void k_cg_update(ElecDev P, const double* __re
                                                    double* __restrict__ blk,
                                                    const double* __restrict__ state)
 {
-    if (state[2] != 0.0) return;
+    const double done = state[2];
     const double alpha = INIT ? 0.0 : state[4], beta = INIT ? 0.0 : state[5];
     const int tid = threadIdx.x;
     __shared__ double part[4][64];
@@ -1362,9 +1416,31 @@ __global__ __launch_bounds__(256) void k_cg_update(ElecDev P, const double* __re
     const int wl = lane / 9, i = lane - 9 * wl;
     const int w = blockIdx.x * CG_WPB + wl;
     const bool act = lane < 9 * CG_WPB && w < P.nw;
-    const int o = 9 * w + i, j = 3 * w + i / 3, c = i % 3;
+    const int o = act ? 9 * w + i : 0, j = 3 * w + i / 3, c = i % 3;
     const double p2 = act ? site_polr2(P, j) : 0.0;
     const bool on = act && p2 > P.toler;
+    // every load of the row is started before the first wait
+    double mm = 0.0, em = 0.0, r0 = 0.0, u0 = 0.0, w0 = 0.0, z0 = 0.0, q0 = 0.0, s0 = 0.0, p0 = 0.0, d0 = 0.0, t0 = 0.0;
+    double mi[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) mi[k] = 0.0;
+    if (wave == 0 && on) {
+        mm = m[o];
+        em = emu[o];
+        r0 = r[o];
+        u0 = u[o];
+        if (!INIT) {
+            w0 = wv[o];
+            z0 = z[o];
+            q0 = qv[o];
+            s0 = sv[o];
+            p0 = pv[o];
+            d0 = dip[o];
+            t0 = tmu[o];
+        }
+#pragma unroll
+        for (int k = 0; k < 9; ++k) mi[k] = minv[45L * w + tri9(i, k)];
+    }
     {
         // this wavefront's quarter of the field chunks
         double sum = 0.0;
@@ -1372,36 +1448,36 @@ __global__ __launch_bounds__(256) void k_cg_update(ElecDev P, const double* __re
             const int c0 = (P.fchunks * wave) / 4, c1 = (P.fchunks * (wave + 1)) / 4;
             const double* f = Fpart + (long)c * P.n + j;
             const long cs = 6L * P.n;
-#pragma unroll 4
+#pragma unroll 8
             for (int ch = c0; ch < c1; ++ch) sum += f[ch * cs];
         }
+        if (done != 0.0) return;
         part[wave][lane] = sum;
     }
     __syncthreads();
     double rr = 0.0, uu = 0.0, wn = 0.0;
     if (wave == 0 && on) {
         const double sum = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
-        const double mm = m[o];
-        const double nv = R4PIE0 * mm / p2 - (emu[o] + (p2 > 1.e-6 ? P.scale * sum : 0.0) + P.self_dd * mm);
+        const double nv = R4PIE0 * mm / p2 - (em + (p2 > 1.e-6 ? P.scale * sum : 0.0) + P.self_dd * mm);
         if (INIT) {
             wn = nv;
             wv[o] = wn;
-            rr = r[o];
-            uu = u[o];
+            rr = r0;
+            uu = u0;
         } else {
-            const double zz = nv + beta * z[o];
-            const double qq = mm + beta * qv[o];
-            const double ss = wv[o] + beta * sv[o];
-            const double pp = u[o] + beta * pv[o];
+            const double zz = nv + beta * z0;
+            const double qq = mm + beta * q0;
+            const double ss = w0 + beta * s0;
+            const double pp = u0 + beta * p0;
             z[o] = zz;
             qv[o] = qq;
             sv[o] = ss;
             pv[o] = pp;
-            dip[o] += alpha * pp;
-            tmu[o] += alpha * (R4PIE0 * pp / p2 - ss);
-            rr = r[o] - alpha * ss;
-            uu = u[o] - alpha * qq;
-            wn = wv[o] - alpha * zz;
+            dip[o] = d0 + alpha * pp;
+            tmu[o] = t0 + alpha * (R4PIE0 * pp / p2 - ss);
+            rr = r0 - alpha * ss;
+            uu = u0 - alpha * qq;
+            wn = w0 - alpha * zz;
             r[o] = rr;
             u[o] = uu;
             wv[o] = wn;
@@ -1411,9 +1487,8 @@ __global__ __launch_bounds__(256) void k_cg_update(ElecDev P, const double* __re
     __syncthreads();
     double mn = 0.0;
     if (wave == 0 && on) {
-        const double* mi = minv + 45L * w;
 #pragma unroll
-        for (int k = 0; k < 9; ++k) mn += mi[tri9(i, k)] * ws[9 * wl + k];
+        for (int k = 0; k < 9; ++k) mn += mi[k] * ws[9 * wl + k];
         m[o] = mn;
     }
     const double zs = p2 * rr / R4PIE0;
