@@ -326,7 +326,7 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
                 kv.insert(kv.end(), rec, rec + 8);
                 const int lmn[3] = {ll, mm, nn};
                 klm.insert(klm.end(), lmn, lmn + 3);
-                if (run_open < 0 || runs[4 * run_open + 3] == 8) {
+                if (run_open < 0 || runs[4 * run_open + 3] == EL_RUN) {
                     run_open = (int)runk.size();
                     const int r4[4] = {ll, mm, nn, 0};
                     runs.insert(runs.end(), r4, r4 + 4);
@@ -374,12 +374,6 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
         E.kchunks = std::max(E.kchunks, std::min(E.nrun, (E.nrun + EL_KCHUNK_RUNS - 1) / EL_KCHUNK_RUNS));
     E.rpc = (E.nrun + E.kchunks - 1) / E.kchunks;
     E.kchunks = (E.nrun + E.rpc - 1) / E.rpc;
-    E.kmaxch = 0;
-    for (int c = 0; c < E.kchunks; ++c) {
-        const int r0 = c * E.rpc, r1 = std::min(E.nrun, r0 + E.rpc);
-        const int k0 = runk[r0], k1 = r1 < E.nrun ? runk[r1] : K;
-        E.kmaxch = std::max(E.kmaxch, k1 - k0);
-    }
     if (build_rs(S, rc, kmax, kv, klm, err)) return -1;
     dfree(E.Fpart);
     ECHK(dalloc(&E.Fpart, std::max((size_t)E.kchunks * 16, (size_t)E.fchunks * 6) * E.n));
@@ -413,7 +407,7 @@ int alloc_direct(ElecState& S, std::string& err)
     ECHK(dalloc(&E.blk, (size_t)E.nblk));
     E.K = E.nrun = 0;
     E.kchunks = E.fchunks = 1;
-    E.rpc = E.kmaxch = 0;
+    E.rpc = 0;
     S.k_alpha = -1.0;   // a later periodic call builds its k list
     S.P.rvolm = 0.0;
     return 0;
@@ -538,7 +532,6 @@ int elec_configure(ElecState& S, int nw, const CellGeom& g, const double* cell, 
     P.kchunks = S.E.kchunks;
     P.kstride = S.E.kstride;
     P.rpc = S.E.rpc;
-    P.kmaxch = S.E.kmaxch;
     P.fchunks = S.E.fchunks;
     P.rs = S.E.rs;
     P.scale = 4.0 * P.rvolm * R4PIE0;

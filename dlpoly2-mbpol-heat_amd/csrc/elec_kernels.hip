@@ -1561,141 +1561,157 @@ __global__ __launch_bounds__(256) void k_el_kscal(ElecDev P, const double* __res
         for (int t = 0; t < 6; ++t)
             v[2 + t] = -virprs * kk[ia[t]] * kk[ib[t]] - 2.0 * akk * kk[ia[t]] * Ms[ib[t]] * summu1 +
                        2.0 * akk * kk[ia[t]] * Mc[ib[t]] * summu2;
+        // what the site pass multiplies with the phases of this k, akk taken in
         double* f = kf + 16 * k;
-        f[0] = Qc;
-        f[1] = Qs;
-        f[2] = summu1;
-        f[3] = summu2;
-        f[4] = skdmuckrs;
-        f[5] = skdmuskrs;
-        f[6] = skdmuckrs;   // dpkMc
-        f[7] = skdmuskrs;   // dpkMs
+        f[0] = akk * summu1;
+        f[1] = akk * summu2;
+        f[2] = akk * Qc;
+        f[3] = akk * Qs;
         for (int q = 0; q < 3; ++q) {
-            f[8 + q] = Mc[q];
-            f[11 + q] = Ms[q];
+            f[4 + q] = akk * Mc[q];
+            f[7 + q] = akk * Ms[q];
         }
+        f[10] = kv[8 * k + 5];   // akv2
     }
     block_sum_store(v, blk + 8 * blockIdx.x);
 }
 
-
-// Final reciprocal pass per site over a chunk of runs (ewald1p.f:550-693, 771-825):
-// forces, ESP parts vesp_k / vesp_dc_k, per-atom energy and per-atom stress (scaled by
-// akk, without the final prefactors).  The chunk's runs and per-k constants (k, akk,
-// akv2, Qc, Qs, summu, k.Mc, k.Ms, Mc, Ms) are staged in LDS.  Partials
-// Fpart[chunk][16][n]: f(3), vk, vdck, e, s(9).
-#define EL_KF 17
-__global__ __launch_bounds__(256) void k_el_kfinal(ElecDev P, const int* __restrict__ runs,
+// Final reciprocal pass per site over a chunk of runs (ewald1p.f:550-693, 771-825): forces, ESP
+// parts vesp_k / vesp_dc_k, per-atom energy and per-atom stress (without the final prefactors).
+// Partials Fpart[chunk][16][n]: f(3), vk, vdck, e, s(9).
+//
+// With S1 = Qc - k.Ms, S2 = Qs + k.Mc, km = k.mu and the phases c, s of site j, everything follows
+// from A = akk (c S1 + s S2) and B = akk (c S2 - s S1):
+//   force   -sum k (q B - km A),   vk + vdck = sum A,
+//   stress  akk [D_ab T - akv2 k_a k_b T + k_a X_b],  akk T = q A + km B,
+//   akk X_b = (s q + c km) akk Mc_b - (c q - s km) akk Ms_b + B mu_b.
+// Along a run k = k0 + t g (g = 2 pi c*, t = 0..7): the sums over t carry the moments t^0, t^1
+// (and t^2 of akv2 T) only, and are multiplied with k0 once per run and with g once per chunk.
+// That leaves 40 FP64 instructions per (k, site) instead of 66, and 6 reads of 16 bytes from LDS
+// per (k, wavefront) instead of 9, which had taken the LDS as long as the arithmetic took the
+// SIMDs: 512 waters 73.6 -> 50.1 us, 2048 waters 767 -> 479 us (430 us of arithmetic at four
+// cycles an instruction).  Slower: two sites per thread (284 registers, one wavefront to a SIMD:
+// 61 and 738 us), four wavefronts to a SIMD (spills: 107 and 1226 us), the factors by scalar loads
+// (their latency: 99 and 828 us).
+__global__ __launch_bounds__(256) void k_el_kfinal(ElecDev P, const int4* __restrict__ runs,
                                                    const int* __restrict__ runk, const double* __restrict__ phc,
                                                    const double* __restrict__ phs, const double* __restrict__ kv,
                                                    const double* __restrict__ kf, const double* __restrict__ chge,
                                                    const double* __restrict__ dip, double* __restrict__ Fpart)
 {
-    extern __shared__ double lds[];
-    const int tid = threadIdx.x;
-    const int j = blockIdx.x * 256 + tid;
+    const int j = blockIdx.x * 256 + threadIdx.x;
     const int chunk = blockIdx.y;
     const int r0 = chunk * P.rpc, r1 = min(P.nrun, r0 + P.rpc);
-    const int nr = max(0, r1 - r0);
-    double* sk = lds;
-    int* sr = reinterpret_cast<int*>(lds + (long)P.kmaxch * EL_KF);
-    const int kbase = nr ? runk[r0] : 0;
-    const int nk = nr ? ((r1 < P.nrun ? runk[r1] : P.K) - kbase) : 0;
-    for (int idx = tid; idx < nk * EL_KF; idx += 256) {
-        const int kk = idx / EL_KF, q = idx - kk * EL_KF;
-        const long k = kbase + kk;
-        double v;
-        if (q < 4) v = kv[8 * k + q];                 // kx ky kz akk
-        else if (q == 4) v = kv[8 * k + 5];           // akv2
-        else if (q < 11) v = kf[16 * k + (q - 5)];    // Qc Qs summu1 summu2 k.Mc k.Ms
-        else v = kf[16 * k + 8 + (q - 11)];           // Mc(3) Ms(3)
-        sk[idx] = v;
+    // the chunk's factors, 12 doubles a k
+    extern __shared__ double lds[];
+    double2* sk = (double2*)lds;
+    const int kb = runk[r0], nk = (r1 < P.nrun ? runk[r1] : P.K) - kb;
+    for (int e = threadIdx.x; e < 6 * nk; e += 256) {
+        const int kk = e / 6;
+        sk[e] = ((const double2*)kf)[8L * (kb + kk) + e - 6 * kk];
     }
-    for (int idx = tid; idx < nr * 4; idx += 256) sr[idx] = runs[4 * r0 + idx];
     __syncthreads();
     if (j >= P.n) return;
     const int ks = P.kstride;
     const bool pol = site_polr2(P, j) > 1.e-6;
     const double q = chge[j];
     const double mu[3] = {pol ? dip[3 * j] : 0.0, pol ? dip[3 * j + 1] : 0.0, pol ? dip[3 * j + 2] : 0.0};
-    // Per k, with km = k.mu, the stress term of ewald1p.f:771-825,
-    //   akk [B_ab (cc + cd + dd) + k_a X_b],  B_ab = delta_ab - akv2 k_a k_b,
-    //   X_b = (s q + c km) Mc_b - (c q - s km) Ms_b + (c (Qs + k.Mc) + s (k.Ms - Qc)) mu_b,
-    // is accumulated as delta_ab D - G_ab + Pm_ab + mu_b R_a with D = sum akk T, G_ab =
-    // sum akk akv2 T k_a k_b, Pm_ab = sum k_a akk (..) and R_a = sum akk (..) k_a
-    // (T = cc + cd + dd); the site energy sum akk q (c Qc + s Qs) is q times acc3.
-    double f3[3] = {0.0, 0.0, 0.0}, vk_ = 0.0, vd_ = 0.0, D = 0.0;
-    double G[6] = {0, 0, 0, 0, 0, 0}, Pm[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, R[3] = {0, 0, 0};
+    const double g[3] = {TWOPI * P.rs.rc[2], TWOPI * P.rs.rc[5], TWOPI * P.rs.rc[8]};
+    const double kg = mu[0] * g[0] + mu[1] * g[1] + mu[2] * g[2];
     const double c1 = phc[((long)2 * ks + 1) * P.n + j], s1 = phs[((long)2 * ks + 1) * P.n + j];
-    int kk = 0;
-    for (int r = 0; r < nr; ++r) {
-        const int l = sr[4 * r], m = sr[4 * r + 1], n0 = sr[4 * r + 2], cnt = sr[4 * r + 3];
+    double vk_ = 0.0, va_ = 0.0;
+    // sums with k0 (per run) and those left for g
+    double F[3] = {0, 0, 0}, R[3] = {0, 0, 0}, Y[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, U[6] = {0, 0, 0, 0, 0, 0};
+    double Fg = 0.0, Rg = 0.0, Yg[3] = {0, 0, 0}, Ug[3] = {0, 0, 0}, Ugg = 0.0;
+    for (int r = r0; r < r1; ++r) {
+        const int4 run = runs[r];
+        const int l = run.x, m = run.y, n0 = run.z, cnt = run.w;
+        const int k = runk[r];
+        const double kx = kv[8L * k], ky = kv[8L * k + 1], kz = kv[8L * k + 2];
         const int am = abs(m), an0 = abs(n0);
-        double ckr, skr;
+        double c, s;
         run_phase(phc[(long)l * P.n + j], phs[(long)l * P.n + j], phc[((long)ks + am) * P.n + j],
                   phs[((long)ks + am) * P.n + j], phc[((long)2 * ks + an0) * P.n + j],
-                  phs[((long)2 * ks + an0) * P.n + j], m, n0, ckr, skr);
-        for (int t = 0; t < cnt; ++t) {
-            const double* f = sk + EL_KF * (kk + t);
-            const double kx = f[0], ky = f[1], kz = f[2];
-            const double akk = f[3], akv2 = f[4];
-            const double Qc = f[5], Qs = f[6], summu1 = f[7], summu2 = f[8];
-            const double dpkMc = f[9], dpkMs = f[10];
-            const double km = mu[0] * kx + mu[1] * ky + mu[2] * kz;
-            const double ssmu = summu1 * (-skr * q - ckr * km) + summu2 * (-skr * km + ckr * q);
-            const double wf = akk * ssmu;
-            f3[0] -= kx * wf;
-            f3[1] -= ky * wf;
-            f3[2] -= kz * wf;
-            const double cq = ckr * Qc + skr * Qs;
-            vk_ += akk * cq;
-            vd_ += akk * (skr * dpkMc - ckr * dpkMs);
-            const double T = q * cq + q * (skr * dpkMc - ckr * dpkMs) + km * (ckr * Qs - skr * Qc) +
-                             km * (ckr * dpkMc + skr * dpkMs);
-            const double aT = akk * T;
-            D += aT;
-            const double u = aT * akv2;
-            const double ux = u * kx, uy = u * ky, uz = u * kz;
-            G[0] += ux * kx;
-            G[1] += ux * ky;
-            G[2] += ux * kz;
-            G[3] += uy * ky;
-            G[4] += uy * kz;
-            G[5] += uz * kz;
-            const double b1 = akk * (skr * q + ckr * km), b2 = akk * (ckr * q - skr * km);
-            const double Y0 = b1 * f[11] - b2 * f[14], Y1 = b1 * f[12] - b2 * f[15], Y2 = b1 * f[13] - b2 * f[16];
-            Pm[0] += kx * Y0;
-            Pm[1] += kx * Y1;
-            Pm[2] += kx * Y2;
-            Pm[3] += ky * Y0;
-            Pm[4] += ky * Y1;
-            Pm[5] += ky * Y2;
-            Pm[6] += kz * Y0;
-            Pm[7] += kz * Y1;
-            Pm[8] += kz * Y2;
-            const double a3 = akk * (ckr * (Qs + dpkMc) + skr * (dpkMs - Qc));
-            R[0] += a3 * kx;
-            R[1] += a3 * ky;
-            R[2] += a3 * kz;
-            const double cn = ckr * c1 - skr * s1;
-            skr = skr * c1 + ckr * s1;
-            ckr = cn;
+                  phs[((long)2 * ks + an0) * P.n + j], m, n0, c, s);
+        const double km0 = mu[0] * kx + mu[1] * ky + mu[2] * kz;
+        double f0 = 0.0, f1 = 0.0, b0 = 0.0, b1 = 0.0, u0 = 0.0, u1 = 0.0, u2 = 0.0;
+        double y0[3] = {0.0, 0.0, 0.0}, y1[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int t = 0; t < EL_RUN; ++t) {
+            if (t >= cnt) break;
+            const double2* fl = sk + 6 * (k - kb + t);
+            const double2 f01 = fl[0], f23 = fl[1], f45 = fl[2], f67 = fl[3], f89 = fl[4];
+            const double f[11] = {f01.x, f01.y, f23.x, f23.y, f45.x, f45.y, f67.x, f67.y, f89.x, f89.y, fl[5].x};
+            const double km = km0 + t * kg;
+            const double A = c * f[0] + s * f[1], B = c * f[1] - s * f[0];
+            const double w = q * B - km * A;
+            const double u = (q * A + km * B) * f[10];
+            const double a = s * q + c * km, b = c * q - s * km;
+            vk_ += c * f[2] + s * f[3];
+            va_ += A;
+            f0 += w;
+            f1 += t * w;
+            b0 += B;
+            b1 += t * B;
+            u0 += u;
+            u1 += t * u;
+            u2 += (t * t) * u;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const double y = a * f[4 + d] - b * f[7 + d];
+                y0[d] += y;
+                y1[d] += t * y;
+            }
+            const double cn = c * c1 - s * s1;
+            s = s * c1 + c * s1;
+            c = cn;
         }
-        kk += cnt;
+        F[0] += kx * f0;
+        F[1] += ky * f0;
+        F[2] += kz * f0;
+        Fg += f1;
+        R[0] += kx * b0;
+        R[1] += ky * b0;
+        R[2] += kz * b0;
+        Rg += b1;
+        const double ux = kx * u0, uy = ky * u0, uz = kz * u0;
+        U[0] += kx * ux;
+        U[1] += kx * uy;
+        U[2] += kx * uz;
+        U[3] += ky * uy;
+        U[4] += ky * uz;
+        U[5] += kz * uz;
+        Ug[0] += kx * u1;
+        Ug[1] += ky * u1;
+        Ug[2] += kz * u1;
+        Ugg += u2;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            Y[d] += kx * y0[d];
+            Y[3 + d] += ky * y0[d];
+            Y[6 + d] += kz * y0[d];
+            Yg[d] += y1[d];
+        }
     }
     double acc[15];
-    acc[0] = f3[0];
-    acc[1] = f3[1];
-    acc[2] = f3[2];
+    double D = q * va_;   // sum akk T
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        acc[a] = -(F[a] + g[a] * Fg);
+        R[a] += g[a] * Rg;
+        D += mu[a] * R[a];
+    }
     acc[3] = vk_;
-    acc[4] = vd_;
+    acc[4] = va_ - vk_;
     acc[5] = q * vk_;
     const int gi[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
-        for (int b = 0; b < 3; ++b)
-            acc[6 + 3 * a + b] = (a == b ? D : 0.0) - G[gi[a][b]] + Pm[3 * a + b] + mu[b] * R[a];
+        for (int b = 0; b < 3; ++b) {
+            const double G = U[gi[a][b]] + g[b] * Ug[a] + g[a] * Ug[b] + g[a] * g[b] * Ugg;
+            acc[6 + 3 * a + b] = (a == b ? D : 0.0) - G + (Y[3 * a + b] + g[a] * Yg[b]) + mu[b] * R[a];
+        }
     double* out = Fpart + (long)chunk * 16 * P.n;
 #pragma unroll
     for (int t = 0; t < 15; ++t) out[(long)t * P.n + j] = acc[t];
@@ -2188,7 +2204,6 @@ namespace {
 inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 // dynamic LDS of the reciprocal-space passes (bytes)
 inline size_t rs_lds(int spc) { return sizeof(double) * std::max(512L * RS_WAVES, 4L * spc); }
-inline size_t kfinal_lds(const ElecDev& P) { return sizeof(double) * ((size_t)P.kmaxch * EL_KF + 2 * (size_t)P.rpc + 2); }
 
 // The real-space field of dip: four wavefronts to a row where rows are long (a cluster's hold
 // every other polarizable site; 300 waters 8.7 -> 7.3 us, 701 waters 28.7 -> 23.4), one where a
@@ -2444,8 +2459,8 @@ int el_launch_final(ElecBuffers& E, const ElecDev& P, int distribute, double g34
         rs_launch_sfac(E, P, {{{E.dip, 3, 0, P.nrow}, {E.dip + 1, 3, 0, P.nrow}, {E.dip + 2, 3, 0, P.nrow}, {E.chge, 1, 0, P.n}}},
                        4, P.rs.nchq, P.rs.spcq, false, E.zero_state, nullptr, 0, 0, s);
         hipLaunchKernelGGL(k_el_kscal, dim3(nkb), dim3(256), 0, s, P, E.kv, E.Spart, E.kf, b_ks);
-        hipLaunchKernelGGL(k_el_kfinal, dim3(ceil_div(P.n, 256), P.kchunks), dim3(256), kfinal_lds(P), s, P, E.runs,
-                           E.runk, E.phc, E.phs, E.kv, E.kf, E.chge, E.dip, E.Fpart);
+        hipLaunchKernelGGL(k_el_kfinal, dim3(ceil_div(P.n, 256), P.kchunks), dim3(256),
+                           sizeof(double2) * 6 * EL_RUN * P.rpc, s, P, (const int4*)E.runs, E.runk, E.phc, E.phs, E.kv, E.kf, E.chge, E.dip, E.Fpart);
         hipLaunchKernelGGL(k_el_ksum, dim3(ceil_div(15L * P.n, 64)), dim3(256), 0, s, P, E.Fpart, E.ksum);
     }
     hipLaunchKernelGGL(k_el_pairs, dim3(P.n), dim3(64), 0, s, P, E.x, E.y, E.z, E.chge, E.dip, E.tab, E.nbrA, E.cntA,

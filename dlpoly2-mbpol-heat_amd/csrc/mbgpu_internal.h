@@ -140,6 +140,12 @@ struct RsPlan {
 #define RS_PAD 4                      // sites past the last that the passes may read
 #define RS_MAX_SPC 1024               // most sites of a chunk (their weights are staged in LDS)
 
+#define EL_RUN 8                      // most k of a run of the final site pass
+
+#define EL_RUN 8                      // most k of a run of the final site pass
+
+#define EL_RUN 8                      // most k of a run of the final site pass
+
 // Kernel-argument block of the polarizable electrostatics (passed by value).
 struct ElecDev {
     int nw, n, nreal, nrow;        // waters, sites (4nw), real atoms (3nw), rows carrying dipoles
@@ -154,7 +160,7 @@ struct ElecDev {
     int compat_qd;                 // qdforce M column as the reference (n_water + imol)
     int capA, capP;                // neighbour-row capacities (all partners / polarizable partners)
     int K, nrun, kchunks;          // k vectors, runs of consecutive n, k chunks of the final pass
-    int rpc, kmaxch;               // runs per k chunk, most k vectors in one chunk (final pass)
+    int rpc;                       // runs per k chunk (final pass)
     int fchunks;                   // partials of a field pass (k-sum: the groups of rs)
     int km[3], kstride;            // kmax per axis, phase-table stride (max kmax + 1)
     RsPlan rs;                     // k-sum: the (l, m) pairs and chunks of the matrix passes
@@ -164,7 +170,7 @@ struct ElecDev {
 // Device buffers of the electrostatics (owned by the context).
 struct ElecBuffers {
     int n = 0, capA = 0, capP = 0, K = 0, nrun = 0, kchunks = 0, ntab = 0, kstride = 0;
-    int rpc = 0, kmaxch = 0;                                   // k chunks of the final pass
+    int rpc = 0;                                               // runs per k chunk of the final pass
     int fchunks = 0;                                           // partials of a field pass
     RsPlan rs{};                                               // k-sum: plan of the matrix passes
     int4* rs_pair = nullptr;                                   // its arrays (see RsPlan)
