@@ -559,9 +559,8 @@ int enqueue_attempt(ElecState& S, const ElecSpme* sp, int solver, bool first, in
     }
     int rc = el_launch_setup(E, P, S.cells, solver == 1, sp == nullptr, s);
     if (!rc) rc = el_launch_prep(E, P, solver == 1, sp, s);
-    if (!rc && solver == 1) rc = el_launch_cg_init(E, P, sp, s);
-    for (int b = 0; !rc && b < nbatch; ++b)
-        rc = solver == 1 ? el_launch_cg_iteration(E, P, b, sp, s) : el_launch_iteration(E, P, b == 0, sp, s);
+    if (!rc && solver == 1) rc = el_launch_cg_start(E, P, nbatch, sp, s);
+    for (int b = 0; !rc && solver != 1 && b < nbatch; ++b) rc = el_launch_iteration(E, P, b == 0, sp, s);
     return rc;
 }
 

@@ -1503,13 +1503,182 @@ __global__ __launch_bounds__(256) void k_cg_update(ElecDev P, const double* __re
     if (tid == 0) blk[5 * blockIdx.x + 4] = fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]));
 }
 
-// The stopping test and scalars of iteration `it` alone (cg_step in one wavefront), for
-// paths whose first kernel of the iteration does not take them.
-__global__ __launch_bounds__(64) void k_cg_check(ElecDev P, int it, int nb, const double* __restrict__ blk,
-                                                 double* __restrict__ state)
+// The whole solve of a small system without reciprocal space in one launch by one block: the first
+// application of A (init: to u, as k_cg_update<INIT>), then iterations it0 .. it0 + count - 1 as
+// cg_step, emu_row and k_cg_update form them, until the dipoles have converged.  Everything an
+// iteration needs stays on the CU: 16 lanes keep the radial factors and separations of a row's
+// partners in registers (four each: the at most 61 partners of at most 63 rows), wavefront v the
+// vectors of the waters 7 v .. 7 v + 6, and m, its field and the partials pass through LDS, where a
+// barrier stands for a launch.  What a later launch continues from is written back.  Bound by
+// the latency of the shuffles and barriers of an iteration.
+// The solve of 9 waters, two launches to each of its about 17 iterations before: an evaluation
+// 265 -> 232 us (of which the two- and three-body terms beside it now take the longer part); of 21
+// waters 272 -> 236 us.  With rows passed in turn to 16 wavefronts that read the factors from
+// memory each time: 240 us at 9 waters, 283 (268 by single launches) at 16.
+#define CG_SOLVE_WATERS 21
+__global__ __launch_bounds__(1024) void k_cg_solve(ElecDev P, bool init, int it0, int count,
+                                                   const double* __restrict__ x, const double* __restrict__ y,
+                                                   const double* __restrict__ z, const int* __restrict__ nbrP,
+                                                   const int* __restrict__ cntP, const double2* __restrict__ tens,
+                                                   const double* __restrict__ tin, const double* __restrict__ minv,
+                                                   double* __restrict__ m, double* __restrict__ dip,
+                                                   double* __restrict__ r, double* __restrict__ u,
+                                                   double* __restrict__ wv, double* __restrict__ zv,
+                                                   double* __restrict__ qv, double* __restrict__ sv,
+                                                   double* __restrict__ pv, double* __restrict__ tmu,
+                                                   double* __restrict__ blk, double* __restrict__ state)
 {
+    constexpr int NWV = (CG_SOLVE_WATERS + CG_WPB - 1) / CG_WPB;   // wavefronts with vector rows
+    static_assert(16 * 3 * CG_SOLVE_WATERS <= 1024 && 3 * CG_SOLVE_WATERS - 3 <= 64, "");
+    __shared__ double lm[9 * CG_SOLVE_WATERS], le[9 * CG_SOLVE_WATERS], lw[NWV][64], lb[5 * NWV], st[16];
+    __shared__ double lt[36 * CG_SOLVE_WATERS];
     if (state[2] != 0.0) return;
-    (void)cg_step(P, it, nb, blk, state, true);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nb = (P.nw + CG_WPB - 1) / CG_WPB;
+    const int wl = lane / 9, i = lane - 9 * wl;
+    const int w = wave * CG_WPB + wl;
+    const bool act = wave < NWV && lane < 9 * CG_WPB && w < P.nw;
+    const int o = act ? 9 * w + i : 0, c = i % 3;
+    const double p2 = act ? site_polr2(P, 3 * w + i / 3) : 0.0;
+    const bool on = act && p2 > P.toler;
+    // the real-space row of these 16 lanes
+    const int row = tid >> 4, rl = tid & 15;
+    int pj[4];
+    double t1[4], t2[4], d[4][3];
+    {
+        const int np = row < P.nrow ? cntP[row] : 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int e = rl + 16 * k;
+            pj[k] = 0;
+            t1[k] = t2[k] = d[k][0] = d[k][1] = d[k][2] = 0.0;
+            if (e < np) {
+                const long q = (long)row * P.capP + e;
+                pj[k] = 3 * nbrP[q];
+                t1[k] = tens[q].x;
+                t2[k] = tens[q].y;
+                (void)sep(P, x, y, z, row, nbrP[q], d[k]);
+            }
+        }
+    }
+    // its two excluded partners of the same water, on lanes 0 and 1 (see emu_row)
+    int xj = -1, xt = 0;
+    if (row < P.nrow && rl < 2) {
+        const int rw = row / 3, si = row - 3 * rw, pt = rl < si ? rl : rl + 1;
+        const int a = min(si, pt), b = max(si, pt);
+        if (site_polr2(P, 3 * rw + pt) > 1.e-6) xj = 3 * (3 * rw + pt);
+        xt = 36 * rw + 6 * (a == 0 ? b - 1 : 3);
+    }
+    for (int e = tid; e < 36 * P.nw; e += 1024) lt[e] = tin[e];
+    double mm = 0.0, rr = 0.0, uu = 0.0, wn = 0.0, zz = 0.0, qq = 0.0, ss = 0.0, pp = 0.0, dd = 0.0, tt = 0.0;
+    double mi[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) mi[k] = 0.0;
+    if (act) {
+        mm = m[o];
+        lm[o] = mm;
+    }
+    if (on) {
+        rr = r[o];
+        uu = u[o];
+        zz = zv[o];
+        qq = qv[o];
+        ss = sv[o];
+        pp = pv[o];
+        dd = dip[o];
+        tt = tmu[o];
+        if (!init) wn = wv[o];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) mi[k] = minv[45L * w + tri9(i, k)];
+    }
+    if (tid < 16) st[tid] = state[tid];
+    if (!init && tid < 5 * nb) lb[tid] = blk[tid];
+    __syncthreads();
+    for (int it = init ? it0 - 1 : it0; it < it0 + count; ++it) {
+        const bool first = it < it0;
+        // (the wavefront that records is past its last use of st; the others read it after a barrier)
+        if (!first && cg_step(P, it, nb, lb, st, wave == 0)) break;
+        {
+            double e[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const double mx = lm[pj[k]], my = lm[pj[k] + 1], mz = lm[pj[k] + 2];
+                const double f = t2[k] * (d[k][0] * mx + d[k][1] * my + d[k][2] * mz);
+                e[0] += f * d[k][0] - t1[k] * mx;
+                e[1] += f * d[k][1] - t1[k] * my;
+                e[2] += f * d[k][2] - t1[k] * mz;
+            }
+            if (xj >= 0) {
+                const double* dt = lt + xt;
+                const double mx = lm[xj] * R4PIE0, my = lm[xj + 1] * R4PIE0, mz = lm[xj + 2] * R4PIE0;
+                e[0] += dt[0] * mx + dt[1] * my + dt[2] * mz;
+                e[1] += dt[1] * mx + dt[3] * my + dt[4] * mz;
+                e[2] += dt[2] * mx + dt[4] * my + dt[5] * mz;
+            }
+            for (int q = 0; q < 3; ++q)
+                for (int k = 8; k > 0; k >>= 1) e[q] += __shfl_xor(e[q], k, 16);
+            if (rl == 0 && row < P.nrow)
+                for (int q = 0; q < 3; ++q) le[3 * row + q] = e[q];
+        }
+        __syncthreads();
+        if (on) {
+            const double nv = R4PIE0 * mm / p2 - (le[o] + P.self_dd * mm);
+            if (first) {
+                wn = nv;
+            } else {
+                const double alpha = st[4], beta = st[5];
+                zz = nv + beta * zz;
+                qq = mm + beta * qq;
+                ss = wn + beta * ss;
+                pp = uu + beta * pp;
+                dd += alpha * pp;
+                tt += alpha * (R4PIE0 * pp / p2 - ss);
+                rr -= alpha * ss;
+                uu -= alpha * qq;
+                wn -= alpha * zz;
+            }
+        }
+        // the new w of a water's rows, which share a wavefront
+        if (wave < NWV) lw[wave][lane] = on ? wn : 0.0;
+        __syncthreads();
+        if (wave < nb) {
+            double mn = 0.0;
+            if (on) {
+#pragma unroll
+                for (int k = 0; k < 9; ++k) mn += mi[k] * lw[wave][9 * wl + k];
+                mm = mn;
+                lm[o] = mn;
+            }
+            const double zs = on ? p2 * rr / R4PIE0 : 0.0;
+            const double v0 = wsum(rr * uu), v1 = wsum(on ? wn * uu : 0.0), v2 = wsum(zs * zs),
+                         v3 = wsum(on && c == 0 ? 1.0 : 0.0);
+            double a = fabs(mn);
+            for (int o2 = 32; o2 > 0; o2 >>= 1) a = fmax(a, __shfl_xor(a, o2, 64));
+            if (lane == 0) {
+                lb[5 * wave] = v0;
+                lb[5 * wave + 1] = v1;
+                lb[5 * wave + 2] = v2;
+                lb[5 * wave + 3] = v3;
+                lb[5 * wave + 4] = a;
+            }
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    if (on) {
+        m[o] = mm;
+        r[o] = rr;
+        u[o] = uu;
+        wv[o] = wn;
+        zv[o] = zz;
+        qv[o] = qq;
+        sv[o] = ss;
+        pv[o] = pp;
+        dip[o] = dd;
+        tmu[o] = tt;
+    }
+    if (tid < 5 * nb) blk[tid] = lb[tid];
+    if (tid < 16) state[tid] = st[tid];
 }
 
 
@@ -2389,27 +2558,53 @@ static void el_cg_update(ElecBuffers& E, const ElecDev& P, const ElecSpme* sp, b
                            E.cg_r, E.cg_u, E.cg_w, E.cg_z, E.cg_q, E.cg_s, E.cg_p, E.cg_tmu, E.cgblk, E.state);
 }
 
-// conjugate-gradient start: residual of the start dipoles (their fields came with the
-// charge fields of the preparation), u = M^-1 r, and
-// the first application of A, to u, for w = A u
-int el_launch_cg_init(ElecBuffers& E, const ElecDev& P, const ElecSpme* sp, hipStream_t s)
+// The one-launch solve takes what its block holds: evaluations of 5 to 21 waters take 230 to 240 us
+// with it and 265 to 273 us with launches per iteration, which larger systems need for their width.
+static inline bool one_launch_solve(const ElecDev& P, const ElecSpme* sp)
 {
-    hipLaunchKernelGGL(k_cg_init, dim3(ceil_div(P.nw, CG_WPB)), dim3(256), 0, s, sp ? one_chunk(P) : P, E.Fpart, E.efk,
-                       E.efdc, E.emu, E.efdd, E.dip, E.cg_minv, E.cg_r, E.cg_u, E.cg_m, E.cg_z, E.cg_q, E.cg_s, E.cg_p,
-                       E.cg_tmu);
-    if (!sp) el_cg_apply_ksum(E, P, false, 0, s);
-    else el_cg_apply_other(E, P, *sp, false, 0, s);
-    el_cg_update(E, P, sp, true, s);
-    return (int)hipGetLastError();
+    return sp && !sp->B && P.nw <= CG_SOLVE_WATERS;
+}
+
+static void el_cg_solve(ElecBuffers& E, const ElecDev& P, bool init, int it0, int count, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cg_solve, dim3(1), dim3(1024), 0, s, P, init, it0, count, E.x, E.y, E.z, E.nbrP, E.cntP, E.tens,
+                       E.tin, E.cg_minv, E.cg_m, E.dip, E.cg_r, E.cg_u, E.cg_w, E.cg_z, E.cg_q, E.cg_s, E.cg_p, E.cg_tmu,
+                       E.cgblk, E.state);
 }
 
 // Iteration `it` (0-based): the stopping test and scalars from the last update's partials,
 // n = A m (real-space rows, structure factors, reciprocal field), then the vector update.
 int el_launch_cg_iteration(ElecBuffers& E, const ElecDev& P, int it, const ElecSpme* sp, hipStream_t s)
 {
+    if (one_launch_solve(P, sp)) {
+        el_cg_solve(E, P, false, it, 1, s);
+        return (int)hipGetLastError();
+    }
     if (sp) el_cg_apply_other(E, P, *sp, true, it, s);
     else el_cg_apply_ksum(E, P, true, it, s);
     el_cg_update(E, P, sp, false, s);
+    return (int)hipGetLastError();
+}
+
+// conjugate-gradient start: residual of the start dipoles (their fields came with the
+// charge fields of the preparation), u = M^-1 r, and
+// the first application of A, to u, for w = A u
+int el_launch_cg_start(ElecBuffers& E, const ElecDev& P, int iters, const ElecSpme* sp, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cg_init, dim3(ceil_div(P.nw, CG_WPB)), dim3(256), 0, s, sp ? one_chunk(P) : P, E.Fpart, E.efk,
+                       E.efdc, E.emu, E.efdd, E.dip, E.cg_minv, E.cg_r, E.cg_u, E.cg_m, E.cg_z, E.cg_q, E.cg_s, E.cg_p,
+                       E.cg_tmu);
+    if (one_launch_solve(P, sp)) {
+        el_cg_solve(E, P, true, 0, iters, s);
+        return (int)hipGetLastError();
+    }
+    if (!sp) el_cg_apply_ksum(E, P, false, 0, s);
+    else el_cg_apply_other(E, P, *sp, false, 0, s);
+    el_cg_update(E, P, sp, true, s);
+    for (int it = 0; it < iters; ++it) {
+        const int rc = el_launch_cg_iteration(E, P, it, sp, s);
+        if (rc) return rc;
+    }
     return (int)hipGetLastError();
 }
 

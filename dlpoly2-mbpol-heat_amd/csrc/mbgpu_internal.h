@@ -228,7 +228,7 @@ int el_launch_prep(ElecBuffers& E, const ElecDev& P, bool cg, const ElecSpme* sp
 int el_launch_iteration(ElecBuffers& E, const ElecDev& P, int first, const ElecSpme* sp, hipStream_t s);
 int el_launch_final(ElecBuffers& E, const ElecDev& P, int distribute, double g34, double gln34, int refresh,
                     const ElecSpme* sp, hipStream_t s);
-int el_launch_cg_init(ElecBuffers& E, const ElecDev& P, const ElecSpme* sp, hipStream_t s);
+int el_launch_cg_start(ElecBuffers& E, const ElecDev& P, int iters, const ElecSpme* sp, hipStream_t s);
 int el_launch_cg_iteration(ElecBuffers& E, const ElecDev& P, int it, const ElecSpme* sp, hipStream_t s);
 int el_time_sfac(ElecBuffers& E, const ElecDev& P, int reps, hipEvent_t a, hipEvent_t b, hipStream_t s);
 void el_launch_zero(double* p, long n, hipStream_t s);
