@@ -1897,33 +1897,6 @@ __global__ __launch_bounds__(256) void k_el_ksum(ElecDev P, const double* __rest
     if (threadIdx.x < 64 && valid) ksum[e] = v;
 }
 
-namespace {
-
-// Sums over the wavefront of 24 values per lane: each step halves the values a lane carries
-// (25 exchanges instead of 144 for 24 butterflies).  Returns the sum of value `k` (on every lane
-// whose k is below 24), always added in the same order.
-__device__ __forceinline__ double wave_sum24(const double (&v)[24], int lane, int& k)
-{
-    double a[12], b[6], c[4], d[2];
-    const bool h5 = lane & 32, h4 = lane & 16, h3 = lane & 8, h2 = lane & 4, h1 = lane & 2;
-#pragma unroll
-    for (int q = 0; q < 12; ++q) a[q] = (h5 ? v[q + 12] : v[q]) + __shfl_xor(h5 ? v[q] : v[q + 12], 32, 64);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) b[q] = (h4 ? a[q + 6] : a[q]) + __shfl_xor(h4 ? a[q] : a[q + 6], 16, 64);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) c[q] = (h3 ? b[q + 3] : b[q]) + __shfl_xor(h3 ? b[q] : b[q + 3], 8, 64);
-    c[3] = 0.0;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) d[q] = (h2 ? c[q + 2] : c[q]) + __shfl_xor(h2 ? c[q] : c[q + 2], 4, 64);
-    double e = (h1 ? d[1] : d[0]) + __shfl_xor(h1 ? d[0] : d[1], 2, 64);
-    e += __shfl_xor(e, 1, 64);
-    const int r = 2 * h2 + h1;
-    k = r < 3 ? 12 * h5 + 6 * h4 + 3 * h3 + r : 24;
-    return e;
-}
-
-}  // namespace
-
 // Real-space pair terms of one row (ewald2p.f:118-600; nthole = 4, lacs, lads): forces,
 // per-atom energy, ESP parts, and the row's force-matrix contraction W_i (real partners
 // only; for an M-site row the partner sums sum_j F and sum_j F (x) x_j, from which the
@@ -2762,42 +2735,6 @@ void el_launch_copy_segs(int nseg, double* const* dst, const double* const* src,
     if (nseg <= 0 || nmax <= 0) return;
     const long blocks = ceil_div(nmax, 256) < 1024 ? ceil_div(nmax, 256) : 1024;
     hipLaunchKernelGGL(k_el_copy_segs, dim3(blocks, nseg), dim3(256), 0, s, S);
-}
-
-// Up to EL_NSEG sums dst_k[i] = a_k[i] + b_k[i], i < n_k, in one launch (segment k in
-// blockIdx.y).
-struct ElSumSegs {
-    double* dst[EL_NSEG];
-    const double* a[EL_NSEG];
-    const double* b[EL_NSEG];
-    long n[EL_NSEG];
-};
-
-__global__ void k_el_sum_segs(ElSumSegs S)
-{
-    const int k = blockIdx.y;
-    double* __restrict__ d = S.dst[k];
-    const double* __restrict__ a = S.a[k];
-    const double* __restrict__ b = S.b[k];
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < S.n[k]; i += (long)gridDim.x * blockDim.x)
-        d[i] = a[i] + b[i];
-}
-
-void el_launch_sum_segs(int nseg, double* const* dst, const double* const* a, const double* const* b, const long* n,
-                        hipStream_t s)
-{
-    ElSumSegs S{};
-    long nmax = 0;
-    for (int k = 0; k < nseg; ++k) {
-        S.dst[k] = dst[k];
-        S.a[k] = a[k];
-        S.b[k] = b[k];
-        S.n[k] = n[k];
-        nmax = n[k] > nmax ? n[k] : nmax;
-    }
-    if (nseg <= 0 || nmax <= 0) return;
-    const long blocks = ceil_div(nmax, 256) < 1024 ? ceil_div(nmax, 256) : 1024;
-    hipLaunchKernelGGL(k_el_sum_segs, dim3(blocks, nseg), dim3(256), 0, s, S);
 }
 
 // dst[i] = src[i], i < n (a kernel rather than a copy call, so that a captured graph holds

@@ -146,6 +146,29 @@ struct RsPlan {
 
 #define EL_RUN 8                      // most k of a run of the final site pass
 
+// Sums over the wavefront of 24 values per lane: each step halves the values a lane carries
+// (25 exchanges instead of 144 for 24 butterflies).  Returns the sum of value `k` (on every lane
+// whose k is below 24), always added in the same order.
+__device__ __forceinline__ double wave_sum24(const double (&v)[24], int lane, int& k)
+{
+    double a[12], b[6], c[4], d[2];
+    const bool h5 = lane & 32, h4 = lane & 16, h3 = lane & 8, h2 = lane & 4, h1 = lane & 2;
+#pragma unroll
+    for (int q = 0; q < 12; ++q) a[q] = (h5 ? v[q + 12] : v[q]) + __shfl_xor(h5 ? v[q] : v[q + 12], 32, 64);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) b[q] = (h4 ? a[q + 6] : a[q]) + __shfl_xor(h4 ? a[q] : a[q + 6], 16, 64);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) c[q] = (h3 ? b[q + 3] : b[q]) + __shfl_xor(h3 ? b[q] : b[q + 3], 8, 64);
+    c[3] = 0.0;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) d[q] = (h2 ? c[q + 2] : c[q]) + __shfl_xor(h2 ? c[q] : c[q + 2], 4, 64);
+    double e = (h1 ? d[1] : d[0]) + __shfl_xor(h1 ? d[0] : d[1], 2, 64);
+    e += __shfl_xor(e, 1, 64);
+    const int r = 2 * h2 + h1;
+    k = r < 3 ? 12 * h5 + 6 * h4 + 3 * h3 + r : 24;
+    return e;
+}
+
 // Kernel-argument block of the polarizable electrostatics (passed by value).
 struct ElecDev {
     int nw, n, nreal, nrow;        // waters, sites (4nw), real atoms (3nw), rows carrying dipoles
@@ -237,9 +260,6 @@ void el_launch_copy(double* dst, const double* src, long n, hipStream_t s);
 // nseg <= EL_NSEG copies (a null source clears its destination) in one launch.
 constexpr int EL_NSEG = 6;
 void el_launch_copy_segs(int nseg, double* const* dst, const double* const* src, const long* n, hipStream_t s);
-// nseg <= EL_NSEG sums dst_k = a_k + b_k in one launch.
-void el_launch_sum_segs(int nseg, double* const* dst, const double* const* a, const double* const* b, const long* n,
-                        hipStream_t s);
 // Read-back of one electrostatics evaluation packed in doubles: the solver state (8), the
 // error flag, the 41 reduced scalars, the particle mesh's two input flags (0 without one).
 constexpr int EL_PK_ST = 0, EL_PK_ERR = 8, EL_PK_SCAL = 9, EL_PK_SPF = 50, EL_PK_N = 52;

@@ -964,20 +964,22 @@ __global__ __launch_bounds__(256) void k_heat_flux(int nreal, const double* __re
                                                    const double* __restrict__ ekin, const double* __restrict__ epot,
                                                    const double* __restrict__ epot2, const double* __restrict__ w,
                                                    const double* __restrict__ w2, const double* __restrict__ sew,
-                                                   double* __restrict__ blk)
+                                                   const double* __restrict__ epot3,
+                                                   const double* __restrict__ w3, double* __restrict__ blk)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     double red[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (i < nreal) {
         const double v[3] = {vx[i], vy[i], vz[i]};
         double e = ekin[i] + epot[i];
-        if (epot2) e += epot2[i];
+        if (epot2) e += epot3 ? epot2[i] + epot3[i] : epot2[i];
         for (int a = 0; a < 3; ++a) red[a] = e * v[a];
         for (int b = 0; b < 3; ++b) {
             double s = 0.0;
             for (int a = 0; a < 3; ++a) {
                 s += v[a] * w[9 * i + 3 * a + b];
-                if (w2) s += v[a] * w2[9 * i + 3 * a + b];
+                const long o = 9L * i + 3 * a + b;
+                if (w2) s += v[a] * (w3 ? w2[o] + w3[o] : w2[o]);
             }
             red[3 + b] = s;
         }
@@ -1073,12 +1075,13 @@ int mb_launch_accumulate(MbBuffers& B, double* fx, double* fy, double* fz, bool 
 
 int mb_launch_heat_flux(int nreal, const double* vx, const double* vy, const double* vz, const double* ekin,
                         const double* epot, const double* epot2, const double* w, const double* w2,
-                        const double* sew, double* blk, int nblk_cap, double* out, hipStream_t s)
+                        const double* sew, const double* epot3, const double* w3, double* blk, int nblk_cap, double* out,
+                        hipStream_t s)
 {
     const int nb = (nreal + 255) / 256;
     if (nb > nblk_cap) return -1;
     hipLaunchKernelGGL(k_heat_flux, dim3(nb), dim3(256), 0, s, nreal, vx, vy, vz, ekin, epot, epot2, w, w2, sew,
-                       blk);
-    hipLaunchKernelGGL(k_reduce_blocks, dim3(1), dim3(512), 0, s, blk, nb, 0, out);
+                       epot3, w3, blk);
+    if (out) hipLaunchKernelGGL(k_reduce_blocks, dim3(1), dim3(512), 0, s, blk, nb, 0, out);
     return (int)hipGetLastError();
 }

@@ -6,16 +6,20 @@
 // GPU organisation (no floating-point atomics; every per-atom sum has one owner):
 //   * k_wt_monomer: one wavefront per water.  Lanes 0..47 build the power tables
 //     x^k (k = 0..15) of the three PS variables in LDS by the same multiplication chain the
-//     reference uses; each lane then takes every 64th of the 244 expansion terms (lanes
-//     0..8 also one mass-correction term), and the wave sums energy, H1 and H2 forces and
-//     virial with xor shuffles.  Lane 0 adds the three bonds and writes the per-atom force,
-//     energy and force-matrix contraction W of O, H1 and H2, and the water's scalars;
+//     reference uses, and the tables of their derivatives; each lane then takes every 64th of the
+//     244 expansion terms (lanes 0..8 also one mass-correction term).  Only four sums are formed,
+//     the energy and its derivatives in the two bond lengths and the angle's cosine: forces and
+//     virial follow from them.  Lanes 0..2 evaluate the three bonds; lane 0 writes the per-atom
+//     force, energy and force-matrix contraction W of O, H1 and H2, and the water's scalars.
+//     Latency bound: 15.9 -> 7.3 us for 9 waters, 18.2 -> 9.2 us for 512 (ten sums with a division
+//     in each of their terms, and per-atom sums indexed in scratch memory, before);
 //   * k_wt_disp: one wavefront per real atom i owns its full dispersion row (both
 //     directions of every pair): lanes stride over all atoms j of other waters, take the
 //     minimum image, and interpolate energy and force from the tables (3-point formula of
 //     srfrce2.f).  The row sums, plus atom i's monomer terms, give its force, energy and W
 //     directly; pair scalars are halved so that each pair counts once;
-//   * k_wt_reduce: one block sums the per-water and per-atom scalars in a fixed order.
+//   * k_wt_reduce: one block sums the per-water and per-atom scalars in a fixed order (bound by
+//     the shuffles of its 18 sums: 10.8 us with a butterfly for each, 3.8 us with wave_sum24).
 // The long-range correction depends only on the cell volume, the atom counts and the
 // parameters and is evaluated on the host.
 #include <math.h>
@@ -37,12 +41,6 @@ constexpr double PS_F5Z = 0.99967788500000, PS_FBASIS = 0.15860145369897;
 constexpr double PS_FCORE = -1.6351695982132, PS_FREST = 1.0;
 constexpr double PS_EOFFSET = 2.0384848702093006e-6 * 2625.50 / 100.0;   // ps_type_couple.f90:251
 constexpr double PI_D = 3.141592653589793;
-
-__device__ __forceinline__ double wsum(double v)
-{
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 
 // f_n(x) = 1 - exp(-x) sum_{k<=n} x^k / k!, with the reference's series for |f| < 1e-8
 // (tang-toennies.f90:5-31)
@@ -116,7 +114,7 @@ __global__ __launch_bounds__(256) void k_wt_monomer(WaterDev P, const double* __
                                                     double* __restrict__ mono, double* __restrict__ wsc)
 {
 #pragma clang fp contract(off)
-    __shared__ double fm[4][16][3];
+    __shared__ double fm[4][16][3], dfm[4][16][3];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int w0 = blockIdx.x * 4 + wv;
     const bool act = w0 < P.nw;                  // whole wavefront; inactive waves still meet the barrier
@@ -133,94 +131,72 @@ __global__ __launch_bounds__(256) void k_wt_monomer(WaterDev P, const double* __
     const double rrab = 1.0 / rab, rrbc = 1.0 / rbc;
     const double u1[3] = {dab[0] * rrab, dab[1] * rrab, dab[2] * rrab};
     const double u2[3] = {dbc[0] * rrbc, dbc[1] * rrbc, dbc[2] * rrbc};
-    const double theta = acos((u1[0] * u2[0] + u1[1] * u2[1]) + u1[2] * u2[2]);
-    const double cost = cos(theta);
+    // the cosine of the angle (the reference's cos(acos(d)): not a number past +-1)
+    const double dot = (u1[0] * u2[0] + u1[1] * u2[1]) + u1[2] * u2[2];
+    const double cost = fabs(dot) <= 1.0 ? dot : nan("");
     const double cose = cos(104.3475 * PI_D / 180.0);
     const double xm = 1.0 / PS_HHMASS;
-    double pt = 0.0, v1 = 0.0, v2 = 0.0, vt = 0.0, fa[3] = {0, 0, 0}, fc[3] = {0, 0, 0};
     // power tables fm[k][v] = x_v^(k-1), fm[0] = 0 (ps_type_couple.f90:64-75): lane k of
-    // each 16-lane group repeats the reference's multiplication chain up to its power
+    // each 16-lane group repeats the reference's multiplication chain up to its power; dfm their
+    // derivatives in the bond lengths (and in x of the third)
     if (lane < 48) {
         const int v = lane >> 4, k = lane & 15;
         const double xv = v == 0 ? (rab - PS_REOH) / PS_REOH : (v == 1 ? (rbc - PS_REOH) / PS_REOH : cost - cose);
-        double p = k == 0 ? 0.0 : 1.0;
-        for (int q = 2; q <= k; ++q) p = p * xv;
+        double p = k == 0 ? 0.0 : 1.0, pm = 0.0;
+        for (int q = 2; q <= k; ++q) {
+            pm = p;
+            p = p * xv;
+        }
         fm[wv][k][v] = p;
+        dfm[wv][k][v] = v == 2 ? (k - 1) * pm : (k - 1) * pm / PS_REOH;
     }
     __syncthreads();
     if (!act) return;
+    // energy and the derivatives in rab, rbc and cos(theta); the forces and the virial follow from
+    // these four sums.  The mass-correction terms (ps_type_couple.f90:163-226) are xm times terms of
+    // the same form.
+    double sums[4] = {0.0, 0.0, 0.0, 0.0};
     if (P.ps_monomer) {
         const double(*F)[3] = fm[wv];
-        for (int j = 1 + lane; j < PS_NTERMS; j += 64) {
-            const int pk = pidx[j];
+        const double(*D)[3] = dfm[wv];
+        auto term = [&](int pk, double c) {
             const int i1 = pk & 255, i2 = (pk >> 8) & 255, i3 = pk >> 16;
-            const double c = psc[j];
+            const double cf = c * F[i3][2];
             const double dum = F[i1][0] * F[i2][1] + F[i2][0] * F[i1][1];
-            pt = pt + c * dum * F[i3][2];
-            for (int q = 0; q < 3; ++q) {
-                const double d1 = (i1 - 1) * F[i1 - 1][0] * u1[q] / PS_REOH;
-                const double d2 = (i2 - 1) * F[i2 - 1][0] * u1[q] / PS_REOH;
-                const double d3 = (i3 - 1) * F[i3 - 1][2] * (u2[q] - cost * u1[q]) / rab;
-                const double dd = d1 * F[i2][1] * F[i3][2] + d2 * F[i1][1] * F[i3][2] + dum * d3;
-                fa[q] = fa[q] - c * dd;
-            }
-            for (int q = 0; q < 3; ++q) {
-                const double d1 = (i2 - 1) * F[i2 - 1][1] * u2[q] / PS_REOH;
-                const double d2 = (i1 - 1) * F[i1 - 1][1] * u2[q] / PS_REOH;
-                const double d3 = (i3 - 1) * F[i3 - 1][2] * (u1[q] - cost * u2[q]) / rbc;
-                const double dd = F[i1][0] * d1 * F[i3][2] + F[i2][0] * d2 * F[i3][2] + dum * d3;
-                fc[q] = fc[q] - c * dd;
-            }
-            vt = vt + c * (rab * F[i2][1] * (i1 - 1) * F[i1 - 1][0] / PS_REOH +
-                           rbc * F[i1][0] * (i2 - 1) * F[i2 - 1][1] / PS_REOH +
-                           rab * F[i1][1] * (i2 - 1) * F[i2 - 1][0] / PS_REOH +
-                           rbc * F[i2][0] * (i1 - 1) * F[i1 - 1][1] / PS_REOH) *
-                          F[i3][2];
-        }
-        if (lane < PS_NMASS) {   // mass-correction terms (ps_type_couple.f90:163-226)
-            const int pk = pidxm[lane];
-            const int i1 = pk & 255, i2 = (pk >> 8) & 255, i3 = pk >> 16;
-            const double c = pcm[lane];
-            v1 = c * F[i1][0] * F[i2][1] * F[i3][2];
-            v2 = c * F[i2][0] * F[i1][1] * F[i3][2];
-            for (int q = 0; q < 3; ++q) {
-                const double d1 = (i1 - 1) * F[i1 - 1][0] * u1[q] / PS_REOH;
-                const double d2 = (i2 - 1) * F[i2 - 1][0] * u1[q] / PS_REOH;
-                const double d3 = (i3 - 1) * F[i3 - 1][2] * (u2[q] - cost * u1[q]) / rab;
-                const double corr = xm * (d1 * F[i2][1] * F[i3][2] + F[i1][0] * F[i2][1] * d3) +
-                                    xm * (d2 * F[i1][1] * F[i3][2] + F[i2][0] * F[i1][1] * d3);
-                fa[q] = fa[q] - c * corr;
-            }
-            for (int q = 0; q < 3; ++q) {
-                const double d1 = (i2 - 1) * F[i2 - 1][1] * u2[q] / PS_REOH;
-                const double d2 = (i1 - 1) * F[i1 - 1][1] * u2[q] / PS_REOH;
-                const double d3 = (i3 - 1) * F[i3 - 1][2] * (u1[q] - cost * u2[q]) / rbc;
-                const double corr = xm * (F[i1][0] * d1 * F[i3][2] + F[i1][0] * F[i2][1] * d3) +
-                                    xm * (F[i2][0] * d2 * F[i3][2] + F[i2][0] * F[i1][1] * d3);
-                fc[q] = fc[q] - c * corr;
-            }
-            vt = vt + c * (xm * rab * F[i2][1] * (i1 - 1) * F[i1 - 1][0] / PS_REOH +
-                           xm * rbc * F[i1][0] * (i2 - 1) * F[i2 - 1][1] / PS_REOH +
-                           xm * rab * F[i1][1] * (i2 - 1) * F[i2 - 1][0] / PS_REOH +
-                           xm * rbc * F[i2][0] * (i1 - 1) * F[i1 - 1][1] / PS_REOH) *
-                          F[i3][2];
-        }
-        pt = wsum(pt);
-        v1 = wsum(v1);
-        v2 = wsum(v2);
-        vt = wsum(vt);
-        for (int q = 0; q < 3; ++q) {
-            fa[q] = wsum(fa[q]);
-            fc[q] = wsum(fc[q]);
-        }
+            sums[0] += cf * dum;
+            sums[1] += cf * (D[i1][0] * F[i2][1] + D[i2][0] * F[i1][1]);
+            sums[2] += cf * (D[i2][1] * F[i1][0] + D[i1][1] * F[i2][0]);
+            sums[3] += c * dum * D[i3][2];
+        };
+        for (int j = 1 + lane; j < PS_NTERMS; j += 64) term(pidx[j], psc[j]);
+        if (lane < PS_NMASS) term(pidxm[lane], xm * pcm[lane]);
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sums[q] += __shfl_xor(sums[q], o, 64);
     }
-    if (lane != 0) return;
-    double pterm = 0.0, vterm = 0.0;
+    const double px[3] = {xo, x1, x2}, py[3] = {yo, y1, y2}, pz[3] = {zo, z1, z2};
+    // bonds (bndfrc.f:136-330): (O,H1), (O,H2) with key 0 params, (H1,H2) with key 1 params, on
+    // lanes 0, 1, 2
+    double bd[3], bom = 0.0, bga = 0.0, br;
+    {
+        const int b = min(lane, 2);
+        bd[0] = (b == 2 ? x1 : xo) - (b == 0 ? x1 : x2);
+        bd[1] = (b == 2 ? y1 : yo) - (b == 0 ? y1 : y2);
+        bd[2] = (b == 2 ? z1 : zo) - (b == 0 ? z1 : z2);
+        image_vec(P.g, bd[0], bd[1], bd[2]);
+        br = sqrt(norm2_nc(bd[0], bd[1], bd[2]));
+        const double rr = br > 1e-6 ? 1.0 / br : 0.0;
+        bond_fn(P.bond_key[b == 2], P.bond_prm[b == 2], br, bom, bga);
+        bga = bga * rr;
+    }
+    double pterm = 0.0, vterm = 0.0, fa[3] = {0, 0, 0}, fc[3] = {0, 0, 0};
     if (P.ps_monomer) {   // prefactor (ps_type_couple.f90:228-258)
-        pt = pt + xm * v1 + xm * v2;
+        const double pt = sums[0], vt = rab * sums[1] + rbc * sums[2];
         const double efac = exp(-PS_B1 * ((rab - PS_REOH) * (rab - PS_REOH) + (rbc - PS_REOH) * (rbc - PS_REOH)));
         pterm = pt * efac + psc[0] + PS_EOFFSET;
         for (int q = 0; q < 3; ++q) {
+            fa[q] = -(sums[1] * u1[q] + sums[3] * (u2[q] - cost * u1[q]) / rab);
+            fc[q] = -(sums[2] * u2[q] + sums[3] * (u1[q] - cost * u2[q]) / rbc);
             fa[q] = fa[q] * efac + 2.0 * PS_B1 * (rab - PS_REOH) * u1[q] * efac * pt;
             fc[q] = fc[q] * efac + 2.0 * PS_B1 * (rbc - PS_REOH) * u2[q] * efac * pt;
         }
@@ -232,27 +208,23 @@ __global__ __launch_bounds__(256) void k_wt_monomer(WaterDev P, const double* __
     double f[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, e[3] = {0, 0, 0}, W[3][9];
     for (int a = 0; a < 3; ++a)
         for (int q = 0; q < 9; ++q) W[a][q] = 0.0;
-    const double px[3] = {xo, x1, x2}, py[3] = {yo, y1, y2}, pz[3] = {zo, z1, z2};
     double st[6] = {0, 0, 0, 0, 0, 0}, eb = 0.0, vb = 0.0;
     // force-matrix entry: force F on atom a due to atom b (un-imaged positions in W)
     auto entry = [&](int a, int b, const double* Fv) {
         const double r[3] = {px[a] - px[b], py[a] - py[b], pz[a] - pz[b]};
+#pragma unroll
         for (int q = 0; q < 3; ++q) f[a][q] += Fv[q];
+#pragma unroll
         for (int p = 0; p < 3; ++p)
+#pragma unroll
             for (int s = 0; s < 3; ++s) W[a][3 * p + s] += Fv[p] * r[s];
     };
-    // bonds (bndfrc.f:136-330): (O,H1), (O,H2) with key 0 params, (H1,H2) with key 1 params
+#pragma unroll
     for (int b = 0; b < 3; ++b) {
         const int t = b == 2 ? 1 : 0;
-        if (P.bond_key[t] == 0) continue;
+        const double d[3] = {__shfl(bd[0], b, 64), __shfl(bd[1], b, 64), __shfl(bd[2], b, 64)};
+        const double r = __shfl(br, b, 64), omega = __shfl(bom, b, 64), gamma = __shfl(bga, b, 64);
         const int ia = b == 2 ? 1 : 0, ib = b == 2 ? 2 : 1 + b;
-        double d[3] = {px[ia] - px[ib], py[ia] - py[ib], pz[ia] - pz[ib]};
-        image_vec(P.g, d[0], d[1], d[2]);
-        const double r = sqrt(norm2_nc(d[0], d[1], d[2]));
-        const double rr = r > 1e-6 ? 1.0 / r : 0.0;
-        double omega, gamma;
-        bond_fn(P.bond_key[t], P.bond_prm[t], r, omega, gamma);
-        gamma = gamma * rr;
         eb += omega;
         vb += gamma * r * r;
         e[ia] += 0.5 * omega;
@@ -282,6 +254,7 @@ __global__ __launch_bounds__(256) void k_wt_monomer(WaterDev P, const double* __
         st[4] += rab * u1[1] * fa[2] + rbc * u2[1] * fc[2];
         st[5] += rab * u1[2] * fa[2] + rbc * u2[2] * fc[2];
     }
+    if (lane != 0) return;
     for (int a = 0; a < 3; ++a) {
         double* m = mono + 13L * (io + a);
         for (int q = 0; q < 3; ++q) m[q] = f[a][q];
@@ -312,8 +285,8 @@ __global__ __launch_bounds__(256) void k_wt_disp(WaterDev P, const double* __res
     if (i >= P.nr) return;
     const double xi = x[i], yi = y[i], zi = z[i];
     const int wi = i / 3, ti = (i % 3) != 0;
-    double a[20];
-    for (int q = 0; q < 20; ++q) a[q] = 0.0;   // f3, e, W9, st6, vir
+    double a[24];
+    for (int q = 0; q < 24; ++q) a[q] = 0.0;   // f3, e, W9, st6, vir
     if (P.dispersion) {
         auto pair = [&](int j) {
 #pragma clang fp contract(off)
@@ -357,23 +330,27 @@ __global__ __launch_bounds__(256) void k_wt_disp(WaterDev P, const double* __res
         } else {
             for (int j = lane; j < P.nr; j += 64) pair(j);
         }
-        for (int q = 0; q < 20; ++q) a[q] = wsum(a[q]);
     }
-    if (lane != 0) return;
-    const double* m = mono + 13L * i;
-    const double f0 = m[0] + a[0], f1 = m[1] + a[1], f2 = m[2] + a[2];
-    fw[i] = f0;
-    fw[P.nr + i] = f1;
-    fw[2L * P.nr + i] = f2;
-    if (fx) fx[i] += f0;
-    if (fy) fy[i] += f1;
-    if (fz) fz[i] += f2;
-    eout[i] = m[3] + 0.5 * a[3];
-    for (int q = 0; q < 9; ++q) wout[9L * i + q] = m[4 + q] + a[4 + q];
+    int k;
+    const double v = wave_sum24(a, lane, k);
+    if ((lane & 1) || k >= 20) return;
+    // the even lane that holds sum k writes what it belongs to
     double* s = asc + 8L * i;
-    s[0] = 0.5 * a[3];
-    s[1] = 0.5 * a[19];
-    for (int q = 0; q < 6; ++q) s[2 + q] = 0.5 * a[13 + q];
+    if (k < 13) {
+        const double t = mono[13L * i + k] + (k == 3 ? 0.5 * v : v);
+        if (k < 3) {
+            fw[(long)k * P.nr + i] = t;
+            double* f = k == 0 ? fx : k == 1 ? fy : fz;
+            if (f) f[i] += t;
+        } else if (k == 3) {
+            eout[i] = t;
+            s[0] = 0.5 * v;
+        } else {
+            wout[9L * i + k - 4] = t;
+        }
+    } else {
+        s[k == 19 ? 1 : k - 11] = 0.5 * v;
+    }
 }
 
 // Fixed-order sums of the per-water [nw][10] and per-atom [nr][8] scalars into out[18].
@@ -381,17 +358,19 @@ __global__ __launch_bounds__(1024) void k_wt_reduce(int nw, int nr, const double
                                                     const double* __restrict__ asc, double* __restrict__ out)
 {
     __shared__ double red[16][18];
-    double v[18];
-    for (int q = 0; q < 18; ++q) v[q] = 0.0;
+    double v[24];
+#pragma unroll
+    for (int q = 0; q < 24; ++q) v[q] = 0.0;
     for (int w = threadIdx.x; w < nw; w += blockDim.x)
+#pragma unroll
         for (int q = 0; q < 10; ++q) v[q] += wsc[10L * w + q];
     for (int i = threadIdx.x; i < nr; i += blockDim.x)
+#pragma unroll
         for (int q = 0; q < 8; ++q) v[10 + q] += asc[8L * i + q];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int q = 0; q < 18; ++q) {
-        const double s = wsum(v[q]);
-        if (lane == 0) red[wv][q] = s;
-    }
+    int k;
+    const double t = wave_sum24(v, lane, k);
+    if (k < 18) red[wv][k] = t;
     __syncthreads();
     if (threadIdx.x < 18) {
         double s = 0.0;
