@@ -52,10 +52,10 @@ FLOP_TRIMER = 113100    # algorithmic FLOP per 3B trimer (value + gradient)
 PEAK_FP64 = 78.6        # TFLOP/s, MI355X FP64 (vector and matrix peaks are equal)
 FLOP_SFAC = 8          # FLOP per (k vector, site) of the Ewald structure factors as matrix products: for the real
                        # and the imaginary part one multiply-add with (l alpha + m beta) and one with gamma
-# HBM bytes per launch of k_el_sfac<false> at this workload, from rocprofv3 --pmc FETCH_SIZE /
+# HBM bytes per launch of k_rs_sfac<2> in the solver at this workload, from rocprofv3 --pmc FETCH_SIZE /
 # WRITE_SIZE (KiB per dispatch) scaled by the same counters on a plain 512 MiB copy (FETCH x 2,
-# WRITE x 1); profiles/k_el_sfac_bench512_traffic.md
-SFAC_TRAFFIC_BYTES = (4190.5 * 2.0 + 7486.5 * 1.0) * 1024
+# WRITE x 1); profiles/k_rs_bench512_traffic.md
+SFAC_TRAFFIC_BYTES = (5865 * 2.0 + 1628 * 1.0) * 1024
 
 
 def _cpu_eval(seed_and_budget):
@@ -554,7 +554,7 @@ def main():
                      "kernel": "k_rs_sfac<2> (dipole structure factors, launched once per solver iteration)",
                      "achieved": achieved, "peak": PEAK_FP64, "unit": "TFLOP/s", "frac": achieved / PEAK_FP64,
                      "traffic": SFAC_TRAFFIC_BYTES,
-                     "traffic_source": "copied from profiles/k_el_sfac_bench512_traffic.md (rocprofv3 --pmc FETCH_SIZE "
+                     "traffic_source": "copied from profiles/k_rs_bench512_traffic.md (rocprofv3 --pmc FETCH_SIZE "
                                        "and WRITE_SIZE of this workload and build, scaled by a plain copy), bytes "
                                        "per launch; not measured in this run",
                      "kernel_ms": ms_sf, "flop_per_launch": flop_sf,
