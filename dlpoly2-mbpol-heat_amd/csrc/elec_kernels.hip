@@ -810,10 +810,11 @@ __device__ __forceinline__ v4d mfma_f64(double a, double b, v4d c)
 }
 
 // One set of weights of a structure-factor launch: dipoles mu[3 j] (dip) or scalars v[j stride],
-// over the first ns sites.
+// over the first ns sites; with pol of the polarizable sites alone (ewald1p.f takes no other
+// site's dipole, and a caller's start dipoles may hold any value there).
 struct RsSrc {
     const double* v;
-    int stride, dip, ns;
+    int stride, dip, ns, pol;
 };
 struct RsSrcs {
     RsSrc s[4];
@@ -861,7 +862,7 @@ __device__ __forceinline__ void rs_sfac_block(const ElecDev& P, const RsSrc src,
         const int i = tid + 64 * RS_WAVES * h;
         const double* v = src.v + (long)(j0 + i) * src.stride;
         mv[h][0] = mv[h][1] = mv[h][2] = 0.0;
-        if (i < nj) {
+        if (i < nj && (!src.pol || site_polr2(P, j0 + i) > 1.e-6)) {
             mv[h][0] = v[0];
             if (src.dip) {
                 mv[h][1] = v[1];
@@ -2465,7 +2466,7 @@ int el_launch_prep(ElecBuffers& E, const ElecDev& P, bool cg, const ElecSpme* sp
         sp_launch_field(*sp->B, *sp->G, P.n, g, 2, sp->kap, E.Fpart, P.n, nullptr, s);
     } else {
         // structure factors of the start dipoles and of the charges, and the iloop = 1 fields
-        rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.n}, {E.chge, 1, 0, P.n}}}, 2, P.rs.nchq, P.rs.spcq, true, E.state, nullptr,
+        rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.n, 1}, {E.chge, 1, 0, P.n, 0}}}, 2, P.rs.nchq, P.rs.spcq, true, E.state, nullptr,
                        0, 0, s);
         rs_launch_field(E, P, 2, P.rs.nchq, s);
     }
@@ -2487,7 +2488,7 @@ int el_launch_iteration(ElecBuffers& E, const ElecDev& P, int first, const ElecS
     } else if (!first) {
         // reciprocal dipole field from the current dipoles (the first iteration's came
         // with the charge field)
-        rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.nrow}}}, 1, P.rs.nch, P.rs.spc, true, E.state, nullptr, 0, 0, s);
+        rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.nrow, 1}}}, 1, P.rs.nch, P.rs.spc, true, E.state, nullptr, 0, 0, s);
         rs_launch_field(E, P, 1, P.rs.nch, s);
         hipLaunchKernelGGL(k_el_kfield_reduce<false>, dim3(ceil_div(3L * P.nrow, 64)), dim3(256), 0, s, P, E.Fpart, E.dip,
                            E.efdd, E.efdc, E.state);
@@ -2505,7 +2506,7 @@ int el_launch_iteration(ElecBuffers& E, const ElecDev& P, int first, const ElecS
 // of iteration `it` first when `check`) and emu in one launch, then the field.
 static void el_cg_apply_ksum(ElecBuffers& E, const ElecDev& P, bool check, int it, hipStream_t s)
 {
-    rs_launch_sfac(E, P, {{{E.cg_m, 3, 1, P.nrow}}}, 1, P.rs.nch, P.rs.spc, true, E.state, check ? E.cgblk : nullptr,
+    rs_launch_sfac(E, P, {{{E.cg_m, 3, 1, P.nrow, 1}}}, 1, P.rs.nch, P.rs.spc, true, E.state, check ? E.cgblk : nullptr,
                    ceil_div(P.nw, CG_WPB), it, s);
     rs_launch_field(E, P, 1, P.rs.nch, s);
 }
@@ -2588,7 +2589,7 @@ int el_time_sfac(ElecBuffers& E, const ElecDev& P, int reps, hipEvent_t a, hipEv
 {
     (void)hipEventRecord(a, s);
     for (int r = 0; r < reps; ++r)
-        rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.nrow}}}, 1, P.rs.nch, P.rs.spc, false, E.zero_state, nullptr, 0, 0, s);
+        rs_launch_sfac(E, P, {{{E.dip, 3, 1, P.nrow, 1}}}, 1, P.rs.nch, P.rs.spc, false, E.zero_state, nullptr, 0, 0, s);
     (void)hipEventRecord(b, s);
     return (int)hipGetLastError();
 }
@@ -2624,8 +2625,9 @@ int el_launch_final(ElecBuffers& E, const ElecDev& P, int distribute, double g34
     }
     if (!sp) {
         // structure factors of mu_x, mu_y, mu_z of the converged dipoles and of the charges
-        rs_launch_sfac(E, P, {{{E.dip, 3, 0, P.nrow}, {E.dip + 1, 3, 0, P.nrow}, {E.dip + 2, 3, 0, P.nrow}, {E.chge, 1, 0, P.n}}},
-                       4, P.rs.nchq, P.rs.spcq, false, E.zero_state, nullptr, 0, 0, s);
+        rs_launch_sfac(E, P,
+                       {{{E.dip, 3, 0, P.nrow, 1}, {E.dip + 1, 3, 0, P.nrow, 1}, {E.dip + 2, 3, 0, P.nrow, 1},
+                         {E.chge, 1, 0, P.n, 0}}}, 4, P.rs.nchq, P.rs.spcq, false, E.zero_state, nullptr, 0, 0, s);
         hipLaunchKernelGGL(k_el_kscal, dim3(nkb), dim3(256), 0, s, P, E.kv, E.Spart, E.kf, b_ks);
         hipLaunchKernelGGL(k_el_kfinal, dim3(ceil_div(P.n, 256), P.kchunks), dim3(256),
                            sizeof(double2) * 6 * EL_RUN * P.rpc, s, P, (const int4*)E.runs, E.runk, E.phc, E.phs, E.kv, E.kf, E.chge, E.dip, E.Fpart);
