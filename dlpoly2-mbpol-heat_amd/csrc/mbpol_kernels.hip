@@ -471,8 +471,9 @@ __device__ __forceinline__ void setup2(int d, int ncap, const double* __restrict
         const V2Def v = c2_vars[n];
         const double dx = s[3 * v.s1] - s[3 * v.s2], dy = s[3 * v.s1 + 1] - s[3 * v.s2 + 1],
                      dz = s[3 * v.s1 + 2] - s[3 * v.s2 + 2];
+        // (r2 rinv is not a number where two sites coincide: r = 0 there, as sqrt(r2) gives)
         const double r2 = dx * dx + dy * dy + dz * dz, rinv = rsqrt(r2);
-        const double e = exp(c2_k[v.k] * ((double)v.d0 - r2 * rinv));
+        const double e = exp(c2_k[v.k] * ((double)v.d0 - (r2 == 0.0 ? 0.0 : r2 * rinv)));
         const double val = v.kind ? e * rinv : e;
         xv[(long)n * ncap + d] = val;
         if (xvf) xvf[(long)n * ncap + d] = (float)val;
