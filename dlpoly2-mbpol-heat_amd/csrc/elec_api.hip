@@ -21,9 +21,11 @@
 #ifndef EL_KCHUNK_RUNS
 #define EL_KCHUNK_RUNS 32     // at most this many k runs per chunk of the final reciprocal pass
 #endif
-// Most solver iterations enqueued (or captured in a graph) at once.  SOR from zero dipoles takes
+// Most solver iterations enqueued (or captured in a graph) at once: EL_BATCH whatever max_iter is,
+// and up to EL_MAX_BATCH as far as max_iter allows (first_batch).  SOR from zero dipoles takes
 // 70 to 80: with a bound of 64 a captured evaluation always ended unconverged and the one-call
 // evaluation was repeated launch by launch (216 waters: 6.05 -> 3.03 ms with the bound at 256).
+#define EL_BATCH 64
 #define EL_MAX_BATCH 256
 #define PI_D 3.141592653589793
 
@@ -608,17 +610,34 @@ const ElecSpme* recip_of(const ElecState& S, ElecSpme& spx, ElecSpme& none)
 }
 }  // namespace
 
+// Solver iterations enqueued between two tests of max_iter once the first batch is done
+static inline int batch_step(int solver) { return solver == 1 ? 4 : 8; }
+
+// The first batch of a solve that is expected to take `last` iterations: last + 2.  max_iter is
+// tested between batches; past EL_BATCH iterations a batch ends where solving on from there in steps
+// would (whole steps, none begun at or after max_iter), so whether a solve is refused does not depend
+// on how far ahead it was enqueued.
+static int first_batch(int last, int max_iter, int solver)
+{
+    const int step = batch_step(solver);
+    auto up = [&](int n) { return EL_BATCH + (std::max(n - EL_BATCH, 0) + step - 1) / step * step; };
+    if (last + 2 <= EL_BATCH) return last + 2;
+    return std::min(EL_MAX_BATCH, std::min(up(last + 2), up(max_iter)));
+}
+
 // Solver iterations a captured evaluation holds (0 before the first evaluation set a count):
-// the last count + 2, kept while it covers the solve and is not far too long (iterations past
-// convergence are no-ops of about a microsecond per kernel; a new capture costs more), so
-// counts that drift by one or two do not capture again.  MBGPU_GRAPH_BATCH=k caps it (a test
-// aid for the continuation after a graph).
-int elec_batch(const ElecState& S)
+// first_batch of the last count, or what the present capture holds while that covers the solve,
+// is not far too long (iterations past convergence are no-ops of about a microsecond per kernel;
+// a new capture costs more, so counts that drift by one or two do not capture again) and is itself
+// a first_batch.  MBGPU_GRAPH_BATCH=k caps it (a test aid for the continuation after a graph).
+int elec_batch(const ElecState& S, int max_iter, int solver)
 {
     int gb = 0;
     if (S.last_iters > 0) {
-        gb = std::min(S.last_iters + 2, EL_MAX_BATCH);
-        if (S.gbatch >= S.last_iters && S.gbatch <= S.last_iters + 8) gb = S.gbatch;
+        gb = first_batch(S.last_iters, max_iter, solver);
+        if (S.gbatch >= S.last_iters && S.gbatch <= S.last_iters + 8 &&
+            S.gbatch == first_batch(S.gbatch - 2, max_iter, solver))
+            gb = S.gbatch;
     }
     if (const char* ev = getenv("MBGPU_GRAPH_BATCH")) gb = gb ? std::min(gb, std::max(1, atoi(ev))) : 0;
     return gb;
@@ -740,7 +759,7 @@ int elec_evaluate(ElecState& S, int max_iter, int distribute, int solver, hipStr
         herr = (int)S.hpk[EL_PK_ERR];
         return hipSuccess;
     };
-    const int gb = elec_batch(S);
+    const int gb = elec_batch(S, max_iter, solver);
     bool from_graph = false;
     // MBGPU_GRAPHS=0 launches kernel by kernel whatever the context's setting (a test aid)
     const char* gv = getenv("MBGPU_GRAPHS");
@@ -786,12 +805,13 @@ int elec_evaluate(ElecState& S, int max_iter, int distribute, int solver, hipStr
     // with clamped counts, so an overflowed attempt runs in bounds and is simply repeated
     // with larger rows, from the same start dipoles (kept in dip0).
     for (int attempt = from_graph ? -1 : (S.gexec && herr ? 1 : 0); attempt >= 0 || from_graph;) {
-        int launched = 0, batch = S.last_iters > 0 ? std::min(S.last_iters + 2, EL_MAX_BATCH) : (solver == 1 ? 8 : 12);
+        int launched = 0,
+            batch = S.last_iters > 0 ? first_batch(S.last_iters, max_iter, solver) : (solver == 1 ? 8 : 12);
         int rc = 0;
         if (from_graph) {
             // continue after the graph's iterations
             launched = S.gbatch;
-            batch = solver == 1 ? 4 : 8;
+            batch = batch_step(solver);
             from_graph = false;
             attempt = -1;
             if (st[2] != 0.0) break;
@@ -813,7 +833,7 @@ int elec_evaluate(ElecState& S, int max_iter, int distribute, int solver, hipStr
                 return rc;
             }
             launched = batch;
-            batch = solver == 1 ? 4 : 8;
+            batch = batch_step(solver);
         }
         bool overflow = false;
         for (;;) {

@@ -1054,7 +1054,7 @@ int evaluate_impl(mbgpu_ctx* c, int imcon, const double cell[9], int nttm2, cons
     if (elec_configure(c->el, nw, g, cell, ep, err)) return fail(-1, "%s", err.c_str());
     c->wt.ready = false;
     if (water_configure(c->wt, nw, g, cell, wp, c->stream, err)) return fail(-1, "%s", err.c_str());
-    const int gb = elec_batch(c->el);
+    const int gb = elec_batch(c->el, ep->max_iter, ep->solver);
     bool fused_ran = false;
     // one enqueue (a graph replay once captured) when every buffer has been sized by an
     // evaluation through the separate entries

@@ -303,7 +303,7 @@ void elec_drop_graph(ElecState& S);
 // pieces of an evaluation for a caller that enqueues it with other work (one graph of a
 // complete evaluation): the solver iterations a capture holds, the device work, the key
 // bytes of that work, and the host side of the end
-int elec_batch(const ElecState& S);
+int elec_batch(const ElecState& S, int max_iter, int solver);
 int elec_enqueue_full(ElecState& S, int distribute, int solver, int gb, hipStream_t s);
 void elec_key_append(const ElecState& S, int distribute, int solver, int gb, std::vector<unsigned char>& k);
 int elec_finish(ElecState& S, const double st[8], const int spflag[2], std::string& err);

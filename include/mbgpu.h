@@ -156,7 +156,10 @@ typedef struct {
     int kmax[3];              /* Ewald kmax1..3 */
     double toler;             /* dipole tolerance, e*A (the reference converts from Debye) */
     double omega;             /* sor_omega: weight of the old dipole in the SOR update */
-    int max_iter;             /* error after this many iterations (the reference: 22581) */
+    int max_iter;             /* error after this many iterations (the reference: 22581).  Tested
+                                 between batches of iterations: a first one (up to 64, the last
+                                 solve's count + 2) and then 8 (solver 1: 4) at a time, so that a
+                                 solve which ends within the batch that reaches max_iter counts */
     double gamma;             /* M-site position parameter (0.426706882) */
     double q_o;               /* oxygen charge (0) */
     double polr[3];           /* smearing polarizabilities of O, H, M (A^3) */
