@@ -99,12 +99,16 @@ void free_buffers(ElecBuffers& E)
     dfree(E.vr); dfree(E.vdcr); dfree(E.vesp); dfree(E.f2); dfree(E.fsite); dfree(E.e1); dfree(E.e2);
     dfree(E.w2); dfree(E.fmsum); dfree(E.fmx); dfree(E.eout); dfree(E.wout);
     dfree(E.sout); dfree(E.blk); dfree(E.scal); dfree(E.err); dfree(E.pk);
-    E.n = E.capA = E.capP = E.K = E.nrun = 0;
+    E.n = E.capA = E.capP = E.K = E.nrun = E.kstride = 0;
 }
 
 // doubles of block partials in E.blk: the final passes' (nkb blocks of 8 per-k sums, 8 per site, 24
 // per 16 waters), or SOR's 2 per 256 rows
 int final_partials(int n, int nw, int nkb) { return 8 * nkb + 8 * n + 24 * ((nw + 15) / 16) + 2 * (n / 256 + 1); }
+
+// A plan's key (S.nw, E.capA, S.tab_alpha, S.k_alpha, E.kstride) says that its buffers are there and
+// hold it: each set-up below clears the key before the first buffer goes and sets it after the last
+// one is filled, so that a call that fails in between leaves nothing a later call would take for whole.
 
 // site-sized buffers (allocated once per context size)
 int alloc_sites(ElecState& S, int nw, std::string& err)
@@ -150,11 +154,12 @@ int alloc_rows(ElecState& S, int capA, int capP, std::string& err)
     dfree(E.nbrA);
     dfree(E.nbrP);
     dfree(E.tens);
-    E.capA = capA;
-    E.capP = capP;
+    E.capA = E.capP = 0;
     ECHK(dalloc(&E.nbrA, (size_t)E.n * capA));
     ECHK(dalloc(&E.nbrP, (size_t)E.n * capP));
     ECHK(dalloc(&E.tens, (size_t)E.n * capP));
+    E.capA = capA;
+    E.capP = capP;
     return 0;
 }
 
@@ -179,6 +184,7 @@ int build_table(ElecState& S, double alpha, double rcut, std::string& err)
             e[n] = rsqi * ((2.0 * fn - 1.0) * e[n - 1] + pow(2.0 * alpha * alpha, fn) * exp2a / alpha / SQRPI);
         }
     }
+    S.tab_alpha = -1.0;
     dfree(E.tab);
     ECHK(dalloc(&E.tab, t.size()));
     ECHK(hipMemcpy(E.tab, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice));
@@ -341,6 +347,7 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
         }
         mmin = -kmax[1];
     }
+    S.k_alpha = -1.0;
     dfree(E.kv);
     dfree(E.runs);
     dfree(E.runk);
@@ -364,9 +371,10 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
     if (ks != E.kstride) {
         dfree(E.phc);
         dfree(E.phs);
-        E.kstride = ks;
+        E.kstride = 0;
         ECHK(dalloc(&E.phc, (size_t)3 * ks * E.n));
         ECHK(dalloc(&E.phs, (size_t)3 * ks * E.n));
+        E.kstride = ks;
     }
     // k split of the site-parallel passes: about 2048 wavefronts over the sites
     E.kchunks = std::max(1, std::min(E.nrun, EL_KCHUNK_WAVES / std::max(1, (E.n + 63) / 64)));
@@ -402,6 +410,7 @@ namespace {
 int alloc_direct(ElecState& S, std::string& err)
 {
     ElecBuffers& E = S.E;
+    S.k_alpha = -1.0;   // a later periodic call builds its k list
     dfree(E.Fpart);
     ECHK(dalloc(&E.Fpart, (size_t)6 * E.n));
     dfree(E.blk);
@@ -410,7 +419,6 @@ int alloc_direct(ElecState& S, std::string& err)
     E.K = E.nrun = 0;
     E.kchunks = E.fchunks = 1;
     E.rpc = 0;
-    S.k_alpha = -1.0;   // a later periodic call builds its k list
     S.P.rvolm = 0.0;
     return 0;
 }
@@ -431,6 +439,8 @@ void elec_release(ElecState& S)
     delete S.spg;
     S.spg = nullptr;
     cells_free(S.cells);
+    S.tab_alpha = S.k_alpha = -1.0;
+    S.nw = 0;
     S.ready = false;
 }
 

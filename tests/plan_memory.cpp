@@ -1,0 +1,258 @@
+// plan_memory.cpp -- the library's set-up on host memory: hipMalloc and the other runtime calls a
+// set-up makes are defined here (the program's definitions come before the runtime's), so that an
+// allocation can be made to fail and every buffer's size, fill and content can be looked at
+// without a GPU.  Nothing is launched.  test_plan_memory.py builds and runs it:
+//   plan_memory CHECK [args]  prints what is wrong, or "ok"
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "mbgpu_internal.h"
+
+namespace {
+
+struct Block {
+    size_t size;
+    int fill;                          // last byte set over all of it, -1: none
+};
+std::map<const void*, Block> live;
+long nalloc = 0, nfree = 0, fail_at = -1;   // allocations made, frees, the allocation that fails
+int wrong = 0;
+
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n)
+{
+    *p = nullptr;
+    if (nalloc++ == fail_at) return hipErrorOutOfMemory;
+    *p = calloc(n, 1);
+    live[*p] = Block{n, -1};
+    return hipSuccess;
+}
+hipError_t hipFree(void* p)
+{
+    if (!live.erase(p)) {
+        printf("free of a block that is not live\n");
+        ++wrong;
+        return hipErrorInvalidValue;
+    }
+    ++nfree;
+    free(p);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned int)
+{
+    *p = calloc(n, 1);
+    return hipSuccess;
+}
+hipError_t hipHostFree(void* p)
+{
+    free(p);
+    return hipSuccess;
+}
+hipError_t hipMemset(void* p, int v, size_t n)
+{
+    memset(p, v, n);
+    auto b = live.find(p);
+    if (b != live.end() && b->second.size == n) b->second.fill = v;
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind)
+{
+    memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t)
+{
+    memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t* s)
+{
+    *s = nullptr;
+    return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned int)
+{
+    *s = nullptr;
+    return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e)
+{
+    *e = nullptr;
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n)
+{
+    *n = 1;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int* d)
+{
+    *d = 0;
+    return hipSuccess;
+}
+}
+
+namespace {
+
+void check(bool ok, const std::string& what)
+{
+    if (ok) return;
+    printf("%s\n", what.c_str());
+    ++wrong;
+}
+
+size_t size_of(const void* p)
+{
+    auto b = live.find(p);
+    return b == live.end() ? 0 : b->second.size;
+}
+
+// ------------------------------------------------------------------ electrostatics ----
+struct Call {
+    const char* name;
+    int nw, imcon;
+    double L, alpha, rcut;
+    int kmax[3], recip;
+};
+const Call calls[] = {
+    {"box", 8, 1, 12.0, 0.55, 1.1, {8, 8, 8}, 0},         // (short cut-offs: short tables)
+    {"other cell", 8, 1, 13.0, 0.55, 1.1, {8, 8, 8}, 0},
+    {"other k list", 8, 2, 12.0, 0.5, 1.0, {11, 9, 17}, 0},
+    {"mesh", 8, 1, 12.0, 0.6, 1.1, {8, 8, 8}, 1},
+    {"cluster", 8, 0, 3.0, 0.0, 3.0, {1, 1, 1}, 0},
+    {"other size", 9, 1, 12.0, 0.55, 1.1, {8, 8, 8}, 0},
+};
+constexpr int NCALLS = sizeof calls / sizeof calls[0];
+
+int configure(ElecState& S, const Call& c)
+{
+    mbgpu_elec_params p = {};
+    p.rcut = c.rcut;
+    p.alpha = c.alpha;
+    for (int i = 0; i < 3; ++i) p.kmax[i] = c.kmax[i];
+    p.toler = 1e-12;
+    p.omega = 0.3;
+    p.max_iter = 100;
+    p.gamma = 0.4267;
+    p.polr[0] = p.polr[2] = p.polr2[0] = 1.31;
+    p.polr[1] = p.polr2[1] = 0.294;
+    p.athole = p.athole13 = 0.055;
+    p.athole12 = 0.626;
+    p.ascc = p.ascd = 0.4;
+    CellGeom g = {};
+    g.imcon = c.imcon;
+    const double cell[9] = {c.L, 0, 0, 0, c.L, 0, 0, 0, c.imcon == 2 ? c.L + 1.0 : c.L};
+    for (int i = 0; i < 9; ++i) g.c[i] = cell[i];
+    S.recip = c.recip;
+    S.sp_order = 6;
+    for (int i = 0; i < 3; ++i) S.sp_grid[i] = 16;
+    std::string err;
+    return elec_configure(S, c.nw, g, cell, &p, err);
+}
+
+// every buffer that an evaluation after a successful configure reads or writes is there, as large
+// as the launch parameters say, and holds what a new state's holds (R)
+void complete(const ElecState& S, const ElecState& R, const Call& c, const std::string& when)
+{
+    const ElecBuffers &E = S.E, &F = R.E;
+    const ElecDev& P = S.P;
+    const size_t n = 4 * c.nw, nr = 3 * c.nw;
+    auto need = [&](const char* name, const void* p, size_t bytes) {
+        check(size_of(p) >= bytes, when + ": " + name + " holds " + std::to_string(size_of(p)) + " of " +
+                                       std::to_string(bytes) + " bytes");
+    };
+    auto same = [&](const char* name, const void* p, const void* q, size_t bytes) {
+        need(name, p, bytes);
+        if (size_of(p) >= bytes) check(memcmp(p, q, bytes) == 0, when + ": " + name + " is another plan's");
+    };
+#define NEED(f, count) need(#f, E.f, sizeof(*E.f) * (size_t)(count))
+#define SAME(f, count) same(#f, E.f, F.f, sizeof(*E.f) * (size_t)(count))
+    check(P.n == (int)n && P.K == R.P.K && P.nrun == R.P.nrun && P.rvolm == R.P.rvolm && P.drewd == R.P.drewd &&
+              P.kchunks == R.P.kchunks && P.fchunks == R.P.fchunks && P.rpc == R.P.rpc,
+          when + ": launch parameters of another plan");
+    NEED(x, n); NEED(y, n); NEED(z, n); NEED(chge, n); NEED(dg, 6 * c.nw); NEED(tin, 36 * c.nw);
+    NEED(cntA, n); NEED(cntP, n); NEED(dip, 3 * n); NEED(dip0, 3 * n); NEED(efk, 3 * n); NEED(emu, 3 * n);
+    NEED(efdc, 3 * n); NEED(efdd, 3 * n); NEED(cg_p, nr * 3); NEED(cg_q, nr * 3); NEED(cg_r, nr * 3);
+    NEED(cg_z, nr * 3); NEED(cg_u, nr * 3); NEED(cg_w, nr * 3); NEED(cg_m, nr * 3); NEED(cg_s, nr * 3);
+    NEED(cg_tmu, nr * 3); NEED(cg_minv, 45 * c.nw); NEED(cgblk, 5 * ((c.nw + 6) / 7)); NEED(ksum, 15 * n);
+    NEED(state, 16); NEED(vr, n); NEED(vdcr, n); NEED(vesp, n); NEED(f2, 3 * n); NEED(fsite, 3 * n); NEED(e1, n);
+    NEED(e2, n); NEED(w2, 9 * n); NEED(fmsum, 3 * n); NEED(fmx, 9 * n); NEED(eout, nr); NEED(wout, 9 * nr);
+    NEED(sout, 9 * nr); NEED(scal, 41); NEED(err, 4); NEED(pk, EL_PK_N);
+    check(P.capA > 0 && P.capP > 0, when + ": no neighbour rows");
+    NEED(nbrA, n * P.capA); NEED(nbrP, n * P.capP); NEED(tens, n * P.capP);
+    const int nkb = c.imcon == 0 ? 0 : std::max((P.K + 63) / 64, P.n / 4);
+    NEED(blk, 8 * nkb + 8 * n + 24 * ((c.nw + 15) / 16));
+    NEED(Fpart, std::max(c.imcon ? 16 * P.kchunks : 0, 6 * P.fchunks) * n);
+    SAME(tab, 4 * (F.ntab + 1));
+    if (c.imcon == 0) return;
+    const RsPlan& Q = P.rs;
+    check(Q.ng == R.P.rs.ng && Q.ntiles == R.P.rs.ntiles && Q.kt == R.P.rs.kt && Q.nch == R.P.rs.nch &&
+              Q.pair == E.rs_pair && Q.ak == E.rs_ak && Q.kpos == E.rs_kpos,
+          when + ": matrix passes of another plan");
+    SAME(kv, 8 * P.K); SAME(runs, 4 * P.nrun); SAME(runk, P.nrun); NEED(kf, 16 * P.K);
+    SAME(rs_pair, 16 * Q.ng); SAME(rs_ak, 16 * Q.ng * (8 * Q.ntiles + 1)); SAME(rs_kpos, P.K);
+    NEED(pht, (n + RS_PAD) * Q.kt); NEED(Spart, 4 * std::max(Q.nch, Q.nchq) * Q.ng * RS_SLOT(Q.ntiles));
+    NEED(phc, 3 * P.kstride * n); NEED(phs, 3 * P.kstride * n);
+    check(P.kstride > std::max({P.km[0], P.km[1], P.km[2]}), when + ": phase tables too short");
+    if (c.recip) check(S.sp && S.spg, when + ": no particle mesh");
+#undef NEED
+#undef SAME
+}
+
+// A, then B with its k-th allocation failing, then A and B again
+void elec_failures()
+{
+    for (int a = -1; a < NCALLS; ++a)
+        for (int b = 0; b < NCALLS; ++b)
+            for (long k = 0;; ++k) {
+                ElecState S, RA, RB;
+                const std::string when = std::string(a < 0 ? "new state" : calls[a].name) + ", then " + calls[b].name +
+                                         " without allocation " + std::to_string(k);
+                fail_at = -1;
+                check(configure(RB, calls[b]) == 0, when + ": reference refused");
+                if (a >= 0) {
+                    check(configure(RA, calls[a]) == 0, when + ": reference refused");
+                    check(configure(S, calls[a]) == 0, when + ": first call refused");
+                }
+                fail_at = nalloc + k;
+                const int rc = configure(S, calls[b]);
+                const bool reached = nalloc > fail_at;
+                fail_at = -1;
+                check((rc != 0) == reached, when + ": returned " + std::to_string(rc));
+                if (a >= 0) {
+                    check(configure(S, calls[a]) == 0, when + ": the call that follows is refused");
+                    complete(S, RA, calls[a], when + ", then " + calls[a].name);
+                }
+                check(configure(S, calls[b]) == 0, when + ": the repeated call is refused");
+                complete(S, RB, calls[b], when + ", repeated");
+                elec_release(S);
+                elec_release(RA);
+                elec_release(RB);
+                if (!reached) break;
+            }
+    check(live.empty(), std::to_string(live.size()) + " blocks left");
+}
+
+}  // namespace
+
+int main(int argc, char** argv)
+{
+    const std::string what = argc > 1 ? argv[1] : "";
+    if (what == "elec_failures") elec_failures();
+    else check(false, "no such check: " + what);
+    if (!wrong) printf("ok\n");
+    return wrong != 0;
+}
