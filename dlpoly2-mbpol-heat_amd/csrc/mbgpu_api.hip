@@ -317,10 +317,14 @@ int alloc_fixed(mbgpu_ctx* c)
     return 0;
 }
 
+// Room for nd dimers and nt trimers.  A capacity is 0 while its buffers are freed and allocated again,
+// so that after a failed allocation clusters_ready is false and the next evaluation comes back here.
 int ensure_clusters(mbgpu_ctx* c, long nd, long nt)
 {
     MbBuffers& B = c->B;
     if (nd > B.dcap) {
+        const long cap = std::max<long>(nd + nd / 2, 1024);
+        B.dcap = 0;
         dfree(B.dimers);
         dfree(B.clus2);
         dfree(B.xv2);
@@ -328,16 +332,18 @@ int ensure_clusters(mbgpu_ctx* c, long nd, long nt)
         dfree(B.e2);
         dfree(B.g2);
         dfree(B.s2);
-        B.dcap = std::max<long>(nd + nd / 2, 1024);
-        HIPCHK(dalloc(&B.dimers, (size_t)2 * B.dcap));
-        HIPCHK(dalloc(&B.clus2, (size_t)18 * B.dcap));
-        HIPCHK(dalloc(&B.xv2, (size_t)31 * B.dcap));
-        HIPCHK(dalloc(&B.part2, (size_t)pip2b_nslices() * 32 * B.dcap));
-        HIPCHK(dalloc(&B.e2, B.dcap));
-        HIPCHK(dalloc(&B.g2, (size_t)18 * B.dcap));
-        HIPCHK(dalloc(&B.s2, (size_t)3 * B.dcap));
+        HIPCHK(dalloc(&B.dimers, (size_t)2 * cap));
+        HIPCHK(dalloc(&B.clus2, (size_t)18 * cap));
+        HIPCHK(dalloc(&B.xv2, (size_t)31 * cap));
+        HIPCHK(dalloc(&B.part2, (size_t)pip2b_nslices() * 32 * cap));
+        HIPCHK(dalloc(&B.e2, cap));
+        HIPCHK(dalloc(&B.g2, (size_t)18 * cap));
+        HIPCHK(dalloc(&B.s2, (size_t)3 * cap));
+        B.dcap = cap;
     }
     if (nt > B.tcap) {
+        const long cap = std::max<long>(nt + nt / 2, 1024);
+        B.tcap = 0;
         dfree(B.trimers);
         dfree(B.clus3);
         dfree(B.xv3);
@@ -345,16 +351,17 @@ int ensure_clusters(mbgpu_ctx* c, long nd, long nt)
         dfree(B.e3);
         dfree(B.g3);
         dfree(B.s3);
-        B.tcap = std::max<long>(nt + nt / 2, 1024);
-        HIPCHK(dalloc(&B.trimers, (size_t)3 * B.tcap));
-        HIPCHK(dalloc(&B.clus3, (size_t)27 * B.tcap));
-        HIPCHK(dalloc(&B.xv3, (size_t)36 * B.tcap));
-        HIPCHK(dalloc(&B.part3, (size_t)pip3b_nslices() * 37 * B.tcap));
-        HIPCHK(dalloc(&B.e3, B.tcap));
-        HIPCHK(dalloc(&B.g3, (size_t)27 * B.tcap));
-        HIPCHK(dalloc(&B.s3, (size_t)3 * B.tcap));
+        HIPCHK(dalloc(&B.trimers, (size_t)3 * cap));
+        HIPCHK(dalloc(&B.clus3, (size_t)27 * cap));
+        HIPCHK(dalloc(&B.xv3, (size_t)36 * cap));
+        HIPCHK(dalloc(&B.part3, (size_t)pip3b_nslices() * 37 * cap));
+        HIPCHK(dalloc(&B.e3, cap));
+        HIPCHK(dalloc(&B.g3, (size_t)27 * cap));
+        HIPCHK(dalloc(&B.s3, (size_t)3 * cap));
+        B.tcap = cap;
     }
     if (B.mixed && (B.fcap2 != B.dcap || B.fcap3 != B.tcap)) {
+        B.fcap2 = B.fcap3 = 0;
         dfree(B.xv2f);
         dfree(B.part2f);
         dfree(B.xv3f);
@@ -368,11 +375,17 @@ int ensure_clusters(mbgpu_ctx* c, long nd, long nt)
     }
     const int nblk = (int)((B.dcap + 127) / 128 + (B.tcap + 127) / 128 + (B.natms + 255) / 256 + 8);
     if (nblk > B.nblk_cap) {
+        B.nblk_cap = 0;
         dfree(B.blk);
-        B.nblk_cap = nblk;
         HIPCHK(dalloc(&B.blk, (size_t)8 * nblk));
+        B.nblk_cap = nblk;
     }
     return 0;
+}
+
+bool clusters_ready(const MbBuffers& B)
+{
+    return B.dcap > 0 && B.tcap > 0 && B.nblk_cap > 0 && (!B.mixed || (B.fcap2 == B.dcap && B.fcap3 == B.tcap));
 }
 
 // Build the lists and size the cluster buffers; returns nd, nt through the context.
@@ -387,7 +400,7 @@ int build_lists(mbgpu_ctx* c)
             return fail(-1, "%s", err.c_str());
     }
     for (int attempt = 0; attempt < 3; ++attempt) {
-        if (B.dcap == 0 && ensure_clusters(c, 1024, 1024)) return -1;
+        if (!clusters_ready(B) && ensure_clusters(c, 1024, 1024)) return -1;
         int rc = mb_launch_lists(B, c->geom, c->stream);
         if (rc) return fail(rc, "list kernels failed: %s", hipGetErrorString((hipError_t)rc));
         int cnt[4];
@@ -850,7 +863,9 @@ int mbgpu_set_precision(mbgpu_ctx* c, int mode)
     if (mode < 0 || mode > 3)
         return fail(-1, "precision mode %d: bit 0 = FP32 2B polynomial, bit 1 = FP32 3B polynomial", mode);
     MbBuffers& B = c->B;
-    if (mode != 0 && !B.cs2f) {
+    if (mode != 0 && !B.have_csf) {
+        dfree(B.cs2f);   // (of a call in which an allocation failed)
+        dfree(B.cs3f);
         const int l2 = pip2b_stream_len(), l3 = pip3b_stream_len();
         std::vector<float> f2(l2), f3(l3);
         for (int i = 0; i < l2; ++i) f2[i] = (float)pip2b_stream_values()[i];
@@ -859,9 +874,14 @@ int mbgpu_set_precision(mbgpu_ctx* c, int mode)
         HIPCHK(dalloc(&B.cs3f, l3));
         HIPCHK(hipMemcpy(B.cs2f, f2.data(), sizeof(float) * l2, hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(B.cs3f, f3.data(), sizeof(float) * l3, hipMemcpyHostToDevice));
+        B.have_csf = 1;
     }
+    const int before = B.mixed;
     B.mixed = mode;
-    if (mode != 0 && B.dcap > 0 && ensure_clusters(c, B.dcap, B.tcap)) return -1;
+    if (mode != 0 && B.dcap > 0 && ensure_clusters(c, B.dcap, B.tcap)) {
+        B.mixed = before;   // (an error changes nothing)
+        return -1;
+    }
     return 0;
 }
 
@@ -1058,7 +1078,7 @@ int evaluate_impl(mbgpu_ctx* c, int imcon, const double cell[9], int nttm2, cons
     bool fused_ran = false;
     // one enqueue (a graph replay once captured) when every buffer has been sized by an
     // evaluation through the separate entries
-    if (B.dcap > 0 && B.nblk_cap > 0 && gb > 0) {
+    if (clusters_ready(B) && gb > 0) {
         const int* spf = c->el.recip && c->el.sp && imcon != 0 ? c->el.sp->flag : nullptr;
         const void* ptrs[18] = {listttm2_dev, x_dev, y_dev, z_dev, dip_dev, vx_dev, vy_dev, vz_dev, e_kin_dev,
                                 c->dep, c->dw, c->dsew, spf, c->dpk, fx_dev, fy_dev, fz_dev, fsite_dev};
@@ -1619,6 +1639,7 @@ int mbgpu_ring_transform_dev(mbgpu_ctx* c, int nbead, long ncoord, const double*
     if (in_dev == out_dev) return fail(-1, "the transform cannot work in place");
     const long need = (long)nbead * nbead;
     if (c->ring_m_cap < need) {
+        c->ring_m_cap = 0;
         dfree(c->ring_m);
         HIPCHK(dalloc(&c->ring_m, (size_t)need));
         c->ring_m_cap = need;
@@ -1642,6 +1663,7 @@ int mbgpu_ring_spring_dev(mbgpu_ctx* c, int nbead, int natom, double coeff, doub
     if (!(force_scale != 0.0)) return fail(-1, "force_scale must be nonzero");
     const long need = 2L * nbead * ((natom + 255) / 256);
     if (c->ring_blk_cap < need) {
+        c->ring_blk_cap = 0;
         dfree(c->ring_blk);
         HIPCHK(dalloc(&c->ring_blk, (size_t)need));
         c->ring_blk_cap = need;

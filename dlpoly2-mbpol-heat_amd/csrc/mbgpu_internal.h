@@ -115,6 +115,7 @@ struct MbBuffers {
     // mixed precision: FP32 variables, slice partials and coefficient streams for the
     // polynomial kernels (the slice sums, chain rule and accumulation stay FP64)
     int mixed = 0;
+    int have_csf = 0;              // the FP32 coefficient streams are filled
     float *xv2f = nullptr, *part2f = nullptr, *cs2f = nullptr;
     float *xv3f = nullptr, *part3f = nullptr, *cs3f = nullptr;
     long fcap2 = 0, fcap3 = 0;     // cluster capacities of the FP32 buffers

@@ -461,6 +461,7 @@ void water_release(WaterState& S)
     dfree(B.vvv); dfree(B.ggg); dfree(B.psc); dfree(B.pcm); dfree(B.pidx); dfree(B.pidxm); dfree(B.scal);
     cells_free(S.cells);
     S.nw = 0;
+    B.ngrid = 0;
     S.have_tab = false;
     S.ready = false;
 }
@@ -542,12 +543,15 @@ int water_configure(WaterState& S, int nw, const CellGeom& g, const double* cell
                                 p->a6[2], p->c8[0], p->c8[1], p->c8[2], p->a8[0], p->a8[1], p->a8[2]};
         const double dlrpot = p->rvdw / (double)(mxgrid - 4);
         if (!S.have_tab || memcmp(key, S.tab_key, sizeof key) != 0) {
+            // (neither key stands while its buffers go and come: see the electrostatics' plans)
+            S.have_tab = false;
             if (B.ngrid != mxgrid + 3) {
+                B.ngrid = 0;
                 dfree(B.vvv);
                 dfree(B.ggg);
+                WCHK(dalloc(&B.vvv, (size_t)3 * (mxgrid + 3)));
+                WCHK(dalloc(&B.ggg, (size_t)3 * (mxgrid + 3)));
                 B.ngrid = mxgrid + 3;
-                WCHK(dalloc(&B.vvv, (size_t)3 * B.ngrid));
-                WCHK(dalloc(&B.ggg, (size_t)3 * B.ngrid));
             }
             const int nk = 3 * B.ngrid;
             hipLaunchKernelGGL(k_wt_table, dim3((nk + 255) / 256), dim3(256), 0, s, mxgrid, B.ngrid, dlrpot,

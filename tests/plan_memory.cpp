@@ -246,12 +246,108 @@ void elec_failures()
     check(live.empty(), std::to_string(live.size()) + " blocks left");
 }
 
+// ----------------------------------------------- water terms, MB-pol (and its precisions) ----
+int configure_water(WaterState& S, double rcut)
+{
+    mbgpu_water_params p = {};
+    p.rcut = p.rvdw = rcut;
+    for (int t = 0; t < 3; ++t) {
+        p.c6[t] = 1000.0;
+        p.a6[t] = p.a8[t] = 9.0;
+    }
+    p.dispersion = p.ps_monomer = 1;
+    CellGeom g = {};
+    g.imcon = 1;
+    const double cell[9] = {12, 0, 0, 0, 12, 0, 0, 0, 12};
+    std::string err;
+    return water_configure(S, 8, g, cell, &p, nullptr, err);
+}
+
+void water_failures()
+{
+    const double cut[2] = {1.0, 1.5};
+    for (int first = 0; first < 2; ++first)
+        for (long k = 0;; ++k) {
+            WaterState S;
+            const std::string when = std::string(first ? "second" : "first") + " cut-off without allocation " +
+                                     std::to_string(k);
+            if (first) check(configure_water(S, cut[0]) == 0, when + ": first call refused");
+            fail_at = nalloc + k;
+            const int rc = configure_water(S, cut[first]);
+            const bool reached = nalloc > fail_at;
+            fail_at = -1;
+            check((rc != 0) == reached, when + ": returned " + std::to_string(rc));
+            for (int again = 0; again < 2; ++again) {
+                check(configure_water(S, cut[again]) == 0, when + ": a call that follows is refused");
+                const size_t table = sizeof(double) * 3 * S.P.ngrid, nr = 24;
+                check(S.P.ngrid == (int)(cut[again] / 0.0001 + 0.5) + 7 && size_of(S.B.vvv) == table &&
+                          size_of(S.B.ggg) == table,
+                      when + ": tables of " + std::to_string(size_of(S.B.vvv)) + " and " +
+                          std::to_string(size_of(S.B.ggg)) + " bytes, not " + std::to_string(table));
+                check(size_of(S.B.mono) == 13 * nr * 8 && size_of(S.B.wsc) && size_of(S.B.asc) && size_of(S.B.fw) &&
+                          size_of(S.B.eout) && size_of(S.B.wout) && size_of(S.B.psc) && size_of(S.B.pcm) &&
+                          size_of(S.B.pidx) && size_of(S.B.pidxm) && size_of(S.B.scal),
+                      when + ": a buffer is missing");
+            }
+            water_release(S);
+            if (!reached) break;
+        }
+    check(live.empty(), std::to_string(live.size()) + " blocks left");
+}
+
+int mbpol(mbgpu_ctx* c)
+{
+    const double cell[9] = {12, 0, 0, 0, 12, 0, 0, 0, 12};
+    const int list[6] = {1, 2, 3, 4, 5, 6};
+    double x[8] = {}, f[8] = {}, e = 0.0, v = 0.0, s[9] = {};
+    return mbgpu_mbpol_forces(c, 1, cell, 6, list, x, x, x, f, f, f, &e, &v, s);
+}
+
+std::multiset<size_t> sizes()
+{
+    std::multiset<size_t> r;
+    for (auto& b : live) r.insert(b.second.size);
+    return r;
+}
+
+// MB-pol's cluster buffers, first in FP64 and then with the FP32 polynomials: whatever fails, the
+// calls that follow hold the same buffers as in a context where nothing failed
+void mbpol_failures()
+{
+    for (int step = 0; step < 3; ++step) {
+        // 0: the first evaluation, 1: the change of precision after it, 2: before it
+        auto call = [&](mbgpu_ctx* c, int s) { return s == 0 ? mbpol(c) : mbgpu_set_precision(c, 3); };
+        std::multiset<size_t> want;
+        for (long k = -1;; ++k) {
+            const std::string when = "MB-pol, step " + std::to_string(step) + " without allocation " + std::to_string(k);
+            mbgpu_ctx* c = mbgpu_create(2, 8);
+            if (step == 1) check(mbpol(c) == 0, when + ": evaluation refused");
+            fail_at = k < 0 ? -1 : nalloc + k;
+            const int rc = call(c, step);
+            const bool reached = k >= 0 && nalloc > fail_at;
+            fail_at = -1;
+            check((rc != 0) == reached, when + ": returned " + std::to_string(rc));
+            check(mbpol(c) == 0, when + ": the evaluation that follows is refused");
+            if (step) check(mbgpu_set_precision(c, 3) == 0, when + ": the precision is refused again");
+            check(mbpol(c) == 0, when + ": the last evaluation is refused");
+            if (k < 0) want = sizes();
+            else check(sizes() == want, when + ": " + std::to_string(live.size()) + " buffers, not the " +
+                                            std::to_string(want.size()) + " of an undisturbed context");
+            mbgpu_destroy(c);
+            check(live.empty(), when + ": blocks left");
+            if (k >= 0 && !reached) break;
+        }
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "elec_failures") elec_failures();
+    else if (what == "water_failures") water_failures();
+    else if (what == "mbpol_failures") mbpol_failures();
     else check(false, "no such check: " + what);
     if (!wrong) printf("ok\n");
     return wrong != 0;

@@ -32,5 +32,6 @@ def run(program, *args, env=()):
     assert r.returncode == 0 and r.stdout.strip() == "ok", (r.stdout + r.stderr)[:4000]
 
 
-def test_failed_allocations_of_the_electrostatics(program):
-    run(program, "elec_failures")
+@pytest.mark.parametrize("part", ["elec", "water", "mbpol"])
+def test_failed_allocations(program, part):
+    run(program, part + "_failures")
