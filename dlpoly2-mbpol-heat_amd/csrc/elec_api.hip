@@ -106,7 +106,7 @@ void free_buffers(ElecBuffers& E)
 // per 16 waters), or SOR's 2 per 256 rows
 int final_partials(int n, int nw, int nkb) { return 8 * nkb + 8 * n + 24 * ((nw + 15) / 16) + 2 * (n / 256 + 1); }
 
-// A plan's key (S.nw, E.capA, S.tab_alpha, S.k_alpha, E.kstride) says that its buffers are there and
+// A plan's key (S.nw, E.capA, S.tab_alpha, S.k_alpha, S.direct, E.kstride) says that its buffers are there and
 // hold it: each set-up below clears the key before the first buffer goes and sets it after the last
 // one is filled, so that a call that fails in between leaves nothing a later call would take for whole.
 
@@ -348,6 +348,7 @@ int build_klist(ElecState& S, const double* cell, const int* kmax, double alpha,
         mmin = -kmax[1];
     }
     S.k_alpha = -1.0;
+    S.direct = false;
     dfree(E.kv);
     dfree(E.runs);
     dfree(E.runk);
@@ -406,16 +407,22 @@ namespace {
 
 // An isolated cluster (imcon 0): no reciprocal space.  The buffers the k-sum set-up would
 // size are sized for the site count alone: the field partials (one chunk of 6 components)
-// and the block partials of the final passes.
+// and the block partials of the final passes.  Kept from call to call (S.direct) until a periodic
+// call sizes them for its k list: freed and allocated again in each, they made every cluster
+// evaluation wait for the whole device, twice, and capture its graph again whenever another
+// thread had taken the blocks in between.
 int alloc_direct(ElecState& S, std::string& err)
 {
     ElecBuffers& E = S.E;
-    S.k_alpha = -1.0;   // a later periodic call builds its k list
-    dfree(E.Fpart);
-    ECHK(dalloc(&E.Fpart, (size_t)6 * E.n));
-    dfree(E.blk);
-    E.nblk = final_partials(E.n, S.nw, (E.n + 3) / 4);
-    ECHK(dalloc(&E.blk, (size_t)E.nblk));
+    if (!S.direct) {
+        S.k_alpha = -1.0;   // a later periodic call builds its k list
+        dfree(E.Fpart);
+        dfree(E.blk);
+        ECHK(dalloc(&E.Fpart, (size_t)6 * E.n));
+        E.nblk = final_partials(E.n, S.nw, (E.n + 3) / 4);
+        ECHK(dalloc(&E.blk, (size_t)E.nblk));
+        S.direct = true;
+    }
     E.K = E.nrun = 0;
     E.kchunks = E.fchunks = 1;
     E.rpc = 0;
@@ -440,6 +447,7 @@ void elec_release(ElecState& S)
     S.spg = nullptr;
     cells_free(S.cells);
     S.tab_alpha = S.k_alpha = -1.0;
+    S.direct = false;
     S.nw = 0;
     S.ready = false;
 }

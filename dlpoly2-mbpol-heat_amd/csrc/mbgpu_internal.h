@@ -283,6 +283,7 @@ struct ElecState {
     double k_cell[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};     // key of the k-vector list
     int k_kmax[3] = {0, 0, 0};
     double k_alpha = -1.0, k_rcut = -1.0;
+    bool direct = false;                // E.Fpart and E.blk are those of an isolated cluster
     double scal[48];                    // host copy of the reduced scalars
     double* hpk = nullptr;              // pinned host copy of E.pk (EL_PK_N doubles)
     double out[20];                     // eng_ew1p, eng_ew2p, eng_ew3p, eng_polar, eng_cpe, vir_cpe,

@@ -246,6 +246,27 @@ void elec_failures()
     check(live.empty(), std::to_string(live.size()) + " blocks left");
 }
 
+// A call with the parameters of the one before frees and allocates nothing.
+void elec_repeats()
+{
+    for (int a = -1; a < NCALLS; ++a)
+        for (int b = 0; b < NCALLS; ++b) {
+            ElecState S;
+            const std::string when = std::string(a < 0 ? "new state" : calls[a].name) + ", then " + calls[b].name;
+            if (a >= 0) check(configure(S, calls[a]) == 0, when + ": first call refused");
+            check(configure(S, calls[b]) == 0, when + ": refused");
+            std::vector<unsigned char> key, key2;
+            elec_key_append(S, 1, 1, 10, key);
+            const long n0 = nalloc, f0 = nfree;
+            check(configure(S, calls[b]) == 0, when + ": refused again");
+            elec_key_append(S, 1, 1, 10, key2);
+            check(nalloc == n0 && nfree == f0, when + ": " + std::to_string(nalloc - n0) + " allocations and " +
+                                                  std::to_string(nfree - f0) + " frees in a repeated call");
+            check(key == key2, when + ": a repeated call has another graph key");
+            elec_release(S);
+        }
+}
+
 // ----------------------------------------------- water terms, MB-pol (and its precisions) ----
 int configure_water(WaterState& S, double rcut)
 {
@@ -346,6 +367,7 @@ int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "elec_failures") elec_failures();
+    else if (what == "elec_repeats") elec_repeats();
     else if (what == "water_failures") water_failures();
     else if (what == "mbpol_failures") mbpol_failures();
     else check(false, "no such check: " + what);

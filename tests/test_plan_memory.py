@@ -4,6 +4,8 @@ libmbgpu.so over a host stand-in of the runtime's memory calls; nothing is launc
 * A device allocation that fails, at every place where one is made, is an error of that call
   alone: the calls that follow, with the parameters before or the same ones again, find every
   buffer, large enough and with their own plan's contents.
+* A set-up with the parameters of the one before makes no allocation and no free, and the key of
+  the captured evaluation stays as it is.
 """
 import os
 import shutil
@@ -35,3 +37,7 @@ def run(program, *args, env=()):
 @pytest.mark.parametrize("part", ["elec", "water", "mbpol"])
 def test_failed_allocations(program, part):
     run(program, part + "_failures")
+
+
+def test_repeated_calls_allocate_nothing(program):
+    run(program, "elec_repeats")
