@@ -18,7 +18,7 @@ namespace {
 
 struct Block {
     size_t size;
-    int fill;                          // last byte set over all of it, -1: none
+    bool filled;                       // 0xff bytes were once set over all of it
 };
 std::map<const void*, Block> live;
 long nalloc = 0, nfree = 0, fail_at = -1;   // allocations made, frees, the allocation that fails
@@ -32,7 +32,7 @@ hipError_t hipMalloc(void** p, size_t n)
     *p = nullptr;
     if (nalloc++ == fail_at) return hipErrorOutOfMemory;
     *p = calloc(n, 1);
-    live[*p] = Block{n, -1};
+    live[*p] = Block{n, false};
     return hipSuccess;
 }
 hipError_t hipFree(void* p)
@@ -60,7 +60,7 @@ hipError_t hipMemset(void* p, int v, size_t n)
 {
     memset(p, v, n);
     auto b = live.find(p);
-    if (b != live.end() && b->second.size == n) b->second.fill = v;
+    if (b != live.end() && b->second.size == n && v == 0xff) b->second.filled = true;
     return hipSuccess;
 }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind)
@@ -267,6 +267,27 @@ void elec_repeats()
         }
 }
 
+// MBGPU_POISON=1 (set by the caller): every buffer but the integer ones is filled when it is made.
+void elec_poison()
+{
+    for (const Call& c : calls) {
+        ElecState S;
+        check(configure(S, c) == 0, std::string(c.name) + ": refused");
+        const ElecBuffers& E = S.E;
+        std::set<const void*> ints = {E.cntA, E.cntP, E.nbrA, E.nbrP, E.err, E.runs, E.runk, E.rs_pair, E.rs_kpos,
+                                      S.cells.key, S.cells.sidx, S.cells.start};
+        if (S.sp) ints.insert({S.sp->gi, S.sp->bin_off, S.sp->bin_site, S.sp->flag});
+        const std::map<const void*, const char*> names = {{E.tens, "tens"}, {E.pht, "pht"}, {E.rs_ak, "rs_ak"}};
+        for (auto& b : live) {
+            auto n = names.find(b.first);
+            check(b.second.filled || ints.count(b.first),
+                  std::string(c.name) + ": " + (n == names.end() ? "a buffer" : n->second) + " of " +
+                      std::to_string(b.second.size) + " bytes is not filled");
+        }
+        elec_release(S);
+    }
+}
+
 // ----------------------------------------------- water terms, MB-pol (and its precisions) ----
 int configure_water(WaterState& S, double rcut)
 {
@@ -368,6 +389,7 @@ int main(int argc, char** argv)
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "elec_failures") elec_failures();
     else if (what == "elec_repeats") elec_repeats();
+    else if (what == "elec_poison") elec_poison();
     else if (what == "water_failures") water_failures();
     else if (what == "mbpol_failures") mbpol_failures();
     else check(false, "no such check: " + what);

@@ -6,6 +6,7 @@ libmbgpu.so over a host stand-in of the runtime's memory calls; nothing is launc
   buffer, large enough and with their own plan's contents.
 * A set-up with the parameters of the one before makes no allocation and no free, and the key of
   the captured evaluation stays as it is.
+* MBGPU_POISON=1 fills every buffer of floating-point numbers, whatever their element type.
 """
 import os
 import shutil
@@ -41,3 +42,7 @@ def test_failed_allocations(program, part):
 
 def test_repeated_calls_allocate_nothing(program):
     run(program, "elec_repeats")
+
+
+def test_poison_fills_every_floating_point_buffer(program):
+    run(program, "elec_poison", env={"MBGPU_POISON": "1"})
