@@ -35,8 +35,9 @@ def slot_bytes(nw, cluster=False):
     """Device memory of a slot of nw waters (estimate from the buffer sizes: MB-pol cluster
     partials dominate in a periodic box, about 0.55 MB per water at liquid density, plus
     fixed tables).  An isolated cluster (imcon 0) takes every site pair into its
-    electrostatics rows: (4 nw)^2 dipole tensors and partner indices, 56 bytes a pair."""
-    return int(0.6 * MB * nw + 24 * MB + (56 * (4 * nw) ** 2 if cluster else 0))
+    electrostatics rows: (4 nw)^2 pairs of radial factors and two partner indices, 24 bytes
+    a pair."""
+    return int(0.6 * MB * nw + 24 * MB + (24 * (4 * nw) ** 2 if cluster else 0))
 
 
 def _pool_key(box):

@@ -288,6 +288,16 @@ void elec_poison()
     }
 }
 
+// Prints the bytes of the neighbour rows of a cluster of nw waters, every pair within rcut.
+void cluster_rows(int nw)
+{
+    ElecState S;
+    const Call c = {"cluster", nw, 0, 40.0, 0.0, 40.0, {1, 1, 1}, 0};
+    check(configure(S, c) == 0, "refused");
+    printf("%zu\n", size_of(S.E.nbrA) + size_of(S.E.nbrP) + size_of(S.E.tens));
+    elec_release(S);
+}
+
 // ----------------------------------------------- water terms, MB-pol (and its precisions) ----
 int configure_water(WaterState& S, double rcut)
 {
@@ -390,6 +400,7 @@ int main(int argc, char** argv)
     if (what == "elec_failures") elec_failures();
     else if (what == "elec_repeats") elec_repeats();
     else if (what == "elec_poison") elec_poison();
+    else if (what == "cluster_rows" && argc > 2) cluster_rows(atoi(argv[2]));
     else if (what == "water_failures") water_failures();
     else if (what == "mbpol_failures") mbpol_failures();
     else check(false, "no such check: " + what);

@@ -6,8 +6,10 @@ libmbgpu.so over a host stand-in of the runtime's memory calls; nothing is launc
   buffer, large enough and with their own plan's contents.
 * A set-up with the parameters of the one before makes no allocation and no free, and the key of
   the captured evaluation stays as it is.
+* The server's estimate of a cluster's memory counts its neighbour rows as large as they are.
 * MBGPU_POISON=1 fills every buffer of floating-point numbers, whatever their element type.
 """
+import importlib
 import os
 import shutil
 import subprocess
@@ -46,3 +48,10 @@ def test_repeated_calls_allocate_nothing(program):
 
 def test_poison_fills_every_floating_point_buffer(program):
     run(program, "elec_poison", env={"MBGPU_POISON": "1"})
+
+
+@pytest.mark.parametrize("nw", [16, 112, 704])
+def test_server_counts_the_rows_of_a_cluster(program, nw):
+    serve = importlib.import_module("dlpoly2-mbpol-heat_amd.serve")
+    r = subprocess.run([program, "cluster_rows", str(nw)], capture_output=True, text=True, timeout=60, check=True)
+    assert serve.slot_bytes(nw, cluster=True) - serve.slot_bytes(nw) == int(r.stdout.split()[0])
