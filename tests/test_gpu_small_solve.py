@@ -1,7 +1,7 @@
 """The solve of the dipoles of an isolated cluster, at the sizes where its kernels change or end:
 one launch holds up to 21 waters (63 rows of 16 lanes, 7 waters to a wavefront, so 1, 7, 8, 21),
-22 take the launches per iteration, and rows of 512 partners and more (128 waters) are shared by
-four wavefronts.  The pair and per-water passes run at the same odd counts.
+22 take the launches per iteration, and rows with room for 512 partners and more (4 sites a water,
+rounded up to 64: 112 waters 448, 113 waters 512) are shared by four wavefronts.  The pair and per-water passes run at the same odd counts.
 
 Bars as test_gpu_cluster: both sides sum the same terms in FP64 in different orders, the solves
 stop below the same RMS step.
@@ -16,7 +16,7 @@ from test_gpu_elec import run_gpu
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nw", [1, 2, 7, 8, 21, 22, 129])
+@pytest.mark.parametrize("nw", [1, 2, 7, 8, 21, 22, 112, 113, 129])
 def test_cluster_sizes(pkg, waterbox, nw):
     box = waterbox.make_cluster(nw, seed=5)
     p = pkg.elec_params.for_cluster(box.L)
