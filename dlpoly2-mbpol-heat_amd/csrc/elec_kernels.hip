@@ -12,12 +12,14 @@
 // per-site sum is owned by one thread or one wavefront and summed in a fixed order):
 //   * real space: full neighbour rows per site (both directions of each pair), so that a
 //     wavefront owns a site's row; the Thole-damped dipole tensors of the polarizable
-//     pairs are built once per evaluation and reused by every solver iteration;
-//   * reciprocal space: the k vectors are grouped into runs of consecutive n at fixed
-//     (l, m); exp(i k.r_j) comes from per-site tables of exp(i l a*.r_j) (a* a reciprocal
-//     vector) and a complex recurrence along n.  Structure factors are k-parallel with a
-//     site split (partials summed in a fixed order); fields and forces are site-parallel
-//     with a k split (likewise);
+//     pairs are kept as two radial factors, built once per evaluation and read by every
+//     solver iteration;
+//   * reciprocal space: exp(i k.r_j) comes from per-site tables of exp(i l a*.r_j) (a* a
+//     reciprocal vector).  The solver's structure factors and fields are FP64 matrix
+//     products over groups of 16 (l, m) pairs and tiles of 8 n, split over chunks of sites
+//     and groups of pairs (partials summed in a fixed order); the final forces and stresses
+//     are site-parallel over runs of consecutive n at fixed (l, m), with a complex
+//     recurrence along n and a split over chunks of runs (likewise);
 //   * the solver loop runs on the device; a done flag set by the convergence check turns
 //     the remaining kernels of a batch of iterations into no-ops.
 #include <math.h>
@@ -30,7 +32,6 @@
 #define R4PIE0 138935.4835            // dl_params.inc
 #define SQRPI 1.7724538509055159      // dl_params.inc
 #define TWOPI (2.0 * 3.141592653589793)
-#define EL_RUN 8                      // k vectors per run (consecutive n)
 
 namespace {
 
@@ -153,10 +154,6 @@ __device__ __forceinline__ bool cg_step(const ElecDev& P, int it, int nb, const 
 
 __device__ __forceinline__ int water_of(const ElecDev& P, int i) { return i < P.nreal ? i / 3 : i - P.nreal; }
 
-__device__ __forceinline__ double site_polr(const ElecDev& P, int i)
-{
-    return i >= P.nreal ? P.polr[2] : ((i % 3) == 0 ? P.polr[0] : P.polr[1]);
-}
 __device__ __forceinline__ double site_polr2(const ElecDev& P, int i)
 {
     return i >= P.nreal ? P.polr2[2] : ((i % 3) == 0 ? P.polr2[0] : P.polr2[1]);

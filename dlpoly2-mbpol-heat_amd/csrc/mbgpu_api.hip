@@ -1080,8 +1080,8 @@ int evaluate_impl(mbgpu_ctx* c, int imcon, const double cell[9], int nttm2, cons
     // evaluation through the separate entries
     if (clusters_ready(B) && gb > 0) {
         const int* spf = c->el.recip && c->el.sp && imcon != 0 ? c->el.sp->flag : nullptr;
-        const void* ptrs[18] = {listttm2_dev, x_dev, y_dev, z_dev, dip_dev, vx_dev, vy_dev, vz_dev, e_kin_dev,
-                                c->dep, c->dw, c->dsew, spf, c->dpk, fx_dev, fy_dev, fz_dev, fsite_dev};
+        const void* ptrs[15] = {listttm2_dev, x_dev, y_dev, z_dev, dip_dev, vx_dev, vy_dev, vz_dev, e_kin_dev,
+                                spf, c->dpk, fx_dev, fy_dev, fz_dev, fsite_dev};
         const char* gv = getenv("MBGPU_GRAPHS");
         const bool graphs = c->el.graphs && !(gv && atoi(gv) == 0);
         hipStream_t a = c->stream, b = c->el_stream;
@@ -1090,7 +1090,7 @@ int evaluate_impl(mbgpu_ctx* c, int imcon, const double cell[9], int nttm2, cons
         auto part_tail = [&] { return full_enqueue_tail(c, vx_dev, vy_dev, vz_dev, e_kin_dev, spf, b); };
         bool replay = false;
         if (graphs) {
-            std::vector<unsigned char> key = full_key(c, ep, gb, ptrs, 18);
+            std::vector<unsigned char> key = full_key(c, ep, gb, ptrs, 15);
             if (!c->fexec[0] || key != c->fkey) {
                 for (hipGraphExec_t& g : c->fexec)
                     if (g) (void)hipGraphExecDestroy(g);

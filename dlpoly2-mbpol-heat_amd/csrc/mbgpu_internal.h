@@ -152,10 +152,6 @@ struct RsPlan {
 
 #define EL_RUN 8                      // most k of a run of the final site pass
 
-#define EL_RUN 8                      // most k of a run of the final site pass
-
-#define EL_RUN 8                      // most k of a run of the final site pass
-
 // Sums over the wavefront of 24 values per lane: each step halves the values a lane carries
 // (25 exchanges instead of 144 for 24 butterflies).  Returns the sum of value `k` (on every lane
 // whose k is below 24), always added in the same order.
@@ -291,7 +287,7 @@ struct ElecState {
     double tab_alpha = -1.0, tab_rcut = -1.0;           // key of the B-function table
     double k_cell[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};     // key of the k-vector list
     int k_kmax[3] = {0, 0, 0};
-    double k_alpha = -1.0, k_rcut = -1.0;
+    double k_alpha = -1.0;
     bool direct = false;                // E.Fpart and E.blk are those of an isolated cluster
     double scal[48];                    // host copy of the reduced scalars
     double* hpk = nullptr;              // pinned host copy of E.pk (EL_PK_N doubles)
