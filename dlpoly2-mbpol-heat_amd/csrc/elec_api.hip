@@ -628,33 +628,37 @@ const ElecSpme* recip_of(const ElecState& S, ElecSpme& spx, ElecSpme& none)
 }
 }  // namespace
 
-// Solver iterations enqueued between two tests of max_iter once the first batch is done
+// max_iter is tested between batches of iterations: a first one, then batch_step at a time.  A first
+// batch past EL_BATCH iterations neither passes the step that reaches max_iter nor is a place to
+// test it unless it ends with a step: whether a solve is refused does not depend on how far ahead it
+// was enqueued.
 static inline int batch_step(int solver) { return solver == 1 ? 4 : 8; }
-
-// The first batch of a solve that is expected to take `last` iterations: last + 2.  max_iter is
-// tested between batches; past EL_BATCH iterations a batch ends where solving on from there in steps
-// would (whole steps, none begun at or after max_iter), so whether a solve is refused does not depend
-// on how far ahead it was enqueued.
-static int first_batch(int last, int max_iter, int solver)
+// iterations from n to the end of its step
+static inline int to_step(int n, int solver)
 {
     const int step = batch_step(solver);
-    auto up = [&](int n) { return EL_BATCH + (std::max(n - EL_BATCH, 0) + step - 1) / step * step; };
-    if (last + 2 <= EL_BATCH) return last + 2;
-    return std::min(EL_MAX_BATCH, std::min(up(last + 2), up(max_iter)));
+    return n > EL_BATCH ? (step - (n - EL_BATCH) % step) % step : 0;
+}
+// the first batch of a solve that is expected to take `last` iterations
+static inline int first_batch(int last, int max_iter, int solver)
+{
+    const int n = std::max(EL_BATCH, std::min(max_iter, EL_MAX_BATCH));
+    return std::min(last + 2, std::min(EL_MAX_BATCH, n + to_step(n, solver)));
 }
 
 // Solver iterations a captured evaluation holds (0 before the first evaluation set a count):
 // first_batch of the last count, or what the present capture holds while that covers the solve,
 // is not far too long (iterations past convergence are no-ops of about a microsecond per kernel;
-// a new capture costs more, so counts that drift by one or two do not capture again) and is itself
-// a first_batch.  MBGPU_GRAPH_BATCH=k caps it (a test aid for the continuation after a graph).
+// a new capture costs more, so counts that drift by one or two do not capture again) and is within
+// the first batch of a solve as long.  MBGPU_GRAPH_BATCH=k caps it (a test aid for the continuation
+// after a graph).
 int elec_batch(const ElecState& S, int max_iter, int solver)
 {
     int gb = 0;
     if (S.last_iters > 0) {
         gb = first_batch(S.last_iters, max_iter, solver);
         if (S.gbatch >= S.last_iters && S.gbatch <= S.last_iters + 8 &&
-            S.gbatch == first_batch(S.gbatch - 2, max_iter, solver))
+            S.gbatch <= first_batch(S.gbatch, max_iter, solver))
             gb = S.gbatch;
     }
     if (const char* ev = getenv("MBGPU_GRAPH_BATCH")) gb = gb ? std::min(gb, std::max(1, atoi(ev))) : 0;
@@ -823,13 +827,11 @@ int elec_evaluate(ElecState& S, int max_iter, int distribute, int solver, hipStr
     // with clamped counts, so an overflowed attempt runs in bounds and is simply repeated
     // with larger rows, from the same start dipoles (kept in dip0).
     for (int attempt = from_graph ? -1 : (S.gexec && herr ? 1 : 0); attempt >= 0 || from_graph;) {
-        int launched = 0,
-            batch = S.last_iters > 0 ? first_batch(S.last_iters, max_iter, solver) : (solver == 1 ? 8 : 12);
+        int launched = 0;
         int rc = 0;
         if (from_graph) {
             // continue after the graph's iterations
             launched = S.gbatch;
-            batch = batch_step(solver);
             from_graph = false;
             attempt = -1;
             if (st[2] != 0.0) break;
@@ -845,14 +847,14 @@ int elec_evaluate(ElecState& S, int max_iter, int distribute, int solver, hipStr
                 P.capA = E.capA;
                 P.capP = E.capP;
             }
-            rc = enqueue_attempt(S, sp, solver, attempt == 0, batch, s);
+            launched = S.last_iters > 0 ? first_batch(S.last_iters, max_iter, solver) : (solver == 1 ? 8 : 12);
+            rc = enqueue_attempt(S, sp, solver, attempt == 0, launched, s);
             if (rc) {
                 err = std::string("electrostatics kernels failed: ") + hipGetErrorString((hipError_t)rc);
                 return rc;
             }
-            launched = batch;
-            batch = batch_step(solver);
         }
+        const bool ahead = launched > EL_BATCH;   // a first batch that may end inside a step
         bool overflow = false;
         for (;;) {
             ECHK(readback(true));
@@ -865,13 +867,15 @@ int elec_evaluate(ElecState& S, int max_iter, int distribute, int solver, hipStr
                 err = "induced dipoles became NaN";
                 return -3;
             }
-            if (st[0] >= (double)max_iter) {
+            const int rest = ahead ? to_step(launched, solver) : 0;
+            if (st[0] >= (double)max_iter && rest == 0) {
                 char buf[160];
                 snprintf(buf, sizeof buf, "induced dipoles did not converge in %d iterations (rms change %.3e)",
                          (int)st[0], st[1]);
                 err = buf;
                 return -3;
             }
+            const int batch = rest ? rest : batch_step(solver);
             for (int b = 0; b < batch; ++b) {
                 rc = solver == 1 ? el_launch_cg_iteration(E, P, launched, sp, s)
                                  : el_launch_iteration(E, P, launched == 0, sp, s);

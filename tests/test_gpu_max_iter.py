@@ -28,7 +28,7 @@ def test_lower_limit_in_a_warm_context(pkg, waterbox, fused, graphs):
     assert n > 100
     f = s.forces()
     reach = lambda limit: 64 + 8 * ((max(limit - 64, 0) + 7) // 8)     # iterations done at the limit
-    for limit in (10, 64, 65, n - 20, n - 8, n):
+    for limit in (10, 64, 65, n - 20, n - 8, n - 1, n):
         print(f"{n} iterations, max_iter {limit}, one call {fused}, graphs {graphs}", flush=True)
         s.set_params(dataclasses.replace(e, max_iter=limit), pkg.water_params.for_box(box.L))
         if reach(limit) < n:
