@@ -303,7 +303,7 @@ def main():
         return
     if args.hw_queues:
         # HIP's default is 4 hardware queues, which the concurrent legs measured fastest with
-        # (16 configurations: 1060 evaluations/s against 925 with 8 queues and 940 with 16);
+        # (16 configurations: 1620 evaluations/s against 1390 with 8 queues and 1450 with 16);
         # must be set before the HIP runtime starts
         os.environ["GPU_MAX_HW_QUEUES"] = str(args.hw_queues)
     import numpy as np
@@ -384,9 +384,9 @@ def main():
 
     # the same configuration through engine.Slot: one library call per evaluation
     # (mbgpu_evaluate_dev, graph replays, electrostatics beside MB-pol and the water terms),
-    # after the separate entries' context is released: with HIP's 4 hardware queues a
-    # context whose two streams are created while another context's exist measured 1.72 ms
-    # instead of 1.48 ms per evaluation (how the runtime maps streams to queues)
+    # after the separate entries' context is released: how the runtime maps streams to HIP's 4
+    # hardware queues can cost a context created beside another the overlap of its two streams
+    # (none with the present kernels: 1.00 to 1.01 ms per evaluation either way)
     ctx.close()
     engine = importlib.import_module("dlpoly2-mbpol-heat_amd.engine")
     one = engine.Slot(box, solver=1 if args.solver == "cg" else 0)
