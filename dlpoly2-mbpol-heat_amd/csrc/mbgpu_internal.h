@@ -34,6 +34,8 @@ inline hipError_t mbgpu_alloc(T** p, size_t n)
     *p = nullptr;
     if (n == 0) n = 1;
     hipError_t e = hipMalloc((void**)p, n * sizeof(T));
+    // (the caller reports it; left as the runtime's last error it would fail a later launch too)
+    if (e != hipSuccess) (void)hipGetLastError();
     const long serial = mbgpu_alloc_serial();
     if constexpr (mbgpu_is_floating<T>::value) {
         const int how = e == hipSuccess ? mbgpu_poison_this(serial) : 0;

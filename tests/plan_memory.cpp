@@ -22,6 +22,7 @@ struct Block {
 };
 std::map<const void*, Block> live;
 long nalloc = 0, nfree = 0, fail_at = -1;   // allocations made, frees, the allocation that fails
+hipError_t last = hipSuccess;               // the runtime's last error, kept until it is asked for
 int wrong = 0;
 
 }  // namespace
@@ -30,7 +31,7 @@ extern "C" {
 hipError_t hipMalloc(void** p, size_t n)
 {
     *p = nullptr;
-    if (nalloc++ == fail_at) return hipErrorOutOfMemory;
+    if (nalloc++ == fail_at) return last = hipErrorOutOfMemory;
     *p = calloc(n, 1);
     live[*p] = Block{n, false};
     return hipSuccess;
@@ -74,7 +75,12 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
     return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) { return hipSuccess; }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void)
+{
+    const hipError_t e = last;
+    last = hipSuccess;
+    return e;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamCreate(hipStream_t* s)
 {
@@ -232,6 +238,7 @@ void elec_failures()
                 const bool reached = nalloc > fail_at;
                 fail_at = -1;
                 check((rc != 0) == reached, when + ": returned " + std::to_string(rc));
+                check(hipGetLastError() == hipSuccess, when + ": the error is left to the next launch");
                 if (a >= 0) {
                     check(configure(S, calls[a]) == 0, when + ": the call that follows is refused");
                     complete(S, RA, calls[a], when + ", then " + calls[a].name);
