@@ -281,9 +281,11 @@ __global__ __launch_bounds__(64) void k_neighbours(int nw, const double* __restr
         for (int base = 0; base < nw; base += 64) take(base + lane < nw ? base + lane : -1);
     }
     if (lane == 0) {
-        cnt2[i] = n2;
-        cnt2l[i] = n2l;
-        cnt3[i] = n3;
+        // (rows past their capacity set the flag; what follows until the host sees it goes by what
+        // the rows hold)
+        cnt2[i] = min(n2, cap2);
+        cnt2l[i] = min(n2l, cap2);
+        cnt3[i] = min(n3, cap3);
         if (n2 > cap2 || n2l > cap2 || n3 > cap3) atomicOr(err, 1);
     }
 }
@@ -870,27 +872,28 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_water(GatherArgs A)
     const int nA = A.cnt2[w], nB = A.cnt2l[w], nC = A.tcnt[w], nD = min(nleaf, GATHER_MAXLEAF);
     const int ntot = nA + nB + nC + nD;
     for (int it = tid; it < ntot; it += GATHER_THREADS) {
-        bool tri;
+        const bool tri = it >= nA + nB;
+        const long nc = tri ? A.nt : A.nd;
         long c;
-        int slot;
+        int slot = 0;
         if (it < nA) {
-            tri = false;
             c = (long)A.off2[w] + it;
-            slot = 0;
-        } else if (it < nA + nB) {
+        } else if (!tri) {
             const int j = A.nbr2l[(long)w * A.cap2 + (it - nA)];
-            tri = false;
             c = (long)A.off2[j] + find_rank(A.nbr2 + (long)j * A.cap2, A.cnt2[j], w);
             slot = 1;
         } else {
-            tri = true;
             c = it < nA + nB + nC ? (long)A.toff[w] + (it - nA - nB) : (long)leaf[it - nA - nB - nC];
+        }
+        // a configuration with more clusters than the records hold (the one-call evaluation sees the
+        // counts afterwards, and starts again with larger ones): nothing past the end is read
+        if (c >= nc) continue;
+        if (tri) {
             const int* tr = A.trimers + 3 * c;
             slot = tr[0] == w ? 0 : (tr[1] == w ? 1 : 2);
         }
         const double frac = tri ? 1.0 / 9.0 : 1.0 / 6.0;
         const double kk = tri ? 9.0 : 6.0;
-        const long nc = tri ? A.nt : A.nd;
         const double E = tri ? A.e3[c] : A.e2[c];
         const double* G = tri ? A.g3 : A.g2;
         const double* Sp = tri ? A.s3 : A.s2;
